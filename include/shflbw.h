@@ -203,7 +203,8 @@ const char* shflbw_spmm_variant_name(int brow, int variant);
  * the buffers of the least recently initialised one (no allocation, no copy when the geometry is the same), whose
  * state must not be executed afterwards.  exec only launches, in order on `stream`.
  * shflbw_spconv_init_variant (variant < 0, and shflbw_spconv_init: the library's choice - variant 2 when B % 8 == 0,
- * else variant 0):
+ * else variant 0, whose three launches are replaced by the one launch of variant 5 - `patch` in the state is then set -
+ * where that is estimated faster; it needs no scratch but its tables):
  *   variant 0 = plane form, three launches: the input is rewritten once per call as channel-major padded
  *     planes (one per stride phase); the SpMM kernel then gathers, for a kept k = (r, s, c), the
  *     plane of channel c at the constant offset of tap (r, s) - the im2col matrix is never built,
@@ -216,7 +217,10 @@ const char* shflbw_spmm_variant_name(int brow, int variant);
  *     input, runs the SpMM and writes NHWC for its own range of output columns, in its own L2; the phases are
  *     counted between the workgroups of an XCD.  Needs a device that deals consecutive workgroups to consecutive
  *     XCDs (checked at init; SHFLBW_ERR_UNSUPPORTED otherwise).  Its waits are bounded: should one run out the launch still ends,
- *     and shflbw_spconv_check reports it.
+ *     and shflbw_spconv_check reports it;
+ *   variant 5 = patch form, one launch (any batch): a workgroup transposes the input patch under its output pixels
+ *     into LDS, runs the products on it and writes NHWC itself.  SHFLBW_ERR_UNSUPPORTED where no patch fits the LDS or
+ *     the plane forms are estimated faster.
  * ------------------------------------------------------------------------- */
 #define SHFLBW_CONV_SCRATCH_DEPTH 4
 typedef struct shflbw_spconv_state {
@@ -263,6 +267,7 @@ typedef struct shflbw_spconv_state {
                          * workgroup joins min(t, 10000) ticks late.  The int at byte 60 of `sync` counts the take-overs. */
     void* sync;
     shflbw_spmm_state spmm;
+    const void* patch; /* patch form: its cut and tables for this geometry, owned by the filter; NULL for the other forms */
 } shflbw_spconv_state;
 
 int shflbw_spconv_init(shflbw_spconv_state* state, const shflbw_weight* filter,

@@ -48,8 +48,11 @@ void release_conv_scratch(shflbw_weight* w)
         if (e.ptr) (void)hipFree(e.ptr);
     for (auto& e : w->conv_bulk)
         if (e.ptr) (void)hipFree(e.ptr);
+    for (auto& e : w->conv_patch)
+        if (e.ptr) (void)hipFree(e.ptr);
     w->conv_ids.clear();
     w->conv_bulk.clear();
+    w->conv_patch.clear();
 }
 
 static int upload_one(void** dst, const void* src, size_t bytes)
@@ -423,7 +426,7 @@ int shflbw_spconv_init(shflbw_spconv_state* state, const shflbw_weight* f, int B
 namespace {
 
 // forms of the convolution (shflbw_spconv_variant_name)
-enum ConvForm { FORM_PLANES = 0, FORM_DIRECT = 1, FORM_BPLANES = 2, FORM_FUSED = 3, FORM_CHWB = 4, FORM_COUNT = 5 };
+enum ConvForm { FORM_PLANES = 0, FORM_DIRECT = 1, FORM_BPLANES = 2, FORM_FUSED = 3, FORM_CHWB = 4, FORM_PATCH = 5, FORM_COUNT = 6 };
 
 // Argument checks of a convolution and every field of the state that does not depend on device scratch.
 int spconv_fill_state(shflbw_spconv_state* state, const shflbw_weight* f, int B, int H, int W, int stride,
@@ -467,7 +470,7 @@ int spconv_fill_state(shflbw_spconv_state* state, const shflbw_weight* f, int B,
     }
     if (variant < 0 || variant >= FORM_COUNT) {
         set_error("spconv_init: variant %d does not exist (0 = plane form, 1 = direct kernel, 2 = batch-innermost plane "
-                  "form, 3 = batch-innermost plane form fused into one launch)", variant);
+                  "form, 3 = batch-innermost plane form fused into one launch, 5 = patch form)", variant);
         return SHFLBW_ERR_INVALID;
     }
     if (variant == FORM_DIRECT) {
@@ -902,6 +905,139 @@ int init_fused(shflbw_spconv_state* state, const shflbw_weight* f, int B, int H,
     return SHFLBW_OK;
 }
 
+// The patch form of one geometry of a filter: cut, LDS offsets of the kept columns and places of the rows in the output,
+// built and uploaded on the first call for a geometry, found afterwards.  *out is null when the form does not take
+// the geometry.
+int conv_patch_for(shflbw_weight* fw, int B, int H, int W, int stride, int Ho, int Wo, const shflbw_weight::ConvPatch** out)
+{
+    *out = nullptr;
+    std::lock_guard<std::mutex> scratch_guard(fw->scratch_lock);
+    for (auto& e : fw->conv_patch)
+        if (e.key[0] == B && e.key[1] == H && e.key[2] == W && e.key[3] == stride) {
+            if (e.plan.valid) *out = &e;
+            return SHFLBW_OK;
+        }
+    shflbw_weight::ConvPatch e{};
+    e.key[0] = B, e.key[1] = H, e.key[2] = W, e.key[3] = stride;
+    const int V = fw->brow, X = fw->nrow / V, F = fw->F, C = fw->C, S = fw->S;
+    const ConvPatchProblem q{V, F, C, fw->R, S, (double)fw->nnzb / X, fw->row_permute ? 1 : 0, B, H, W, Ho, Wo, stride, device_compute_units()};
+    if (conv_patch_plan(q, &e.plan)) {
+        const ConvPatchPlan& p = e.plan;
+        const int RW = conv_patch_unit_rows(V), per_panel = V / RW, nunits = F / RW;
+        SHFLBW_HIP_TRY(conv_patch_kernel(RW, p.col_blocks, p.waves)->prepare());
+        e.dense = !fw->row_permute || p.chunks == 1;
+        size_t batches = 0;
+        for (int i = 0; i < X; i++) batches += (size_t)((fw->indptr[i + 1] - fw->indptr[i] + 31) / 32) * per_panel;
+        const size_t held = batches + CONV_PATCH_TAIL_BATCHES;
+        const size_t o_offs = up256(held * 32 * RW * sizeof(uint16_t)), o_first = o_offs + up256(held * 32 * sizeof(uint16_t));
+        const size_t o_filt = o_first + up256((size_t)(nunits + 1) * sizeof(int)), o_dst = o_filt + up256((size_t)F * sizeof(int));
+        e.bytes = o_dst + up256((size_t)F * sizeof(unsigned short));
+        // (an image beyond three quarters of an XCD's L2 is left to the ring past that)
+        e.plan.touch_bytes = (unsigned)std::min<size_t>(o_filt, 3u << 20) - 4;
+        e.plan.touch_step = (unsigned)(p.jobs_per_xcd * p.waves * 64) * 128u;
+        std::vector<unsigned char> h(e.bytes, 0);
+        uint16_t* A = (uint16_t*)h.data();
+        uint16_t* offs = (uint16_t*)(h.data() + o_offs);
+        int* first = (int*)(h.data() + o_first);
+        int* filt = (int*)(h.data() + o_filt);
+        unsigned short* dst = (unsigned short*)(h.data() + o_dst);
+        // bank pairs the positions one pass of a transposing read touches lie in, for a row that starts in pair 0
+        const int group = RW == 16 ? 8 : 4, quads = 32 / group;
+        uint32_t foot = 0;
+        for (int t = 0; t < quads; t++) {
+            const int i = t / p.row_len, j = t % p.row_len;
+            if (i < p.tile_h) foot |= 1u << ((i * p.step_h * p.patch_w + j * p.step_w) & 31);
+        }
+        // slots of the groups a batch's reads are made of, group after group: a pass reads slots 8 (lane / 16 or
+        // lane / 32) + 0..3 of a step, the second read of a fragment the four behind them
+        int slot_of[32];
+        for (int t = 0; t < 32; t++)
+            slot_of[t] = RW == 16 ? (t / 16) * 16 + ((t / 8) & 1) * 4 + ((t / 4) & 1) * 8 + t % 4 : t;
+        std::vector<int> pair_of, order;
+        size_t b = 0;
+        for (int panel = 0; panel < X; panel++) {
+            const int begin = fw->indptr[panel], nnz = fw->indptr[panel + 1] - begin;
+            auto offset_of = [&](int k) {
+                const int c = k % C, tap = k / C;
+                return c * p.pitch + ((tap / S) * p.patch_w + tap % S) * 8;
+            };
+            pair_of.resize(nnz);
+            for (int i = 0; i < nnz; i++) pair_of[i] = (offset_of(fw->indices[begin + i]) >> 3) & 31;
+            conv_patch_order(pair_of, foot, group, order);
+            for (int part = 0; part < per_panel; part++) {
+                first[panel * per_panel + part] = (int)b;
+                for (int t = 0; t < (nnz + 31) / 32 * 32; t++) {
+                    const int s = slot_of[t % 32];
+                    uint16_t* o = offs + (b + t / 32) * 32;
+                    uint16_t* a = A + (b + t / 32) * 32 * RW;
+                    const int in_step = RW == 16 ? s : s % 16, step = RW == 16 ? 0 : s / 16;
+                    const int pair = (in_step / 8) * 4 + in_step % 4, hi = (in_step % 8) / 4;
+                    // a lane addresses slots s and s + 4 of a step and loads the offsets of all steps of a batch at once
+                    o[RW == 16 ? pair * 2 + hi : pair * 4 + step * 2 + hi] = (uint16_t)((t < nnz ? offset_of(fw->indices[begin + order[t]]) : C * p.pitch) >> 3);
+                    if (t >= nnz) continue;
+                    const uint16_t* v = fw->values.data() + (size_t)(begin + order[t]) * V + part * RW;
+                    if (RW == 16)
+                        for (int r = 0; r < 16; r++) a[((s / 8) * 16 + r) * 8 + s % 8] = v[r];
+                    else
+                        for (int r = 0; r < RW; r++) a[(((size_t)step * (RW / 32) + r / 32) * 64 + (in_step / 8) * 32 + r % 32) * 8 + s % 8] = v[r];
+                }
+                b += (nnz + 31) / 32;
+            }
+        }
+        first[nunits] = (int)b;
+        for (int row0 = 0; row0 < F; row0 += p.rows_wg) {
+            const int rows = std::min(p.rows_wg, F - row0);
+            order.resize(rows);
+            for (int i = 0; i < rows; i++) order[i] = i;
+            auto filter_of = [&](int i) { return fw->row_permute ? fw->row_permute_ids[row0 + i] : row0 + i; };
+            std::sort(order.begin(), order.end(), [&](int x, int y) { return filter_of(x) < filter_of(y); });
+            for (int place = 0; place < rows; place++) {
+                filt[row0 + place] = filter_of(order[place]);
+                dst[row0 + order[place]] = (unsigned short)place;
+            }
+        }
+        SHFLBW_HIP_TRY(hipMalloc(&e.ptr, e.bytes));
+        if (hipMemcpy(e.ptr, h.data(), e.bytes, hipMemcpyHostToDevice) != hipSuccess) {
+            (void)hipFree(e.ptr);
+            set_error("spconv_init: cannot upload the offsets of the patch form");
+            return SHFLBW_ERR_HIP;
+        }
+        e.packedA = e.ptr;
+        e.offs = (const unsigned short*)((const char*)e.ptr + o_offs);
+        e.first_batch = (const int*)((const char*)e.ptr + o_first);
+        e.filt = (const int*)((const char*)e.ptr + o_filt);
+        e.dst = (const unsigned short*)((const char*)e.ptr + o_dst);
+    }
+    fw->conv_patch.push_back(e);
+    if (e.plan.valid) *out = &fw->conv_patch.back();
+    return SHFLBW_OK;
+}
+
+// Form 5.  `reported`: what the state's variant says (the library's own choice keeps naming the plane form whose
+// place the patch form takes).  SHFLBW_ERR_UNSUPPORTED when the form does not take the geometry.
+int init_patch(shflbw_spconv_state* state, const shflbw_weight* f, int B, int H, int W, int stride, const void* IFMap,
+               void* OFMap, int reported)
+{
+    int rc = spconv_fill_state(state, f, B, H, W, stride, IFMap, OFMap, FORM_PATCH);
+    if (rc != SHFLBW_OK) return rc;
+    const shflbw_weight::ConvPatch* e = nullptr;
+    if ((rc = conv_patch_for(const_cast<shflbw_weight*>(f), B, H, W, stride, state->Ho, state->Wo, &e)) != SHFLBW_OK) return rc;
+    if (!e) {
+        set_error("spconv_init: the input patch of a workgroup does not fit the LDS (%d channels, %d x %d filter)", f->C, f->R, f->S);
+        return SHFLBW_ERR_UNSUPPORTED;
+    }
+    state->patch = e;
+    state->variant = reported;
+    state->ncols = B * state->Ho * state->Wo;
+    state->shared_mem_size = (size_t)e->plan.lds_bytes;
+    state->grid_dim[0] = (unsigned)e->plan.jobs;
+    state->block_dim[0] = (unsigned)(e->plan.waves * 64);
+    state->grid_dim[1] = state->grid_dim[2] = 1;
+    state->block_dim[1] = state->block_dim[2] = 1;
+    state->init_success = 1;
+    return SHFLBW_OK;
+}
+
 // launch arguments every form shares
 void fill_conv_launch_args(const shflbw_spconv_state* state, SpconvLaunchArgs* out)
 {
@@ -969,7 +1105,10 @@ int shflbw_spconv_init_variant(shflbw_spconv_state* state, const shflbw_weight* 
             const long Ho = (H + 2 * (f->R / 2) - f->R) / stride + 1, Wo = (W + 2 * (f->S / 2) - f->S) / stride + 1;
             if (Ho > 0 && Wo > 0) variant = FORM_BPLANES;
         }
+        const int rc = init_patch(state, f, B, H, W, stride, IFMap, OFMap, variant);
+        if (rc != SHFLBW_ERR_UNSUPPORTED) return rc;
     }
+    if (variant == FORM_PATCH) return init_patch(state, f, B, H, W, stride, IFMap, OFMap, FORM_PATCH);
     if (variant == FORM_BPLANES) return init_batch_planes(state, f, B, H, W, stride, IFMap, OFMap, FORM_BPLANES);
     if (variant == FORM_FUSED) return init_fused(state, f, B, H, W, stride, IFMap, OFMap);
     if (variant == FORM_PLANES) return init_planes(state, f, B, H, W, stride, IFMap, OFMap);
@@ -999,9 +1138,26 @@ int shflbw_spconv_exec(const shflbw_spconv_state* state, void* stream)
         set_error("spconv_exec: state was not initialised successfully");
         return SHFLBW_ERR_STATE;
     }
+    hipError_t e = hipSuccess;
+    if (state->patch) {
+        const auto& pe = *(const shflbw_weight::ConvPatch*)state->patch;
+        const ConvPatchKernel* k = conv_patch_kernel(conv_patch_unit_rows(state->brow), pe.plan.col_blocks, pe.plan.waves);
+        if (!k) return SHFLBW_ERR_UNSUPPORTED;
+        ConvPatchArgs p;
+        p.p = pe.plan;
+        p.C = state->args.C, p.F = state->args.F, p.R = state->args.R, p.S = state->args.S;
+        p.in = (const half_t*)state->args.IFMap;
+        p.out = (half_t*)state->args.OFMap;
+        p.packedA = (const half8_t*)pe.packedA;
+        p.first_batch = pe.first_batch;
+        p.offs = pe.offs, p.dst = pe.dst, p.filt = pe.filt, p.dense = pe.dense;
+        e = k->launch(p, (hipStream_t)stream);
+        if (e == hipSuccess) return SHFLBW_OK;
+        set_error("spconv_exec: launch failed: %s", hipGetErrorString(e));
+        return SHFLBW_ERR_HIP;
+    }
     SpconvLaunchArgs a;
     fill_conv_launch_args(state, &a);
-    hipError_t e = hipSuccess;
     if (state->variant == FORM_CHWB || state->variant == FORM_BPLANES) {
         const ConvChwbKernel* k = conv_chwb_kernel(state->brow, state->middle_tile_cols, 0, 0, 0);
         if (!k) return SHFLBW_ERR_UNSUPPORTED;
@@ -1171,6 +1327,7 @@ static const char* const g_spconv_forms[FORM_COUNT] = {
     "bplanes+spmm+transpose", // 2: NHWC tensors, planes and result with the batch innermost (batch a multiple of 8): three launches
     "bplanes-fused",          // 3: the steps of form 2 in one persistent launch, every XCD on its own columns
     "chwb-planes+spmm",       // 4: the reference's batch-innermost tensors (shflbw_spconv_init_chwb only): padded copy, SpMM
+    "patch",                  // 5: one launch, the input patch of a workgroup's pixels in LDS, channel-major
 };
 
 int shflbw_spconv_variant_count(void) { return FORM_COUNT; }
@@ -1196,8 +1353,9 @@ int shflbw_weight_scratch_bytes(const shflbw_weight* w, size_t* bytes, int* buff
     size_t total = 0;
     for (auto& e : w->conv_ids) total += e.bytes;
     for (auto& e : w->conv_bulk) total += e.bytes;
+    for (auto& e : w->conv_patch) total += e.bytes;
     if (bytes) *bytes = total;
-    if (buffers) *buffers = (int)(w->conv_ids.size() + w->conv_bulk.size());
+    if (buffers) *buffers = (int)(w->conv_ids.size() + w->conv_bulk.size() + w->conv_patch.size());
     return SHFLBW_OK;
 }
 

@@ -1,0 +1,80 @@
+// Launch-side description of the patch form of the convolution (host + device shared): one launch over NHWC tensors, a
+// workgroup keeps the input patch its output pixels read in LDS, channel-major.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include <vector>
+
+#include "kernel_common.h"
+
+namespace shflbw {
+
+// How a convolution is cut into workgroups.  Output positions are taken in blocks of tile_h x tile_w (at most
+// 16 or 8) per image; four blocks ("units", any image, any place) make a column tile: column 4 p + u of the GEMM tile is
+// position p of unit u.  The four units of a position lie side by side in LDS (8 bytes), which is what one lane of
+// the transposing LDS read supplies, so a tap is a plain offset whatever the stride, the batch and the alignment.
+struct ConvPatchPlan {
+    int valid;
+    int col_blocks;       // 32-column blocks of a tile: 2 (16 positions x 4 units) or 1 (8 positions)
+    int waves;            // waves of a workgroup
+    int tile_h, tile_w;   // output positions of a unit
+    int row_len;          // GEMM positions per tile row (>= tile_w; the surplus positions are no pixels)
+    int blocks_w, blocks_hw, units;
+    int step_h, step_w;   // patch positions between neighbouring output positions
+    int patch_w, npos;    // columns and positions of the input patch of a unit
+    int pitch;            // LDS bytes of one channel: 8 per position, an odd multiple of 8
+    int groups, ksplit;   // waves = groups (rows) x ksplit (parts of the kept columns, a power of two: 1 << kshift)
+    int kshift;
+    int panels_per_wave;  // row units one wave computes one after the other
+    int rows_wg, chunks;  // filters of a workgroup, workgroups per column tile
+    int jobs, jobs_per_xcd;
+    int H, W, Ho, Wo, stride, pad_h, pad_w; // extents as the kernel walks them (a 1 x 1 filter at stride 1: one row)
+    int skip;             // stride wider than the filter in some direction
+    unsigned in_bytes;
+    unsigned touch_bytes, touch_step; // last byte of the filter image a workgroup brings into the L2; bytes one round of an XCD's threads covers
+    int lds_bytes;
+    unsigned magic_bhw, magic_bw, magic_pw, magic_row, magic_chunks, magic_pg;
+};
+
+// What the plan depends on.
+struct ConvPatchProblem {
+    int V, F, C, R, S;
+    double kept_per_panel; // kept columns of a row panel on average
+    int permuted;          // rows of the filter are permuted
+    int B, H, W, Ho, Wo, stride, cus;
+};
+// Fills `plan`; false when no patch fits the LDS or the sizes leave 32-bit indexes (the plane forms take over).
+bool conv_patch_plan(const ConvPatchProblem& q, ConvPatchPlan* plan);
+
+// Order of the kept columns of a row panel that keeps the LDS reads of a group of rows apart (see the definition).
+void conv_patch_order(const std::vector<int>& pair_of, uint32_t foot, int group, std::vector<int>& order);
+
+struct ConvPatchArgs {
+    ConvPatchPlan p;
+    int C, F, R, S;
+    const half_t* in;
+    half_t* out;
+    // the filter as this form reads it: row units (a row panel; two for block height 128) of batches of 32 slots
+    const half8_t* packedA;        // per batch the A fragments in register order
+    const int* first_batch;        // per row unit its first batch, and the number of batches behind the last unit
+    const unsigned short* offs;    // per batch the LDS offsets (in 8 bytes) of channel row and tap, in the order the lanes load them
+    const unsigned short* dst;     // per stored row: its place among the staged rows of its workgroup
+    const int* filt;               // per chunk and place: the filter (used when not dense)
+    int dense;                     // the filters of a chunk are consecutive in the output
+};
+
+struct ConvPatchKernel {
+    int RW, col_blocks, waves;
+    int per_cu; // workgroups of it the registers of a compute unit hold
+    int ring, items; // batches a wave keeps in flight, patch items a thread keeps in flight
+    hipError_t (*launch)(const ConvPatchArgs&, hipStream_t);
+    hipError_t (*prepare)();
+};
+const ConvPatchKernel* conv_patch_kernel(int rows, int col_blocks, int waves);
+
+constexpr int CONV_PATCH_LDS_MAX = 160 * 1024;
+constexpr int CONV_PATCH_SLACK = 256;       // LDS bytes behind the row of zeros
+constexpr int CONV_PATCH_TAIL_BATCHES = 8;  // batches of padding behind the last one: waves fetch ahead of their end
+inline int conv_patch_unit_rows(int V) { return V == 128 ? 64 : V; }
+
+} // namespace shflbw

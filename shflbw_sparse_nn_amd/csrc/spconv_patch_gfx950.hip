@@ -1,0 +1,696 @@
+// Patch form of the Shfl-BW convolution: NHWC in, NHWC out, one launch.
+//
+// The plane forms rewrite the input channel-major in memory and the result pixel-major: two passes over memory and
+// two more launches around an SpMM that itself takes half of the time.  Here a workgroup owns 64 (or 32) output
+// pixels and a set of filters:
+//   1. it copies the input patch under its pixels (halo included) into LDS and transposes it on the way: one row
+//      per channel, the four units of a position side by side in 8 bytes;
+//   2. every wave streams the A fragments of its own row panels and the LDS offsets of their kept columns straight
+//      into registers (several batches in flight) and reads its B fragments from the rows the offsets name
+//      (transposing LDS reads; tap, stride and position are one added offset), MFMA, fp32 accumulators;
+//   3. the fp16 results go through LDS (pixel rows, filters in output order) to whole runs of the NHWC output.
+// What bounds it: the A stream (64 bytes per clock and compute unit from the L2) and the MFMAs are level for block
+// height 64, the LDS reads for 32 and 16; on small layers the chain of launch, patch, first fragments and stores.
+#include "spconv_patch.h"
+
+#include <algorithm>
+#include <type_traits>
+#include <cmath>
+
+namespace shflbw {
+
+// RW: rows of a row unit - one row panel, half of one for block height 128
+template <int RW>
+struct ConvPatchCfg {
+    static constexpr bool R16 = RW == 16;
+    static constexpr int MBW = RW == 64 ? 2 : 1;     // A fragments per MFMA step
+    static constexpr int STEPS = R16 ? 1 : 2;        // MFMA steps per batch of 32 slots
+    static constexpr int NA = STEPS * MBW;           // A fragments per batch
+    static constexpr int OPS = NA + 1;               // loads per batch
+    static constexpr int NPMAX = 64 / RW;            // row units a wave may compute one after the other
+};
+
+template <int RW, int NB, int NW, int NBUF, int U, int WPE>
+__global__ void __launch_bounds__(NW * 64, WPE) spconv_patch_kernel(ConvPatchArgs a)
+{
+    using Cfg = ConvPatchCfg<RW>;
+    constexpr bool R16 = Cfg::R16;
+    constexpr int NA = Cfg::NA, NPMAX = Cfg::NPMAX, MBW = Cfg::MBW, STEPS = Cfg::STEPS;
+    constexpr int NCB = R16 ? NB * 2 : NB;           // column blocks of a wave: 16 or 32 columns
+    constexpr int AV = R16 ? 4 : 16;                 // accumulator values per lane and block
+    constexpr int NQ = MBW * NCB * AV / 4;           // quads of accumulator values per lane
+    // U: items of the patch a thread keeps in flight; WPE: waves per SIMD the registers are kept to
+    constexpr int RING_OPS = NBUF * Cfg::OPS;
+    static_assert(NBUF % 2 == 0 && NBUF <= CONV_PATCH_TAIL_BATCHES && RING_OPS + 2 < 64, "fragment sets alternate; vmcnt is a 6-bit counter");
+
+    extern __shared__ __attribute__((aligned(1024))) char lds_raw[];
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(SHFLBW_LDS char*)lds_raw;
+    const ConvPatchPlan& P = a.p;
+    const int tid = threadIdx.x, lane = tid & 63, li = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+
+    // XCD x owns a contiguous range of the jobs (column tile, chunk of filters), chunk-minor: the workgroups that write
+    // interleaved filters of the same pixels share an L2, where their partial lines meet
+    const int xcd = blockIdx.x & 7, job = xcd * P.jobs_per_xcd + (int)(blockIdx.x >> 3);
+    if (job >= min(P.jobs, (xcd + 1) * P.jobs_per_xcd)) return;
+    int tile, ch;
+    fast_divmod(job, P.chunks, P.magic_chunks, tile, ch);
+
+    // ---- this wave's row units and its share of their batches (32 slots each, one unit behind the other in memory)
+    const int grp = wave >> P.kshift, ks = wave & (P.ksplit - 1);
+    const int np = P.panels_per_wave, nunits = a.F / RW;
+    const int ufirst = (ch * P.groups + grp) * np;
+    const SHFLBW_CONST int* first_batch = (const SHFLBW_CONST int*)(uintptr_t)a.first_batch;
+    int bound[NPMAX + 1]; // batches of unit j: [bound[j], bound[j + 1])
+#pragma unroll
+    for (int j = 0; j <= NPMAX; j++) bound[j] = first_batch[min(ufirst + min(j, np), nunits)];
+    if (NPMAX == 1 || P.ksplit > 1) {
+        const int n = bound[1] - bound[0], b0 = bound[0];
+        bound[0] = b0 + ((n * ks) >> P.kshift);
+#pragma unroll
+        for (int j = 1; j <= NPMAX; j++) bound[j] = b0 + ((n * (ks + 1)) >> P.kshift);
+    }
+    int left = bound[NPMAX] - bound[0];
+    int fpos = bound[0];
+    const int fend = bound[NPMAX];
+
+    // ---- the unit of this lane's column (lane % 4): its first output and input pixel.  A unit past the end lies outside.
+    SHFLBW_LDS int* tout = (SHFLBW_LDS int*)(uintptr_t)lds0;
+    const uint32_t slab = lds0 + 32 * NB * 4;
+    int uh[4], uw[4], ub[4];
+    {
+        const int unit = tile * 4 + (lane & 3);
+        int img, rem, bi, bj;
+        fast_divmod(unit, P.blocks_hw, P.magic_bhw, img, rem);
+        fast_divmod(rem, P.blocks_w, P.magic_bw, bi, bj);
+        const bool ok = unit < P.units;
+        const int oh = ok ? bi * P.tile_h : P.Ho, ow = bj * P.tile_w;
+        const int h = ok ? oh * P.stride - P.pad_h : P.H, w = ow * P.stride - P.pad_w;
+        const int b = (int)((unsigned)((img * P.H + h) * P.W + w) * (unsigned)(a.C * 2));
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            uh[u] = __builtin_amdgcn_readlane(h, u);
+            uw[u] = __builtin_amdgcn_readlane(w, u);
+            ub[u] = __builtin_amdgcn_readlane(b, u);
+        }
+        if (tid < 32 * NB) { // output pixel of every column of the tile, -1: none
+            int i, j;
+            fast_divmod(tid >> 2, P.row_len, P.magic_row, i, j);
+            tout[tid] = i < P.tile_h && j < P.tile_w && oh + i < P.Ho && ow + j < P.Wo ? (img * P.Ho + oh + i) * P.Wo + ow + j : -1;
+        }
+    }
+
+    struct Batch {
+        half8_t a[NA];
+        typename std::conditional<R16, int, int2_t>::type i; // LDS offsets in units of 8 bytes, 16 bits each: slots s, s + 4 of every step
+    };
+    struct Frags {
+        half8_t b[STEPS][NCB];
+    };
+    // ---- every load up to the end of the products is inline assembly with hand-written waits: the patch, the places
+    // and the ring of batches share one counter, and the compiler would wait for all of them at the first use of one
+    const uint32_t lane16 = (uint32_t)lane * 16;
+    const uint32_t offl = R16 ? (uint32_t)((lane >> 4) * 4 + (li >> 2)) * 4 : (uint32_t)((lane >> 5) * 4 + (li >> 2)) * 8;
+    // Past the wave's last batch the loads are issued without a lane: no traffic, and the waits go on counting the same
+    // number of them.
+    auto fetch = [&](Batch& b) __attribute__((always_inline)) {
+        const char* A = (const char*)a.packedA + (size_t)fpos * (32 * RW * 2);
+        const char* I = (const char*)a.offs + (size_t)fpos * 64;
+        if constexpr (NA == 4)
+            asm volatile("s_cmp_lt_i32 %[p], %[e]\n\t"
+                         "s_cselect_b64 exec, -1, 0\n\t"
+                         "global_load_dwordx4 %[a0], %[l], %[A]\n\t"
+                         "global_load_dwordx4 %[a1], %[l], %[A] offset:1024\n\t"
+                         "global_load_dwordx4 %[a2], %[l], %[A] offset:2048\n\t"
+                         "global_load_dwordx4 %[a3], %[l], %[A] offset:3072\n\t"
+                         "global_load_dwordx2 %[i], %[o], %[I]\n\t"
+                         "s_mov_b64 exec, -1"
+                         : [a0] "=&v"(b.a[0]), [a1] "=&v"(b.a[1]), [a2] "=&v"(b.a[2]), [a3] "=&v"(b.a[3]), [i] "=&v"(b.i)
+                         : [p] "s"(fpos), [e] "s"(fend), [l] "v"(lane16), [A] "s"(A), [o] "v"(offl), [I] "s"(I)
+                         : "scc");
+        else if constexpr (NA == 2)
+            asm volatile("s_cmp_lt_i32 %[p], %[e]\n\t"
+                         "s_cselect_b64 exec, -1, 0\n\t"
+                         "global_load_dwordx4 %[a0], %[l], %[A]\n\t"
+                         "global_load_dwordx4 %[a1], %[l], %[A] offset:1024\n\t"
+                         "global_load_dwordx2 %[i], %[o], %[I]\n\t"
+                         "s_mov_b64 exec, -1"
+                         : [a0] "=&v"(b.a[0]), [a1] "=&v"(b.a[1]), [i] "=&v"(b.i)
+                         : [p] "s"(fpos), [e] "s"(fend), [l] "v"(lane16), [A] "s"(A), [o] "v"(offl), [I] "s"(I)
+                         : "scc");
+        else
+            asm volatile("s_cmp_lt_i32 %[p], %[e]\n\t"
+                         "s_cselect_b64 exec, -1, 0\n\t"
+                         "global_load_dwordx4 %[a0], %[l], %[A]\n\t"
+                         "global_load_dword %[i], %[o], %[I]\n\t"
+                         "s_mov_b64 exec, -1"
+                         : [a0] "=&v"(b.a[0]), [i] "=&v"(b.i)
+                         : [p] "s"(fpos), [e] "s"(fend), [l] "v"(lane16), [A] "s"(A), [o] "v"(offl), [I] "s"(I)
+                         : "scc");
+        fpos++;
+    };
+    auto pass_through = [](Batch& b) __attribute__((always_inline)) {
+        asm volatile("" : "+v"(b.i));
+#pragma unroll
+        for (int q = 0; q < NA; q++) asm volatile("" : "+v"(b.a[q]));
+    };
+    // waits until at most `younger` batches fetched behind this one are outstanding
+    auto arrived = [&](Batch& b, auto younger) __attribute__((always_inline)) {
+        asm volatile("s_waitcnt vmcnt(%0)" : : "n"(decltype(younger)::value * Cfg::OPS));
+        pass_through(b);
+    };
+    Batch buf[NBUF];
+    int touched0, touched1;
+
+    // places of this wave's rows in the staged output
+    int dst[NPMAX][MBW];
+#pragma unroll
+    for (int j = 0; j < NPMAX; j++)
+#pragma unroll
+        for (int mb = 0; mb < MBW; mb++) {
+            const uint32_t at = (uint32_t)min((ufirst + j) * RW + mb * 32 + (lane & (R16 ? 15 : 31)), a.F - 1) * 2;
+            asm volatile("global_load_ushort %0, %1, %2" : "=v"(dst[j][mb]) : "v"(at), "s"(a.dst));
+        }
+
+    // ---- the patch: a lane takes 8 channels of one position in all four units (four 16-byte loads; bytes outside the
+    // image come back as zeros from the bounds check of the buffer) and writes them as eight 8-byte pieces, one per
+    // channel row.  The pitch is an odd multiple of 8 bytes: the 4 channel groups x 8 positions of half a wave fall into
+    // different banks.
+    {
+        const int C8 = a.C >> 3, npos = P.npos, pitch = P.pitch, PG = (npos + 7) >> 3;
+        const int combos = PG * ((C8 + 7) >> 3);
+        const int ol = (lane & 3) | ((lane >> 5) << 2), pl = (lane >> 2) & 7;
+        const int4_t rsrc = {(int)(uint32_t)(uintptr_t)a.in, (int)(uint32_t)((uintptr_t)a.in >> 32), (int)P.in_bytes, 0x00027000};
+        half8_t v[U][4];
+        uint32_t to[U];
+        auto load_round = [&](int q0) __attribute__((always_inline)) {
+#pragma unroll
+            for (int k = 0; k < U; k++) {
+                const int q = q0 + k * NW;
+                int og, pg, pi, pj;
+                fast_divmod(q, PG, P.magic_pg, og, pg);
+                const int oct = og * 8 + ol, pos = pg * 8 + pl;
+                fast_divmod(pos, P.patch_w, P.magic_pw, pi, pj);
+                if (P.skip) { // a stride wider than the filter: input rows and columns no tap reads are left out
+                    if (P.stride > a.R) pi = (pi / a.R) * P.stride + pi % a.R;
+                    if (P.stride > a.S) pj = (pj / a.S) * P.stride + pj % a.S;
+                }
+                const bool in_patch = oct < C8 && pos < npos; // false for every q past the last
+                to[k] = in_patch ? (uint32_t)(oct * 8) * pitch + pos * 8 : 0xffffffffu;
+                const uint32_t rel = (uint32_t)((pi * P.W + pj) * a.C + oct * 8) * 2;
+                if (k > 0 && q >= combos) continue;
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const bool ok = in_patch && (unsigned)(uh[u] + pi) < (unsigned)P.H && (unsigned)(uw[u] + pj) < (unsigned)P.W;
+                    const uint32_t at = ok ? rel + (uint32_t)ub[u] : 0xffffffffu;
+                    asm volatile("buffer_load_dwordx4 %0, %1, %2, 0 offen" : "=v"(v[k][u]) : "v"(at), "s"(rsrc));
+                }
+            }
+        };
+        auto write_round = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int k = 0; k < U; k++) {
+#pragma unroll
+                for (int u = 0; u < 4; u++) asm volatile("" : "+v"(v[k][u]));
+                if (to[k] != 0xffffffffu) {
+                    uint32_t at = slab + to[k];
+                    const int4_t d0 = __builtin_bit_cast(int4_t, v[k][0]), d1 = __builtin_bit_cast(int4_t, v[k][1]),
+                                 d2 = __builtin_bit_cast(int4_t, v[k][2]), d3 = __builtin_bit_cast(int4_t, v[k][3]);
+#pragma unroll
+                    for (int e = 0; e < 8; e++) {
+                        const unsigned sel = (e & 1) ? 0x07060302u : 0x05040100u;
+                        int2_t w;
+                        w.x = (int)__builtin_amdgcn_perm((unsigned)d1[e >> 1], (unsigned)d0[e >> 1], sel);
+                        w.y = (int)__builtin_amdgcn_perm((unsigned)d3[e >> 1], (unsigned)d2[e >> 1], sel);
+                        *(SHFLBW_LDS int2_t*)(uintptr_t)at = w;
+                        at += pitch;
+                    }
+                }
+            }
+        };
+        int q0 = wave;
+        for (; q0 + NW * U < combos; q0 += NW * U) {
+            load_round(q0);
+            asm volatile("s_waitcnt vmcnt(0)");
+            write_round();
+        }
+        load_round(q0); // the last round, maybe empty for this wave
+#pragma unroll
+        for (int j = 0; j < NBUF; j++) fetch(buf[j]);
+        // The filter is not in the L2 when a launch starts, and the workgroups of an XCD walk it in step: left to the ring,
+        // every batch would cost all of them a trip to memory.  Each thread touches a line of its own once, which brings
+        // the whole image into the XCD's L2 while the patch is on its way.
+        const uint32_t line = ((blockIdx.x >> 3) * (NW * 64) + tid) * 128;
+        asm volatile("global_load_dword %0, %1, %2" : "=v"(touched0) : "v"(min(line, P.touch_bytes)), "s"(a.packedA));
+        asm volatile("global_load_dword %0, %1, %2" : "=v"(touched1) : "v"(min(line + P.touch_step, P.touch_bytes)), "s"(a.packedA));
+        asm volatile("s_waitcnt vmcnt(%0)" : : "n"(RING_OPS + 2));
+        write_round();
+#pragma unroll
+        for (int j = 0; j < NPMAX; j++)
+#pragma unroll
+            for (int mb = 0; mb < MBW; mb++) asm volatile("" : "+v"(dst[j][mb])); // older than the ring: arrived
+        // the row of zeros the padding slots read, and behind it what columns without a pixel may touch
+        for (int i = tid; i < (pitch >> 3) + CONV_PATCH_SLACK / 8; i += NW * 64)
+            *(SHFLBW_LDS int2_t*)(uintptr_t)(slab + (uint32_t)a.C * pitch + i * 8) = int2_t{0, 0};
+    }
+    __syncthreads(); // the patch
+
+    // ---- products
+    uint32_t colc[NCB]; // LDS offset of the lane's four columns
+#pragma unroll
+    for (int nb = 0; nb < NCB; nb++) {
+        const int pos = R16 ? nb * 4 + (li & 3) : nb * 8 + ((lane >> 4) & 1) * 4 + (li & 3);
+        int i, j;
+        fast_divmod(pos, P.row_len, P.magic_row, i, j);
+        colc[nb] = slab + (i < P.tile_h ? (uint32_t)(i * P.step_h * P.patch_w + j * P.step_w) * 8 : 0u);
+    }
+    typedef float accv_t __attribute__((ext_vector_type(AV)));
+    accv_t acc[MBW][NCB];
+    half4_t kept[NPMAX][NQ]; // finished panels, rounded to fp16
+    auto clear = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int mb = 0; mb < MBW; mb++)
+#pragma unroll
+            for (int nb = 0; nb < NCB; nb++)
+#pragma unroll
+                for (int i = 0; i < AV; i++) acc[mb][nb][i] = 0.f;
+    };
+    clear();
+#pragma unroll
+    for (int j = 0; j < NPMAX; j++)
+#pragma unroll
+        for (int q = 0; q < NQ; q++) kept[j][q] = half4_t{0, 0, 0, 0};
+    {
+        auto read_frags = [&](const Batch& b, Frags& f) __attribute__((always_inline)) {
+#pragma unroll
+            for (int h = 0; h < STEPS; h++)
+#pragma unroll
+                for (int nb = 0; nb < NCB; nb++) {
+                    uint32_t both;
+                    if constexpr (R16) both = (uint32_t)b.i;
+                    else both = (uint32_t)b.i[h];
+                    const half4_t l = lds_read_tr16(((both & 0xffff) << 3) + colc[nb]);
+                    const half4_t u = lds_read_tr16(((both >> 16) << 3) + colc[nb]);
+                    f.b[h][nb] = __builtin_shufflevector(l, u, 0, 1, 2, 3, 4, 5, 6, 7);
+                }
+        };
+        auto mma = [&](const Frags& f, const Batch& b) __attribute__((always_inline)) {
+#pragma unroll
+            for (int h = 0; h < STEPS; h++)
+#pragma unroll
+                for (int mb = 0; mb < MBW; mb++)
+#pragma unroll
+                    for (int nb = 0; nb < NCB; nb++) {
+                        if constexpr (R16)
+                            acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.b[h][nb], b.a[0], acc[mb][nb], 0, 0, 0);
+                        else
+                            acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.b[h][nb], b.a[h * MBW + mb], acc[mb][nb], 0, 0, 0);
+                    }
+        };
+        // end of a unit: its sums to fp16 (with a split over the kept columns a wave has one unit, whose fp32 sums stay
+        // in acc), then the next unit that has batches
+        int cur = 0, pos = bound[0], end = bound[1];
+        auto next_unit = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = 0; j < NPMAX; j++) // units without a batch in front are passed over
+                if (cur < NPMAX && pos == end) {
+                    if (P.ksplit > 1) { cur = NPMAX; break; }
+#pragma unroll
+                    for (int t = 0; t < NPMAX; t++)
+                        if (t == cur) {
+#pragma unroll
+                            for (int q = 0; q < NQ; q++)
+#pragma unroll
+                                for (int e = 0; e < 4; e++) {
+                                    const int i = q * 4 + e;
+                                    kept[t][q][e] = (half_t)acc[i / (NCB * AV)][(i / AV) % NCB][i % AV];
+                                }
+                        }
+                    clear();
+                    cur++;
+                    int e = bound[NPMAX];
+#pragma unroll
+                    for (int t = 0; t < NPMAX; t++) e = t == cur ? bound[t + 1] : e;
+                    end = e;
+                }
+        };
+        if constexpr (NPMAX > 1) next_unit();
+        Frags fr[2];
+        if (left > 0) {
+            arrived(buf[0], std::integral_constant<int, NBUF - 1>{});
+            read_frags(buf[0], fr[0]);
+        }
+        // MFMAs of a batch first, the LDS reads of the next one spread behind them
+        auto interleave = [&]() __attribute__((always_inline)) {
+            constexpr int NRD = STEPS * NCB * 2, NMM = STEPS * MBW * NCB, RPM = (NRD + NMM - 1) / NMM;
+#pragma unroll
+            for (int i = 0; i < NMM; i++) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // one MFMA
+                __builtin_amdgcn_sched_group_barrier(0x100, RPM, 0); // LDS reads
+            }
+        };
+        for (; left > NBUF; left -= NBUF) {
+#pragma unroll
+            for (int j = 0; j < NBUF; j++) {
+                arrived(buf[(j + 1) % NBUF], std::integral_constant<int, NBUF - 2>{});
+                read_frags(buf[(j + 1) % NBUF], fr[(j + 1) & 1]);
+                mma(fr[j & 1], buf[j]);
+                interleave();
+                fetch(buf[j]);
+                if constexpr (NPMAX > 1)
+                    if (++pos == end) next_unit();
+            }
+        }
+        // the rest: what it needs is in the ring
+        auto rest = [&](auto self, auto jj) __attribute__((always_inline)) {
+            constexpr int j = decltype(jj)::value;
+            if constexpr (j < NBUF) {
+                if (j < left) {
+                    if constexpr (j + 1 < NBUF)
+                        if (j + 1 < left) {
+                            arrived(buf[j + 1], std::integral_constant<int, NBUF - 2 - j>{});
+                            read_frags(buf[j + 1], fr[(j + 1) & 1]);
+                        }
+                    mma(fr[j & 1], buf[j]);
+                    if constexpr (NPMAX > 1)
+                        if (++pos == end) next_unit();
+                }
+                self(self, std::integral_constant<int, j + 1>{});
+            }
+        };
+        rest(rest, std::integral_constant<int, 0>{});
+        // no load may land in a register that has found another use
+        asm volatile("s_waitcnt vmcnt(0)" : "+v"(touched0), "+v"(touched1));
+#pragma unroll
+        for (int j = 0; j < NBUF; j++) pass_through(buf[j]);
+    }
+
+    // ---- results: one LDS row per filter, in output order (a lane holds four columns, the four units of a position, of
+    // one filter per 8-byte write); the patch is no longer needed
+    __syncthreads();
+    const uint32_t SP = a.dense ? NB * 64 + 16 : NB * 64 + 8;
+    uint32_t stage = slab;
+    if (P.ksplit > 1) { // sum the parts: every wave adds up its share of the quads of its group
+        stage = slab + NW * NQ * 1024;
+#pragma unroll
+        for (int q = 0; q < NQ; q++) {
+            float4_t v;
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] = acc[(q * 4 + e) / (NCB * AV)][((q * 4 + e) / AV) % NCB][(q * 4 + e) % AV];
+            *(SHFLBW_LDS float4_t*)(uintptr_t)(slab + (wave * NQ + q) * 1024 + lane * 16) = v;
+        }
+        __syncthreads();
+    }
+    auto put = [&](int j, int q, half4_t h) __attribute__((always_inline)) { // quad q of the lane's values of panel j
+        const int i = q * 4, mb = i / (NCB * AV), nb = (i / AV) % NCB, ig = (i % AV) / 4;
+        const uint32_t col = R16 ? nb * 16 + (lane >> 4) * 4 : nb * 32 + ig * 8 + (lane >> 5) * 4;
+        *(SHFLBW_LDS half4_t*)(uintptr_t)(stage + dst[j][mb] * SP + col * 2) = h;
+    };
+    if (P.ksplit > 1) {
+        if (ufirst < nunits)
+#pragma unroll
+            for (int q = 0; q < NQ; q++) {
+                if ((q & (P.ksplit - 1)) != ks) continue;
+                float4_t s = {0.f, 0.f, 0.f, 0.f};
+                for (int k = 0; k < P.ksplit; k++) {
+                    const float4_t v = *(SHFLBW_LDS float4_t*)(uintptr_t)(slab + ((grp * P.ksplit + k) * NQ + q) * 1024 + lane * 16);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) s[e] += v[e];
+                }
+                half4_t h;
+#pragma unroll
+                for (int e = 0; e < 4; e++) h[e] = (half_t)s[e];
+                put(0, q, h);
+            }
+    } else {
+#pragma unroll
+        for (int j = 0; j < NPMAX; j++)
+            if (j < np && ufirst + j < nunits) {
+#pragma unroll
+                for (int q = 0; q < NQ; q++) {
+                    half4_t h = kept[j][q];
+                    if constexpr (NPMAX == 1) {
+#pragma unroll
+                        for (int e = 0; e < 4; e++) h[e] = (half_t)acc[(q * 4 + e) / (NCB * AV)][((q * 4 + e) / AV) % NCB][(q * 4 + e) % AV];
+                    }
+                    put(j, q, h);
+                }
+            }
+    }
+    __syncthreads();
+    const int row0 = ch * P.rows_wg, rows = min(P.rows_wg, a.F - row0);
+    if (a.dense) { // transposing reads: a lane gets 8 consecutive filters of one of 16 pixels, twice, 32 filters apart; lanes
+                   // 8..15 of each 16 then trade places so that a store writes whole 128-byte lines of 8 pixels
+        const int nit = NB * 2 * ((rows + 63) >> 6);
+        for (int it = wave; it < nit; it += NW) {
+            const int cb = it & (NB * 2 - 1), r0 = (it / (NB * 2)) * 64, g8 = (lane >> 4) * 8;
+            int4_t v[2];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const uint32_t at = stage + (uint32_t)(min(r0 + h * 32 + g8, rows - 8) + (li >> 2)) * SP + cb * 32 + (li & 3) * 8;
+                const half4_t lo = lds_read_tr16(at), hi = lds_read_tr16(at + 4 * SP);
+                v[h] = __builtin_bit_cast(int4_t, (half8_t)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+            }
+            int4_t first, second;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                first[e] = __builtin_amdgcn_update_dpp(v[0][e], v[1][e], 0x128, 0xf, 0xc, false);  // row_ror:8 into lanes 8..15
+                second[e] = __builtin_amdgcn_update_dpp(v[1][e], v[0][e], 0x128, 0xf, 0x3, false); // ... into lanes 0..7
+            }
+            const int r = r0 + g8 + (li >> 3) * 32;
+            const int pix0 = tout[cb * 16 + (li & 7)], pix1 = tout[cb * 16 + 8 + (li & 7)];
+            if (pix0 >= 0 && r < rows) store_result_16B<true>(a.out + (size_t)pix0 * a.F + row0 + r, __builtin_bit_cast(half8_t, first));
+            if (pix1 >= 0 && r < rows) store_result_16B<true>(a.out + (size_t)pix1 * a.F + row0 + r, __builtin_bit_cast(half8_t, second));
+        }
+    } else { // a chunk's filters are scattered over the pixel: 2-byte pieces in ascending order, merged in the L2
+        constexpr int MAXQ = 8;
+        int f[MAXQ];
+#pragma unroll
+        for (int q = 0; q < MAXQ; q++) f[q] = q * 64 + lane < rows ? a.filt[row0 + q * 64 + lane] : -1;
+        for (int pos = wave; pos < 8 * NB; pos += NW) {
+            half_t* o[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int pix = __builtin_amdgcn_readfirstlane(tout[pos * 4 + u]);
+                o[u] = pix >= 0 ? a.out + (size_t)pix * a.F : nullptr;
+            }
+#pragma unroll
+            for (int q = 0; q < MAXQ; q++)
+                if (f[q] >= 0) {
+                    const half4_t v = *(SHFLBW_LDS half4_t*)(uintptr_t)(stage + (q * 64 + lane) * SP + pos * 8);
+#pragma unroll
+                    for (int u = 0; u < 4; u++)
+                        if (o[u]) o[u][f[q]] = v[u];
+                }
+        }
+    }
+}
+
+template <int RW, int NB, int NW, int NBUF, int U, int WPE>
+static hipError_t launch_patch(const ConvPatchArgs& a, hipStream_t stream)
+{
+    hipLaunchKernelGGL((spconv_patch_kernel<RW, NB, NW, NBUF, U, WPE>), dim3(a.p.jobs_per_xcd * 8), dim3(NW * 64), a.p.lds_bytes, stream, a);
+    return hipGetLastError();
+}
+
+template <int RW, int NB, int NW, int NBUF, int U, int WPE>
+static hipError_t prepare_patch()
+{
+    return hipFuncSetAttribute((const void*)spconv_patch_kernel<RW, NB, NW, NBUF, U, WPE>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               CONV_PATCH_LDS_MAX);
+}
+
+#define SHFLBW_PATCH(RW, NB, NW, NBUF, U, WPE) {RW, NB, NW, WPE * 4 / NW, NBUF, U, &launch_patch<RW, NB, NW, NBUF, U, WPE>, &prepare_patch<RW, NB, NW, NBUF, U, WPE>}
+
+static const ConvPatchKernel g_patch[] = {
+    SHFLBW_PATCH(16, 2, 8, 8, 5, 2), SHFLBW_PATCH(32, 2, 8, 8, 5, 2), SHFLBW_PATCH(64, 2, 8, 4, 5, 2),
+    SHFLBW_PATCH(16, 1, 8, 8, 5, 2), SHFLBW_PATCH(32, 1, 8, 8, 5, 2), SHFLBW_PATCH(64, 1, 8, 4, 5, 2),
+    SHFLBW_PATCH(16, 2, 4, 2, 2, 3), SHFLBW_PATCH(32, 2, 4, 2, 2, 2), SHFLBW_PATCH(64, 2, 4, 2, 2, 3),
+    SHFLBW_PATCH(16, 1, 4, 2, 2, 4), SHFLBW_PATCH(32, 1, 4, 2, 2, 4), SHFLBW_PATCH(64, 1, 4, 2, 2, 4),
+};
+
+// Estimated microseconds of the plane forms (three launches): the launches, the gathers of the SpMM, the two layout
+// passes.  The weights come from a fit to 124 measured layers (20 % rms).
+static double conv_planes_estimate(const ConvPatchProblem& q)
+{
+    const int s = q.stride;
+    const double PW = q.Wo + (q.S - 1) / s, PH = q.Ho + (q.R - 1) / s, n = (double)q.B * q.Ho * PW;
+    const double kept = (q.kept_per_panel + 32) * (q.F / q.V);
+    const double in = 2.0 * q.B * q.H * q.W * q.C, planes = 2.0 * s * s * q.C * PH * PW * q.B, out = 2.0 * q.F * (n + (double)q.B * q.Ho * q.Wo);
+    return 12.0 + kept * n * 2 / 15.1e6 + (in + planes) / 9.2e6 + out / 4.65e6;
+}
+
+// The cut with the least estimated time: rounds of workgroups times the sum of a workgroup's phases.  The weights come from
+// a fit to 124 layers measured with 20 to 40 cuts each (10 % rms; the cut it picks is 4 % slower than the best one
+// measured on average).  Where the plane forms are estimated faster - many filters over few resident pixels (wide
+// filters over many channels), filters of several workgroups interleaved in the output - the form is not taken:
+// 7 x 54 x 54 x 584 -> 1024, 5 x 5, stride 2 takes 152 us here, 54 us there; 16 x 14 x 14 x 512 -> 2048 20 and 23 us.
+bool conv_patch_plan(const ConvPatchProblem& q, ConvPatchPlan* plan)
+{
+    ConvPatchPlan best{};
+    double best_cost = 0;
+    const bool flat = q.R == 1 && q.S == 1 && q.stride == 1; // every pixel for itself: one long row
+    const unsigned long long in_bytes = (unsigned long long)q.B * q.H * q.W * q.C * 2;
+    if (in_bytes > 0xffffff00ull || (unsigned long long)q.B * q.Ho * q.Wo > 0x7fffffffull) return false;
+    const int B = flat ? 1 : q.B, H = flat ? 1 : q.H, W = flat ? q.B * q.H * q.W : q.W;
+    const int Ho = flat ? 1 : q.Ho, Wo = flat ? W : q.Wo;
+    const int eh = std::min(q.stride, q.R), ew = std::min(q.stride, q.S);
+    const int rw = conv_patch_unit_rows(q.V), npmax = 64 / rw, nunits = q.F / rw;
+    const double batches = std::max(1.0, std::ceil(q.kept_per_panel / 32.0));
+    for (const ConvPatchKernel& k : g_patch) {
+        if (k.RW != rw) continue;
+        const int positions = 8 * k.col_blocks;
+        for (int th = 1; th <= std::min(positions, Ho); th++)
+            for (int tw = 1; tw <= std::min(positions / th, Wo); tw++) {
+                // rows of 8 or 16 positions: the 8 positions half a wave reads lie in a row (what the order of the slots counts
+                // on); else positions are packed
+                const int rl = tw <= 8 && th <= positions / 8 ? 8 : th == 1 ? 16 : tw;
+                ConvPatchPlan p{};
+                p.col_blocks = k.col_blocks, p.waves = k.waves;
+                p.tile_h = th, p.tile_w = tw, p.row_len = rl;
+                p.blocks_w = (Wo + tw - 1) / tw;
+                const long blocks_hw = (long)((Ho + th - 1) / th) * p.blocks_w, units = B * blocks_hw;
+                if (units > 0x3fffffffL) continue;
+                p.blocks_hw = (int)blocks_hw;
+                p.units = (int)units;
+                const long tiles = (units + 3) / 4;
+                p.patch_w = (tw - 1) * ew + q.S;
+                p.npos = ((th - 1) * eh + q.R) * p.patch_w;
+                p.pitch = 8 * (p.npos | 1);
+                const long slab = (long)(q.C + 1) * p.pitch + CONV_PATCH_SLACK;
+                if (slab > CONV_PATCH_LDS_MAX) continue;
+                for (int groups = k.waves; groups >= 1; groups >>= 1)
+                    for (int np = 1; np <= npmax; np <<= 1) {
+                        p.groups = groups, p.ksplit = k.waves / groups, p.panels_per_wave = np;
+                        if (p.ksplit > 1 && np > 1) continue;
+                        if (groups > 1 && groups * np >= 2 * nunits) continue; // half of the waves would idle
+                        for (p.kshift = 0; (1 << p.kshift) < p.ksplit; p.kshift++) {}
+                        p.rows_wg = groups * np * rw;
+                        p.chunks = (q.F + p.rows_wg - 1) / p.rows_wg;
+                        const long jobs = tiles * p.chunks;
+                        if (jobs > 0x3fffffffL) continue;
+                        p.jobs = (int)jobs, p.jobs_per_xcd = (p.jobs + 7) / 8;
+                        const int cols = 32 * k.col_blocks;
+                        const long quads = (long)rw * cols / 64 / 4;
+                        const long stage = (long)p.rows_wg * (cols * 2 + 16) + (p.ksplit > 1 ? k.waves * quads * 1024 : 0);
+                        const long lds = 128 * k.col_blocks + std::max(slab, stage);
+                        if (lds > CONV_PATCH_LDS_MAX) continue;
+                        p.lds_bytes = (int)lds;
+                        // ---- estimated microseconds
+                        const int wgs = (int)std::min<long>(CONV_PATCH_LDS_MAX / lds, k.per_cu);
+                        const double per_cu = std::ceil((double)jobs / q.cus), act = std::min<double>(wgs, per_cu);
+                        const double rounds = std::ceil((double)jobs / ((double)q.cus * wgs));
+                        const double w = k.waves * act; // waves of a compute unit
+                        const double nb = std::ceil(np * batches / p.ksplit);
+                        const int steps = rw == 16 ? 1 : 2, mbw = rw == 64 ? 2 : 1, ncb = rw == 16 ? 2 * k.col_blocks : k.col_blocks;
+                        const bool apart = rl == 8 || rl == 16; // rows of half a wave's positions lie in a line
+                        const double t_mfma = steps * mbw * ncb * (rw == 16 ? 16 : 32) * w / 4 * 0.00045;
+                        const double t_stream = w * (steps * mbw * 1024 + (rw == 16 ? 256 : 512)) / 64 * 0.0004;
+                        const double t_lds = w * steps * ncb * 4 * (apart ? 1.2 : 2.0) * 0.00081;
+                        const double t_longest = std::max(std::max(t_mfma, t_stream), std::max(t_lds, 0.37 / k.ring));
+                        const double t_main = nb * (t_longest + 0.2 * (t_mfma + t_stream + t_lds - std::min(t_longest, t_mfma + t_stream + t_lds)));
+                        const double rounds_patch = std::ceil((double)((p.npos + 7) / 8 * ((q.C + 63) / 64)) / (k.waves * k.items));
+                        const double t_patch = act * q.C * p.npos * 8 * 5.3e-6 + rounds_patch * 0.7;
+                        const double values = (double)cols * std::min(p.rows_wg, q.F) * act;
+                        const double t_out = values * (!q.permuted || p.chunks == 1 ? 5.0e-5 : 1.5e-4) +
+                                             (p.ksplit > 1 ? k.waves * rw * cols * 4.0 * act * 1.0e-5 : 0);
+                        const double one = 1.0 + (k.waves == 8 ? 1.15 : 0) + t_patch + t_main + t_out;
+                        const double cost = 2.9 + one * (1 + (rounds - 1) * 1.16) + jobs * 1.0e-5;
+                        if (!best.valid || cost < best_cost) {
+                            best = p, best_cost = cost;
+                            best.valid = 1;
+                        }
+                    }
+            }
+    }
+    if (!best.valid) return false;
+    if (best_cost > conv_planes_estimate(q)) return false;
+    best.H = H, best.W = W, best.Ho = Ho, best.Wo = Wo, best.stride = q.stride;
+    best.pad_h = q.R / 2, best.pad_w = q.S / 2;
+    best.step_h = eh, best.step_w = ew;
+    best.skip = q.stride > q.R || q.stride > q.S;
+    best.in_bytes = (unsigned)in_bytes;
+    best.touch_bytes = best.touch_step = 0; // set with the size of the image
+    best.magic_bhw = udiv_magic(best.blocks_hw);
+    best.magic_bw = udiv_magic(best.blocks_w);
+    best.magic_pw = udiv_magic(best.patch_w);
+    best.magic_row = udiv_magic(best.row_len);
+    best.magic_chunks = udiv_magic(best.chunks);
+    best.magic_pg = udiv_magic((best.npos + 7) / 8);
+    *plan = best;
+    return true;
+}
+
+// Order of the kept columns of one row panel: the rows one pass of a transposing LDS read touches (32 lanes: four rows
+// of 8 positions, for row units of 16 eight rows of 4) should fall into different banks.  A row starts in one of 32
+// bank pairs; `foot` marks the pairs its positions touch when it starts in pair 0.  Exact tilings of the 32 pairs by
+// shifted copies of `foot` are looked for first; groups are then filled from the tiling and shift whose
+// scarcest member has the most rows left, and from whatever collides least once no tiling can be filled.
+// pair_of: start pairs of the kept columns; returns their order, whole groups of `group` at a time.
+static void tilings(uint32_t foot, int group, std::vector<int>& shifts, uint32_t used, std::vector<std::vector<int>>& found)
+{
+    if ((int)shifts.size() == group) {
+        found.push_back(shifts);
+        return;
+    }
+    for (int s = shifts.back() + 1; s < 32 && found.size() < 64; s++) {
+        const uint32_t m = s ? (foot << s) | (foot >> (32 - s)) : foot;
+        if (used & m) continue;
+        shifts.push_back(s);
+        tilings(foot, group, shifts, used | m, found);
+        shifts.pop_back();
+    }
+}
+
+void conv_patch_order(const std::vector<int>& pair_of, uint32_t foot, int group, std::vector<int>& order)
+{
+    const int n = (int)pair_of.size();
+    order.clear();
+    order.reserve(n);
+    std::vector<int> at[32];
+    for (int i = n - 1; i >= 0; i--) at[pair_of[i]].push_back(i);
+    std::vector<std::vector<int>> found;
+    std::vector<int> shifts{0};
+    tilings(foot, group, shifts, foot, found);
+    auto rot = [&](int s) { return s ? (foot << s) | (foot >> (32 - s)) : foot; };
+    while ((int)order.size() < n) {
+        int best = 0, best_shift = 0;
+        const std::vector<int>* with = nullptr;
+        for (const auto& t : found)
+            for (int s = 0; s < 32; s++) {
+                int least = n;
+                for (int d : t) least = std::min(least, (int)at[(s + d) & 31].size());
+                if (least > best) best = least, best_shift = s, with = &t;
+            }
+        if (with) {
+            for (int d : *with) {
+                auto& from = at[(best_shift + d) & 31];
+                order.push_back(from.back());
+                from.pop_back();
+            }
+            continue;
+        }
+        int load[32] = {};
+        for (int g = 0; g < group && (int)order.size() < n; g++) {
+            int pick = -1, pick_worst = 0;
+            for (int s = 0; s < 32; s++) {
+                if (at[s].empty()) continue;
+                int worst = 0;
+                for (int b = 0; b < 32; b++) worst = std::max(worst, load[b] + (int)((rot(s) >> b) & 1));
+                if (pick < 0 || worst < pick_worst || (worst == pick_worst && at[s].size() > at[pick].size())) pick = s, pick_worst = worst;
+            }
+            for (int b = 0; b < 32; b++) load[b] += (rot(pick) >> b) & 1;
+            order.push_back(at[pick].back());
+            at[pick].pop_back();
+        }
+    }
+}
+
+const ConvPatchKernel* conv_patch_kernel(int rows, int col_blocks, int waves)
+{
+    for (const ConvPatchKernel& k : g_patch)
+        if (k.RW == rows && k.col_blocks == col_blocks && k.waves == waves) return &k;
+    return nullptr;
+}
+
+} // namespace shflbw

@@ -2,11 +2,13 @@
 // Host side of the Shfl-BW format: reference block_sparse/spmm/blockwise_format.h:13-68.
 #pragma once
 #include <cstdint>
+#include <list>
 #include <mutex>
 #include <string>
 #include <vector>
 
 #include "shflbw.h"
+#include "spconv_patch.h"
 
 struct shflbw_weight {
     // shape and pattern (blockwise_format.h:15-22)
@@ -68,7 +70,22 @@ struct shflbw_weight {
         unsigned long long stamp; // value of bulk_clock when it was last handed out
     };
     static constexpr int CONV_BULK_DEPTH = SHFLBW_CONV_SCRATCH_DEPTH;
+    //  * ConvPatch: cut, filter image (in an order of its own) and output places of the patch form, keyed like the ids
+    //    (plan.valid == 0: the form does not take that geometry); states point at the entries, which stay where they are.
+    struct ConvPatch {
+        int key[4]; // B, H, W, stride
+        shflbw::ConvPatchPlan plan;
+        void* ptr; // fragments | offsets | first batches | filters | places
+        size_t bytes;
+        const void* packedA;
+        const int* first_batch;
+        const unsigned short* offs;
+        const int* filt;
+        const unsigned short* dst;
+        int dense;
+    };
     std::vector<ConvIds> conv_ids;
+    std::list<ConvPatch> conv_patch;
     std::vector<ConvBulk> conv_bulk;
     unsigned long long bulk_clock = 0;
     std::mutex scratch_lock;

@@ -1,0 +1,91 @@
+"""GPU parity of the patch form of the convolution (one launch, the input patch of a workgroup in LDS) against the CPU
+oracle: integer operands, bit for bit.  The shapes sit where the form can go wrong: edges of the pixel blocks and of the
+four-unit tiles, channel counts that leave part of a 64-channel group, strides wider than the filter, every block
+height, one and several workgroups per column tile with and without a permutation, kept columns split over waves."""
+import numpy as np
+import pytest
+
+import shflbw_sparse_nn_amd as S
+from oracle import oracle as O
+import workloads as P
+from workloads import run_spconv
+
+pytestmark = pytest.mark.gpu
+PATCH = 5
+
+
+def _check(torch, w, x, R, Sx, C, stride):
+    got = run_spconv(torch, w, R, Sx, C, x, stride, PATCH)
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref = O.float_to_half(P.conv_oracle(w, R, Sx, C, x, stride))
+    nan = np.isnan(ref)
+    assert np.array_equal(np.isnan(got), nan)
+    np.testing.assert_array_equal(got[~nan].view(np.uint16), ref[~nan].view(np.uint16))
+
+
+@pytest.mark.parametrize("Bn,H,W,C,F,R,Sx,stride,V,d,permute", [
+    (1, 1, 1, 8, 16, 1, 1, 1, 16, 1.0, True),          # one pixel, one panel
+    (1, 5, 5, 8, 32, 3, 3, 1, 32, 0.5, True),          # fewer blocks than a tile has units
+    (3, 9, 9, 8, 128, 1, 1, 1, 128, 0.6, False),       # 1 x 1: one long row of pixels over all images
+    (2, 8, 8, 24, 64, 5, 3, 1, 32, 0.2, True),         # three groups of eight channels
+    (2, 9, 7, 16, 48, 3, 3, 1, 16, 0.4, True),
+    (1, 11, 9, 16, 64, 3, 3, 3, 64, 0.5, True),
+    (2, 6, 20, 8, 32, 1, 7, 1, 32, 0.4, True),
+    (8, 9, 8, 16, 64, 4, 2, 2, 32, 0.3, True),         # even filter extents
+    (5, 9, 9, 40, 704, 1, 1, 2, 64, 0.25, True),       # stride wider than the filter, eleven panels
+    (5, 13, 3, 136, 64, 2, 2, 3, 64, 0.25, True),
+    (3, 9, 9, 40, 2048, 3, 3, 1, 16, 0.25, True),      # filters of several workgroups interleaved in a pixel
+    (3, 9, 9, 40, 1536, 3, 3, 1, 128, 0.25, True),
+    (3, 9, 9, 40, 1088, 3, 3, 1, 32, 0.25, False),     # ... consecutive
+    (1, 7, 7, 512, 64, 3, 3, 1, 64, 0.1, True),        # one panel: its kept columns over all waves of a workgroup
+    (2, 30, 31, 32, 96, 3, 3, 1, 32, 0.02, True),      # panels with almost no kept column
+    (24, 28, 28, 32, 64, 3, 3, 1, 64, 0.2, True),      # several workgroups of a compute unit at a time
+])
+def test_exact_shapes(torch_gpu, Bn, H, W, C, F, R, Sx, stride, V, d, permute):
+    w = P.make_weight(F, R * Sx * C, V, d, permute, 2021, integer=True)
+    x = np.random.default_rng(5).integers(-4, 5, size=(Bn, H, W, C)).astype(np.float16)
+    _check(torch_gpu, w, x, R, Sx, C, stride)
+
+
+@pytest.mark.parametrize("V", [16, 32, 64, 128])
+def test_empty_panels_and_non_finite_input(torch_gpu, V):
+    """Panels without a kept column give zeros; an Inf or NaN in the input reaches the outputs it reaches in the oracle and
+    no other (padding slots read a row of zeros)."""
+    Bn, H, W, C, R, Sx = 2, 9, 10, 16, 3, 3
+    X, K = 6, R * Sx * C
+    counts = np.array([0, 33, 0, 5, 64, 0])
+    rng = np.random.default_rng(5)
+    indptr = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    indices = np.concatenate([np.sort(rng.choice(K, c, replace=False)) for c in counts]).astype(np.int32)
+    values = rng.integers(1, 5, size=int(counts.sum()) * V).astype(np.float16)  # no zero: 0 * inf is NaN in the oracle too
+    w = dict(nrow=X * V, ncol=K, brow=V, bcol=1, nnzb=int(counts.sum()), indptr=indptr, indices=indices, values=values,
+             row_permute_ids=O.row_permutation(X * V, 5))
+    x = rng.integers(-4, 5, size=(Bn, H, W, C)).astype(np.float16)
+    _check(torch_gpu, w, x, R, Sx, C, 1)
+    x[0, 4, 5, 3], x[1, 0, 0, 15], x[1, 8, 9, 0] = np.inf, -np.inf, np.nan
+    _check(torch_gpu, w, x, R, Sx, C, 1)
+
+
+def test_the_library_runs_it_and_it_needs_no_buffers(torch_gpu):
+    """shflbw_spconv_init takes the patch form on an ordinary layer (the state keeps naming the plane form it stands in
+    for); states over many tensors share its tables; weights of too many channels for the LDS keep the plane form."""
+    torch = torch_gpu
+    w = P.make_weight(64, 9 * 64, 32, 0.2, True, 3, integer=True)
+    f = P.upload_weight(w, 3, 3, 64, cls=S.BlockwiseSpFilter)
+    x = torch.zeros((8, 14, 14, 64), dtype=torch.float16, device="cuda")
+    ops = []
+    for _ in range(3):
+        op = S.SpconvBlockwiseOp()
+        y = torch.full((8, 14, 14, 64), float("nan"), dtype=torch.float16, device="cuda")
+        st = op.initialize(f, 8, 14, 14, 1, x.data_ptr(), y.data_ptr())
+        assert st.patch and st.variant == 2
+        op(torch.cuda.current_stream().cuda_stream)
+        ops.append((op, y))
+    torch.cuda.synchronize()
+    assert len({op._state.patch for op, _ in ops}) == 1 and all((y == 0).all() for _, y in ops)
+    wide = P.make_weight(64, 25 * 1024, 64, 0.01, True, 3, integer=True)
+    fw = P.upload_weight(wide, 5, 5, 1024, cls=S.BlockwiseSpFilter)
+    xw = torch.zeros((1, 8, 8, 1024), dtype=torch.float16, device="cuda")
+    op = S.SpconvBlockwiseOp()
+    st = op.initialize(fw, 1, 8, 8, 1, xw.data_ptr(), ops[0][1].data_ptr())
+    assert not st.patch and st.variant == 0
