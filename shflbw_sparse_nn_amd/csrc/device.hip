@@ -8,6 +8,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -32,12 +33,10 @@ static void release_conv_scratch(shflbw_weight* w);
 
 void clear_device(shflbw_weight* w)
 {
-    void** bufs[] = {&w->d_meta, &w->d_values, &w->d_group_ptr, &w->d_packed_indices, &w->d_packed_indices_pm,
-                     &w->d_packed_values, &w->d_packed_slab};
-    for (void** b : bufs) {
-        if (*b) (void)hipFree(*b);
+    if (w->d_image) (void)hipFree(w->d_image);
+    for (void** b : {&w->d_image, &w->d_meta, &w->d_values, &w->d_group_ptr, &w->d_packed_indices, &w->d_packed_indices_pm,
+                     &w->d_packed_values, &w->d_packed_slab})
         *b = nullptr;
-    }
     release_conv_scratch(w);
 }
 
@@ -55,27 +54,36 @@ void release_conv_scratch(shflbw_weight* w)
     w->conv_patch.clear();
 }
 
-static int upload_one(void** dst, const void* src, size_t bytes)
-{
-    // zero-length arrays (an empty matrix) still get a valid pointer
-    SHFLBW_HIP_TRY(hipMalloc(dst, bytes ? bytes : 16));
-    if (bytes) SHFLBW_HIP_TRY(hipMemcpy(*dst, src, bytes, hipMemcpyHostToDevice));
-    return SHFLBW_OK;
-}
-
+// One allocation and one copy for all arrays of a weight (seven of each cost more than packing a small weight).
 int upload(shflbw_weight* w)
 {
-    int rc;
-    if ((rc = upload_one(&w->d_meta, w->meta_h.data(), w->meta_h.size() * sizeof(int))) ||
-        (rc = upload_one(&w->d_values, w->values.data(), w->values.size() * sizeof(uint16_t))) ||
-        (rc = upload_one(&w->d_group_ptr, w->panel_desc.data(), w->panel_desc.size() * sizeof(int))) ||
-        (rc = upload_one(&w->d_packed_indices, w->packed_indices.data(), w->packed_indices.size() * sizeof(int))) ||
-        (rc = upload_one(&w->d_packed_indices_pm, w->packed_indices_pm.data(),
-                         w->packed_indices_pm.size() * sizeof(int))) ||
-        (rc = upload_one(&w->d_packed_values, w->packed_values.data(), w->packed_values.size() * sizeof(uint16_t))) ||
-        (rc = upload_one(&w->d_packed_slab, w->packed_slab.data(), w->packed_slab.size() * sizeof(int)))) {
+    struct Part {
+        void** dst;
+        const void* src;
+        size_t bytes, at;
+    } parts[] = {
+        {&w->d_meta, w->meta_h.data(), w->meta_h.size() * sizeof(int), 0},
+        {&w->d_values, w->values.data(), w->values.size() * sizeof(uint16_t), 0},
+        {&w->d_group_ptr, w->panel_desc.data(), w->panel_desc.size() * sizeof(int), 0},
+        {&w->d_packed_indices, w->packed_indices.data(), w->packed_indices.size() * sizeof(int), 0},
+        {&w->d_packed_indices_pm, w->packed_indices_pm.data(), w->packed_indices_pm.size() * sizeof(int), 0},
+        {&w->d_packed_values, w->packed_values.data(), w->packed_values.size() * sizeof(uint16_t), 0},
+        {&w->d_packed_slab, w->packed_slab.data(), w->packed_slab.size() * sizeof(int), 0},
+    };
+    size_t total = 0;
+    for (Part& p : parts) {
+        p.at = total;
+        total += (p.bytes + 16 + 255) / 256 * 256; // zero-length arrays (an empty matrix) still get a valid pointer
+    }
+    std::unique_ptr<unsigned char[]> host(new unsigned char[total]);
+    for (Part& p : parts)
+        if (p.bytes) memcpy(host.get() + p.at, p.src, p.bytes);
+    SHFLBW_HIP_TRY(hipMalloc(&w->d_image, total));
+    for (Part& p : parts) *p.dst = (char*)w->d_image + p.at;
+    if (hipMemcpy(w->d_image, host.get(), total, hipMemcpyHostToDevice) != hipSuccess) {
         clear_device(w);
-        return rc;
+        set_error("sync_device: cannot upload %zu bytes", total);
+        return SHFLBW_ERR_HIP;
     }
     return SHFLBW_OK;
 }
@@ -954,6 +962,7 @@ int conv_patch_for(shflbw_weight* fw, int B, int H, int W, int stride, int Ho, i
         for (int t = 0; t < 32; t++)
             slot_of[t] = RW == 16 ? (t / 16) * 16 + ((t / 8) & 1) * 4 + ((t / 4) & 1) * 8 + t % 4 : t;
         std::vector<int> pair_of, order;
+        static const uint16_t zeros[64] = {};
         size_t b = 0;
         for (int panel = 0; panel < X; panel++) {
             const int begin = fw->indptr[panel], nnz = fw->indptr[panel + 1] - begin;
@@ -966,20 +975,31 @@ int conv_patch_for(shflbw_weight* fw, int B, int H, int W, int stride, int Ho, i
             conv_patch_order(pair_of, foot, group, order);
             for (int part = 0; part < per_panel; part++) {
                 first[panel * per_panel + part] = (int)b;
-                for (int t = 0; t < (nnz + 31) / 32 * 32; t++) {
-                    const int s = slot_of[t % 32];
-                    uint16_t* o = offs + (b + t / 32) * 32;
-                    uint16_t* a = A + (b + t / 32) * 32 * RW;
-                    const int in_step = RW == 16 ? s : s % 16, step = RW == 16 ? 0 : s / 16;
-                    const int pair = (in_step / 8) * 4 + in_step % 4, hi = (in_step % 8) / 4;
-                    // a lane addresses slots s and s + 4 of a step and loads the offsets of all steps of a batch at once
-                    o[RW == 16 ? pair * 2 + hi : pair * 4 + step * 2 + hi] = (uint16_t)((t < nnz ? offset_of(fw->indices[begin + order[t]]) : C * p.pitch) >> 3);
-                    if (t >= nnz) continue;
-                    const uint16_t* v = fw->values.data() + (size_t)(begin + order[t]) * V + part * RW;
-                    if (RW == 16)
-                        for (int r = 0; r < 16; r++) a[((s / 8) * 16 + r) * 8 + s % 8] = v[r];
-                    else
-                        for (int r = 0; r < RW; r++) a[(((size_t)step * (RW / 32) + r / 32) * 64 + (in_step / 8) * 32 + r % 32) * 8 + s % 8] = v[r];
+                for (int t0 = 0; t0 < nnz; t0 += 32) {
+                    uint16_t* o = offs + (b + t0 / 32) * 32;
+                    uint16_t* a = A + (b + t0 / 32) * 32 * RW;
+                    const uint16_t* src[32];
+                    for (int t = 0; t < 32; t++) {
+                        const int s = slot_of[t], in_step = RW == 16 ? s : s % 16, step = RW == 16 ? 0 : s / 16;
+                        const int pair = (in_step / 8) * 4 + in_step % 4, hi = (in_step % 8) / 4;
+                        const bool held = t0 + t < nnz;
+                        const int i = held ? order[t0 + t] : 0;
+                        // a lane addresses slots s and s + 4 of a step and loads the offsets of all steps of a batch at once
+                        o[RW == 16 ? pair * 2 + hi : pair * 4 + step * 2 + hi] = (uint16_t)((held ? offset_of(fw->indices[begin + i]) : C * p.pitch) >> 3);
+                        src[s] = held ? fw->values.data() + (size_t)(begin + i) * V + part * RW : zeros;
+                    }
+                    for (int s = 0; s < 32; s += 8) {
+                        const uint16_t* v[8];
+                        for (int j = 0; j < 8; j++) v[j] = src[s + j];
+                        if (RW == 16) {
+                            interleave8(v, 16, a + (s / 8) * 16 * 8);
+                            continue;
+                        }
+                        for (int mb = 0; mb < RW / 32; mb++) {
+                            interleave8(v, 32, a + ((size_t)((s / 16) * (RW / 32) + mb) * 64 + (s % 16) / 8 * 32) * 8);
+                            for (int j = 0; j < 8; j++) v[j] += 32;
+                        }
+                    }
                 }
                 b += (nnz + 31) / 32;
             }

@@ -627,17 +627,17 @@ bool conv_patch_plan(const ConvPatchProblem& q, ConvPatchPlan* plan)
 // shifted copies of `foot` are looked for first; groups are then filled from the tiling and shift whose
 // scarcest member has the most rows left, and from whatever collides least once no tiling can be filled.
 // pair_of: start pairs of the kept columns; returns their order, whole groups of `group` at a time.
-static void tilings(uint32_t foot, int group, std::vector<int>& shifts, uint32_t used, std::vector<std::vector<int>>& found)
+static void tilings(const uint32_t (&rot)[32], int group, std::vector<int>& shifts, uint32_t used, std::vector<std::vector<int>>& found)
 {
     if ((int)shifts.size() == group) {
         found.push_back(shifts);
         return;
     }
-    for (int s = shifts.back() + 1; s < 32 && found.size() < 64; s++) {
-        const uint32_t m = s ? (foot << s) | (foot >> (32 - s)) : foot;
-        if (used & m) continue;
+    const uint32_t lowest = ~used & (used + 1); // the first pair without a row: some copy has to cover it
+    for (int s = 1; s < 32 && found.size() < 3; s++) {
+        if (!(rot[s] & lowest) || (rot[s] & used)) continue;
         shifts.push_back(s);
-        tilings(foot, group, shifts, used | m, found);
+        tilings(rot, group, shifts, used | rot[s], found);
         shifts.pop_back();
     }
 }
@@ -647,41 +647,45 @@ void conv_patch_order(const std::vector<int>& pair_of, uint32_t foot, int group,
     const int n = (int)pair_of.size();
     order.clear();
     order.reserve(n);
-    std::vector<int> at[32];
-    for (int i = n - 1; i >= 0; i--) at[pair_of[i]].push_back(i);
+    int begin[33] = {}, count[32] = {}; // rows by start pair: by_pair[begin[s] ..], count[s] of them left
+    for (int i = 0; i < n; i++) count[pair_of[i]]++;
+    for (int s = 0; s < 32; s++) begin[s + 1] = begin[s] + count[s];
+    std::vector<int> by_pair(n);
+    int fill[32];
+    std::copy(begin, begin + 32, fill);
+    for (int i = 0; i < n; i++) by_pair[fill[pair_of[i]]++] = i;
+    auto take = [&](int s) { order.push_back(by_pair[begin[s + 1] - count[s]--]); };
+    uint32_t rot[32];
+    for (int s = 0; s < 32; s++) rot[s] = s ? (foot << s) | (foot >> (32 - s)) : foot;
     std::vector<std::vector<int>> found;
     std::vector<int> shifts{0};
-    tilings(foot, group, shifts, foot, found);
-    auto rot = [&](int s) { return s ? (foot << s) | (foot >> (32 - s)) : foot; };
-    while ((int)order.size() < n) {
+    tilings(rot, group, shifts, foot, found);
+    while (true) {
         int best = 0, best_shift = 0;
         const std::vector<int>* with = nullptr;
         for (const auto& t : found)
             for (int s = 0; s < 32; s++) {
                 int least = n;
-                for (int d : t) least = std::min(least, (int)at[(s + d) & 31].size());
+                for (int d : t) least = std::min(least, count[(s + d) & 31]);
                 if (least > best) best = least, best_shift = s, with = &t;
             }
-        if (with) {
-            for (int d : *with) {
-                auto& from = at[(best_shift + d) & 31];
-                order.push_back(from.back());
-                from.pop_back();
-            }
-            continue;
-        }
-        int load[32] = {};
+        if (!with) break;
+        for (; best > 0; best--)
+            for (int d : *with) take((best_shift + d) & 31);
+    }
+    while ((int)order.size() < n) {
+        uint32_t level[9] = {}; // level[m]: pairs at least m of the picked rows touch
         for (int g = 0; g < group && (int)order.size() < n; g++) {
             int pick = -1, pick_worst = 0;
             for (int s = 0; s < 32; s++) {
-                if (at[s].empty()) continue;
-                int worst = 0;
-                for (int b = 0; b < 32; b++) worst = std::max(worst, load[b] + (int)((rot(s) >> b) & 1));
-                if (pick < 0 || worst < pick_worst || (worst == pick_worst && at[s].size() > at[pick].size())) pick = s, pick_worst = worst;
+                if (!count[s]) continue;
+                int worst = 1;
+                while (worst <= g && (level[worst] & rot[s])) worst++;
+                if (pick < 0 || worst < pick_worst || (worst == pick_worst && count[s] > count[pick])) pick = s, pick_worst = worst;
             }
-            for (int b = 0; b < 32; b++) load[b] += (rot(pick) >> b) & 1;
-            order.push_back(at[pick].back());
-            at[pick].pop_back();
+            for (int m = group; m > 1; m--) level[m] |= level[m - 1] & rot[pick];
+            level[1] |= rot[pick];
+            take(pick);
         }
     }
 }

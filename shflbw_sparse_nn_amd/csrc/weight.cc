@@ -272,22 +272,18 @@ int build_packed_image(shflbw_weight* w)
         }
         uint16_t* dst = w->packed_values.data() + slot0 * V;
         const uint16_t* src = w->values.data() + (size_t)begin * V;
-        if (V >= 32) {
-            const int MB = V / 32;
-            for (int q = 0; q < nnz; q++) {
-                const int s = q / 16, half_k = (q % 16) / 8, j = q % 8;
-                for (int r = 0; r < V; r++) {
-                    const int mb = r / 32, lane = half_k * 32 + r % 32;
-                    dst[(((size_t)s * MB + mb) * 64 + lane) * 8 + j] = src[(size_t)ord[q] * V + r];
+        static const uint16_t zeros[128] = {};
+        for (int q = 0; q < nnz; q += 8) { // eight slots: one 16-byte piece per row
+            const uint16_t* v[8];
+            for (int j = 0; j < 8; j++) v[j] = q + j < nnz ? src + (size_t)ord[q + j] * V : zeros;
+            if (V >= 32) {
+                const int MB = V / 32, s = q / 16, half_k = (q % 16) / 8;
+                for (int mb = 0; mb < MB; mb++) {
+                    interleave8(v, 32, dst + (((size_t)s * MB + mb) * 64 + half_k * 32) * 8);
+                    for (int j = 0; j < 8; j++) v[j] += 32;
                 }
-            }
-        } else {
-            for (int q = 0; q < nnz; q++) {
-                const int s = q / 32, quarter = (q % 32) / 8, j = q % 8;
-                for (int r = 0; r < 16; r++) {
-                    const int lane = quarter * 16 + r;
-                    dst[((size_t)s * 64 + lane) * 8 + j] = src[(size_t)ord[q] * 16 + r];
-                }
+            } else {
+                interleave8(v, 16, dst + ((size_t)(q / 32) * 64 + (q % 32) / 8 * 16) * 8);
             }
         }
     }

@@ -38,7 +38,8 @@ struct shflbw_weight {
     bool initialized = false, device_synced = false;
     std::string config_str;
 
-    // device buffers (owned)
+    // device buffers: parts of d_image (owned)
+    void* d_image = nullptr;
     void* d_meta = nullptr;
     void* d_values = nullptr;
     void* d_group_ptr = nullptr; // holds panel_desc
@@ -116,6 +117,30 @@ inline int slab_row_offset(int k, int ncol)
 // Which quarter of the LDS banks the 64 bytes of slab row k that one transposing read touches fall into (the other
 // 64 bytes of the row: the same quarter with the lowest bit flipped): rows of different class never collide.
 inline int slab_bank_class(int k) { return (k & 1) * 2 + ((k >> 2) & 1); }
+
+// out[8 r + j] = v[j][r] for r < rows (a multiple of 8): eight kept vectors side by side, as the matrix cores take them
+// (8 x 8 transposes; value by value this was most of the time of packing a weight)
+inline void interleave8(const uint16_t* const (&v)[8], int rows, uint16_t* out)
+{
+    typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
+    for (int r = 0; r < rows; r += 8) {
+        u16x8 a[8], b[8];
+        for (int j = 0; j < 8; j++) __builtin_memcpy(&a[j], v[j] + r, 16);
+        for (int j = 0; j < 4; j++) { // pairs (j, j + 4), then (j, j + 2), then neighbours
+            b[2 * j] = __builtin_shufflevector(a[j], a[j + 4], 0, 8, 1, 9, 2, 10, 3, 11);
+            b[2 * j + 1] = __builtin_shufflevector(a[j], a[j + 4], 4, 12, 5, 13, 6, 14, 7, 15);
+        }
+        for (int j = 0; j < 4; j++) {
+            a[2 * j] = __builtin_shufflevector(b[j], b[j + 4], 0, 8, 1, 9, 2, 10, 3, 11);
+            a[2 * j + 1] = __builtin_shufflevector(b[j], b[j + 4], 4, 12, 5, 13, 6, 14, 7, 15);
+        }
+        for (int j = 0; j < 4; j++) {
+            b[2 * j] = __builtin_shufflevector(a[j], a[j + 4], 0, 8, 1, 9, 2, 10, 3, 11);
+            b[2 * j + 1] = __builtin_shufflevector(a[j], a[j + 4], 4, 12, 5, 13, 6, 14, 7, 15);
+        }
+        __builtin_memcpy(out + r * 8, b, 128);
+    }
+}
 
 // builds group_ptr / packed_indices / packed_values from the host arrays
 int build_packed_image(shflbw_weight* w);
