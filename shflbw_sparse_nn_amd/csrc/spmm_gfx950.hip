@@ -259,7 +259,8 @@ __device__ __forceinline__ int ks_sel(const int (&ks)[N_], int base, int sub, in
     return k;
 }
 
-template <int V, int WN, int NCONS, int NPROD, int KT, int NSTAGE>
+// RES: beta != 0
+template <int V, int WN, int NCONS, int NPROD, int KT, int NSTAGE, bool RES>
 __global__ void
 __launch_bounds__((NCONS + NPROD) * 64, (SpmmWsCfg<V, WN, NCONS, NPROD, KT, NSTAGE>::WGS_PER_CU * (NCONS + NPROD) + 3) / 4)
 spmm_shflbw_ws_kernel(SpmmLaunchArgs a)
@@ -287,9 +288,9 @@ spmm_shflbw_ws_kernel(SpmmLaunchArgs a)
     }
 
     if constexpr (V == 16)
-        ws_consumer16<Cfg, WN, NCONS>(a, lds0, lane, wave, id_first, id_end, S);
+        ws_consumer16<Cfg, WN, NCONS, false, false, RES>(a, lds0, lane, wave, id_first, id_end, S);
     else
-        ws_consumer<Cfg, V, WN, NCONS>(a, lds0, lane, wave, id_first, id_end, S);
+        ws_consumer<Cfg, V, WN, NCONS, false, false, RES>(a, lds0, lane, wave, id_first, id_end, S);
 }
 
 template <int V, int WN, int NCONS, int NPROD, int KT, int NSTAGE>
@@ -307,8 +308,12 @@ static hipError_t launch_ws(const SpmmLaunchArgs& a, hipStream_t stream)
     grid = (grid / 8) * 8;
     const int need = ((T + 7) / 8) * 8;
     if (grid > need) grid = need;
-    hipLaunchKernelGGL((spmm_shflbw_ws_kernel<V, WN, NCONS, NPROD, KT, NSTAGE>), dim3(grid),
-                       dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream, b);
+    if (a.beta != 0.f)
+        hipLaunchKernelGGL((spmm_shflbw_ws_kernel<V, WN, NCONS, NPROD, KT, NSTAGE, true>), dim3(grid),
+                           dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream, b);
+    else
+        hipLaunchKernelGGL((spmm_shflbw_ws_kernel<V, WN, NCONS, NPROD, KT, NSTAGE, false>), dim3(grid),
+                           dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream, b);
     return hipGetLastError();
 }
 
@@ -316,7 +321,10 @@ template <int V, int WN, int NCONS, int NPROD, int KT, int NSTAGE>
 static hipError_t prepare_ws()
 {
     using Cfg = SpmmWsCfg<V, WN, NCONS, NPROD, KT, NSTAGE>;
-    return hipFuncSetAttribute((const void*)spmm_shflbw_ws_kernel<V, WN, NCONS, NPROD, KT, NSTAGE>,
+    const hipError_t e = hipFuncSetAttribute((const void*)spmm_shflbw_ws_kernel<V, WN, NCONS, NPROD, KT, NSTAGE, false>,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS_BYTES);
+    if (e != hipSuccess) return e;
+    return hipFuncSetAttribute((const void*)spmm_shflbw_ws_kernel<V, WN, NCONS, NPROD, KT, NSTAGE, true>,
                                hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS_BYTES);
 }
 

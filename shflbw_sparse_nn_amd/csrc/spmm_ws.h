@@ -146,7 +146,12 @@ struct TileWalker {
 // LDS; a consumer executes one barrier before its first stage and one more per stage.
 // XCD_LOCAL: the result is read back by workgroups of the same XCD in the same launch and is stored without device
 // scope (it stays in that XCD's L2); DMAP: see output_column().
-template <typename Cfg, int V, int WN, int NCONS, bool XCD_LOCAL = false, bool DMAP = false>
+// RES: beta != 0.  The pieces of C a lane adds are loaded over the tile's stages (PRE of its epilogue's steps of two
+// pieces, the others as the first ones are used up).  Loaded in the epilogue every step waited for memory once, and loaded
+// at one point of the stage loop they hold up the gathers behind them: 8192 x 4096 x 16384, block height 128, density 0.1:
+// 272 us in the epilogue, 255 at one point, 249 spread; 4096^3, block height 64: 34.3, 34.0, 31.7.  Streaming loads lose
+// what is left of C in the Infinity Cache (34.8).
+template <typename Cfg, int V, int WN, int NCONS, bool XCD_LOCAL = false, bool DMAP = false, bool RES = false>
 __device__ __forceinline__ void ws_consumer(const SpmmLaunchArgs& a, uint32_t lds0, int lane, int cw, int id_first,
                                             int id_end, int S)
 {
@@ -164,6 +169,22 @@ __device__ __forceinline__ void ws_consumer(const SpmmLaunchArgs& a, uint32_t ld
     const uint32_t epi = lds0 + Cfg::RING_BYTES + cw * Cfg::EPI_WAVE_BYTES;
     constexpr int KSPS = Cfg::KSPS; // k16 steps per LDS stage: rows 16h.. of the B area and A block h belong to step h
     static_assert(KSPS == 1 || KSPS == 2, "one or two k16 steps per LDS stage");
+
+    constexpr int PR = 4;                 // 16-byte pieces per 32-column row segment
+    constexpr int RPS = 64 / PR;          // rows per store instruction
+    constexpr int ER = Cfg::EPI_ROWS;     // rows staged at a time: 32 (whole block) or 16 (half, by lanes)
+    constexpr int NIT = ER / RPS;
+    // Whole lines: with an even number of 32-column blocks, 16 rows of two neighbouring blocks are staged at a time
+    // (rows of 128 bytes + 16) and eight lanes store one 128-byte line of a row: half as many write requests to the
+    // L2s as with 64-byte row segments (4096 x 4096 x 4096, density 0.1: -2 %, -11 % at N = 16384, where every epilogue
+    // runs beside other workgroups' gathers).  Not where two workgroups share a compute unit (128 registers per wave: it
+    // spills).
+    constexpr bool LINES = SHFLBW_EPI_LINES && NB % 2 == 0 && 16 * (128 + 16) <= Cfg::EPI_WAVE_BYTES && Cfg::WGS_PER_CU == 1;
+    constexpr int CIT = LINES ? 2 : NIT;                            // pieces of C per epilogue step
+    constexpr int STEPS = LINES ? MB * NB : MB * NB * (32 / ER);    // epilogue steps of a tile
+    // ... whose pieces are in flight (beside 128 accumulators all eight would spill; waves with 128 registers have no room)
+    constexpr int PRE = !RES || Cfg::WGS_PER_CU != 1 || Cfg::THREADS > 512 ? 0 : STEPS < 6 ? STEPS : 6;
+    constexpr int PRE1 = PRE > 0 ? PRE : 1;
 
     struct Frags {
         half8_t a[MB], b[NB];
@@ -210,6 +231,21 @@ __device__ __forceinline__ void ws_consumer(const SpmmLaunchArgs& a, uint32_t ld
             rid[q] = a.row_ids ? a.row_ids[panel * V + r] : panel * V + r;
         }
 
+        // ---- the pieces of C of epilogue step `st` (in the order the epilogue below takes them)
+        half8_t cpre[PRE > 0 ? PRE : 1][2];
+        auto load_c = [&](int st) __attribute__((always_inline)) {
+            const int nbs = LINES ? NB / 2 : NB, hhs = LINES ? 2 : 32 / ER;
+            const int mb = st / (nbs * hhs), in = st % (nbs * hhs);
+            const int np = LINES ? in / hhs : in % nbs, hh = LINES ? in % hhs : in / nbs;
+            const int col = n0 + cw * WN + (LINES ? np * 64 + (lane & 7) * 8 : np * 32 + (lane % PR) * 8);
+#pragma unroll
+            for (int it = 0; it < CIT; it++) {
+                const int rr = mb * 32 + (LINES ? hh * 16 + it * 8 + (lane >> 3) : hh * ER + it * RPS + lane / PR);
+                const size_t roff = (size_t)__shfl(rid[rr >> 6], rr & 63) * a.ldd;
+                if (col < N) cpre[st % PRE1][it] = *(const half8_t*)(a.C + roff + col);
+            }
+        };
+
         auto mma = [&](const Frags& f) __attribute__((always_inline)) {
 #pragma unroll
             for (int mb = 0; mb < MB; mb++)
@@ -250,47 +286,49 @@ __device__ __forceinline__ void ws_consumer(const SpmmLaunchArgs& a, uint32_t ld
             load_frags(sb, 0, f0);
             primed = true;
         }
-        if (KSPS == 1) {
-            int s = 0;
-            for (; s + 1 < ntl; s += 2) {
-                stage(f0, f1);
+        // n pairs of k16 steps
+        auto pairs = [&](int n) __attribute__((always_inline)) {
+            for (int p = 0; p < n; p++) {
+                if (KSPS == 1) {
+                    stage(f0, f1);
+                } else {
+                    // two k16 steps per LDS stage: the odd step's fragments come from the stage already
+                    // present, only the step into the next stage passes a barrier.  A tile with an odd
+                    // number of steps computes one padded step (zero A values).
+                    load_frags(sb, 1, f1);
+                    mma(f0);
+                    interleave_reads();
+                }
                 stage(f1, f0);
             }
-            if (s < ntl) {
-                stage(f0, f1);
-                f0 = f1;
+        };
+        const int npairs = KSPS == 1 ? ntl >> 1 : (ntl + 1) >> 1;
+        if constexpr (PRE > 0) {
+            const int per = npairs / (PRE + 1);
+#pragma unroll
+            for (int st = 0; st < PRE; st++) {
+                pairs(per);
+                load_c(st);
             }
+            pairs(npairs - PRE * per);
         } else {
-            // two k16 steps per LDS stage: the odd step's fragments come from the stage already
-            // present, only the step into the next stage passes a barrier.  A tile with an odd
-            // number of steps computes one padded step (zero A values).
-            for (int p = 0; p < (ntl + 1) >> 1; p++) {
-                load_frags(sb, 1, f1);
-                mma(f0);
-                interleave_reads();
-                stage(f1, f0);
-            }
+            pairs(npairs);
+        }
+        if (KSPS == 1 && (ntl & 1)) {
+            stage(f0, f1);
+            f0 = f1;
         }
 
         // ---- epilogue of this wave's V x WN sub-tile, one 32 x 32 accumulator block at a time:
         // fp16 (one rounding) -> private LDS area (a lane holds 4 consecutive columns of one row
         // per 8-byte write) -> 16-byte pieces of 64-byte row segments -> scattered rows of D.  The
         // staging area is small on purpose: the LDS belongs to the stage ring.
-        constexpr int PR = 4;                 // 16-byte pieces per 32-column row segment
-        constexpr int RPS = 64 / PR;          // rows per store instruction
-        constexpr int ER = Cfg::EPI_ROWS;     // rows staged at a time: 32 (whole block) or 16 (half, by lanes)
-        constexpr int NIT = ER / RPS;
         const int pc = lane % PR;
         const int col0 = n0 + cw * WN + pc * 8;
         const uint32_t wr = epi + (lane & (ER - 1)) * Cfg::EPI_ROWB + (lane >> 5) * 8;
         const uint32_t rd = epi + (lane / PR) * Cfg::EPI_ROWB + pc * 16;
         // specialised on "alpha == 1" and "beta == 0" so that the common path has no branch (a
         // branch per piece would put a full wait at every join)
-        // Whole lines: with an even number of 32-column blocks, 16 rows of two neighbouring blocks are staged at a time
-        // (rows of 128 bytes + 16) and eight lanes store one 128-byte line of a row: half as many write requests to the
-        // L2s as with 64-byte row segments (cfg1 -2 %, 11 % at N = 16384, where every epilogue runs beside other
-        // workgroups' gathers).  Not where two workgroups share a compute unit (128 registers per wave: it spills).
-        constexpr bool LINES = SHFLBW_EPI_LINES && NB % 2 == 0 && 16 * (128 + 16) <= Cfg::EPI_WAVE_BYTES && Cfg::WGS_PER_CU == 1;
         constexpr int LROWB = 128 + 16;
         const uint32_t wrl = epi + (lane & 15) * LROWB + (lane >> 5) * 8;
         const uint32_t rdl = epi + (lane >> 3) * LROWB + (lane & 7) * 16;
@@ -334,14 +372,23 @@ __device__ __forceinline__ void ws_consumer(const SpmmLaunchArgs& a, uint32_t ld
                     if (DMAP) keep = keep && output_column(a, col);
                     if (keep) {
                         if (ADDC) {
+                            const int st = (mb * (NB / 2) + np) * 2 + hh;
+                            if (PRE == 0) {
 #pragma unroll
-                            for (int it = 0; it < 2; it++) c[it] = *(const half8_t*)(a.C + roff[it] + col);
+                                for (int it = 0; it < 2; it++) c[it] = *(const half8_t*)(a.C + roff[it] + col);
+                            }
 #pragma unroll
                             for (int it = 0; it < 2; it++)
 #pragma unroll
                                 for (int e = 0; e < 8; e++)
-                                    v[it][e] = (half_t)((float)v[it][e] + beta * (float)c[it][e]);
+                                    v[it][e] = (half_t)((float)v[it][e] + beta * (float)(PRE ? cpre[st % PRE1] : c)[it][e]);
                         }
+                    }
+                    if constexpr (PRE > 0) {
+                        const int st = (mb * (NB / 2) + np) * 2 + hh;
+                        if (st + PRE < STEPS) load_c(st + PRE);
+                    }
+                    if (keep) {
 #pragma unroll
                         for (int it = 0; it < 2; it++) store_result_16B<!XCD_LOCAL>(a.D + roff[it] + col, v[it]);
                     }
@@ -389,14 +436,23 @@ __device__ __forceinline__ void ws_consumer(const SpmmLaunchArgs& a, uint32_t ld
                     if (DMAP) keep = keep && output_column(a, col);
                     if (keep) {
                         if (ADDC) {
+                            const int st = (mb * (32 / ER) + hh) * NB + nb;
+                            if (PRE == 0) {
 #pragma unroll
-                            for (int it = 0; it < NIT; it++) c[it] = *(const half8_t*)(a.C + roff[it] + col);
+                                for (int it = 0; it < NIT; it++) c[it] = *(const half8_t*)(a.C + roff[it] + col);
+                            }
 #pragma unroll
                             for (int it = 0; it < NIT; it++)
 #pragma unroll
                                 for (int e = 0; e < 8; e++)
-                                    v[it][e] = (half_t)((float)v[it][e] + beta * (float)c[it][e]);
+                                    v[it][e] = (half_t)((float)v[it][e] + beta * (float)(PRE ? cpre[st % PRE1] : c)[it][e]);
                         }
+                    }
+                    if constexpr (PRE > 0) {
+                        const int st = (mb * (32 / ER) + hh) * NB + nb;
+                        if (st + PRE < STEPS) load_c(st + PRE);
+                    }
+                    if (keep) {
 #pragma unroll
                         for (int it = 0; it < NIT; it++) store_result_16B<!XCD_LOCAL>(a.D + roff[it] + col, v[it]);
                     }
@@ -411,15 +467,15 @@ __device__ __forceinline__ void ws_consumer(const SpmmLaunchArgs& a, uint32_t ld
         using T = std::true_type;
         using F = std::false_type;
         // one straight-line sequence over all 32-row blocks per specialisation
-        if (beta == 0.f && alpha == 1.f) {
-#pragma unroll
-            for (int mb = 0; mb < MB; mb++) epi_block(mb, F{}, F{});
-        } else if (beta == 0.f) {
-#pragma unroll
-            for (int mb = 0; mb < MB; mb++) epi_block(mb, T{}, F{});
-        } else {
+        if constexpr (RES) {
 #pragma unroll
             for (int mb = 0; mb < MB; mb++) epi_block(mb, T{}, T{});
+        } else if (alpha == 1.f) {
+#pragma unroll
+            for (int mb = 0; mb < MB; mb++) epi_block(mb, F{}, F{});
+        } else {
+#pragma unroll
+            for (int mb = 0; mb < MB; mb++) epi_block(mb, T{}, F{});
         }
     }
 }
@@ -427,7 +483,7 @@ __device__ __forceinline__ void ws_consumer(const SpmmLaunchArgs& a, uint32_t ld
 // Consumer role for block height 16: 16x16x32 tiles, one 32-slot step per LDS stage, same barrier
 // protocol and ring as ws_consumer.  Wave `cw` owns the 16 x WN sub-tile at column cw*WN.  A lane of
 // the result holds output row lane % 16 and, per 16-column block, the 4 columns 4*(lane/16) + 0..3.
-template <typename Cfg, int WN, int NCONS, bool XCD_LOCAL = false, bool DMAP = false>
+template <typename Cfg, int WN, int NCONS, bool XCD_LOCAL = false, bool DMAP = false, bool RES = false>
 __device__ __forceinline__ void ws_consumer16(const SpmmLaunchArgs& a, uint32_t lds0, int lane, int cw, int id_first,
                                               int id_end, int S)
 {
@@ -495,12 +551,29 @@ __device__ __forceinline__ void ws_consumer16(const SpmmLaunchArgs& a, uint32_t 
             load_frags(sb, f0);
             primed = true;
         }
-        int s = 0;
-        for (; s + 1 < ntl; s += 2) {
-            stage(f0, f1);
-            stage(f1, f0);
+        auto pairs = [&](int n) __attribute__((always_inline)) {
+            for (int p = 0; p < n; p++) {
+                stage(f0, f1);
+                stage(f1, f0);
+            }
+        };
+        // the pieces of C, loaded half way through the tile's stages (as ws_consumer does)
+        half8_t c[WN / 64][2];
+        if constexpr (RES) {
+            pairs(ntl >> 2);
+#pragma unroll
+            for (int h = 0; h < WN / 64; h++)
+#pragma unroll
+                for (int it = 0; it < 2; it++) {
+                    const int col = n0 + cw * WN + h * 64 + (lane & 7) * 8;
+                    const size_t roff = (size_t)__shfl(orow, it * 8 + (lane >> 3)) * a.ldd;
+                    if (col < N) c[h][it] = *(const half8_t*)(a.C + roff + col);
+                }
+            pairs((ntl >> 1) - (ntl >> 2));
+        } else {
+            pairs(ntl >> 1);
         }
-        if (s < ntl) {
+        if (ntl & 1) {
             stage(f0, f1);
             f0 = f1;
         }
@@ -520,7 +593,7 @@ __device__ __forceinline__ void ws_consumer16(const SpmmLaunchArgs& a, uint32_t 
             for (int q = 0; q < 4; q++) {
                 half4_t hv;
 #pragma unroll
-                for (int e = 0; e < 4; e++) hv[e] = (half_t)scaled(acc[h * 4 + q][e], alpha, beta != 0.f);
+                for (int e = 0; e < 4; e++) hv[e] = (half_t)scaled(acc[h * 4 + q][e], alpha, RES);
                 *(SHFLBW_LDS half4_t*)(uintptr_t)(wr + q * 32) = hv;
             }
             half8_t v[2];
@@ -530,14 +603,11 @@ __device__ __forceinline__ void ws_consumer16(const SpmmLaunchArgs& a, uint32_t 
             bool keep = col < N;
             if (DMAP) keep = keep && output_column(a, col);
             if (keep) {
-                if (beta != 0.f) {
-                    half8_t c[2];
-#pragma unroll
-                    for (int it = 0; it < 2; it++) c[it] = *(const half8_t*)(a.C + roff[it] + col);
+                if (RES) {
 #pragma unroll
                     for (int it = 0; it < 2; it++)
 #pragma unroll
-                        for (int e = 0; e < 8; e++) v[it][e] = (half_t)((float)v[it][e] + beta * (float)c[it][e]);
+                        for (int e = 0; e < 8; e++) v[it][e] = (half_t)((float)v[it][e] + beta * (float)c[h][it][e]);
                 }
 #pragma unroll
                 for (int it = 0; it < 2; it++) store_result_16B<!XCD_LOCAL>(a.D + roff[it] + col, v[it]);
