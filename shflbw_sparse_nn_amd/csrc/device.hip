@@ -133,8 +133,10 @@ static const SpconvVariant* find_spconv_variant(int brow, int variant, int* n_fo
     return hit;
 }
 
-// the persistent role-split variants ("ws..." names) form gather addresses from 32-bit byte offsets
-static bool spmm_variant_offsets32(const SpmmVariant* v) { return v && v->name[0] == 'w'; }
+static bool spmm_variant_splits(const SpmmVariant* v) { return v && strncmp(v->name, "split", 5) == 0; }
+// the persistent role-split variants ("ws..." names) form gather addresses from 32-bit byte offsets; the split form is for
+// few columns and holds to the same bound
+static bool spmm_variant_offsets32(const SpmmVariant* v) { return v && (v->name[0] == 'w' || spmm_variant_splits(v)); }
 
 // Tile choice when the caller does not force one: the table lists the preferred (persistent, 512 columns
 // wide) variant of every block size first.  When its tiles would occupy at most half of the compute units,
@@ -152,7 +154,7 @@ static bool spmm_variant_offsets32(const SpmmVariant* v) { return v && v->name[0
 //    at the same time and share it in their L2 (16 tiles: 15 % slower).
 // Inside these bounds: equal to 28 % faster (M = 4096, K = 1024, N = 4096, density 0.2: 15.1 against 16.5 us;
 // M = 8192, density 0.3: 31.3 against 38.7 us).
-static int auto_spmm_variant(const shflbw_weight* w, int N, bool allow_slab)
+static int auto_gather_variant(const shflbw_weight* w, int N, bool allow_slab, int compute_units)
 {
     const int brow = w->brow, X = w->nrow / w->brow;
     int count = 0;
@@ -162,7 +164,7 @@ static int auto_spmm_variant(const shflbw_weight* w, int N, bool allow_slab)
         for (int i = 0; i < count; i++) {
             if (all[i].V != brow) continue;
             if (all[i].max_k >= w->ncol) {
-                const int cus = (device_compute_units() / 8) * 8;
+                const int cus = (compute_units / 8) * 8;
                 const int n_tiles = (N + all[i].BN - 1) / all[i].BN;
                 const int chunks = std::max(1, std::min(X, cus / n_tiles)); // as the launcher deals the panels
                 const double panels_per_wg = (double)X / chunks;
@@ -184,16 +186,50 @@ static int auto_spmm_variant(const shflbw_weight* w, int N, bool allow_slab)
     };
     // small problems: 128-column tiles while they do not outnumber the compute units (39 shapes of block heights 32, 64
     // and 128 measured against the wider tiles: 6-17 % faster up to one tile per compute unit, 10-25 % slower from two on)
-    if ((long)X * ((N + 127) / 128) <= device_compute_units()) {
+    if ((long)X * ((N + 127) / 128) <= compute_units) {
         const int narrow = role_split_with(128);
         if (narrow >= 0) return narrow;
     }
     const SpmmVariant* first = find_spmm_variant(brow, 0, nullptr);
     if (!first || first->BN != 512) return 0;
     const long wide_tiles = (long)X * ((N + 511) / 512);
-    if (wide_tiles > device_compute_units() / 2) return 0;
+    if (wide_tiles > compute_units / 2) return 0;
     const int medium = role_split_with(256);
     return medium >= 0 ? medium : 0;
+}
+
+// Few columns: the split form (its waves split the kept vectors) where it is estimated to be at least a tenth faster than the
+// variant above.  Both estimates are us, fitted to 4 block heights x 7 weights x 6 widths from 8 to 512 columns:
+//  split: 4 + rounds * (0.6 + 0.03 * steps) with 32-column tiles (0.04 for block height 16), (0.9 + 0.052 * steps) with 64;
+//    rounds = workgroups per compute unit, steps of 16 kept vectors (32 for block height 16);
+//  above: 3.6 + rounds * (0.3 + 0.2 * stages) with 128-column tiles, (1.35 + 0.22 * stages) with wider ones for block height 32,
+//    1.7 from 64, (0.85 + 0.27 * stages) for 16; stages of 32 kept vectors.
+// 2048 x 8192, density 0.5, 8 columns: 8.1-10 us split, 30-37 us above; 8192 x 4096, density 0.3: 6.8 and 11.6-26; 4096 x 4096,
+// density 0.1: 5.1-5.4 and 6.2-7.4, with 256 columns 7.0 and 6.4; 16384 x 1024, density 0.1, block height 64, 64 columns: 5.7 and 4.7.
+static int auto_spmm_variant(const shflbw_weight* w, int N, bool spmm, int compute_units)
+{
+    const int general = auto_gather_variant(w, N, spmm, compute_units);
+    const int X = w->nrow / w->brow;
+    if (!spmm || N > 512 || X <= 0) return general;
+    int split = 0; // the split form is the last variant of its block height
+    find_spmm_variant(w->brow, 0, &split);
+    split--;
+    const SpmmVariant* g = find_spmm_variant(w->brow, general, nullptr);
+    if (!g || !spmm_variant_splits(find_spmm_variant(w->brow, split, nullptr))) return general;
+    const double cus = compute_units, vectors = (double)w->nnzb / X;
+    const bool v16 = w->brow == 16;
+    auto rounds = [cus](double workgroups) {
+        const double r = workgroups / cus;
+        return r <= 1 ? 1 : r <= 2 ? 2 : r;
+    };
+    const double edge = g->BN <= 128 ? 0.3 : v16 ? 0.85 : w->brow == 32 ? 1.35 : 1.7;
+    const double stage = g->BN <= 128 ? 0.2 : v16 ? 0.27 : 0.22;
+    const double t_general = 3.6 + rounds(X * (double)((N + g->BN - 1) / g->BN)) * (edge + stage * vectors / 32);
+    const double blocks = w->nrow / (v16 ? 16.0 : 32.0), narrow = blocks * ((N + 31) / 32);
+    const double steps = vectors / (v16 ? 32 : 16);
+    const double t_split = v16 || N <= 32 || narrow <= cus ? 4 + rounds(narrow) * (0.6 + (v16 ? 0.04 : 0.03) * steps)
+                                                           : 4 + rounds(blocks * ((N + 63) / 64)) * (0.9 + 0.052 * steps);
+    return t_split < 0.9 * t_general ? split : general;
 }
 
 // Geometry of the plane form of a convolution and the layout of its device scratch.
@@ -320,11 +356,11 @@ static int spmm_init_impl(shflbw_spmm_state* state, const shflbw_weight* w, int 
         set_error("spmm_init: B, C and D must be 16-byte aligned");
         return SHFLBW_ERR_INVALID;
     }
-    const int X = w->nrow / w->brow;
+    const int X = w->nrow / w->brow, compute_units = device_compute_units();
     // the role-split kernels address the rows of B with 32-bit byte offsets
     const bool wide_b = (unsigned long long)w->ncol * (unsigned long long)N * 2ull + (unsigned long long)N * 2ull > 0xffffffffull;
     if (variant < 0) {
-        variant = auto_spmm_variant(w, N, !gather_only);
+        variant = auto_spmm_variant(w, N, !gather_only, compute_units);
         if (wide_b) { // first variant of this block size with 64-bit addressing
             int n = 0;
             find_spmm_variant(w->brow, 0, &n);
@@ -353,7 +389,9 @@ static int spmm_init_impl(shflbw_spmm_state* state, const shflbw_weight* w, int 
         set_error("spmm_init: B (%d x %d fp16) exceeds the 4 GiB the tile variant %s can address", w->ncol, N, v->name);
         return SHFLBW_ERR_UNSUPPORTED;
     }
-    SHFLBW_HIP_TRY(v->prepare());
+    SpmmLaunchArgs la;
+    la.M = w->nrow, la.N = N, la.X = X, la.beta = beta, la.num_cus = compute_units;
+    SHFLBW_HIP_TRY(v->prepare(la));
 
     shflbw_device_ref ref;
     shflbw_weight_device_ref(w, &ref);

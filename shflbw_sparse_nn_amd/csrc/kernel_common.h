@@ -76,6 +76,15 @@ __device__ __forceinline__ void global_to_lds_16B_sbase(const void* sbase, uint3
                  : "m0", "scc");
 }
 
+// the same copy with 4 bytes per lane: 256 bytes of consecutive LDS
+__device__ __forceinline__ void global_to_lds_4B(const void* gptr, uint32_t lds_base)
+{
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off"
+                 :
+                 : "v"(gptr), "s"(lds_base)
+                 : "m0");
+}
+
 // s_waitcnt on the vector-memory counter that the compiler also treats as a memory fence, for
 // waits that publish LDS contents written by copies the compiler does not know about
 template <int N>

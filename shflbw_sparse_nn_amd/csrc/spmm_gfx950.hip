@@ -23,6 +23,7 @@
 #include "spmm_launch.h"
 #include <algorithm>
 #include "spmm_slab.h"
+#include "spmm_split.h"
 #include "spmm_ws.h"
 
 namespace shflbw {
@@ -318,14 +319,12 @@ static hipError_t launch_ws(const SpmmLaunchArgs& a, hipStream_t stream)
 }
 
 template <int V, int WN, int NCONS, int NPROD, int KT, int NSTAGE>
-static hipError_t prepare_ws()
+static hipError_t prepare_ws(const SpmmLaunchArgs& a)
 {
     using Cfg = SpmmWsCfg<V, WN, NCONS, NPROD, KT, NSTAGE>;
-    const hipError_t e = hipFuncSetAttribute((const void*)spmm_shflbw_ws_kernel<V, WN, NCONS, NPROD, KT, NSTAGE, false>,
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS_BYTES);
-    if (e != hipSuccess) return e;
-    return hipFuncSetAttribute((const void*)spmm_shflbw_ws_kernel<V, WN, NCONS, NPROD, KT, NSTAGE, true>,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS_BYTES);
+    const void* f = a.beta != 0.f ? (const void*)spmm_shflbw_ws_kernel<V, WN, NCONS, NPROD, KT, NSTAGE, true>
+                                  : (const void*)spmm_shflbw_ws_kernel<V, WN, NCONS, NPROD, KT, NSTAGE, false>;
+    return hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS_BYTES);
 }
 
 #define SHFLBW_WS_VARIANT(V, WN, NC, NP, KT, NS)                                                             \
@@ -355,7 +354,7 @@ static hipError_t launch_slab(const SpmmLaunchArgs& a, hipStream_t stream)
     return hipGetLastError();
 }
 
-static hipError_t prepare_slab()
+static hipError_t prepare_slab(const SpmmLaunchArgs&)
 {
     return hipFuncSetAttribute((const void*)spmm_shflbw_slab_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                                SpmmSlabCfg::LDS_MAX);
@@ -365,6 +364,14 @@ static hipError_t prepare_slab()
     {                                                                                                             \
         SpmmSlabCfg::V, SpmmSlabCfg::BN, SpmmSlabCfg::THREADS, SpmmSlabCfg::LDS_MAX, "slab32x64", &launch_slab,    \
             &prepare_slab, SpmmSlabCfg::MAX_K                                                                     \
+    }
+
+// split form (few columns; the waves of a workgroup split the kept vectors)
+#define SHFLBW_SPLIT_VARIANT(V)                                                                               \
+    {                                                                                                         \
+        V, SpmmSplitCfg<V == 16, 1>::BN, SpmmSplitCfg<V == 16, 1>::MAX_WAVES * 64,                              \
+            SpmmSplitCfg<V == 16, 1>::lds_bytes(SpmmSplitCfg<V == 16, 1>::MAX_WAVES), "split" #V "x32",          \
+            &launch_split<V == 16>, &prepare_split<V == 16>                                                    \
     }
 
 // ---------------------------------------------------------------------------------------
@@ -383,7 +390,7 @@ static hipError_t launch_variant(const SpmmLaunchArgs& a, hipStream_t stream)
 }
 
 template <int V, int WN, int NWAVES, int KT, int NSTAGE>
-static hipError_t prepare_variant()
+static hipError_t prepare_variant(const SpmmLaunchArgs&)
 {
     using Cfg = SpmmCfg<V, WN, NWAVES, KT, NSTAGE>;
     return hipFuncSetAttribute((const void*)spmm_shflbw_kernel<V, WN, NWAVES, KT, NSTAGE>,
@@ -414,6 +421,7 @@ static const SpmmVariant g_variants[] = {
     SHFLBW_VARIANT(64, 64, 2, 32, 3),
     SHFLBW_VARIANT(64, 32, 4, 32, 3),
     SHFLBW_WS_VARIANT(64, 32, 4, 4, 32, 6), // 128-column tiles: problems too small for the wider ones
+    SHFLBW_SPLIT_VARIANT(64), // few columns
     // block 32
     SHFLBW_WS_VARIANT(32, 128, 4, 4, 32, 4),
     SHFLBW_WS_VARIANT(32, 128, 4, 4, 16, 6),
@@ -425,14 +433,17 @@ static const SpmmVariant g_variants[] = {
     SHFLBW_VARIANT(32, 64, 2, 32, 3),
     SHFLBW_SLAB_VARIANT(), // weights of at most SLAB_MAX_K columns
     SHFLBW_WS_VARIANT(32, 32, 4, 4, 32, 6), // 128-column tiles: problems too small for the wider ones
+    SHFLBW_SPLIT_VARIANT(32), // few columns
     // block 16
     SHFLBW_WS_VARIANT(16, 128, 4, 4, 32, 4),
+    SHFLBW_SPLIT_VARIANT(16), // few columns
     // block 128
     SHFLBW_WS_VARIANT(128, 64, 4, 4, 32, 6),
     SHFLBW_WS_VARIANT(128, 64, 4, 4, 32, 5),
     SHFLBW_VARIANT(128, 64, 4, 32, 3),
     SHFLBW_VARIANT(128, 32, 4, 32, 3),
     SHFLBW_WS_VARIANT(128, 32, 4, 4, 32, 6), // 128-column tiles: problems too small for the wider ones
+    SHFLBW_SPLIT_VARIANT(128), // few columns
 };
 
 // The row of zeros the padding slots gather.  `g_zero_row` is the host-side handle of the symbol; kernels get
