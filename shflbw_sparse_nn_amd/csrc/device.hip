@@ -154,12 +154,21 @@ static bool spmm_variant_offsets32(const SpmmVariant* v) { return v && (v->name[
 //    at the same time and share it in their L2 (16 tiles: 15 % slower).
 // Inside these bounds: equal to 28 % faster (M = 4096, K = 1024, N = 4096, density 0.2: 15.1 against 16.5 us;
 // M = 8192, density 0.3: 31.3 against 38.7 us).
+// Block height 16 has no narrower tiles than 512 columns beside it and gathers twice as much per product: there the slab
+// variant is taken from 128 columns on (below, the split form) when (192 shapes)
+//  * a workgroup runs at least 24 panels (32 to 132: 1.0-1.9 times as fast) with at least one kept vector per column of A, or 16 panels
+//    with 2.5 (18 panels: 0.9 at 0.6 vectors, 1.2 at 5.5; 6 to 9 panels: 0.6-1.1), four where a fifth of the compute units would have
+//    no job (3.2: 8 % slower, 6.4: 5 % faster),
+//  * panels keep at least 32 vectors, or D is below 100 MB: with less to do per panel both wait for the stores of D, and the
+//    wider row segments of the role-split kernel are 5-15 % ahead (33728 x 96 x 2048: 40 against 47 us) where rows of D start at
+//    whole lines (15760 x 127 x 3864: 31 against 41 us).
+// 33728 x 777 x 1000, density 0.1: 31 against 38 us; 8192 x 384 x 4096: 20 against 29 us; 33728 x 1128 x 136, 0.2: 17 and 31 us.
 static int auto_gather_variant(const shflbw_weight* w, int N, bool allow_slab, int compute_units)
 {
     const int brow = w->brow, X = w->nrow / w->brow;
     int count = 0;
     const SpmmVariant* all = spmm_variants(&count);
-    if (allow_slab && brow == 32 && !w->packed_slab.empty() && w->ncol >= 384 && X > 0) {
+    if (allow_slab && !w->packed_slab.empty() && X > 0 && (brow == 16 ? N >= 128 : w->ncol >= 384)) {
         int seen = 0;
         for (int i = 0; i < count; i++) {
             if (all[i].V != brow) continue;
@@ -169,7 +178,11 @@ static int auto_gather_variant(const shflbw_weight* w, int N, bool allow_slab, i
                 const int chunks = std::max(1, std::min(X, cus / n_tiles)); // as the launcher deals the panels
                 const double panels_per_wg = (double)X / chunks;
                 const double vectors_per_column = panels_per_wg * w->nnzb / ((double)X * w->ncol);
-                if (vectors_per_column >= 3.0 && n_tiles >= 32) return seen;
+                const double vectors = (double)w->nnzb / X;
+                if (brow == 16 ? panels_per_wg >= 16 && vectors_per_column >= (n_tiles * chunks < 0.8 * cus ? 4.0 : panels_per_wg < 24 ? 2.5 : 1.0) &&
+                                     (vectors >= 32 || 2.0 * w->nrow * N <= 100e6 || N % 64 != 0)
+                               : vectors_per_column >= 3.0 && n_tiles >= 32)
+                    return seen;
             }
             seen++;
         }
@@ -215,7 +228,7 @@ static int auto_spmm_variant(const shflbw_weight* w, int N, bool spmm, int compu
     find_spmm_variant(w->brow, 0, &split);
     split--;
     const SpmmVariant* g = find_spmm_variant(w->brow, general, nullptr);
-    if (!g || !spmm_variant_splits(find_spmm_variant(w->brow, split, nullptr))) return general;
+    if (!g || g->max_k > 0 || !spmm_variant_splits(find_spmm_variant(w->brow, split, nullptr))) return general;
     const double cus = compute_units, vectors = (double)w->nnzb / X;
     const bool v16 = w->brow == 16;
     auto rounds = [cus](double workgroups) {

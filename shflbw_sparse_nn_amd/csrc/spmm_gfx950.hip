@@ -337,9 +337,10 @@ static hipError_t prepare_ws(const SpmmLaunchArgs& a)
 // ---------------------------------------------------------------------------------------
 // slab form (all rows of a 64-column slab of B in LDS): launcher
 // ---------------------------------------------------------------------------------------
+template <int V>
 static hipError_t launch_slab(const SpmmLaunchArgs& a, hipStream_t stream)
 {
-    using Cfg = SpmmSlabCfg;
+    using Cfg = SpmmSlabCfg<V>;
     if (a.K > Cfg::MAX_K || !a.slab_ids || a.K <= 0) return hipErrorInvalidValue;
     SpmmLaunchArgs b = a;
     b.n_tiles = (a.N + Cfg::BN - 1) / Cfg::BN;
@@ -350,20 +351,21 @@ static hipError_t launch_slab(const SpmmLaunchArgs& a, hipStream_t stream)
     b.slab_chunks = std::max(1, std::min(a.X, std::max(cus / b.n_tiles, (a.M + rows_per_wg - 1) / rows_per_wg)));
     const int T = b.n_tiles * b.slab_chunks;
     const int grid = std::min(cus, ((T + 7) / 8) * 8);
-    hipLaunchKernelGGL(spmm_shflbw_slab_kernel, dim3(grid), dim3(Cfg::THREADS), Cfg::lds_bytes(a.K), stream, b);
+    hipLaunchKernelGGL((spmm_shflbw_slab_kernel<V>), dim3(grid), dim3(Cfg::THREADS), Cfg::lds_bytes(a.K), stream, b);
     return hipGetLastError();
 }
 
+template <int V>
 static hipError_t prepare_slab(const SpmmLaunchArgs&)
 {
-    return hipFuncSetAttribute((const void*)spmm_shflbw_slab_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               SpmmSlabCfg::LDS_MAX);
+    return hipFuncSetAttribute((const void*)spmm_shflbw_slab_kernel<V>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               SpmmSlabCfg<V>::LDS_MAX);
 }
 
-#define SHFLBW_SLAB_VARIANT()                                                                                     \
+#define SHFLBW_SLAB_VARIANT(V)                                                                                    \
     {                                                                                                             \
-        SpmmSlabCfg::V, SpmmSlabCfg::BN, SpmmSlabCfg::THREADS, SpmmSlabCfg::LDS_MAX, "slab32x64", &launch_slab,    \
-            &prepare_slab, SpmmSlabCfg::MAX_K                                                                     \
+        V, SpmmSlabCfg<V>::BN, SpmmSlabCfg<V>::THREADS, SpmmSlabCfg<V>::LDS_MAX, "slab" #V "x64", &launch_slab<V>,  \
+            &prepare_slab<V>, SpmmSlabCfg<V>::MAX_K                                                               \
     }
 
 // split form (few columns; the waves of a workgroup split the kept vectors)
@@ -431,11 +433,12 @@ static const SpmmVariant g_variants[] = {
     SHFLBW_VARIANT(32, 128, 2, 32, 3),
     SHFLBW_VARIANT(32, 128, 4, 16, 3),
     SHFLBW_VARIANT(32, 64, 2, 32, 3),
-    SHFLBW_SLAB_VARIANT(), // weights of at most SLAB_MAX_K columns
+    SHFLBW_SLAB_VARIANT(32), // weights of at most SLAB_MAX_K columns
     SHFLBW_WS_VARIANT(32, 32, 4, 4, 32, 6), // 128-column tiles: problems too small for the wider ones
     SHFLBW_SPLIT_VARIANT(32), // few columns
     // block 16
     SHFLBW_WS_VARIANT(16, 128, 4, 4, 32, 4),
+    SHFLBW_SLAB_VARIANT(16), // weights of at most SLAB_MAX_K columns
     SHFLBW_SPLIT_VARIANT(16), // few columns
     // block 128
     SHFLBW_WS_VARIANT(128, 64, 4, 4, 32, 6),

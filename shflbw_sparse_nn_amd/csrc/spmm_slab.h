@@ -1,4 +1,4 @@
-// Slab form of the SpMM for block height 32 and weights with few columns (K <= SLAB_MAX_K): a workgroup copies
+// Slab form of the SpMM for block heights 32 and 16 and weights with few columns (K <= SLAB_MAX_K): a workgroup copies
 // all K rows of a 64-column slab of B into LDS once and then runs many row panels over it, so a row of B crosses
 // the path from the L2 to the compute unit once per workgroup instead of once per panel that keeps it.  What
 // streams instead are the A fragments (64 bytes per kept vector, straight into registers) and the kept-column
@@ -12,22 +12,31 @@
 // offsets name (transposing reads; the 32-byte units of row r are XOR-ed with (r / 2) % 4, and the host orders a
 // panel's vectors so that the four rows one read touches lie in different bank groups) and issues two MFMAs.
 // A panel's 32 x 64 result goes through the wave's private staging area to D like in the role-split kernel.
+// Block height 16 (one 16x16x32 step of 32 slots per batch): a gathered value feeds only 16 MACs in the role-split kernel,
+// which is bound by the path from the L2 there (33728 x 777 x 1000, density 0.1: 329 MB of gathers for 67 MB of result,
+// 38 us; here 31, and 20 instead of 29 us at 8192 x 384 x 4096).
 #pragma once
+#include <type_traits>
+
 #include "kernel_common.h"
 #include "spmm_launch.h"
 #include "weight_internal.h"
 
 namespace shflbw {
 
+template <int V_>
 struct SpmmSlabCfg {
-    static constexpr int V = 32;
+    static constexpr int V = V_;
+    static constexpr bool V16 = V == 16;
+    static constexpr int NA = V16 ? 1 : 2;   // A fragments, and MFMA steps, per batch of 32 slots
     static constexpr int BN = 64;            // columns of the slab
     static constexpr int ROWB = BN * 2;      // bytes of a slab row
     static constexpr int NW = 8;             // waves of a workgroup
     static constexpr int THREADS = NW * 64;
-    static constexpr int NB = BN / 32;
+    static constexpr int NB = V16 ? BN / 16 : BN / 32; // accumulator blocks
     static constexpr int NBUF = 8;           // batches a wave keeps in flight (even: the fragment sets alternate)
-    static constexpr int FETCH_OPS = 3;      // loads per batch: two A fragments and a quad of offsets
+    static constexpr int FETCH_OPS = NA + 1; // loads per batch: A fragments and the offsets of a lane's slots
+    static constexpr int PANEL_PASSES = V / 16;           // 16 rows of a panel's result are staged at a time
     static constexpr int RID_REGS = 8;       // a wave's panels have at most RID_REGS * 64 rows
     static constexpr int EPI_ROWB = BN * 2 + 16;          // a staged row: all 64 columns and 16 bytes of padding
     static constexpr int EPI_WAVE_BYTES = 16 * EPI_ROWB;  // 16 rows at a time
@@ -39,9 +48,12 @@ struct SpmmSlabCfg {
     static constexpr int lds_bytes(int K) { return (((K + 7) & ~7) + 1) * ROWB + NW * EPI_WAVE_BYTES; }
 };
 
-__global__ void __launch_bounds__(SpmmSlabCfg::THREADS) spmm_shflbw_slab_kernel(SpmmLaunchArgs a)
+template <int V_>
+__global__ void __launch_bounds__(SpmmSlabCfg<V_>::THREADS) spmm_shflbw_slab_kernel(SpmmLaunchArgs a)
 {
-    using Cfg = SpmmSlabCfg;
+    using Cfg = SpmmSlabCfg<V_>;
+    constexpr bool V16 = Cfg::V16;
+    constexpr int NA = Cfg::NA;
     constexpr int V = Cfg::V, NB = Cfg::NB, NBUF = Cfg::NBUF, ROWB = Cfg::ROWB, NW = Cfg::NW, BN = Cfg::BN;
     extern __shared__ __attribute__((aligned(1024))) char lds_raw[];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(SHFLBW_LDS char*)lds_raw;
@@ -60,24 +72,28 @@ __global__ void __launch_bounds__(SpmmSlabCfg::THREADS) spmm_shflbw_slab_kernel(
     const int job_end = min(T, (xcd + 1) * per);
 
     // lane constants of the transposing reads: a 16-lane group reads 4 rows x 32 bytes; lanes 16..31 the next
-    // 32 bytes, lanes 32..63 the rows of slots 8..15
+    // 32 bytes, lanes 32..63 the rows of slots 8..15 (block height 16: the four groups the same 32 bytes of the rows of
+    // slots 0.., 8.., 16.. and 24..)
     const int li = lane & 15;
-    const uint32_t lc = (uint32_t)((((lane >> 4) & 1) << 5) | ((li & 3) << 3));
+    const uint32_t lc = (uint32_t)((V16 ? 0 : ((lane >> 4) & 1) << 5) | ((li & 3) << 3));
     // which two slots (s, s + 4) of a step this lane addresses: pair number (lane / 32) * 4 + (lane % 16) / 4, 32 bytes
     // of offsets per pair and 64-slot group, 16 per batch
-    const uint32_t pair32 = (uint32_t)(((lane >> 5) * 4 + (li >> 2)) * 32);
+    const uint32_t pair32 = V16 ? (uint32_t)((((lane >> 4) & 1) * 4 + (li >> 2)) * 32 + (lane >> 5) * 8)
+                                : (uint32_t)(((lane >> 5) * 4 + (li >> 2)) * 32);
     const uint32_t lane16 = (uint32_t)lane * 16;
     // epilogue: a lane writes 4 columns (per 32-column block) of row lane % 16, reads 16-byte piece lane % 8 of row lane / 8
-    const uint32_t wr = epi + (lane & 15) * Cfg::EPI_ROWB + (lane >> 5) * 8;
+    const uint32_t wr = epi + (lane & 15) * Cfg::EPI_ROWB + (V16 ? lane >> 4 : lane >> 5) * 8;
     const uint32_t rd = epi + (lane >> 3) * Cfg::EPI_ROWB + (lane & 7) * 16;
     const float alpha = a.alpha, beta = a.beta;
 
+    using ids_t = typename std::conditional<V16, int2_t, int4_t>::type;
+    using acc_t = typename std::conditional<V16, float4_t, float16_t>::type;
     struct Batch {
-        half8_t a[2]; // A fragments of the two steps
-        int4_t i;     // slab offsets: {step 0: slot s, s + 4; step 1: slot s, s + 4}
+        half8_t a[NA]; // A fragments of the steps
+        ids_t i;       // slab offsets: {step 0: slot s, s + 4; step 1: slot s, s + 4}
     };
     struct Frags {
-        half8_t b[2][NB]; // B fragments of the two steps
+        half8_t b[NA][NB]; // B fragments of the steps
     };
 
     bool first = true;
@@ -116,18 +132,19 @@ __global__ void __launch_bounds__(SpmmSlabCfg::THREADS) spmm_shflbw_slab_kernel(
         }
 
         // ---- consumer side of the stream: panel p, n_left batches of it still to compute
-        float16_t acc[NB];
+        acc_t acc[NB];
         int p = pa, n_left = 0;
         auto open_panel = [&]() __attribute__((always_inline)) {
             n_left = (desc[p].x + 1) >> 1; // batches of two steps; an odd last step has zero weights behind it
 #pragma unroll
             for (int nb = 0; nb < NB; nb++)
 #pragma unroll
-                for (int i = 0; i < 16; i++) acc[nb][i] = 0.f;
+                for (int i = 0; i < (V16 ? 4 : 16); i++) acc[nb][i] = 0.f;
         };
         // fp32 -> fp16 (one rounding) -> staging area, 16 rows of all 64 columns at a time -> rows of D, eight lanes
-        // to a row: every store instruction writes whole 128-byte lines (half lines, written at different times,
-        // cost 1.4 x the bytes at the memory side with streaming stores)
+        // to a row: every store instruction writes whole 128-byte lines where N is a multiple of 64.  Elsewhere the ends of
+        // a row segment are half lines, which streaming stores bring to memory twice (8192 x 777 x 3000, block height 16,
+        // density 0.1: 32.5 us with them, 23.2 with ordinary stores, 22.5 with device scope; N = 4096: 24, 21 and 20)
         auto epilogue = [&]() __attribute__((always_inline)) {
             const int i0 = (p - pa) * V; // first row of the panel among the wave's rows
             int rid = ridreg[0];
@@ -135,20 +152,20 @@ __global__ void __launch_bounds__(SpmmSlabCfg::THREADS) spmm_shflbw_slab_kernel(
             for (int q = 1; q < Cfg::RID_REGS; q++) rid = (i0 >> 6) == q ? ridreg[q] : rid;
             const int col = n0 + (lane & 7) * 8;
 #pragma unroll
-            for (int hh = 0; hh < 2; hh++) { // rows 16 hh .. 16 hh + 15: held by the lanes with bit 4 equal to hh
+            for (int hh = 0; hh < Cfg::PANEL_PASSES; hh++) { // rows 16 hh .. 16 hh + 15: held by the lanes with bit 4 equal to hh
                 size_t roff[2];
 #pragma unroll
                 for (int it = 0; it < 2; it++)
                     roff[it] = (size_t)__shfl(rid, (i0 & 63) + hh * 16 + it * 8 + (lane >> 3)) * a.ldd;
-                if (((lane >> 4) & 1) == hh) {
+                if (V16 || ((lane >> 4) & 1) == hh) {
 #pragma unroll
                     for (int nb = 0; nb < NB; nb++)
 #pragma unroll
-                        for (int ig = 0; ig < 4; ig++) {
+                        for (int ig = 0; ig < (V16 ? 1 : 4); ig++) {
                             half4_t h;
 #pragma unroll
                             for (int e = 0; e < 4; e++) h[e] = (half_t)scaled(acc[nb][ig * 4 + e], alpha, beta != 0.f);
-                            *(SHFLBW_LDS half4_t*)(uintptr_t)(wr + nb * 64 + ig * 16) = h;
+                            *(SHFLBW_LDS half4_t*)(uintptr_t)(wr + nb * (V16 ? 32 : 64) + ig * 16) = h;
                         }
                 }
                 // Lanes exchange data through the staging area.  For the compiler every lane is a thread of its own: it
@@ -172,8 +189,8 @@ __global__ void __launch_bounds__(SpmmSlabCfg::THREADS) spmm_shflbw_slab_kernel(
                         }
                     }
 #pragma unroll
-                    for (int it = 0; it < 2; it++) // streaming stores: D must not push A and the slabs out of the L2
-                        __builtin_nontemporal_store(v[it], (half8_t*)(a.D + roff[it] + col));
+                    for (int it = 0; it < 2; it++) // D must not push A and the slabs out of the L2
+                        store_result_16B(a.D + roff[it] + col, v[it]);
                 }
             }
         };
@@ -211,8 +228,12 @@ __global__ void __launch_bounds__(SpmmSlabCfg::THREADS) spmm_shflbw_slab_kernel(
             const char* A = (const char*)a.packedA + (size_t)lpos * (32 * V * 2);
             const char* I = (const char*)a.slab_ids + (size_t)(lpos >> 1) * 256 + (lpos & 1) * 16;
             asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(b.a[0]) : "v"(lane16), "s"(A));
-            asm volatile("global_load_dwordx4 %0, %1, %2 offset:1024" : "=v"(b.a[1]) : "v"(lane16), "s"(A));
-            asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(b.i) : "v"(pair32), "s"(I));
+            if constexpr (V16) {
+                asm volatile("global_load_dwordx2 %0, %1, %2" : "=v"(b.i) : "v"(pair32), "s"(I));
+            } else {
+                asm volatile("global_load_dwordx4 %0, %1, %2 offset:1024" : "=v"(b.a[NA - 1]) : "v"(lane16), "s"(A));
+                asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(b.i) : "v"(pair32), "s"(I));
+            }
             if (lrun && ++lpos == lend) {
                 lrun = false;
                 lpos--; // stay on the last batch unless another panel follows
@@ -230,7 +251,10 @@ __global__ void __launch_bounds__(SpmmSlabCfg::THREADS) spmm_shflbw_slab_kernel(
         // waits until the batch fetched NBUF - 2 fetches before the latest has arrived; the registers pass through
         // the statement so that nothing that reads them can be scheduled in front of the wait
         auto arrived = [&](Batch& b) __attribute__((always_inline)) {
-            asm volatile("s_waitcnt vmcnt(%3)" : "+v"(b.a[0]), "+v"(b.a[1]), "+v"(b.i) : "n"((NBUF - 2) * Cfg::FETCH_OPS));
+            if constexpr (V16)
+                asm volatile("s_waitcnt vmcnt(%2)" : "+v"(b.a[0]), "+v"(b.i) : "n"((NBUF - 2) * Cfg::FETCH_OPS));
+            else
+                asm volatile("s_waitcnt vmcnt(%3)" : "+v"(b.a[0]), "+v"(b.a[NA - 1]), "+v"(b.i) : "n"((NBUF - 2) * Cfg::FETCH_OPS));
         };
         Batch buf[NBUF];
         if (more) {
@@ -246,28 +270,31 @@ __global__ void __launch_bounds__(SpmmSlabCfg::THREADS) spmm_shflbw_slab_kernel(
 
         // B fragments: two transposing reads per fragment, from the rows the offsets name
         auto read_frags = [&](const Batch& b, Frags& f) __attribute__((always_inline)) {
-            const int ids[4] = {b.i.x, b.i.y, b.i.z, b.i.w};
 #pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const uint32_t alo = lds0 + ((uint32_t)ids[2 * h] ^ lc), ahi = lds0 + ((uint32_t)ids[2 * h + 1] ^ lc);
+            for (int h = 0; h < NA; h++) {
+                const uint32_t alo = lds0 + ((uint32_t)b.i[2 * h] ^ lc), ahi = lds0 + ((uint32_t)b.i[2 * h + 1] ^ lc);
 #pragma unroll
                 for (int nb = 0; nb < NB; nb++) {
-                    const half4_t l = lds_read_tr16(alo ^ (nb << 6));
-                    const half4_t u = lds_read_tr16(ahi ^ (nb << 6));
+                    const half4_t l = lds_read_tr16(alo ^ (nb << (V16 ? 5 : 6)));
+                    const half4_t u = lds_read_tr16(ahi ^ (nb << (V16 ? 5 : 6)));
                     f.b[h][nb] = __builtin_shufflevector(l, u, 0, 1, 2, 3, 4, 5, 6, 7);
                 }
             }
         };
         auto mma = [&](const Frags& f, const Batch& b) __attribute__((always_inline)) {
 #pragma unroll
-            for (int h = 0; h < 2; h++)
+            for (int h = 0; h < NA; h++)
 #pragma unroll
-                for (int nb = 0; nb < NB; nb++)
-                    acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.b[h][nb], b.a[h], acc[nb], 0, 0, 0);
+                for (int nb = 0; nb < NB; nb++) {
+                    if constexpr (V16)
+                        acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.b[h][nb], b.a[h], acc[nb], 0, 0, 0);
+                    else
+                        acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.b[h][nb], b.a[h], acc[nb], 0, 0, 0);
+                }
         };
         // the reads of a batch's fragments are issued one batch ahead of its MFMAs, also across the end of a panel
         Frags fr[2];
-        asm volatile("s_waitcnt vmcnt(0)" : "+v"(buf[0].a[0]), "+v"(buf[0].a[1]), "+v"(buf[0].i)); // nothing reads them earlier
+        asm volatile("s_waitcnt vmcnt(0)" : "+v"(buf[0].a[0]), "+v"(buf[0].a[NA - 1]), "+v"(buf[0].i)); // nothing reads them earlier
         read_frags(buf[0], fr[0]);
         for (bool done = false; !done;) {
 #pragma unroll

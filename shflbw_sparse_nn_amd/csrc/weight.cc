@@ -194,6 +194,26 @@ static int check_pattern(int nrow, int ncol, int brow, int bcol, int nnzb, const
     return SHFLBW_OK;
 }
 
+// Order of a panel's kept vectors for the slab form of block height 16: a transposing read touches 32 bytes of the slab rows of
+// slots 0..3 and 8..11 (or 4..7 and 12..15) of a 16-slot half step at a time, which lie in different banks when the rows differ
+// modulo 8.  Eights are drawn from the residues with ids left, in turn, and dealt to those slots.
+static void order_for_slab16(const int* ids, int nnz, int* ord)
+{
+    std::vector<int> by_residue(nnz);
+    int at[9] = {}, fill[8];
+    for (int q = 0; q < nnz; q++) at[(ids[q] & 7) + 1]++;
+    for (int c = 0; c < 8; c++) at[c + 1] += at[c], fill[c] = at[c];
+    for (int q = 0; q < nnz; q++) by_residue[fill[ids[q] & 7]++] = q;
+    std::vector<int> drawn(nnz);
+    for (int q = 0; q < nnz;)
+        for (int c = 0; c < 8; c++)
+            if (at[c] < fill[c]) drawn[q++] = by_residue[at[c]++];
+    for (int q = 0; q < nnz; q++) {
+        const int base = q & ~15, s = q & 15, t = s & 7; // t-th of the eight number s / 8
+        ord[base + 16 <= nnz ? base + (s >> 3) * 4 + (t < 4 ? t : t + 4) : q] = drawn[q];
+    }
+}
+
 // ---------------------------------------------------------------------------------
 // private image.  Panel i keeps nnz_i vectors; they are padded to a multiple of 64
 // slots.  packed_indices: the column ids, tail slots hold -1 (their values are zero and
@@ -230,7 +250,7 @@ int build_packed_image(shflbw_weight* w)
     w->packed_indices.assign(slots, 0);
     w->packed_indices_pm.assign(slots, 0);
     w->packed_values.assign(slots * V, 0);
-    const bool slab = V == 32 && w->ncol <= SLAB_MAX_K;
+    const bool slab = (V == 32 || V == 16) && w->ncol <= SLAB_MAX_K;
     w->packed_slab.assign(slab ? slots : 0, 0);
     for (int i = 0; i < X; i++) {
         const int begin = w->indptr[i], nnz = w->indptr[i + 1] - begin;
@@ -241,7 +261,9 @@ int build_packed_image(shflbw_weight* w)
         // groups (slab_bank_class): every quad takes the next id of each of the classes with the most ids left.
         std::vector<int> ord(nnz);
         for (int q = 0; q < nnz; q++) ord[q] = q;
-        if (slab) {
+        if (slab && V == 16) {
+            order_for_slab16(w->indices.data() + begin, nnz, ord.data());
+        } else if (slab) {
             std::vector<int> of_class[4];
             for (int q = nnz - 1; q >= 0; q--) of_class[slab_bank_class(w->indices[begin + q])].push_back(q); // back() = smallest id
             for (int q = 0; q < nnz;) {
