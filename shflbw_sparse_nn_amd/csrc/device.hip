@@ -103,19 +103,28 @@ static int device_compute_units()
     return cached[dev];
 }
 
+// The variants of a block height lie side by side in the table.  Every initialisation and launch looks one up: the ranges
+// are found once.
 static const SpmmVariant* find_spmm_variant(int brow, int variant, int* n_for_brow)
 {
-    int count = 0;
-    const SpmmVariant* all = spmm_variants(&count);
-    const SpmmVariant* hit = nullptr;
-    int seen = 0;
-    for (int i = 0; i < count; i++) {
-        if (all[i].V != brow) continue;
-        if (seen == variant) hit = &all[i];
-        seen++;
-    }
-    if (n_for_brow) *n_for_brow = seen;
-    return hit;
+    struct Ranges {
+        const SpmmVariant* first[4] = {};
+        int n[4] = {};
+        static int of(int brow) { return brow == 16 ? 0 : brow == 32 ? 1 : brow == 64 ? 2 : brow == 128 ? 3 : -1; }
+        Ranges()
+        {
+            int count = 0;
+            const SpmmVariant* all = spmm_variants(&count);
+            for (int i = 0; i < count; i++) {
+                const int r = of(all[i].V);
+                if (n[r]++ == 0) first[r] = &all[i];
+            }
+        }
+    };
+    static const Ranges ranges;
+    const int r = Ranges::of(brow), n = r < 0 ? 0 : ranges.n[r];
+    if (n_for_brow) *n_for_brow = n;
+    return variant >= 0 && variant < n ? ranges.first[r] + variant : nullptr;
 }
 
 static const SpconvVariant* find_spconv_variant(int brow, int variant, int* n_for_brow)
@@ -167,11 +176,9 @@ static int auto_gather_variant(const shflbw_weight* w, int N, bool allow_slab, i
 {
     const int brow = w->brow, X = w->nrow / w->brow;
     int count = 0;
-    const SpmmVariant* all = spmm_variants(&count);
+    const SpmmVariant* all = find_spmm_variant(brow, 0, &count);
     if (allow_slab && !w->packed_slab.empty() && X > 0 && (brow == 16 ? N >= 128 : w->ncol >= 384)) {
-        int seen = 0;
         for (int i = 0; i < count; i++) {
-            if (all[i].V != brow) continue;
             if (all[i].max_k >= w->ncol) {
                 const int cus = (compute_units / 8) * 8;
                 const int n_tiles = (N + all[i].BN - 1) / all[i].BN;
@@ -182,19 +189,14 @@ static int auto_gather_variant(const shflbw_weight* w, int N, bool allow_slab, i
                 if (brow == 16 ? panels_per_wg >= 16 && vectors_per_column >= (n_tiles * chunks < 0.8 * cus ? 4.0 : panels_per_wg < 24 ? 2.5 : 1.0) &&
                                      (vectors >= 32 || 2.0 * w->nrow * N <= 100e6 || N % 64 != 0)
                                : vectors_per_column >= 3.0 && n_tiles >= 32)
-                    return seen;
+                    return i;
             }
-            seen++;
         }
     }
     // the role-split variant of this block size with tiles of `bn` columns, -1 when there is none
     auto role_split_with = [&](int bn) {
-        int seen = 0;
-        for (int i = 0; i < count; i++) {
-            if (all[i].V != brow) continue;
-            if (all[i].name[0] == 'w' && all[i].BN == bn) return seen; // "ws..." names
-            seen++;
-        }
+        for (int i = 0; i < count; i++)
+            if (all[i].name[0] == 'w' && all[i].BN == bn) return i; // "ws..." names
         return -1;
     };
     // small problems: 128-column tiles while they do not outnumber the compute units (39 shapes of block heights 32, 64
