@@ -31,7 +31,7 @@ struct shflbw_weight {
     std::vector<int> packed_indices; // 64 * group_ptr[X]; tail slots hold -1 (a row of zeros)
     std::vector<int> packed_indices_pm; // each 64-slot group reordered: [16p + 4j + r] = packed_indices[16j + 4p + r]
     std::vector<uint16_t> packed_values; // 64 * brow * group_ptr[X]; MFMA fragment order, tail zero
-    // slab form of the SpMM (block sizes 32 and 64, ncol <= SLAB_MAX_K; empty otherwise): the ids of every 64-slot
+    // slab form of the SpMM (block sizes 32 and 16, ncol <= SLAB_MAX_K; empty otherwise): the ids of every 64-slot
     // group as LDS byte offsets of slab rows, in the order the lanes of a wave load them (see build_packed_image)
     std::vector<int> packed_slab;
 
