@@ -376,11 +376,11 @@ static int spmm_init_impl(shflbw_spmm_state* state, const shflbw_weight* w, int 
     const bool wide_b = (unsigned long long)w->ncol * (unsigned long long)N * 2ull + (unsigned long long)N * 2ull > 0xffffffffull;
     if (variant < 0) {
         variant = auto_spmm_variant(w, N, !gather_only, compute_units);
-        if (wide_b) { // first variant of this block size with 64-bit addressing
+        if (wide_b) { // first variant of this block size with 64-bit addressing (block height 16 has none: refused below)
             int n = 0;
             find_spmm_variant(w->brow, 0, &n);
             for (int i = 0; i < n; i++)
-                if (!spmm_variant_offsets32(find_spmm_variant(w->brow, i, nullptr))) {
+                if (const SpmmVariant* c = find_spmm_variant(w->brow, i, nullptr); !spmm_variant_offsets32(c) && c->max_k == 0) {
                     variant = i;
                     break;
                 }
