@@ -378,7 +378,7 @@ static int spmm_init_impl(shflbw_spmm_state* state, const shflbw_weight* w, int 
         variant = auto_spmm_variant(w, N, !gather_only, compute_units);
         if (wide_b) { // first variant of this block size with 64-bit addressing (block height 16 has none: refused below)
             int n = 0;
-            find_spmm_variant(w->brow, 0, &n);
+            find_spmm_variant(w->brow, variant = 0, &n);
             for (int i = 0; i < n; i++)
                 if (const SpmmVariant* c = find_spmm_variant(w->brow, i, nullptr); !spmm_variant_offsets32(c) && c->max_k == 0) {
                     variant = i;
