@@ -23,6 +23,7 @@ struct ConvPatchPlan {
     int step_h, step_w;   // patch positions between neighbouring output positions
     int patch_w, npos;    // columns and positions of the input patch of a unit
     int pitch;            // LDS bytes of one channel: 8 per position, an odd multiple of 8
+    int slack;            // LDS bytes behind the row of zeros that columns without a pixel may touch
     int groups, ksplit;   // waves = groups (rows) x ksplit (parts of the kept columns, a power of two: 1 << kshift)
     int kshift;
     int panels_per_wave;  // row units one wave computes one after the other
@@ -73,7 +74,7 @@ struct ConvPatchKernel {
 const ConvPatchKernel* conv_patch_kernel(int rows, int col_blocks, int waves);
 
 constexpr int CONV_PATCH_LDS_MAX = 160 * 1024;
-constexpr int CONV_PATCH_SLACK = 256;       // LDS bytes behind the row of zeros
+constexpr int CONV_PATCH_SLACK = 256;       // least LDS bytes behind the row of zeros
 constexpr int CONV_PATCH_TAIL_BATCHES = 8;  // batches of padding behind the last one: waves fetch ahead of their end
 inline int conv_patch_unit_rows(int V) { return V == 128 ? 64 : V; }
 

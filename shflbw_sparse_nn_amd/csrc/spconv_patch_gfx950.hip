@@ -250,7 +250,7 @@ __global__ void __launch_bounds__(NW * 64, WPE) spconv_patch_kernel(ConvPatchArg
 #pragma unroll
             for (int mb = 0; mb < MBW; mb++) asm volatile("" : "+v"(dst[j][mb])); // older than the ring: arrived
         // the row of zeros the padding slots read, and behind it what columns without a pixel may touch
-        for (int i = tid; i < (pitch >> 3) + CONV_PATCH_SLACK / 8; i += NW * 64)
+        for (int i = tid; i < (pitch + P.slack) >> 3; i += NW * 64)
             *(SHFLBW_LDS int2_t*)(uintptr_t)(slab + (uint32_t)a.C * pitch + i * 8) = int2_t{0, 0};
     }
     __syncthreads(); // the patch
@@ -557,7 +557,12 @@ bool conv_patch_plan(const ConvPatchProblem& q, ConvPatchPlan* plan)
                 p.patch_w = (tw - 1) * ew + q.S;
                 p.npos = ((th - 1) * eh + q.R) * p.patch_w;
                 p.pitch = 8 * (p.npos | 1);
-                const long slab = (long)(q.C + 1) * p.pitch + CONV_PATCH_SLACK;
+                // the furthest byte a lane reads: the last tap of the last channel, or the row of zeros, under the last
+                // position of a row (positions from tile_w on are no pixels, but are read)
+                const long last_row = std::max((long)q.C * p.pitch, (q.C - 1L) * p.pitch + ((q.R - 1L) * p.patch_w + q.S - 1) * 8);
+                const long last = last_row + ((th - 1L) * eh * p.patch_w + (rl - 1L) * ew) * 8 + 8;
+                p.slack = (int)std::max<long>(CONV_PATCH_SLACK, last - (q.C + 1L) * p.pitch);
+                const long slab = (long)(q.C + 1) * p.pitch + p.slack;
                 if (slab > CONV_PATCH_LDS_MAX) continue;
                 for (int groups = k.waves; groups >= 1; groups >>= 1)
                     for (int np = 1; np <= npmax; np <<= 1) {

@@ -1,0 +1,91 @@
+// The planner of the convolution's patch form on the CPU: what a workgroup of the cut it picks would read from LDS, for
+// seeded random layers.  The walk below restates the kernel's addressing (position -> column offset, kept column -> row).
+#include <algorithm>
+#include <cstdio>
+#include <cstring>
+#include <random>
+
+#include "csrc/spconv_patch.h"
+
+using namespace shflbw;
+
+namespace {
+
+struct Layer {
+    int V, F, C, R, S, permuted, B, H, W, stride;
+    double density;
+};
+
+ConvPatchProblem problem(const Layer& l)
+{
+    return ConvPatchProblem{l.V, l.F, l.C, l.R, l.S, l.density * l.R * l.S * l.C, l.permuted, l.B, l.H, l.W,
+                            (l.H + 2 * (l.R / 2) - l.R) / l.stride + 1, (l.W + 2 * (l.S / 2) - l.S) / l.stride + 1, l.stride, 256};
+}
+
+// Ordinary layers, and (one in four) the corners: strides as wide as the filter, filters of one row, narrow maps.
+Layer random_layer(std::mt19937& rng)
+{
+    auto pick = [&](std::initializer_list<int> v) { return v.begin()[rng() % v.size()]; };
+    Layer l{};
+    l.V = pick({16, 32, 64, 128});
+    l.F = l.V * (1 + (int)(rng() % 16));
+    l.C = 8 * (1 + (int)(rng() % 64));
+    l.permuted = rng() % 2;
+    l.B = 1 + (int)(rng() % 64);
+    l.density = 0.05 + (rng() % 100) / 110.0;
+    if (rng() % 4) {
+        l.R = pick({1, 3, 3, 5, 7}), l.S = rng() % 4 ? l.R : pick({1, 2, 3, 4, 7});
+        l.H = 3 + (int)(rng() % 56), l.W = rng() % 2 ? l.H : 3 + (int)(rng() % 56);
+        l.stride = 1 + (int)(rng() % 3);
+    } else {
+        l.R = pick({1, 1, 2, 7}), l.S = pick({1, 2, 5, 6, 7, 9, 11});
+        l.H = 1 + (int)(rng() % 24), l.W = 1 + (int)(rng() % 24);
+        l.stride = 1 + (int)(rng() % 11);
+    }
+    if (l.H + 2 * (l.R / 2) < l.R || l.W + 2 * (l.S / 2) < l.S) return random_layer(rng);
+    return l;
+}
+
+// One byte past the last one that any lane of the kernel reads from the patch, counted from its first row.
+long patch_end(const Layer& l, const ConvPatchPlan& p)
+{
+    long col = 0;
+    for (int pos = 0; pos < 8 * p.col_blocks; pos++) {
+        const int i = pos / p.row_len, j = pos % p.row_len;
+        if (i < p.tile_h) col = std::max(col, (long)(i * p.step_h * p.patch_w + j * p.step_w) * 8);
+    }
+    long row = (long)l.C * p.pitch; // the row of zeros
+    for (int r = 0; r < l.R; r++)
+        for (int s = 0; s < l.S; s++) row = std::max(row, (l.C - 1L) * p.pitch + (r * p.patch_w + s) * 8);
+    return row + col + 8;
+}
+
+int reads_stay_inside()
+{
+    std::mt19937 rng(2024);
+    int bad = 0, taken = 0;
+    for (int t = 0; t < 20000; t++) {
+        // first the one-row filter whose stride leaves one output column per unit
+        const Layer l = t == 0 ? Layer{32, 32, 8, 1, 7, 1, 4, 4, 7, 7, 0.5} : random_layer(rng);
+        ConvPatchPlan p;
+        if (!conv_patch_plan(problem(l), &p)) continue;
+        taken++;
+        const long place = 128 * p.col_blocks, end = patch_end(l, p);
+        if (place + end > p.lds_bytes || p.lds_bytes > CONV_PATCH_LDS_MAX) {
+            if (bad++ < 5)
+                printf("Failed: V %d F %d C %d %dx%d map %dx%d stride %d: reads to %ld of %d bytes\n", l.V, l.F, l.C, l.R, l.S, l.H, l.W,
+                       l.stride, place + end, p.lds_bytes);
+        }
+    }
+    printf("reads: %d cuts, %d past the LDS of the workgroup\n", taken, bad);
+    return bad + (taken < 5000);
+}
+
+} // namespace
+
+int main()
+{
+    const int bad = reads_stay_inside();
+    printf(bad ? "FAILED\n" : "ALL PASSED\n");
+    return bad != 0;
+}
