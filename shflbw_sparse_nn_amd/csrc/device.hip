@@ -405,7 +405,7 @@ static int spmm_init_impl(shflbw_spmm_state* state, const shflbw_weight* w, int 
         return SHFLBW_ERR_UNSUPPORTED;
     }
     SpmmLaunchArgs la;
-    la.M = w->nrow, la.N = N, la.X = X, la.beta = beta, la.num_cus = compute_units;
+    la.M = w->nrow, la.N = N, la.X = X, la.num_cus = compute_units;
     SHFLBW_HIP_TRY(v->prepare(la));
 
     shflbw_device_ref ref;

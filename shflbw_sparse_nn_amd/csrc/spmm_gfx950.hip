@@ -16,6 +16,7 @@
 //    the vector-memory counter only ever counts the LDS copies and the waits are exact;
 //  * fp32 accumulators are rounded once to fp16, staged through LDS and scattered as whole
 //    row segments through the permutation.
+#include <atomic>
 #include <mutex>
 #include <type_traits>
 
@@ -318,13 +319,23 @@ static hipError_t launch_ws(const SpmmLaunchArgs& a, hipStream_t stream)
     return hipGetLastError();
 }
 
+// Both instances: the beta of a state is a plain field, and the launch goes by what it holds then.  Once per device, so that
+// an initialisation makes no call into the driver for a limit that is already raised.
 template <int V, int WN, int NCONS, int NPROD, int KT, int NSTAGE>
-static hipError_t prepare_ws(const SpmmLaunchArgs& a)
+static hipError_t prepare_ws(const SpmmLaunchArgs&)
 {
     using Cfg = SpmmWsCfg<V, WN, NCONS, NPROD, KT, NSTAGE>;
-    const void* f = a.beta != 0.f ? (const void*)spmm_shflbw_ws_kernel<V, WN, NCONS, NPROD, KT, NSTAGE, true>
-                                  : (const void*)spmm_shflbw_ws_kernel<V, WN, NCONS, NPROD, KT, NSTAGE, false>;
-    return hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS_BYTES);
+    static std::atomic<unsigned long long> raised{0}; // one bit per device
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    const unsigned long long bit = dev < 64 ? 1ull << dev : 0;
+    if (raised.load(std::memory_order_acquire) & bit) return hipSuccess;
+    for (const void* f : {(const void*)spmm_shflbw_ws_kernel<V, WN, NCONS, NPROD, KT, NSTAGE, false>,
+                          (const void*)spmm_shflbw_ws_kernel<V, WN, NCONS, NPROD, KT, NSTAGE, true>})
+        if ((e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS_BYTES)) != hipSuccess) return e;
+    raised.fetch_or(bit, std::memory_order_release);
+    return hipSuccess;
 }
 
 #define SHFLBW_WS_VARIANT(V, WN, NC, NP, KT, NS)                                                             \

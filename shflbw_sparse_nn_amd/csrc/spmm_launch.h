@@ -37,7 +37,7 @@ struct SpmmVariant {
     int lds_bytes;   // dynamic LDS
     const char* name;
     hipError_t (*launch)(const SpmmLaunchArgs&, hipStream_t);
-    hipError_t (*prepare)(const SpmmLaunchArgs&); // raises the dynamic-LDS limit of the kernel that `launch` takes (M, N, X, beta are set)
+    hipError_t (*prepare)(const SpmmLaunchArgs&); // raises the dynamic-LDS limit of the kernels that `launch` may take (M, N, X are set)
     int max_k;               // 0, or the most columns of A the variant takes (it holds all rows of B in LDS)
 };
 
