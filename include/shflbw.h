@@ -220,7 +220,7 @@ const char* shflbw_spmm_variant_name(int brow, int variant);
  *     and shflbw_spconv_check reports it;
  *   variant 5 = patch form, one launch (any batch): a workgroup transposes the input patch under its output pixels
  *     into LDS, runs the products on it and writes NHWC itself.  SHFLBW_ERR_UNSUPPORTED where no patch fits the LDS or
- *     the plane forms are estimated faster.
+ *     the tensors leave 32-bit indexes.
  * ------------------------------------------------------------------------- */
 #define SHFLBW_CONV_SCRATCH_DEPTH 4
 typedef struct shflbw_spconv_state {

@@ -967,22 +967,27 @@ int init_fused(shflbw_spconv_state* state, const shflbw_weight* f, int B, int H,
 }
 
 // The patch form of one geometry of a filter: cut, LDS offsets of the kept columns and places of the rows in the output,
-// built and uploaded on the first call for a geometry, found afterwards.  *out is null when the form does not take
-// the geometry.
-int conv_patch_for(shflbw_weight* fw, int B, int H, int W, int stride, int Ho, int Wo, const shflbw_weight::ConvPatch** out)
+// built and uploaded on the first call that takes a geometry, found afterwards.  *out is null when no patch fits and, unless
+// `forced`, when the plane forms are estimated faster.
+int conv_patch_for(shflbw_weight* fw, int B, int H, int W, int stride, int Ho, int Wo, bool forced, const shflbw_weight::ConvPatch** out)
 {
     *out = nullptr;
     std::lock_guard<std::mutex> scratch_guard(fw->scratch_lock);
-    for (auto& e : fw->conv_patch)
-        if (e.key[0] == B && e.key[1] == H && e.key[2] == W && e.key[3] == stride) {
-            if (e.plan.valid) *out = &e;
-            return SHFLBW_OK;
-        }
-    shflbw_weight::ConvPatch e{};
-    e.key[0] = B, e.key[1] = H, e.key[2] = W, e.key[3] = stride;
     const int V = fw->brow, X = fw->nrow / V, F = fw->F, C = fw->C, S = fw->S;
-    const ConvPatchProblem q{V, F, C, fw->R, S, (double)fw->nnzb / X, fw->row_permute ? 1 : 0, B, H, W, Ho, Wo, stride, device_compute_units()};
-    if (conv_patch_plan(q, &e.plan)) {
+    shflbw_weight::ConvPatch* known = nullptr;
+    for (auto& c : fw->conv_patch)
+        if (c.key[0] == B && c.key[1] == H && c.key[2] == W && c.key[3] == stride) known = &c;
+    if (!known) {
+        const ConvPatchProblem q{V, F, C, fw->R, S, (double)fw->nnzb / X, fw->row_permute ? 1 : 0, B, H, W, Ho, Wo, stride, device_compute_units()};
+        shflbw_weight::ConvPatch c{};
+        c.key[0] = B, c.key[1] = H, c.key[2] = W, c.key[3] = stride;
+        conv_patch_plan(q, &c.plan);
+        fw->conv_patch.push_back(c);
+        known = &fw->conv_patch.back();
+    }
+    if (!known->plan.valid || !(forced || known->plan.preferred)) return SHFLBW_OK;
+    if (!known->ptr) {
+        shflbw_weight::ConvPatch e = *known;
         const ConvPatchPlan& p = e.plan;
         const int RW = conv_patch_unit_rows(V), per_panel = V / RW, nunits = F / RW;
         SHFLBW_HIP_TRY(conv_patch_kernel(RW, p.col_blocks, p.waves)->prepare());
@@ -1080,23 +1085,25 @@ int conv_patch_for(shflbw_weight* fw, int B, int H, int W, int stride, int Ho, i
         e.first_batch = (const int*)((const char*)e.ptr + o_first);
         e.filt = (const int*)((const char*)e.ptr + o_filt);
         e.dst = (const unsigned short*)((const char*)e.ptr + o_dst);
+        *known = e;
     }
-    fw->conv_patch.push_back(e);
-    if (e.plan.valid) *out = &fw->conv_patch.back();
+    *out = known;
     return SHFLBW_OK;
 }
 
 // Form 5.  `reported`: what the state's variant says (the library's own choice keeps naming the plane form whose
-// place the patch form takes).  SHFLBW_ERR_UNSUPPORTED when the form does not take the geometry.
+// place the patch form takes).  `forced`: whatever the estimate says.  SHFLBW_ERR_UNSUPPORTED when the form does not take the
+// geometry.
 int init_patch(shflbw_spconv_state* state, const shflbw_weight* f, int B, int H, int W, int stride, const void* IFMap,
-               void* OFMap, int reported)
+               void* OFMap, int reported, bool forced)
 {
     int rc = spconv_fill_state(state, f, B, H, W, stride, IFMap, OFMap, FORM_PATCH);
     if (rc != SHFLBW_OK) return rc;
     const shflbw_weight::ConvPatch* e = nullptr;
-    if ((rc = conv_patch_for(const_cast<shflbw_weight*>(f), B, H, W, stride, state->Ho, state->Wo, &e)) != SHFLBW_OK) return rc;
+    if ((rc = conv_patch_for(const_cast<shflbw_weight*>(f), B, H, W, stride, state->Ho, state->Wo, forced, &e)) != SHFLBW_OK) return rc;
     if (!e) {
-        set_error("spconv_init: the input patch of a workgroup does not fit the LDS (%d channels, %d x %d filter)", f->C, f->R, f->S);
+        set_error(forced ? "spconv_init: no input patch of a workgroup fits the LDS (%d channels, %d x %d filter), or the tensors leave 32-bit indexes"
+                         : "spconv_init: the patch form does not take this layer (%d channels, %d x %d filter)", f->C, f->R, f->S);
         return SHFLBW_ERR_UNSUPPORTED;
     }
     state->patch = e;
@@ -1178,10 +1185,10 @@ int shflbw_spconv_init_variant(shflbw_spconv_state* state, const shflbw_weight* 
             const long Ho = (H + 2 * (f->R / 2) - f->R) / stride + 1, Wo = (W + 2 * (f->S / 2) - f->S) / stride + 1;
             if (Ho > 0 && Wo > 0) variant = FORM_BPLANES;
         }
-        const int rc = init_patch(state, f, B, H, W, stride, IFMap, OFMap, variant);
+        const int rc = init_patch(state, f, B, H, W, stride, IFMap, OFMap, variant, false);
         if (rc != SHFLBW_ERR_UNSUPPORTED) return rc;
     }
-    if (variant == FORM_PATCH) return init_patch(state, f, B, H, W, stride, IFMap, OFMap, FORM_PATCH);
+    if (variant == FORM_PATCH) return init_patch(state, f, B, H, W, stride, IFMap, OFMap, FORM_PATCH, true);
     if (variant == FORM_BPLANES) return init_batch_planes(state, f, B, H, W, stride, IFMap, OFMap, FORM_BPLANES);
     if (variant == FORM_FUSED) return init_fused(state, f, B, H, W, stride, IFMap, OFMap);
     if (variant == FORM_PLANES) return init_planes(state, f, B, H, W, stride, IFMap, OFMap);

@@ -14,7 +14,8 @@ namespace shflbw {
 // position p of unit u.  The four units of a position lie side by side in LDS (8 bytes), which is what one lane of
 // the transposing LDS read supplies, so a tap is a plain offset whatever the stride, the batch and the alignment.
 struct ConvPatchPlan {
-    int valid;
+    int valid;            // some patch fits the LDS
+    int preferred;        // ... and is estimated faster than the plane forms
     int col_blocks;       // 32-column blocks of a tile: 2 (16 positions x 4 units) or 1 (8 positions)
     int waves;            // waves of a workgroup
     int tile_h, tile_w;   // output positions of a unit
@@ -44,7 +45,7 @@ struct ConvPatchProblem {
     int permuted;          // rows of the filter are permuted
     int B, H, W, Ho, Wo, stride, cus;
 };
-// Fills `plan`; false when no patch fits the LDS or the sizes leave 32-bit indexes (the plane forms take over).
+// Fills `plan`; false when no patch fits the LDS or the sizes leave 32-bit indexes.
 bool conv_patch_plan(const ConvPatchProblem& q, ConvPatchPlan* plan);
 
 // Order of the kept columns of a row panel that keeps the LDS reads of a group of rows apart (see the definition).

@@ -523,7 +523,7 @@ static double conv_planes_estimate(const ConvPatchProblem& q)
 // The cut with the least estimated time: rounds of workgroups times the sum of a workgroup's phases.  The weights come from
 // a fit to 124 layers measured with 20 to 40 cuts each (10 % rms; the cut it picks is 4 % slower than the best one
 // measured on average).  Where the plane forms are estimated faster - many filters over few resident pixels (wide
-// filters over many channels), filters of several workgroups interleaved in the output - the form is not taken:
+// filters over many channels), filters of several workgroups interleaved in the output - the cut is not `preferred`:
 // 7 x 54 x 54 x 584 -> 1024, 5 x 5, stride 2 takes 152 us here, 54 us there; 16 x 14 x 14 x 512 -> 2048 20 and 23 us.
 bool conv_patch_plan(const ConvPatchProblem& q, ConvPatchPlan* plan)
 {
@@ -609,7 +609,7 @@ bool conv_patch_plan(const ConvPatchProblem& q, ConvPatchPlan* plan)
             }
     }
     if (!best.valid) return false;
-    if (best_cost > conv_planes_estimate(q)) return false;
+    best.preferred = best_cost <= conv_planes_estimate(q);
     best.H = H, best.W = W, best.Ho = Ho, best.Wo = Wo, best.stride = q.stride;
     best.pad_h = q.R / 2, best.pad_w = q.S / 2;
     best.step_h = eh, best.step_w = ew;

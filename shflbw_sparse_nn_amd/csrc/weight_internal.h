@@ -72,7 +72,7 @@ struct shflbw_weight {
     };
     static constexpr int CONV_BULK_DEPTH = SHFLBW_CONV_SCRATCH_DEPTH;
     //  * ConvPatch: cut, filter image (in an order of its own) and output places of the patch form, keyed like the ids
-    //    (plan.valid == 0: the form does not take that geometry); states point at the entries, which stay where they are.
+    //    (ptr == null: nothing has taken the form for that geometry); states point at the entries, which stay where they are.
     struct ConvPatch {
         int key[4]; // B, H, W, stride
         shflbw::ConvPatchPlan plan;

@@ -89,3 +89,30 @@ def test_the_library_runs_it_and_it_needs_no_buffers(torch_gpu):
     op = S.SpconvBlockwiseOp()
     st = op.initialize(fw, 1, 8, 8, 1, xw.data_ptr(), ops[0][1].data_ptr())
     assert not st.patch and st.variant == 0
+
+
+@pytest.mark.parametrize("Bn,H,C,F,V,stride", [(1, 5, 512, 64, 64, 2), (4, 8, 512, 128, 128, 2)])
+def test_variant_5_runs_where_the_library_would_not_choose_it(torch_gpu, Bn, H, C, F, V, stride):
+    """A layer whose patch fits the LDS but whose plane forms are estimated faster: the library takes a plane form, an explicit
+    request runs the patch form, and neither changes what the other gets."""
+    torch = torch_gpu
+    w = P.make_weight(F, 25 * C, V, 0.4, True, 3, integer=True)
+    x = np.random.default_rng(5).integers(-4, 5, size=(Bn, H, H, C)).astype(np.float16)
+    ref = O.float_to_half(P.conv_oracle(w, 5, 5, C, x, stride))
+    f = P.upload_weight(w, 5, 5, C, cls=S.BlockwiseSpFilter)
+    dX = P.to_dev(torch, x)
+    for variant in (-1, PATCH, -1, PATCH):
+        dY = torch.full(ref.shape, float("nan"), dtype=torch.float16, device="cuda")
+        op = S.SpconvBlockwiseOp(variant)
+        st = op.initialize(f, Bn, H, H, stride, dX.data_ptr(), dY.data_ptr())
+        assert bool(st.patch) == (variant == PATCH)
+        op(torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(dY.cpu().numpy().view(np.uint16), ref.view(np.uint16))
+
+
+def test_variant_5_is_refused_where_no_patch_fits(torch_gpu):
+    w = P.make_weight(64, 25 * 1024, 64, 0.01, True, 3, integer=True)
+    with pytest.raises(S.capi.ShflbwError) as e:
+        run_spconv(torch_gpu, w, 5, 5, 1024, np.zeros((1, 8, 8, 1024), dtype=np.float16), 1, PATCH)
+    assert e.value.status == S.capi.ERR_UNSUPPORTED and "LDS" in str(e.value)
