@@ -392,7 +392,7 @@ def bench_conv(args, name, np, torch, S, P, full, cpu):
                                     "the first %d panels" % XS, O.max_threads())
 
     eff_tflops = eff_flops / t / 1e12
-    kernel = S.spconv_variant_name(5 if op._state.patch else op._state.variant)  # the library's choice may run the patch form
+    kernel = S.spconv_variant_name(op._state.variant)  # the form the library chose
     traffic = measured_traffic(name, kernel) if args.traffic is None else round(float(args.traffic))
     return {
         "metric": "effective sparse TFLOP/s + %% fp16 MFMA peak, SpConv2D %s" % name,

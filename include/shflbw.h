@@ -202,9 +202,8 @@ const char* shflbw_spmm_variant_name(int brow, int variant);
  * SHFLBW_CONV_SCRATCH_DEPTH such buffers exist per filter: initialising a state over one more tensor pair recycles
  * the buffers of the least recently initialised one (no allocation, no copy when the geometry is the same), whose
  * state must not be executed afterwards.  exec only launches, in order on `stream`.
- * shflbw_spconv_init_variant (variant < 0, and shflbw_spconv_init: the library's choice - variant 2 when B % 8 == 0,
- * else variant 0, whose three launches are replaced by the one launch of variant 5 - `patch` in the state is then set -
- * where that is estimated faster; it needs no scratch but its tables):
+ * shflbw_spconv_init_variant (variant < 0, and shflbw_spconv_init: the library's choice - variant 5 where it is estimated
+ * faster than the plane forms, else variant 2 when B % 8 == 0, else variant 0; the state's `variant` says which it was):
  *   variant 0 = plane form, three launches: the input is rewritten once per call as channel-major padded
  *     planes (one per stride phase); the SpMM kernel then gathers, for a kept k = (r, s, c), the
  *     plane of channel c at the constant offset of tap (r, s) - the im2col matrix is never built,
@@ -228,7 +227,7 @@ typedef struct shflbw_spconv_state {
     unsigned grid_dim[3];
     unsigned block_dim[3];
     int init_success;
-    int variant;
+    int variant; /* the form that exec runs (shflbw_spconv_variant_name) */
     struct {
         int B, H, W, C, F, R, S, stride;
         const void* A_values;

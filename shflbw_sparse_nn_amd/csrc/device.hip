@@ -1091,11 +1091,9 @@ int conv_patch_for(shflbw_weight* fw, int B, int H, int W, int stride, int Ho, i
     return SHFLBW_OK;
 }
 
-// Form 5.  `reported`: what the state's variant says (the library's own choice keeps naming the plane form whose
-// place the patch form takes).  `forced`: whatever the estimate says.  SHFLBW_ERR_UNSUPPORTED when the form does not take the
-// geometry.
+// Form 5.  `forced`: whatever the estimate says.  SHFLBW_ERR_UNSUPPORTED when the form does not take the geometry.
 int init_patch(shflbw_spconv_state* state, const shflbw_weight* f, int B, int H, int W, int stride, const void* IFMap,
-               void* OFMap, int reported, bool forced)
+               void* OFMap, bool forced)
 {
     int rc = spconv_fill_state(state, f, B, H, W, stride, IFMap, OFMap, FORM_PATCH);
     if (rc != SHFLBW_OK) return rc;
@@ -1107,7 +1105,6 @@ int init_patch(shflbw_spconv_state* state, const shflbw_weight* f, int B, int H,
         return SHFLBW_ERR_UNSUPPORTED;
     }
     state->patch = e;
-    state->variant = reported;
     state->ncols = B * state->Ho * state->Wo;
     state->shared_mem_size = (size_t)e->plan.lds_bytes;
     state->grid_dim[0] = (unsigned)e->plan.jobs;
@@ -1176,19 +1173,16 @@ int shflbw_spconv_init_variant(shflbw_spconv_state* state, const shflbw_weight* 
         set_error("spconv_init: form 4 works on C-H-W-B / F-H-W-B tensors; call shflbw_spconv_init_chwb");
         return SHFLBW_ERR_INVALID;
     }
-    // the library's choice: the batch-innermost form wherever the batch allows it (one copy of the planes instead of
-    // two, no dead plane rows in the result; with the tile width of its SpMM chosen by the size of the GEMM it is level
-    // with the plane form on the smallest layers and ahead from a few hundred output pixels on), else the plane form
+    // the library's choice: the patch form wherever it is estimated faster; else the batch-innermost form wherever the batch
+    // allows it (one copy of the planes instead of two, no dead plane rows in the result; with the tile width of its SpMM
+    // chosen by the size of the GEMM it is level with the plane form on the smallest layers and ahead from a few hundred
+    // output pixels on), else the plane form
     if (variant < 0) {
-        variant = FORM_PLANES;
-        if (f && f->R > 0 && B > 0 && B % 8 == 0 && H > 0 && W > 0 && stride > 0) {
-            const long Ho = (H + 2 * (f->R / 2) - f->R) / stride + 1, Wo = (W + 2 * (f->S / 2) - f->S) / stride + 1;
-            if (Ho > 0 && Wo > 0) variant = FORM_BPLANES;
-        }
-        const int rc = init_patch(state, f, B, H, W, stride, IFMap, OFMap, variant, false);
+        const int rc = init_patch(state, f, B, H, W, stride, IFMap, OFMap, false);
         if (rc != SHFLBW_ERR_UNSUPPORTED) return rc;
+        variant = B % 8 == 0 ? FORM_BPLANES : FORM_PLANES;
     }
-    if (variant == FORM_PATCH) return init_patch(state, f, B, H, W, stride, IFMap, OFMap, FORM_PATCH, true);
+    if (variant == FORM_PATCH) return init_patch(state, f, B, H, W, stride, IFMap, OFMap, true);
     if (variant == FORM_BPLANES) return init_batch_planes(state, f, B, H, W, stride, IFMap, OFMap, FORM_BPLANES);
     if (variant == FORM_FUSED) return init_fused(state, f, B, H, W, stride, IFMap, OFMap);
     if (variant == FORM_PLANES) return init_planes(state, f, B, H, W, stride, IFMap, OFMap);
@@ -1219,7 +1213,7 @@ int shflbw_spconv_exec(const shflbw_spconv_state* state, void* stream)
         return SHFLBW_ERR_STATE;
     }
     hipError_t e = hipSuccess;
-    if (state->patch) {
+    if (state->variant == FORM_PATCH) {
         const auto& pe = *(const shflbw_weight::ConvPatch*)state->patch;
         const ConvPatchKernel* k = conv_patch_kernel(conv_patch_unit_rows(state->brow), pe.plan.col_blocks, pe.plan.waves);
         if (!k) return SHFLBW_ERR_UNSUPPORTED;

@@ -327,12 +327,13 @@ def test_direct_kernel_refuses_inputs_it_cannot_index(torch_gpu):
 
 @pytest.mark.parametrize("Bn,H,expected", [(8, 8, 2), (8, 16, 2), (12, 16, 0), (32, 8, 2), (20, 8, 0)])
 def test_the_library_picks_the_batch_innermost_form_for_batches_of_eights(torch_gpu, Bn, H, expected):
-    """shflbw_spconv_init: form 2 needs a batch that is a multiple of 8; other batches get form 0."""
+    """shflbw_spconv_init where the patch form does not fit the LDS (25 taps of 1024 channels): form 2 needs a batch that is a
+    multiple of 8; other batches get form 0."""
     import shflbw_sparse_nn_amd as S
     torch = torch_gpu
-    C, F = 8, 32
-    w = P.make_weight(F, 9 * C, 32, 0.5, True, 3, integer=True)
-    f = P.upload_weight(w, 3, 3, C, cls=S.BlockwiseSpFilter)
+    C, F = 1024, 32
+    w = P.make_weight(F, 25 * C, 32, 0.01, True, 3, integer=True)
+    f = P.upload_weight(w, 5, 5, C, cls=S.BlockwiseSpFilter)
     dX = torch.zeros((Bn, H, H, C), dtype=torch.float16, device="cuda")
     dY = torch.zeros((Bn, H, H, F), dtype=torch.float16, device="cuda")
     op = S.SpconvBlockwiseOp()
@@ -372,8 +373,9 @@ def test_batch_innermost_form_tile_widths(torch_gpu, Bn, H, C, F, V, tile_cols):
 
 
 def test_library_choice_seeded_random_shapes(torch_gpu):
-    """Twenty-four seeded NHWC problems with the form the library picks (form 2 for batches of eights, form 0 otherwise;
-    the SpMM in the middle with tiles of 128, 256 or 512 columns): filter extents 1..5, strides 1..3, all block heights."""
+    """Twenty-four seeded NHWC problems with the form the library picks (the patch form on all of them, by its estimate) and
+    with the plane form it would pick otherwise (form 2 for batches of eights, form 0 for others; the SpMM in the middle with
+    tiles of 128, 256 or 512 columns): filter extents 1..5, strides 1..3, all block heights."""
     import shflbw_sparse_nn_amd as S
     torch = torch_gpu
     rng = np.random.default_rng(2718)
@@ -392,15 +394,16 @@ def test_library_choice_seeded_random_shapes(torch_gpu):
         ref = O.float_to_half(P.conv_oracle(w, R, S_, C, x, stride))
         f = P.upload_weight(w, R, S_, C, cls=S.BlockwiseSpFilter)
         dX = P.to_dev(torch, x)
-        dY = torch.full(ref.shape, float("nan"), dtype=torch.float16, device="cuda")
-        op = S.SpconvBlockwiseOp()
-        st = op.initialize(f, Bn, H, W, stride, dX.data_ptr(), dY.data_ptr())
-        forms.add(st.variant)
-        print("case", case, (Bn, H, W, C, F, R, S_, stride, V, d), "form", st.variant, "tiles of", st.middle_tile_cols, flush=True)
-        assert op.output_hw == ref.shape[1:3]
-        op(torch.cuda.current_stream().cuda_stream)
-        torch.cuda.synchronize()
-        op.check()
-        np.testing.assert_array_equal(dY.cpu().numpy().view(np.uint16), ref.view(np.uint16), err_msg="case %d" % case)
-    assert forms == {0, 2}
-
+        for variant in (-1, 2 if Bn % 8 == 0 else 0):
+            dY = torch.full(ref.shape, float("nan"), dtype=torch.float16, device="cuda")
+            op = S.SpconvBlockwiseOp(variant)
+            st = op.initialize(f, Bn, H, W, stride, dX.data_ptr(), dY.data_ptr())
+            forms.add(st.variant)
+            print("case", case, (Bn, H, W, C, F, R, S_, stride, V, d), "form", st.variant, "tiles of", st.middle_tile_cols, flush=True)
+            assert st.variant == (5 if variant < 0 else variant)
+            assert op.output_hw == ref.shape[1:3]
+            op(torch.cuda.current_stream().cuda_stream)
+            torch.cuda.synchronize()
+            op.check()
+            np.testing.assert_array_equal(dY.cpu().numpy().view(np.uint16), ref.view(np.uint16), err_msg="case %d" % case)
+    assert forms == {0, 2, 5}

@@ -67,8 +67,8 @@ def test_empty_panels_and_non_finite_input(torch_gpu, V):
 
 
 def test_the_library_runs_it_and_it_needs_no_buffers(torch_gpu):
-    """shflbw_spconv_init takes the patch form on an ordinary layer (the state keeps naming the plane form it stands in
-    for); states over many tensors share its tables; weights of too many channels for the LDS keep the plane form."""
+    """shflbw_spconv_init takes the patch form on an ordinary layer and the state says so; states over many tensors share its tables;
+    weights of too many channels for the LDS keep the plane form."""
     torch = torch_gpu
     w = P.make_weight(64, 9 * 64, 32, 0.2, True, 3, integer=True)
     f = P.upload_weight(w, 3, 3, 64, cls=S.BlockwiseSpFilter)
@@ -78,7 +78,7 @@ def test_the_library_runs_it_and_it_needs_no_buffers(torch_gpu):
         op = S.SpconvBlockwiseOp()
         y = torch.full((8, 14, 14, 64), float("nan"), dtype=torch.float16, device="cuda")
         st = op.initialize(f, 8, 14, 14, 1, x.data_ptr(), y.data_ptr())
-        assert st.patch and st.variant == 2
+        assert st.patch and st.variant == PATCH and S.spconv_variant_name(st.variant) == "patch"
         op(torch.cuda.current_stream().cuda_stream)
         ops.append((op, y))
     torch.cuda.synchronize()
@@ -105,7 +105,7 @@ def test_variant_5_runs_where_the_library_would_not_choose_it(torch_gpu, Bn, H, 
         dY = torch.full(ref.shape, float("nan"), dtype=torch.float16, device="cuda")
         op = S.SpconvBlockwiseOp(variant)
         st = op.initialize(f, Bn, H, H, stride, dX.data_ptr(), dY.data_ptr())
-        assert bool(st.patch) == (variant == PATCH)
+        assert (st.variant == PATCH) == (variant == PATCH) and st.variant in (0, PATCH)
         op(torch.cuda.current_stream().cuda_stream)
         torch.cuda.synchronize()
         np.testing.assert_array_equal(dY.cpu().numpy().view(np.uint16), ref.view(np.uint16))
