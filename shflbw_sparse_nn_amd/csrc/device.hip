@@ -997,16 +997,23 @@ int conv_patch_for(shflbw_weight* fw, int B, int H, int W, int stride, int Ho, i
         const size_t held = batches + CONV_PATCH_TAIL_BATCHES;
         const size_t o_offs = up256(held * 32 * RW * sizeof(uint16_t)), o_first = o_offs + up256(held * 32 * sizeof(uint16_t));
         const size_t o_filt = o_first + up256((size_t)(nunits + 1) * sizeof(int)), o_dst = o_filt + up256((size_t)F * sizeof(int));
-        e.bytes = o_dst + up256((size_t)F * sizeof(unsigned short));
+        const size_t o_src = o_dst + up256((size_t)F * sizeof(unsigned short));
+        e.bytes = o_src + up256(batches * 32 * sizeof(int));
         // (an image beyond three quarters of an XCD's L2 is left to the ring past that)
         e.plan.touch_bytes = (unsigned)std::min<size_t>(o_filt, 3u << 20) - 4;
         e.plan.touch_step = (unsigned)(p.jobs_per_xcd * p.waves * 64) * 128u;
-        std::vector<unsigned char> h(e.bytes, 0);
-        uint16_t* A = (uint16_t*)h.data();
-        uint16_t* offs = (uint16_t*)(h.data() + o_offs);
-        int* first = (int*)(h.data() + o_first);
-        int* filt = (int*)(h.data() + o_filt);
-        unsigned short* dst = (unsigned short*)(h.data() + o_dst);
+        // The fragments, many times the size of the tables, are packed on the device from the weight's values once packing and
+        // copying them costs more than a launch and a wait (first initialisation of a filter, fragments packed on the host / on
+        // the device: 72 KB 29 / 43 us, 144 KB 38 / 48, 288 KB 59 / 58 and 47 / 47, 576 KB 79 / 59, 1843 KB 329 / 211).
+        const bool on_host = o_offs <= 256u << 10;
+        const size_t o_host = on_host ? 0 : o_offs; // what is made here starts there
+        std::vector<unsigned char> h(e.bytes - o_host, 0);
+        uint16_t* A = (uint16_t*)h.data(); // on_host
+        uint16_t* offs = (uint16_t*)(h.data() + (o_offs - o_host));
+        int* first = (int*)(h.data() + (o_first - o_host));
+        int* filt = (int*)(h.data() + (o_filt - o_host));
+        unsigned short* dst = (unsigned short*)(h.data() + (o_dst - o_host));
+        int* src = (int*)(h.data() + (o_src - o_host));
         // bank pairs the positions one pass of a transposing read touches lie in, for a row that starts in pair 0
         const int group = RW == 16 ? 8 : 4, quads = 32 / group;
         uint32_t foot = 0;
@@ -1015,40 +1022,46 @@ int conv_patch_for(shflbw_weight* fw, int B, int H, int W, int stride, int Ho, i
             if (i < p.tile_h) foot |= 1u << ((i * p.step_h * p.patch_w + j * p.step_w) & 31);
         }
         // slots of the groups a batch's reads are made of, group after group: a pass reads slots 8 (lane / 16 or
-        // lane / 32) + 0..3 of a step, the second read of a fragment the four behind them
-        int slot_of[32];
-        for (int t = 0; t < 32; t++)
-            slot_of[t] = RW == 16 ? (t / 16) * 16 + ((t / 8) & 1) * 4 + ((t / 4) & 1) * 8 + t % 4 : t;
+        // lane / 32) + 0..3 of a step, the second read of a fragment the four behind them.  A lane addresses slots s and
+        // s + 4 of a step and loads the offsets of all steps of a batch at once.
+        int slot_of[32], place_of[32];
+        for (int t = 0; t < 32; t++) {
+            const int s = RW == 16 ? (t / 16) * 16 + ((t / 8) & 1) * 4 + ((t / 4) & 1) * 8 + t % 4 : t;
+            const int in_step = RW == 16 ? s : s % 16, step = RW == 16 ? 0 : s / 16;
+            const int pair = (in_step / 8) * 4 + in_step % 4, hi = (in_step % 8) / 4;
+            slot_of[t] = s;
+            place_of[t] = RW == 16 ? pair * 2 + hi : pair * 4 + step * 2 + hi;
+        }
+        // LDS offset (in 8 bytes) of every column, tap after tap
+        std::vector<uint16_t> at(fw->ncol);
+        for (int r = 0, k = 0; r < fw->R; r++)
+            for (int t = 0; t < S; t++)
+                for (int c = 0; c < C; c++, k++) at[k] = (uint16_t)((c * p.pitch >> 3) + r * p.patch_w + t);
+        const uint16_t zero_row = (uint16_t)(C * p.pitch >> 3);
+        const ConvPatchOrder keep_apart(foot, group);
         std::vector<int> pair_of, order;
         static const uint16_t zeros[64] = {};
         size_t b = 0;
         for (int panel = 0; panel < X; panel++) {
             const int begin = fw->indptr[panel], nnz = fw->indptr[panel + 1] - begin;
-            auto offset_of = [&](int k) {
-                const int c = k % C, tap = k / C;
-                return c * p.pitch + ((tap / S) * p.patch_w + tap % S) * 8;
-            };
             pair_of.resize(nnz);
-            for (int i = 0; i < nnz; i++) pair_of[i] = (offset_of(fw->indices[begin + i]) >> 3) & 31;
-            conv_patch_order(pair_of, foot, group, order);
+            for (int i = 0; i < nnz; i++) pair_of[i] = at[fw->indices[begin + i]] & 31;
+            keep_apart.of(pair_of, order);
             for (int part = 0; part < per_panel; part++) {
                 first[panel * per_panel + part] = (int)b;
                 for (int t0 = 0; t0 < nnz; t0 += 32) {
                     uint16_t* o = offs + (b + t0 / 32) * 32;
-                    uint16_t* a = A + (b + t0 / 32) * 32 * RW;
-                    const uint16_t* src[32];
+                    int* from = src + (b + t0 / 32) * 32;
                     for (int t = 0; t < 32; t++) {
-                        const int s = slot_of[t], in_step = RW == 16 ? s : s % 16, step = RW == 16 ? 0 : s / 16;
-                        const int pair = (in_step / 8) * 4 + in_step % 4, hi = (in_step % 8) / 4;
                         const bool held = t0 + t < nnz;
-                        const int i = held ? order[t0 + t] : 0;
-                        // a lane addresses slots s and s + 4 of a step and loads the offsets of all steps of a batch at once
-                        o[RW == 16 ? pair * 2 + hi : pair * 4 + step * 2 + hi] = (uint16_t)((held ? offset_of(fw->indices[begin + i]) : C * p.pitch) >> 3);
-                        src[s] = held ? fw->values.data() + (size_t)(begin + i) * V + part * RW : zeros;
+                        const int i = begin + (held ? order[t0 + t] : 0);
+                        o[place_of[t]] = held ? at[fw->indices[i]] : zero_row;
+                        from[slot_of[t]] = held ? i * per_panel + part : -1;
                     }
-                    for (int s = 0; s < 32; s += 8) {
+                    for (int s = 0; on_host && s < 32; s += 8) {
                         const uint16_t* v[8];
-                        for (int j = 0; j < 8; j++) v[j] = src[s + j];
+                        for (int j = 0; j < 8; j++) v[j] = from[s + j] < 0 ? zeros : fw->values.data() + (size_t)from[s + j] * RW;
+                        uint16_t* a = A + (b + t0 / 32) * 32 * RW;
                         if (RW == 16) {
                             interleave8(v, 16, a + (s / 8) * 16 * 8);
                             continue;
@@ -1063,21 +1076,23 @@ int conv_patch_for(shflbw_weight* fw, int B, int H, int W, int stride, int Ho, i
             }
         }
         first[nunits] = (int)b;
-        for (int row0 = 0; row0 < F; row0 += p.rows_wg) {
-            const int rows = std::min(p.rows_wg, F - row0);
-            order.resize(rows);
-            for (int i = 0; i < rows; i++) order[i] = i;
-            auto filter_of = [&](int i) { return fw->row_permute ? fw->row_permute_ids[row0 + i] : row0 + i; };
-            std::sort(order.begin(), order.end(), [&](int x, int y) { return filter_of(x) < filter_of(y); });
-            for (int place = 0; place < rows; place++) {
-                filt[row0 + place] = filter_of(order[place]);
-                dst[row0 + order[place]] = (unsigned short)place;
-            }
+        // places of a chunk's rows: filters in ascending order
+        std::vector<int> row_of(F), next(p.chunks, 0);
+        for (int i = 0; i < F; i++) row_of[fw->row_permute ? fw->row_permute_ids[i] : i] = i;
+        for (int filter = 0; filter < F; filter++) {
+            const int chunk = row_of[filter] / p.rows_wg, place = next[chunk]++;
+            filt[chunk * p.rows_wg + place] = filter;
+            dst[row_of[filter]] = (unsigned short)place;
         }
         SHFLBW_HIP_TRY(hipMalloc(&e.ptr, e.bytes));
-        if (hipMemcpy(e.ptr, h.data(), e.bytes, hipMemcpyHostToDevice) != hipSuccess) {
+        hipError_t err = hipMemcpy((char*)e.ptr + o_host, h.data(), h.size(), hipMemcpyHostToDevice);
+        if (err == hipSuccess && !on_host) {
+            err = launch_patch_pack((const half_t*)fw->d_values, (const int*)((char*)e.ptr + o_src), (half8_t*)e.ptr, RW, batches, nullptr);
+            if (err == hipSuccess) err = hipStreamSynchronize(nullptr); // any stream may launch on the image
+        }
+        if (err != hipSuccess) {
             (void)hipFree(e.ptr);
-            set_error("spconv_init: cannot upload the offsets of the patch form");
+            set_error("spconv_init: cannot build the tables of the patch form: %s", hipGetErrorString(err));
             return SHFLBW_ERR_HIP;
         }
         e.packedA = e.ptr;

@@ -49,7 +49,18 @@ struct ConvPatchProblem {
 bool conv_patch_plan(const ConvPatchProblem& q, ConvPatchPlan* plan);
 
 // Order of the kept columns of a row panel that keeps the LDS reads of a group of rows apart (see the definition).
-void conv_patch_order(const std::vector<int>& pair_of, uint32_t foot, int group, std::vector<int>& order);
+struct ConvPatchOrder {
+    ConvPatchOrder(uint32_t foot, int group);
+    // pair_of: start pairs of the kept columns; `order` becomes their order, whole groups of `group` at a time
+    void of(const std::vector<int>& pair_of, std::vector<int>& order) const;
+
+private:
+    uint32_t foot;
+    int group;
+    std::vector<std::vector<int>> tilings; // up to three exact ones, as shifts
+    uint32_t touching(uint32_t set) const;
+    void find_tilings(std::vector<int>& shifts, uint32_t used);
+};
 
 struct ConvPatchArgs {
     ConvPatchPlan p;
@@ -64,6 +75,10 @@ struct ConvPatchArgs {
     const int* filt;               // per chunk and place: the filter (used when not dense)
     int dense;                     // the filters of a chunk are consecutive in the output
 };
+
+// Packs the A fragments of `batches` batches from the weight's values (kept vectors one behind the other).  src: per batch and
+// slot the row unit's part of a kept vector, as a multiple of `rows` values; -1: zeros (a padding slot).
+hipError_t launch_patch_pack(const half_t* values, const int* src, half8_t* packedA, int rows, size_t batches, hipStream_t stream);
 
 struct ConvPatchKernel {
     int RW, col_blocks, waves;

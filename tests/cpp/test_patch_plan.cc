@@ -81,11 +81,90 @@ int reads_stay_inside()
     return bad + (taken < 5000);
 }
 
+// The order of a panel's kept columns by the rule as it is stated at ConvPatchOrder, one start pair at a time.
+struct PlainOrder {
+    uint32_t foot;
+    int group;
+
+    uint32_t row(int s) const { return s ? (foot << s) | (foot >> (32 - s)) : foot; }
+
+    void tilings(std::vector<int>& shifts, uint32_t used, std::vector<std::vector<int>>& found) const
+    {
+        if ((int)shifts.size() == group) {
+            found.push_back(shifts);
+            return;
+        }
+        const uint32_t lowest = ~used & (used + 1);
+        for (int s = 1; s < 32 && found.size() < 3; s++)
+            if ((row(s) & lowest) && !(row(s) & used)) {
+                shifts.push_back(s);
+                tilings(shifts, used | row(s), found);
+                shifts.pop_back();
+            }
+    }
+
+    std::vector<int> of(const std::vector<int>& pair_of) const
+    {
+        std::vector<int> order;
+        std::vector<std::vector<int>> left(32), found;
+        for (size_t i = pair_of.size(); i-- > 0;) left[pair_of[i]].push_back((int)i);
+        auto take = [&](int s) { order.push_back(left[s].back()), left[s].pop_back(); };
+        std::vector<int> shifts{0};
+        tilings(shifts, foot, found);
+        while (true) { // the tiling and shift whose scarcest member has the most rows left, the first of equals
+            int best = 0, at = 0, shift = 0;
+            for (size_t t = 0; t < found.size(); t++)
+                for (int s = 0; s < 32; s++) {
+                    int least = 1 << 30;
+                    for (int d : found[t]) least = std::min(least, (int)left[(s + d) & 31].size());
+                    if (least > best) best = least, at = (int)t, shift = s;
+                }
+            if (!best) break;
+            for (; best > 0; best--)
+                for (int d : found[at]) take((shift + d) & 31);
+        }
+        while (order.size() < pair_of.size()) { // a row that meets the fewest rows of its group; of those the one with most rows left
+            std::vector<int> touched(32, 0);
+            for (int g = 0; g < group && order.size() < pair_of.size(); g++) {
+                int pick = -1, meets = 0;
+                for (int s = 0; s < 32; s++) {
+                    if (left[s].empty()) continue;
+                    int worst = 0;
+                    for (int b = 0; b < 32; b++)
+                        if (row(s) >> b & 1) worst = std::max(worst, touched[b]);
+                    if (pick < 0 || worst < meets || (worst == meets && left[s].size() > left[pick].size())) pick = s, meets = worst;
+                }
+                for (int b = 0; b < 32; b++) touched[b] += row(pick) >> b & 1;
+                take(pick);
+            }
+        }
+        return order;
+    }
+};
+
+int orders_follow_the_rule()
+{
+    std::mt19937 rng(7);
+    int bad = 0;
+    for (int t = 0; t < 3000; t++) {
+        const int group = rng() % 2 ? 4 : 8, n = (int)(rng() % (t % 10 ? 90 : 700)), step = 1 + (int)(rng() % 31);
+        uint32_t foot = 0; // a row of positions `step` pairs apart, or (one in four) positions anywhere
+        for (int i = 0; i < 32 / group; i++) foot |= 1u << (t % 4 ? i * step & 31 : (int)(rng() % 32));
+        std::vector<int> pair_of(n), order;
+        const int spread = rng() % 3 ? 32 : 1 + (int)(rng() % 32); // some panels keep few start pairs
+        for (int& s : pair_of) s = (int)(rng() % spread);
+        ConvPatchOrder(foot, group).of(pair_of, order);
+        if (order != PlainOrder{foot, group}.of(pair_of) && bad++ < 5) printf("Failed: order of %d rows, foot %08x, groups of %d\n", n, foot, group);
+    }
+    printf("orders: %d differ from the rule\n", bad);
+    return bad;
+}
+
 } // namespace
 
 int main()
 {
-    const int bad = reads_stay_inside();
+    const int bad = reads_stay_inside() + orders_follow_the_rule();
     printf(bad ? "FAILED\n" : "ALL PASSED\n");
     return bad != 0;
 }

@@ -116,3 +116,29 @@ def test_variant_5_is_refused_where_no_patch_fits(torch_gpu):
     with pytest.raises(S.capi.ShflbwError) as e:
         run_spconv(torch_gpu, w, 5, 5, 1024, np.zeros((1, 8, 8, 1024), dtype=np.float16), 1, PATCH)
     assert e.value.status == S.capi.ERR_UNSUPPORTED and "LDS" in str(e.value)
+
+
+@pytest.mark.parametrize("Bn,H,C,F,V,d,stride", [(1, 28, 128, 128, 32, 0.25, 1), (16, 14, 512, 2048, 64, 0.1, 1),
+                                                 (32, 28, 256, 512, 32, 0.3, 2), (16, 28, 64, 256, 16, 0.25, 1)])
+def test_first_initialisation_of_a_filter_costs_no_more_than_the_plane_form(torch_gpu, Bn, H, C, F, V, d, stride):
+    """A program that meets a new filter pays for its tables in the call: planning, ordering and packing the patch form's
+    image stay below what the plane form's first initialisation takes (medians over new filters, in turn, which stay alive as
+    those of a network do; half as much again is allowed for noise of the host)."""
+    import time
+    torch = torch_gpu
+    w = P.make_weight(F, 9 * C, V, d, True, 3, integer=True)
+    dX = torch.zeros((Bn, H, H, C), dtype=torch.float16, device="cuda")
+    dY = torch.zeros((Bn, H, H, F), dtype=torch.float16, device="cuda")
+    took, alive = {PATCH: [], 0: []}, []
+    for _ in range(31):
+        for variant in took:
+            f = P.upload_weight(w, 3, 3, C, cls=S.BlockwiseSpFilter)
+            op = S.SpconvBlockwiseOp(variant)
+            alive.append(op)
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            op.initialize(f, Bn, H, H, stride, dX.data_ptr(), dY.data_ptr())
+            took[variant].append(time.perf_counter() - t)
+    patch, planes = (np.median(took[v][10:]) * 1e6 for v in (PATCH, 0))
+    print("first initialisation: patch form %.0f us, plane form %.0f us" % (patch, planes), flush=True)
+    assert patch < 1.5 * planes
