@@ -218,10 +218,16 @@ const char* shflbw_spmm_variant_name(int brow, int variant);
  *     XCDs (checked at init; SHFLBW_ERR_UNSUPPORTED otherwise).  Its waits are bounded: should one run out the launch still ends,
  *     and shflbw_spconv_check reports it;
  *   variant 5 = patch form, one launch (any batch): a workgroup transposes the input patch under its output pixels
- *     into LDS, runs the products on it and writes NHWC itself.  SHFLBW_ERR_UNSUPPORTED where no patch fits the LDS or
- *     the tensors leave 32-bit indexes.
+ *     into LDS, runs the products on it and writes NHWC itself.  It needs no buffers, but an image of the filter in an order
+ *     that suits the shape of the patch; geometries with patches of one shape share it, and a filter holds at most
+ *     SHFLBW_CONV_PATCH_IMAGES of them, never recycled (each is about as large as the filter's values).  Where they are all
+ *     taken, a geometry gets the best of the shapes that are held, or (the library's choice) a plane form.
+ *     SHFLBW_ERR_UNSUPPORTED where no patch fits the LDS or the tensors leave 32-bit indexes, SHFLBW_ERR_CAPACITY where no
+ *     image that is held fits and there is no room for another (shflbw_weight_release_scratch makes room).
  * ------------------------------------------------------------------------- */
 #define SHFLBW_CONV_SCRATCH_DEPTH 4
+#define SHFLBW_CONV_PATCH_IMAGES 16
+#define SHFLBW_PATCH_LAUNCH_WORDS 40
 typedef struct shflbw_spconv_state {
     size_t shared_mem_size;
     unsigned grid_dim[3];
@@ -266,7 +272,8 @@ typedef struct shflbw_spconv_state {
                          * workgroup joins min(t, 10000) ticks late.  The int at byte 60 of `sync` counts the take-overs. */
     void* sync;
     shflbw_spmm_state spmm;
-    const void* patch; /* patch form: its cut and tables for this geometry, owned by the filter; NULL for the other forms */
+    const void* patch; /* patch form: the image of the filter it reads (device memory owned by the filter); NULL for the other forms */
+    unsigned long long patch_launch[SHFLBW_PATCH_LAUNCH_WORDS]; /* patch form, private: how exec launches it */
 } shflbw_spconv_state;
 
 int shflbw_spconv_init(shflbw_spconv_state* state, const shflbw_weight* filter,

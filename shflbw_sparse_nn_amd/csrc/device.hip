@@ -11,6 +11,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "shflbw.h"
@@ -47,11 +48,15 @@ void release_conv_scratch(shflbw_weight* w)
         if (e.ptr) (void)hipFree(e.ptr);
     for (auto& e : w->conv_bulk)
         if (e.ptr) (void)hipFree(e.ptr);
-    for (auto& e : w->conv_patch)
+    for (auto& e : w->patch_images)
+        if (e.ptr) (void)hipFree(e.ptr);
+    for (auto& e : w->patch_places)
         if (e.ptr) (void)hipFree(e.ptr);
     w->conv_ids.clear();
     w->conv_bulk.clear();
-    w->conv_patch.clear();
+    w->patch_images.clear();
+    w->patch_places.clear();
+    w->patch_geometries.clear();
 }
 
 // One allocation and one copy for all arrays of a weight (seven of each cost more than packing a small weight).
@@ -966,143 +971,213 @@ int init_fused(shflbw_spconv_state* state, const shflbw_weight* f, int B, int H,
     return SHFLBW_OK;
 }
 
-// The patch form of one geometry of a filter: cut, LDS offsets of the kept columns and places of the rows in the output,
-// built and uploaded on the first call that takes a geometry, found afterwards.  *out is null when no patch fits and, unless
-// `forced`, when the plane forms are estimated faster.
-int conv_patch_for(shflbw_weight* fw, int B, int H, int W, int stride, int Ho, int Wo, bool forced, const shflbw_weight::ConvPatch** out)
+// The filters of every workgroup of `rows_wg` rows in output order, and the place of each row among them.
+void fill_patch_places(const shflbw_weight* fw, int rows_wg, int* filt, unsigned short* dst)
+{
+    const int F = fw->F;
+    std::vector<int> row_of(F), next((F + rows_wg - 1) / rows_wg, 0);
+    for (int i = 0; i < F; i++) row_of[fw->row_permute ? fw->row_permute_ids[i] : i] = i;
+    for (int filter = 0; filter < F; filter++) {
+        const int chunk = row_of[filter] / rows_wg, place = next[chunk]++;
+        filt[chunk * rows_wg + place] = filter;
+        dst[row_of[filter]] = (unsigned short)place;
+    }
+}
+
+const shflbw_weight::PatchPlaces* find_patch_places(const shflbw_weight* fw, int rows_wg)
+{
+    for (auto& e : fw->patch_places)
+        if (e.rows_wg == rows_wg) return &e;
+    return nullptr;
+}
+
+// The places of a cut: found, or built and uploaded.  The caller holds the weight's scratch_lock.
+int patch_places_for(shflbw_weight* fw, int rows_wg, const shflbw_weight::PatchPlaces** out)
+{
+    if ((*out = find_patch_places(fw, rows_wg))) return SHFLBW_OK;
+    shflbw_weight::PatchPlaces e{rows_wg, nullptr, 0, nullptr, nullptr};
+    const size_t o_dst = up256((size_t)fw->F * sizeof(int));
+    e.bytes = o_dst + up256((size_t)fw->F * sizeof(unsigned short));
+    std::vector<unsigned char> h(e.bytes, 0);
+    fill_patch_places(fw, rows_wg, (int*)h.data(), (unsigned short*)(h.data() + o_dst));
+    SHFLBW_HIP_TRY(hipMalloc(&e.ptr, e.bytes));
+    if (hipMemcpy(e.ptr, h.data(), e.bytes, hipMemcpyHostToDevice) != hipSuccess) {
+        (void)hipFree(e.ptr);
+        set_error("spconv_init: cannot upload the output places of the patch form");
+        return SHFLBW_ERR_HIP;
+    }
+    e.filt = (const int*)e.ptr;
+    e.dst = (const unsigned short*)((const char*)e.ptr + o_dst);
+    fw->patch_places.push_back(e);
+    *out = &fw->patch_places.back();
+    return SHFLBW_OK;
+}
+
+// The filter as the patch form reads it, for patches of the shape of `p`: built on the first call for a shape, found
+// afterwards; null in *out where CONV_PATCH_IMAGES others are held.  With it go the places of that cut, one copy for both.  The
+// caller holds the weight's scratch_lock.
+int patch_image_for(shflbw_weight* fw, const ConvPatchPlan& p, const shflbw_weight::PatchImage** out)
 {
     *out = nullptr;
-    std::lock_guard<std::mutex> scratch_guard(fw->scratch_lock);
     const int V = fw->brow, X = fw->nrow / V, F = fw->F, C = fw->C, S = fw->S;
-    shflbw_weight::ConvPatch* known = nullptr;
-    for (auto& c : fw->conv_patch)
-        if (c.key[0] == B && c.key[1] == H && c.key[2] == W && c.key[3] == stride) known = &c;
-    if (!known) {
-        const ConvPatchProblem q{V, F, C, fw->R, S, (double)fw->nnzb / X, fw->row_permute ? 1 : 0, B, H, W, Ho, Wo, stride, device_compute_units()};
-        shflbw_weight::ConvPatch c{};
-        c.key[0] = B, c.key[1] = H, c.key[2] = W, c.key[3] = stride;
-        conv_patch_plan(q, &c.plan);
-        fw->conv_patch.push_back(c);
-        known = &fw->conv_patch.back();
+    const int RW = conv_patch_unit_rows(V), per_panel = V / RW, nunits = F / RW;
+    const ConvPatchShape shape = conv_patch_shape(RW, p);
+    for (auto& e : fw->patch_images)
+        if (e.shape == shape) {
+            *out = &e;
+            return SHFLBW_OK;
+        }
+    if ((int)fw->patch_images.size() >= shflbw_weight::CONV_PATCH_IMAGES) return SHFLBW_OK;
+    shflbw_weight::PatchImage e{};
+    e.shape = shape;
+    size_t batches = 0;
+    for (int i = 0; i < X; i++) batches += (size_t)((fw->indptr[i + 1] - fw->indptr[i] + 31) / 32) * per_panel;
+    const size_t held = batches + CONV_PATCH_TAIL_BATCHES;
+    const size_t o_offs = up256(held * 32 * RW * sizeof(uint16_t)), o_first = o_offs + up256(held * 32 * sizeof(uint16_t));
+    const size_t o_filt = o_first + up256((size_t)(nunits + 1) * sizeof(int)), o_dst = o_filt + up256((size_t)F * sizeof(int));
+    const size_t o_src = o_dst + up256((size_t)F * sizeof(unsigned short));
+    e.bytes = o_src + up256(batches * 32 * sizeof(int));
+    e.touch = o_filt;
+    // The fragments, many times the size of the tables, are packed on the device from the weight's values once packing and
+    // copying them costs more than a launch and a wait (first initialisation of a filter, fragments packed on the host / on
+    // the device: 72 KB 29 / 43 us, 144 KB 38 / 48, 288 KB 59 / 58 and 47 / 47, 576 KB 79 / 59, 1843 KB 329 / 211).
+    const bool on_host = o_offs <= 256u << 10;
+    const size_t o_host = on_host ? 0 : o_offs; // what is made here starts there
+    std::vector<unsigned char> h(e.bytes - o_host, 0);
+    uint16_t* A = (uint16_t*)h.data(); // on_host
+    uint16_t* offs = (uint16_t*)(h.data() + (o_offs - o_host));
+    int* first = (int*)(h.data() + (o_first - o_host));
+    int* src = (int*)(h.data() + (o_src - o_host));
+    // slots of the groups a batch's reads are made of, group after group: a pass reads slots 8 (lane / 16 or
+    // lane / 32) + 0..3 of a step, the second read of a fragment the four behind them.  A lane addresses slots s and
+    // s + 4 of a step and loads the offsets of all steps of a batch at once.
+    int slot_of[32], place_of[32];
+    for (int t = 0; t < 32; t++) {
+        const int s = RW == 16 ? (t / 16) * 16 + ((t / 8) & 1) * 4 + ((t / 4) & 1) * 8 + t % 4 : t;
+        const int in_step = RW == 16 ? s : s % 16, step = RW == 16 ? 0 : s / 16;
+        const int pair = (in_step / 8) * 4 + in_step % 4, hi = (in_step % 8) / 4;
+        slot_of[t] = s;
+        place_of[t] = RW == 16 ? pair * 2 + hi : pair * 4 + step * 2 + hi;
     }
-    if (!known->plan.valid || !(forced || known->plan.preferred)) return SHFLBW_OK;
-    if (!known->ptr) {
-        shflbw_weight::ConvPatch e = *known;
-        const ConvPatchPlan& p = e.plan;
-        const int RW = conv_patch_unit_rows(V), per_panel = V / RW, nunits = F / RW;
-        SHFLBW_HIP_TRY(conv_patch_kernel(RW, p.col_blocks, p.waves)->prepare());
-        e.dense = !fw->row_permute || p.chunks == 1;
-        size_t batches = 0;
-        for (int i = 0; i < X; i++) batches += (size_t)((fw->indptr[i + 1] - fw->indptr[i] + 31) / 32) * per_panel;
-        const size_t held = batches + CONV_PATCH_TAIL_BATCHES;
-        const size_t o_offs = up256(held * 32 * RW * sizeof(uint16_t)), o_first = o_offs + up256(held * 32 * sizeof(uint16_t));
-        const size_t o_filt = o_first + up256((size_t)(nunits + 1) * sizeof(int)), o_dst = o_filt + up256((size_t)F * sizeof(int));
-        const size_t o_src = o_dst + up256((size_t)F * sizeof(unsigned short));
-        e.bytes = o_src + up256(batches * 32 * sizeof(int));
-        // (an image beyond three quarters of an XCD's L2 is left to the ring past that)
-        e.plan.touch_bytes = (unsigned)std::min<size_t>(o_filt, 3u << 20) - 4;
-        e.plan.touch_step = (unsigned)(p.jobs_per_xcd * p.waves * 64) * 128u;
-        // The fragments, many times the size of the tables, are packed on the device from the weight's values once packing and
-        // copying them costs more than a launch and a wait (first initialisation of a filter, fragments packed on the host / on
-        // the device: 72 KB 29 / 43 us, 144 KB 38 / 48, 288 KB 59 / 58 and 47 / 47, 576 KB 79 / 59, 1843 KB 329 / 211).
-        const bool on_host = o_offs <= 256u << 10;
-        const size_t o_host = on_host ? 0 : o_offs; // what is made here starts there
-        std::vector<unsigned char> h(e.bytes - o_host, 0);
-        uint16_t* A = (uint16_t*)h.data(); // on_host
-        uint16_t* offs = (uint16_t*)(h.data() + (o_offs - o_host));
-        int* first = (int*)(h.data() + (o_first - o_host));
-        int* filt = (int*)(h.data() + (o_filt - o_host));
-        unsigned short* dst = (unsigned short*)(h.data() + (o_dst - o_host));
-        int* src = (int*)(h.data() + (o_src - o_host));
-        // bank pairs the positions one pass of a transposing read touches lie in, for a row that starts in pair 0
-        const int group = RW == 16 ? 8 : 4, quads = 32 / group;
-        uint32_t foot = 0;
-        for (int t = 0; t < quads; t++) {
-            const int i = t / p.row_len, j = t % p.row_len;
-            if (i < p.tile_h) foot |= 1u << ((i * p.step_h * p.patch_w + j * p.step_w) & 31);
-        }
-        // slots of the groups a batch's reads are made of, group after group: a pass reads slots 8 (lane / 16 or
-        // lane / 32) + 0..3 of a step, the second read of a fragment the four behind them.  A lane addresses slots s and
-        // s + 4 of a step and loads the offsets of all steps of a batch at once.
-        int slot_of[32], place_of[32];
-        for (int t = 0; t < 32; t++) {
-            const int s = RW == 16 ? (t / 16) * 16 + ((t / 8) & 1) * 4 + ((t / 4) & 1) * 8 + t % 4 : t;
-            const int in_step = RW == 16 ? s : s % 16, step = RW == 16 ? 0 : s / 16;
-            const int pair = (in_step / 8) * 4 + in_step % 4, hi = (in_step % 8) / 4;
-            slot_of[t] = s;
-            place_of[t] = RW == 16 ? pair * 2 + hi : pair * 4 + step * 2 + hi;
-        }
-        // LDS offset (in 8 bytes) of every column, tap after tap
-        std::vector<uint16_t> at(fw->ncol);
-        for (int r = 0, k = 0; r < fw->R; r++)
-            for (int t = 0; t < S; t++)
-                for (int c = 0; c < C; c++, k++) at[k] = (uint16_t)((c * p.pitch >> 3) + r * p.patch_w + t);
-        const uint16_t zero_row = (uint16_t)(C * p.pitch >> 3);
-        const ConvPatchOrder keep_apart(foot, group);
-        std::vector<int> pair_of, order;
-        static const uint16_t zeros[64] = {};
-        size_t b = 0;
-        for (int panel = 0; panel < X; panel++) {
-            const int begin = fw->indptr[panel], nnz = fw->indptr[panel + 1] - begin;
-            pair_of.resize(nnz);
-            for (int i = 0; i < nnz; i++) pair_of[i] = at[fw->indices[begin + i]] & 31;
-            keep_apart.of(pair_of, order);
-            for (int part = 0; part < per_panel; part++) {
-                first[panel * per_panel + part] = (int)b;
-                for (int t0 = 0; t0 < nnz; t0 += 32) {
-                    uint16_t* o = offs + (b + t0 / 32) * 32;
-                    int* from = src + (b + t0 / 32) * 32;
-                    for (int t = 0; t < 32; t++) {
-                        const bool held = t0 + t < nnz;
-                        const int i = begin + (held ? order[t0 + t] : 0);
-                        o[place_of[t]] = held ? at[fw->indices[i]] : zero_row;
-                        from[slot_of[t]] = held ? i * per_panel + part : -1;
+    // LDS offset (in 8 bytes) of every column, tap after tap
+    std::vector<uint16_t> at(fw->ncol);
+    for (int r = 0, k = 0; r < fw->R; r++)
+        for (int t = 0; t < S; t++)
+            for (int c = 0; c < C; c++, k++) at[k] = (uint16_t)((c * p.pitch >> 3) + r * p.patch_w + t);
+    const uint16_t zero_row = (uint16_t)(C * p.pitch >> 3);
+    const ConvPatchOrder keep_apart(shape.foot, conv_patch_group(RW));
+    std::vector<int> pair_of, order;
+    static const uint16_t zeros[64] = {};
+    size_t b = 0;
+    for (int panel = 0; panel < X; panel++) {
+        const int begin = fw->indptr[panel], nnz = fw->indptr[panel + 1] - begin;
+        pair_of.resize(nnz);
+        for (int i = 0; i < nnz; i++) pair_of[i] = at[fw->indices[begin + i]] & 31;
+        keep_apart.of(pair_of, order);
+        for (int part = 0; part < per_panel; part++) {
+            first[panel * per_panel + part] = (int)b;
+            for (int t0 = 0; t0 < nnz; t0 += 32) {
+                uint16_t* o = offs + (b + t0 / 32) * 32;
+                int* from = src + (b + t0 / 32) * 32;
+                for (int t = 0; t < 32; t++) {
+                    const bool held = t0 + t < nnz;
+                    const int i = begin + (held ? order[t0 + t] : 0);
+                    o[place_of[t]] = held ? at[fw->indices[i]] : zero_row;
+                    from[slot_of[t]] = held ? i * per_panel + part : -1;
+                }
+                for (int s = 0; on_host && s < 32; s += 8) {
+                    const uint16_t* v[8];
+                    for (int j = 0; j < 8; j++) v[j] = from[s + j] < 0 ? zeros : fw->values.data() + (size_t)from[s + j] * RW;
+                    uint16_t* a = A + (b + t0 / 32) * 32 * RW;
+                    if (RW == 16) {
+                        interleave8(v, 16, a + (s / 8) * 16 * 8);
+                        continue;
                     }
-                    for (int s = 0; on_host && s < 32; s += 8) {
-                        const uint16_t* v[8];
-                        for (int j = 0; j < 8; j++) v[j] = from[s + j] < 0 ? zeros : fw->values.data() + (size_t)from[s + j] * RW;
-                        uint16_t* a = A + (b + t0 / 32) * 32 * RW;
-                        if (RW == 16) {
-                            interleave8(v, 16, a + (s / 8) * 16 * 8);
-                            continue;
-                        }
-                        for (int mb = 0; mb < RW / 32; mb++) {
-                            interleave8(v, 32, a + ((size_t)((s / 16) * (RW / 32) + mb) * 64 + (s % 16) / 8 * 32) * 8);
-                            for (int j = 0; j < 8; j++) v[j] += 32;
-                        }
+                    for (int mb = 0; mb < RW / 32; mb++) {
+                        interleave8(v, 32, a + ((size_t)((s / 16) * (RW / 32) + mb) * 64 + (s % 16) / 8 * 32) * 8);
+                        for (int j = 0; j < 8; j++) v[j] += 32;
                     }
                 }
-                b += (nnz + 31) / 32;
             }
+            b += (nnz + 31) / 32;
         }
-        first[nunits] = (int)b;
-        // places of a chunk's rows: filters in ascending order
-        std::vector<int> row_of(F), next(p.chunks, 0);
-        for (int i = 0; i < F; i++) row_of[fw->row_permute ? fw->row_permute_ids[i] : i] = i;
-        for (int filter = 0; filter < F; filter++) {
-            const int chunk = row_of[filter] / p.rows_wg, place = next[chunk]++;
-            filt[chunk * p.rows_wg + place] = filter;
-            dst[row_of[filter]] = (unsigned short)place;
-        }
-        SHFLBW_HIP_TRY(hipMalloc(&e.ptr, e.bytes));
-        hipError_t err = hipMemcpy((char*)e.ptr + o_host, h.data(), h.size(), hipMemcpyHostToDevice);
-        if (err == hipSuccess && !on_host) {
-            err = launch_patch_pack((const half_t*)fw->d_values, (const int*)((char*)e.ptr + o_src), (half8_t*)e.ptr, RW, batches, nullptr);
-            if (err == hipSuccess) err = hipStreamSynchronize(nullptr); // any stream may launch on the image
-        }
-        if (err != hipSuccess) {
-            (void)hipFree(e.ptr);
-            set_error("spconv_init: cannot build the tables of the patch form: %s", hipGetErrorString(err));
-            return SHFLBW_ERR_HIP;
-        }
-        e.packedA = e.ptr;
-        e.offs = (const unsigned short*)((const char*)e.ptr + o_offs);
-        e.first_batch = (const int*)((const char*)e.ptr + o_first);
-        e.filt = (const int*)((const char*)e.ptr + o_filt);
-        e.dst = (const unsigned short*)((const char*)e.ptr + o_dst);
-        *known = e;
     }
-    *out = known;
+    first[nunits] = (int)b;
+    const bool with_places = !find_patch_places(fw, p.rows_wg);
+    if (with_places) fill_patch_places(fw, p.rows_wg, (int*)(h.data() + (o_filt - o_host)), (unsigned short*)(h.data() + (o_dst - o_host)));
+    SHFLBW_HIP_TRY(hipMalloc(&e.ptr, e.bytes));
+    hipError_t err = hipMemcpy((char*)e.ptr + o_host, h.data(), h.size(), hipMemcpyHostToDevice);
+    if (err == hipSuccess && !on_host) {
+        err = launch_patch_pack((const half_t*)fw->d_values, (const int*)((char*)e.ptr + o_src), (half8_t*)e.ptr, RW, batches, nullptr);
+        if (err == hipSuccess) err = hipStreamSynchronize(nullptr); // any stream may launch on the image
+    }
+    if (err != hipSuccess) {
+        (void)hipFree(e.ptr);
+        set_error("spconv_init: cannot build the filter image of the patch form: %s", hipGetErrorString(err));
+        return SHFLBW_ERR_HIP;
+    }
+    e.offs = (const unsigned short*)((const char*)e.ptr + o_offs);
+    e.first_batch = (const int*)((const char*)e.ptr + o_first);
+    fw->patch_images.push_back(e);
+    if (with_places)
+        fw->patch_places.push_back({p.rows_wg, nullptr, 0, (const int*)((const char*)e.ptr + o_filt), (const unsigned short*)((const char*)e.ptr + o_dst)});
+    *out = &fw->patch_images.back();
+    return SHFLBW_OK;
+}
+
+// The cut of one geometry of a filter and its launch arguments, as a copy.  SHFLBW_ERR_UNSUPPORTED when no patch fits or,
+// unless `forced`, the plane forms are estimated faster; SHFLBW_ERR_CAPACITY when that is so only because the filter's images
+// are all taken by other shapes.
+int conv_patch_for(shflbw_weight* fw, int B, int H, int W, int stride, int Ho, int Wo, bool forced, ConvPatchArgs* out)
+{
+    std::lock_guard<std::mutex> scratch_guard(fw->scratch_lock);
+    auto& all = fw->patch_geometries;
+    shflbw_weight::PatchGeometry* g = nullptr;
+    for (auto& e : all)
+        if (e.key[0] == B && e.key[1] == H && e.key[2] == W && e.key[3] == stride) g = &e;
+    const ConvPatchProblem q{fw->brow, fw->F, fw->C, fw->R, fw->S, (double)fw->nnzb / (fw->nrow / fw->brow), fw->row_permute ? 1 : 0,
+                             B, H, W, Ho, Wo, stride, device_compute_units()};
+    if (!g) {
+        if ((int)all.size() < shflbw_weight::CONV_PATCH_GEOMETRIES)
+            g = &*all.insert(all.end(), shflbw_weight::PatchGeometry{});
+        else
+            g = &*std::min_element(all.begin(), all.end(), [](const auto& x, const auto& y) { return x.stamp < y.stamp; });
+        *g = shflbw_weight::PatchGeometry{{B, H, W, stride}, {}, 0, {}, 0};
+        conv_patch_plan(q, &g->plan);
+    }
+    g->stamp = ++fw->bulk_clock;
+    if (!g->plan.valid || !(forced || g->plan.preferred)) return SHFLBW_ERR_UNSUPPORTED;
+    if (!g->bound) {
+        const int RW = conv_patch_unit_rows(fw->brow);
+        ConvPatchPlan plan = g->plan;
+        const shflbw_weight::PatchImage* image = nullptr;
+        int rc = patch_image_for(fw, plan, &image);
+        if (rc != SHFLBW_OK) return rc;
+        if (!image) { // no room for another shape: the best cut among those that are held
+            std::vector<ConvPatchShape> held;
+            for (auto& e : fw->patch_images) held.push_back(e.shape);
+            if (!conv_patch_plan(q, &plan, &held) || !(forced || plan.preferred)) return SHFLBW_ERR_CAPACITY;
+            if ((rc = patch_image_for(fw, plan, &image)) != SHFLBW_OK) return rc;
+        }
+        const shflbw_weight::PatchPlaces* places = nullptr;
+        if ((rc = patch_places_for(fw, plan.rows_wg, &places)) != SHFLBW_OK) return rc;
+        SHFLBW_HIP_TRY(conv_patch_kernel(RW, plan.col_blocks, plan.waves)->prepare());
+        // (an image beyond three quarters of an XCD's L2 is left to the ring past that)
+        plan.touch_bytes = (unsigned)std::min<size_t>(image->touch, 3u << 20) - 4;
+        plan.touch_step = (unsigned)(plan.jobs_per_xcd * plan.waves * 64) * 128u;
+        ConvPatchArgs& a = g->args;
+        a.p = plan;
+        a.C = fw->C, a.F = fw->F, a.R = fw->R, a.S = fw->S;
+        a.in = nullptr, a.out = nullptr; // each launch's own
+        a.packedA = (const half8_t*)image->ptr;
+        a.first_batch = image->first_batch;
+        a.offs = image->offs;
+        a.dst = places->dst;
+        a.filt = places->filt;
+        a.dense = !fw->row_permute || plan.chunks == 1;
+        g->bound = 1;
+    }
+    *out = g->args;
     return SHFLBW_OK;
 }
 
@@ -1112,18 +1187,22 @@ int init_patch(shflbw_spconv_state* state, const shflbw_weight* f, int B, int H,
 {
     int rc = spconv_fill_state(state, f, B, H, W, stride, IFMap, OFMap, FORM_PATCH);
     if (rc != SHFLBW_OK) return rc;
-    const shflbw_weight::ConvPatch* e = nullptr;
-    if ((rc = conv_patch_for(const_cast<shflbw_weight*>(f), B, H, W, stride, state->Ho, state->Wo, forced, &e)) != SHFLBW_OK) return rc;
-    if (!e) {
+    ConvPatchArgs args;
+    rc = conv_patch_for(const_cast<shflbw_weight*>(f), B, H, W, stride, state->Ho, state->Wo, forced, &args);
+    if (rc == SHFLBW_ERR_UNSUPPORTED)
         set_error(forced ? "spconv_init: no input patch of a workgroup fits the LDS (%d channels, %d x %d filter), or the tensors leave 32-bit indexes"
                          : "spconv_init: the patch form does not take this layer (%d channels, %d x %d filter)", f->C, f->R, f->S);
-        return SHFLBW_ERR_UNSUPPORTED;
-    }
-    state->patch = e;
+    if (rc == SHFLBW_ERR_CAPACITY)
+        set_error("spconv_init: the filter holds %d images of the patch form already, none of which suits this layer "
+                  "(shflbw_weight_release_scratch frees them)", shflbw_weight::CONV_PATCH_IMAGES);
+    if (rc != SHFLBW_OK) return rc;
+    static_assert(sizeof(ConvPatchArgs) <= sizeof(state->patch_launch) && std::is_trivially_copyable<ConvPatchArgs>::value, "kept in the state");
+    memcpy(state->patch_launch, &args, sizeof(args));
+    state->patch = args.packedA;
     state->ncols = B * state->Ho * state->Wo;
-    state->shared_mem_size = (size_t)e->plan.lds_bytes;
-    state->grid_dim[0] = (unsigned)e->plan.jobs;
-    state->block_dim[0] = (unsigned)(e->plan.waves * 64);
+    state->shared_mem_size = (size_t)args.p.lds_bytes;
+    state->grid_dim[0] = (unsigned)args.p.jobs;
+    state->block_dim[0] = (unsigned)(args.p.waves * 64);
     state->grid_dim[1] = state->grid_dim[2] = 1;
     state->block_dim[1] = state->block_dim[2] = 1;
     state->init_success = 1;
@@ -1194,7 +1273,7 @@ int shflbw_spconv_init_variant(shflbw_spconv_state* state, const shflbw_weight* 
     // output pixels on), else the plane form
     if (variant < 0) {
         const int rc = init_patch(state, f, B, H, W, stride, IFMap, OFMap, false);
-        if (rc != SHFLBW_ERR_UNSUPPORTED) return rc;
+        if (rc != SHFLBW_ERR_UNSUPPORTED && rc != SHFLBW_ERR_CAPACITY) return rc;
         variant = B % 8 == 0 ? FORM_BPLANES : FORM_PLANES;
     }
     if (variant == FORM_PATCH) return init_patch(state, f, B, H, W, stride, IFMap, OFMap, true);
@@ -1229,17 +1308,12 @@ int shflbw_spconv_exec(const shflbw_spconv_state* state, void* stream)
     }
     hipError_t e = hipSuccess;
     if (state->variant == FORM_PATCH) {
-        const auto& pe = *(const shflbw_weight::ConvPatch*)state->patch;
-        const ConvPatchKernel* k = conv_patch_kernel(conv_patch_unit_rows(state->brow), pe.plan.col_blocks, pe.plan.waves);
-        if (!k) return SHFLBW_ERR_UNSUPPORTED;
         ConvPatchArgs p;
-        p.p = pe.plan;
-        p.C = state->args.C, p.F = state->args.F, p.R = state->args.R, p.S = state->args.S;
+        memcpy(&p, state->patch_launch, sizeof(p));
+        const ConvPatchKernel* k = conv_patch_kernel(conv_patch_unit_rows(state->brow), p.p.col_blocks, p.p.waves);
+        if (!k) return SHFLBW_ERR_UNSUPPORTED;
         p.in = (const half_t*)state->args.IFMap;
         p.out = (half_t*)state->args.OFMap;
-        p.packedA = (const half8_t*)pe.packedA;
-        p.first_batch = pe.first_batch;
-        p.offs = pe.offs, p.dst = pe.dst, p.filt = pe.filt, p.dense = pe.dense;
         e = k->launch(p, (hipStream_t)stream);
         if (e == hipSuccess) return SHFLBW_OK;
         set_error("spconv_exec: launch failed: %s", hipGetErrorString(e));
@@ -1442,9 +1516,11 @@ int shflbw_weight_scratch_bytes(const shflbw_weight* w, size_t* bytes, int* buff
     size_t total = 0;
     for (auto& e : w->conv_ids) total += e.bytes;
     for (auto& e : w->conv_bulk) total += e.bytes;
-    for (auto& e : w->conv_patch) total += e.bytes;
+    for (auto& e : w->patch_images) total += e.bytes;
+    int places = 0; // those that are no part of an image
+    for (auto& e : w->patch_places) total += e.bytes, places += e.ptr != nullptr;
     if (bytes) *bytes = total;
-    if (buffers) *buffers = (int)(w->conv_ids.size() + w->conv_bulk.size() + w->conv_patch.size());
+    if (buffers) *buffers = (int)(w->conv_ids.size() + w->conv_bulk.size() + w->patch_images.size()) + places;
     return SHFLBW_OK;
 }
 

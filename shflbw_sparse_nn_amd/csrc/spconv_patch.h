@@ -45,8 +45,18 @@ struct ConvPatchProblem {
     int permuted;          // rows of the filter are permuted
     int B, H, W, Ho, Wo, stride, cus;
 };
-// Fills `plan`; false when no patch fits the LDS or the sizes leave 32-bit indexes.
-bool conv_patch_plan(const ConvPatchProblem& q, ConvPatchPlan* plan);
+// What the order of a filter image depends on: the patch as the LDS reads walk it.
+struct ConvPatchShape {
+    int pitch, patch_w;
+    uint32_t foot; // bank pairs that the positions one pass of a transposing read touches lie in, for a row that starts in pair 0
+    bool operator==(const ConvPatchShape& o) const { return pitch == o.pitch && patch_w == o.patch_w && foot == o.foot; }
+};
+ConvPatchShape conv_patch_shape(int rows, const ConvPatchPlan& p);
+// rows of one pass of a transposing read: four of 8 positions, for row units of 16 eight of 4
+inline int conv_patch_group(int rows) { return rows == 16 ? 8 : 4; }
+
+// Fills `plan`; false when no patch fits the LDS (with `held`: none of these shapes) or the sizes leave 32-bit indexes.
+bool conv_patch_plan(const ConvPatchProblem& q, ConvPatchPlan* plan, const std::vector<ConvPatchShape>* held = nullptr);
 
 // Order of the kept columns of a row panel that keeps the LDS reads of a group of rows apart (see the definition).
 struct ConvPatchOrder {

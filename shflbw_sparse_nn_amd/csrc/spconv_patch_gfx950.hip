@@ -549,12 +549,22 @@ static double conv_planes_estimate(const ConvPatchProblem& q)
     return 12.0 + kept * n * 2 / 15.1e6 + (in + planes) / 9.2e6 + out / 4.65e6;
 }
 
+ConvPatchShape conv_patch_shape(int rows, const ConvPatchPlan& p)
+{
+    ConvPatchShape shape{p.pitch, p.patch_w, 0};
+    for (int t = 0; t < 32 / conv_patch_group(rows); t++) {
+        const int i = t / p.row_len, j = t % p.row_len;
+        if (i < p.tile_h) shape.foot |= 1u << ((i * p.step_h * p.patch_w + j * p.step_w) & 31);
+    }
+    return shape;
+}
+
 // The cut with the least estimated time: rounds of workgroups times the sum of a workgroup's phases.  The weights come from
 // a fit to 124 layers measured with 20 to 40 cuts each (10 % rms; the cut it picks is 4 % slower than the best one
 // measured on average).  Where the plane forms are estimated faster - many filters over few resident pixels (wide
 // filters over many channels), filters of several workgroups interleaved in the output - the cut is not `preferred`:
 // 7 x 54 x 54 x 584 -> 1024, 5 x 5, stride 2 takes 152 us here, 54 us there; 16 x 14 x 14 x 512 -> 2048 20 and 23 us.
-bool conv_patch_plan(const ConvPatchProblem& q, ConvPatchPlan* plan)
+bool conv_patch_plan(const ConvPatchProblem& q, ConvPatchPlan* plan, const std::vector<ConvPatchShape>* held)
 {
     ConvPatchPlan best{};
     double best_cost = 0;
@@ -586,6 +596,8 @@ bool conv_patch_plan(const ConvPatchProblem& q, ConvPatchPlan* plan)
                 p.patch_w = (tw - 1) * ew + q.S;
                 p.npos = ((th - 1) * eh + q.R) * p.patch_w;
                 p.pitch = 8 * (p.npos | 1);
+                p.step_h = eh, p.step_w = ew;
+                if (held && std::find(held->begin(), held->end(), conv_patch_shape(rw, p)) == held->end()) continue;
                 // the furthest byte a lane reads: the last tap of the last channel, or the row of zeros, under the last
                 // position of a row (positions from tile_w on are no pixels, but are read)
                 const long last_row = std::max((long)q.C * p.pitch, (q.C - 1L) * p.pitch + ((q.R - 1L) * p.patch_w + q.S - 1) * 8);
@@ -644,7 +656,6 @@ bool conv_patch_plan(const ConvPatchProblem& q, ConvPatchPlan* plan)
     best.preferred = best_cost <= conv_planes_estimate(q);
     best.H = H, best.W = W, best.Ho = Ho, best.Wo = Wo, best.stride = q.stride;
     best.pad_h = q.R / 2, best.pad_w = q.S / 2;
-    best.step_h = eh, best.step_w = ew;
     best.skip = q.stride > q.R || q.stride > q.S;
     best.in_bytes = (unsigned)in_bytes;
     best.touch_bytes = best.touch_step = 0; // set with the size of the image
@@ -701,7 +712,7 @@ void ConvPatchOrder::of(const std::vector<int>& pair_of, std::vector<int>& order
     const int n = (int)pair_of.size();
     order.resize(n);
     int* out = order.data();
-    int* const end = out + n;
+    const int* const end = out + n;
     int begin[33] = {}, count[32] = {}; // rows by start pair: by_pair[begin[s] ..], count[s] of them left
     for (int i = 0; i < n; i++) count[pair_of[i]]++;
     for (int s = 0; s < 32; s++) begin[s + 1] = begin[s] + count[s];
@@ -733,7 +744,8 @@ void ConvPatchOrder::of(const std::vector<int>& pair_of, std::vector<int>& order
             for (int d : *with) take((__builtin_ctz(shifts) + d) & 31);
     }
     const uint32_t meets = touching(foot); // the starts of rows that meet the row from pair 0
-    for (int most = (int)left.size() - 1; out < end;) {
+    int most = (int)left.size() - 1;
+    while (out < end) {
         uint32_t level[9] = {}; // level[m]: pairs at least m of the picked rows touch
         uint32_t meeting = 0;   // the starts of rows that meet a picked one
         for (int g = 0; g < group && out < end; g++) {

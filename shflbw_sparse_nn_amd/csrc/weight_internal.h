@@ -2,7 +2,6 @@
 // Host side of the Shfl-BW format: reference block_sparse/spmm/blockwise_format.h:13-68.
 #pragma once
 #include <cstdint>
-#include <list>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -71,22 +70,40 @@ struct shflbw_weight {
         unsigned long long stamp; // value of bulk_clock when it was last handed out
     };
     static constexpr int CONV_BULK_DEPTH = SHFLBW_CONV_SCRATCH_DEPTH;
-    //  * ConvPatch: cut, filter image (in an order of its own) and output places of the patch form, keyed like the ids
-    //    (ptr == null: nothing has taken the form for that geometry); states point at the entries, which stay where they are.
-    struct ConvPatch {
-        int key[4]; // B, H, W, stride
-        shflbw::ConvPatchPlan plan;
-        void* ptr; // fragments | offsets | first batches | filters | places
-        size_t bytes;
-        const void* packedA;
+    //  * PatchImage: the filter as the patch form reads it.  Its order depends on the shape of the patch alone, so
+    //    geometries whose cuts agree in that share it; at most CONV_PATCH_IMAGES exist per weight, and none is recycled:
+    //    states hold its addresses.  (Forty batches and resolutions of one layer need 12 to 14 shapes, five layers tried; with
+    //    room for 8, up to a quarter of them ran another cut than their best, 1.1 times as long on average and 1.6 at worst.)
+    //  * PatchPlaces: the filters of a workgroup in output order, one per number of filters (a handful of powers of two).
+    //  * PatchGeometry: cut and launch arguments of the geometries initialised last, so that a further initialisation plans
+    //    nothing.  States hold copies: an entry may go at any time.
+    struct PatchImage {
+        shflbw::ConvPatchShape shape;
+        void* ptr; // fragments | offsets | first batches | places of the first cut | what the fragments were packed from
+        size_t bytes, touch; // touch: bytes a launch reads
         const int* first_batch;
         const unsigned short* offs;
+    };
+    struct PatchPlaces {
+        int rows_wg;
+        void* ptr; // filters | places; null when they are a part of an image
+        size_t bytes;
         const int* filt;
         const unsigned short* dst;
-        int dense;
     };
+    struct PatchGeometry {
+        int key[4]; // B, H, W, stride
+        shflbw::ConvPatchPlan plan;
+        int bound;  // args are those of the plan; 0: nothing has taken the form for that geometry
+        shflbw::ConvPatchArgs args;
+        unsigned long long stamp;
+    };
+    static constexpr int CONV_PATCH_IMAGES = SHFLBW_CONV_PATCH_IMAGES;
+    static constexpr int CONV_PATCH_GEOMETRIES = 64;
+    std::vector<PatchImage> patch_images;
+    std::vector<PatchPlaces> patch_places;
+    std::vector<PatchGeometry> patch_geometries;
     std::vector<ConvIds> conv_ids;
-    std::list<ConvPatch> conv_patch;
     std::vector<ConvBulk> conv_bulk;
     unsigned long long bulk_clock = 0;
     std::mutex scratch_lock;

@@ -160,11 +160,43 @@ int orders_follow_the_rule()
     return bad;
 }
 
+// With shapes to choose from, the plan has one of them; with its own shape among them it is the plan it would be without.
+int plans_keep_to_held_shapes()
+{
+    std::mt19937 rng(99);
+    int bad = 0, other = 0;
+    for (int t = 0; t < 3000; t++) {
+        Layer l = random_layer(rng);
+        const ConvPatchProblem q = problem(l);
+        const int rows = conv_patch_unit_rows(l.V);
+        ConvPatchPlan free{}, p{};
+        if (!conv_patch_plan(q, &free)) continue;
+        const ConvPatchShape own = conv_patch_shape(rows, free);
+        std::vector<ConvPatchShape> held;
+        if (conv_patch_plan(q, &p, &held)) bad++;
+        // shapes of the same layer over other maps, as a filter that serves them holds them
+        for (int i = 0; i < 4; i++) {
+            Layer m = l;
+            m.B = 1 + (int)(rng() % 64), m.H = l.R + (int)(rng() % 40), m.W = l.S + (int)(rng() % 40);
+            if (conv_patch_plan(problem(m), &p) && !(conv_patch_shape(rows, p) == own)) held.push_back(conv_patch_shape(rows, p));
+        }
+        if (conv_patch_plan(q, &p, &held)) {
+            other++;
+            bad += std::find(held.begin(), held.end(), conv_patch_shape(rows, p)) == held.end() || p.lds_bytes > CONV_PATCH_LDS_MAX ||
+                   128 * p.col_blocks + patch_end(l, p) > p.lds_bytes;
+        }
+        held.push_back(own);
+        bad += !conv_patch_plan(q, &p, &held) || memcmp(&p, &free, sizeof(p)) != 0;
+    }
+    printf("held shapes: %d plans with another shape, %d wrong\n", other, bad);
+    return bad + (other < 500);
+}
+
 } // namespace
 
 int main()
 {
-    const int bad = reads_stay_inside() + orders_follow_the_rule();
+    const int bad = reads_stay_inside() + orders_follow_the_rule() + plans_keep_to_held_shapes();
     printf(bad ? "FAILED\n" : "ALL PASSED\n");
     return bad != 0;
 }

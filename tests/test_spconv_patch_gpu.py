@@ -142,3 +142,72 @@ def test_first_initialisation_of_a_filter_costs_no_more_than_the_plane_form(torc
     patch, planes = (np.median(took[v][10:]) * 1e6 for v in (PATCH, 0))
     print("first initialisation: patch form %.0f us, plane form %.0f us" % (patch, planes), flush=True)
     assert patch < 1.5 * planes
+
+
+def test_a_filter_serves_many_geometries_from_a_bounded_number_of_images(torch_gpu):
+    """A serving loop over many batches and resolutions: geometries whose patches have one shape share an image of the filter,
+    a filter holds at most SHFLBW_CONV_PATCH_IMAGES (16), and a geometry met after that runs on one of those.  What is held
+    does not grow on a second round, and a state made first is still good at the end."""
+    import ctypes
+    torch = torch_gpu
+    C, F, V = 24, 64, 16
+    w = P.make_weight(F, 9 * C, V, 0.3, True, 3, integer=True)
+    f = P.upload_weight(w, 3, 3, C, cls=S.BlockwiseSpFilter)
+    stream = torch.cuda.current_stream().cuda_stream
+    rng = np.random.default_rng(5)
+
+    def held():
+        b, n = ctypes.c_size_t(0), ctypes.c_int(0)
+        S.capi.check(S.capi.load().shflbw_weight_scratch_bytes(f._h, ctypes.byref(b), ctypes.byref(n)))
+        return b.value, n.value
+
+    first, images, sizes = None, set(), []
+    for rnd in range(2):
+        for stride, H in ((1, 4), (2, 9), (1, 5), (2, 14), (1, 7), (2, 25), (1, 10), (1, 14), (2, 30), (1, 20), (1, 28), (1, 33)):
+            for Bn in (1, 2, 3, 5, 8, 13, 24):
+                x = rng.integers(-4, 5, size=(Bn, H, H + 1, C)).astype(np.float16)
+                ref = O.float_to_half(P.conv_oracle(w, 3, 3, C, x, stride))
+                dX, dY = P.to_dev(torch, x), torch.full(ref.shape, float("nan"), dtype=torch.float16, device="cuda")
+                op = S.SpconvBlockwiseOp()
+                st = op.initialize(f, Bn, H, H + 1, stride, dX.data_ptr(), dY.data_ptr())
+                assert st.variant == PATCH
+                images.add(st.patch)
+                op(stream)
+                torch.cuda.synchronize()
+                np.testing.assert_array_equal(dY.cpu().numpy().view(np.uint16), ref.view(np.uint16), err_msg="%d x %d" % (Bn, H))
+                first = first or (op, dX, dY, ref)
+        sizes.append(held())
+        print("round", rnd, "images", len(images), "bytes, buffers", sizes[-1], flush=True)
+    assert len(images) == 16 and sizes[0] == sizes[1]
+    one = 2 * w["nnzb"] * V  # the values alone; an image adds offsets, sources and padding
+    assert sizes[0][0] <= 16 * (2 * one + 64 * 1024), sizes
+    op, _, dY, ref = first
+    dY.fill_(float("nan"))
+    op(stream)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(dY.cpu().numpy().view(np.uint16), ref.view(np.uint16))
+    f.release_scratch()
+    assert held() == (0, 0)
+
+
+def test_requests_for_shapes_beyond_those_held(torch_gpu):
+    """All images taken: an explicit request that none of them suits says so (and leaves the others alone); the library takes a
+    plane form; released, the filter takes the patch form again."""
+    torch = torch_gpu
+    C, F, V = 24, 64, 16
+    w = P.make_weight(F, 9 * C, V, 0.3, True, 3, integer=True)
+    f = P.upload_weight(w, 3, 3, C, cls=S.BlockwiseSpFilter)
+    t = torch.zeros(64 * 80 * 80 * 64, dtype=torch.float16, device="cuda")
+    images = set()
+    for H in range(4, 70):
+        for Bn, stride in ((1, 1), (3, 2), (16, 1), (1, 2), (6, 1), (16, 2)):
+            images.add(S.SpconvBlockwiseOp().initialize(f, Bn, H, H, stride, t.data_ptr(), t.data_ptr()).patch)
+    assert len(images) == 16 and None not in images
+    # at stride 3 neighbouring positions lie 3 apart: another foot than any patch at strides 1 and 2
+    refused = S.SpconvBlockwiseOp(PATCH)
+    with pytest.raises(S.capi.ShflbwError) as e:
+        refused.initialize(f, 2, 30, 30, 3, t.data_ptr(), t.data_ptr())
+    assert e.value.status == S.capi.ERR_CAPACITY and "16 images" in str(e.value)
+    assert S.SpconvBlockwiseOp().initialize(f, 2, 30, 30, 3, t.data_ptr(), t.data_ptr()).variant == 0
+    f.release_scratch()
+    assert S.SpconvBlockwiseOp().initialize(f, 2, 30, 30, 3, t.data_ptr(), t.data_ptr()).variant == PATCH
