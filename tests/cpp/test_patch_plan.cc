@@ -2,6 +2,7 @@
 // seeded random layers.  The walk below restates the kernel's addressing (position -> column offset, kept column -> row).
 #include <algorithm>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <random>
 
@@ -194,8 +195,21 @@ int plans_keep_to_held_shapes()
 
 } // namespace
 
-int main()
+// test_patch_plan: the checks above.  test_patch_plan cut V F C R S nnzb permuted B H W stride: the cut of one layer, as
+// rows of a row unit, 32-column blocks, waves, row units of a wave, parts of the kept columns, workgroups of a column tile.
+int main(int argc, char** argv)
 {
+    if (argc == 13 && !strcmp(argv[1], "cut")) {
+        int v[11];
+        for (int i = 0; i < 11; i++) v[i] = atoi(argv[2 + i]);
+        Layer l{v[0], v[1], v[2], v[3], v[4], v[6], v[7], v[8], v[9], v[10], 0};
+        ConvPatchProblem q = problem(l);
+        q.kept_per_panel = (double)v[5] / (l.F / l.V);
+        ConvPatchPlan p{};
+        if (!conv_patch_plan(q, &p)) return 1;
+        printf("%d %d %d %d %d %d\n", conv_patch_unit_rows(l.V), p.col_blocks, p.waves, p.panels_per_wave, p.ksplit, p.chunks);
+        return 0;
+    }
     const int bad = reads_stay_inside() + orders_follow_the_rule() + plans_keep_to_held_shapes();
     printf(bad ? "FAILED\n" : "ALL PASSED\n");
     return bad != 0;

@@ -48,7 +48,8 @@ def test_spmm_exec_in_a_graph(torch_gpu):
     _replays(torch, op, [to_dev(torch, B) for B in Bs], dB, dD, refs)
 
 
-@pytest.mark.parametrize("variant", [0, 2, 3])  # three launches, batch-innermost three launches, one fused launch
+# three launches, batch-innermost three launches, one fused launch, the patch form and the library's choice (the patch form here)
+@pytest.mark.parametrize("variant", [0, 2, 3, 5, -1])
 def test_spconv_exec_in_a_graph(torch_gpu, variant):
     torch = torch_gpu
     Bn, H, W, C, F, R, Sx, stride, V = 8, 14, 14, 64, 128, 3, 3, 2, 64
@@ -59,7 +60,8 @@ def test_spconv_exec_in_a_graph(torch_gpu, variant):
     dX = torch.empty((Bn, H, W, C), dtype=torch.float16, device="cuda")
     dY = torch.empty(refs[0].shape, dtype=torch.float16, device="cuda")
     op = S.SpconvBlockwiseOp(variant)
-    op.initialize(f, Bn, H, W, stride, dX.data_ptr(), dY.data_ptr())
+    st = op.initialize(f, Bn, H, W, stride, dX.data_ptr(), dY.data_ptr())
+    assert st.variant == (5 if variant < 0 else variant)
     _replays(torch, op, [to_dev(torch, x) for x in xs], dX, dY, refs)
 
 

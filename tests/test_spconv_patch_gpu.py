@@ -1,7 +1,11 @@
 """GPU parity of the patch form of the convolution (one launch, the input patch of a workgroup in LDS) against the CPU
 oracle: integer operands, bit for bit.  The shapes sit where the form can go wrong: edges of the pixel blocks and of the
 four-unit tiles, channel counts that leave part of a 64-channel group, strides wider than the filter, every block
-height, one and several workgroups per column tile with and without a permutation, kept columns split over waves."""
+height, one and several workgroups per column tile with and without a permutation, kept columns split over waves; and, by
+the cut that the planner picks, every kernel of the form, several row units a wave and every number of parts."""
+import os
+import subprocess
+
 import numpy as np
 import pytest
 
@@ -45,6 +49,61 @@ def test_exact_shapes(torch_gpu, Bn, H, W, C, F, R, Sx, stride, V, d, permute):
     w = P.make_weight(F, R * Sx * C, V, d, permute, 2021, integer=True)
     x = np.random.default_rng(5).integers(-4, 5, size=(Bn, H, W, C)).astype(np.float16)
     _check(torch_gpu, w, x, R, Sx, C, stride)
+
+
+def _cut(w, R, Sx, C, x, stride):
+    """(rows of a row unit, 32-column blocks, waves, row units of a wave, parts of the kept columns) the planner picks."""
+    exe = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "bin", "test_patch_plan")
+    args = [w["brow"], w["nrow"], C, R, Sx, w["nnzb"], int(w["row_permute_ids"] is not None), *x.shape[:3], stride]
+    return tuple(map(int, subprocess.check_output([exe, "cut"] + [str(int(a)) for a in args], text=True).split()))[:5]
+
+
+@pytest.mark.parametrize("cut,Bn,H,W,C,F,R,stride,V,d,permute", [
+    ((16, 1, 4, 2, 1), 29, 10, 17, 160, 96, 3, 2, 16, 0.05, True),
+    ((16, 1, 4, 4, 1), 18, 30, 25, 80, 144, 3, 1, 16, 0.1, True),
+    ((16, 2, 4, 2, 1), 15, 22, 25, 80, 80, 3, 1, 16, 0.1, True),
+    ((16, 2, 4, 4, 1), 27, 20, 25, 56, 176, 5, 1, 16, 0.05, True),
+    ((16, 1, 8, 1, 1), 13, 8, 26, 264, 128, 3, 2, 16, 0.05, True),
+    ((16, 1, 8, 1, 4), 11, 15, 11, 232, 32, 5, 2, 16, 0.05, True),
+    ((16, 1, 8, 2, 1), 24, 19, 17, 168, 144, 3, 2, 16, 0.05, True),
+    ((16, 1, 8, 4, 1), 18, 28, 22, 160, 320, 3, 2, 16, 0.05, True),
+    ((16, 2, 8, 1, 1), 37, 28, 30, 168, 80, 3, 2, 16, 0.05, True),
+    ((16, 2, 8, 1, 8), 36, 15, 15, 136, 16, 5, 1, 16, 0.05, True),
+    ((16, 2, 8, 2, 1), 22, 28, 13, 160, 144, 3, 1, 16, 0.05, True),
+    ((16, 2, 8, 4, 1), 35, 19, 13, 160, 272, 3, 1, 16, 0.05, True),
+    ((32, 1, 4, 2, 1), 29, 9, 15, 192, 160, 3, 2, 32, 0.05, True),
+    ((32, 2, 4, 2, 1), 14, 21, 25, 56, 160, 5, 1, 32, 0.05, True),
+    ((32, 1, 8, 1, 2), 28, 20, 10, 232, 288, 3, 2, 32, 0.05, True),
+    ((32, 1, 8, 1, 8), 1, 4, 6, 280, 32, 5, 2, 32, 0.2, True),
+    ((32, 1, 8, 2, 1), 20, 26, 11, 208, 288, 3, 2, 32, 0.05, True),
+    ((32, 2, 8, 1, 1), 25, 11, 28, 160, 160, 3, 1, 32, 0.05, False),
+    ((32, 2, 8, 1, 4), 26, 10, 5, 272, 544, 3, 1, 32, 0.05, True),
+    ((32, 2, 8, 2, 1), 33, 9, 25, 40, 288, 3, 1, 32, 0.2, True),
+    ((64, 1, 8, 1, 1), 23, 12, 20, 208, 320, 3, 2, 64, 0.05, True),
+    ((64, 1, 8, 1, 4), 27, 15, 25, 264, 128, 3, 2, 64, 0.05, True),
+    ((64, 2, 8, 1, 1), 19, 19, 21, 160, 320, 3, 1, 64, 0.05, True),
+    ((64, 2, 8, 1, 8), 40, 7, 28, 208, 64, 5, 1, 64, 0.05, True),
+    ((64, 2, 8, 1, 4), 40, 28, 31, 272, 128, 3, 2, 128, 0.05, True),
+    ((64, 2, 4, 1, 1), 35, 10, 9, 56, 384, 5, 1, 64, 0.05, False),
+    ((64, 1, 4, 1, 2), 3, 22, 7, 72, 512, 5, 2, 128, 0.05, False),
+])
+def test_exact_by_cut(torch_gpu, cut, Bn, H, W, C, F, R, stride, V, d, permute):
+    """The 8-wave kernels (deeper ring, more of the patch in flight) and waves with several row units one after the other; the
+    third and every fourth panel from there on keep nothing, one other keeps a single column."""
+    w = P.make_weight(F, R * R * C, V, d, permute, 2021, integer=True)
+    x = np.random.default_rng(5).integers(-4, 5, size=(Bn, H, W, C)).astype(np.float16)
+    assert _cut(w, R, R, C, x, stride) == cut
+    _check(torch_gpu, w, x, R, R, C, stride)
+    X = F // V
+    counts = np.diff(w["indptr"])
+    counts[2::4] = 0
+    counts[X // 2] = min(1, counts[X // 2])
+    sel = np.concatenate([np.arange(b, b + n) for b, n in zip(w["indptr"], counts)]).astype(np.int64)
+    w2 = dict(w, nnzb=int(counts.sum()), indptr=np.concatenate([[0], np.cumsum(counts)]).astype(np.int32),
+              indices=w["indices"][sel], values=w["values"].reshape(-1, V)[sel].reshape(-1))
+    if cut[3] > 1:
+        assert _cut(w2, R, R, C, x, stride) == cut
+    _check(torch_gpu, w2, x, R, R, C, stride)
 
 
 @pytest.mark.parametrize("V", [16, 32, 64, 128])
