@@ -196,8 +196,8 @@ const char* shflbw_spmm_variant_name(int brow, int variant);
  *   H, W are the INPUT extents; padding is R/2, S/2 ("same" for stride 1, as the
  *   reference's col2im, spconv/conv_format.h:77-81); Ho = (H + 2*(R/2) - R)/stride + 1.
  * Preconditions: filter synced, bcol == 1, C % 8 == 0, F % 8 == 0.
- * init allocates device scratch inside the filter object (freed with it or by shflbw_weight_release_scratch):
- * the gather ids once per (form, B, H, W, stride), and per (form, geometry, IFMap, OFMap) the buffers the launches
+ * init allocates device scratch inside the filter object (freed with it or by shflbw_weight_release_scratch).  The patch form
+ * (variant 5 below): images of the filter, shared by geometries.  The others: the gather ids once per (form, B, H, W, stride), and per (form, geometry, IFMap, OFMap) the buffers the launches
  * write - states over different tensors never share those and may run on different streams.  At most
  * SHFLBW_CONV_SCRATCH_DEPTH such buffers exist per filter: initialising a state over one more tensor pair recycles
  * the buffers of the least recently initialised one (no allocation, no copy when the geometry is the same), whose
@@ -291,7 +291,8 @@ int shflbw_spconv_init_chwb(shflbw_spconv_state* state, const shflbw_weight* fil
                             int B, int H, int W, int stride, const void* IFMap, void* OFMap);
 /* No counterpart in the reference.  For callers that cannot allocate device memory: code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc.  One complete convolution in the plane
- * form, the same launches as shflbw_spconv_init + shflbw_spconv_exec, with all scratch (the planes, the
+ * form, the same launches as variant 0 of shflbw_spconv_init_variant + shflbw_spconv_exec (bit for bit the same result;
+ * the library's own choice may be another form, whose sums are formed in another order), with all scratch (the planes, the
  * filter-major result, the rewritten ids, which a small kernel computes on the device) in a fixed device
  * array inside the library: SHFLBW_STATIC_SCRATCH_BYTES on every GPU the library runs on, held until the
  * process ends.  Calls no hipMalloc / hipFree and copies nothing from the host; launches on `stream` only.

@@ -174,9 +174,10 @@ static bool spmm_variant_offsets32(const SpmmVariant* v) { return v && (v->name[
 //    with 2.5 (18 panels: 0.9 at 0.6 vectors, 1.2 at 5.5; 6 to 9 panels: 0.6-1.1), four where a fifth of the compute units would have
 //    no job (3.2: 8 % slower, 6.4: 5 % faster),
 //  * panels keep at least 32 vectors, or D is below 100 MB: with less to do per panel both wait for the stores of D, and the
-//    wider row segments of the role-split kernel are 5-15 % ahead (33728 x 96 x 2048: 40 against 47 us) where rows of D start at
-//    whole lines (15760 x 127 x 3864: 31 against 41 us).
-// 33728 x 777 x 1000, density 0.1: 31 against 38 us; 8192 x 384 x 4096: 20 against 29 us; 33728 x 1128 x 136, 0.2: 17 and 31 us.
+//    wider row segments of the role-split kernel are 5-15 % ahead (33728 x 96 x 2048: 38 against 46 us) where rows of D start at
+//    whole lines (15760 x 127 x 3864: 41 against 31 us).
+// On one box, density 0.1: 33728 x 777 x 1000 29.6 against 32.8 us; 8192 x 384 x 4096 17.3 against 28.7; 8192 x 777 x 3000 19.0 against
+// 24.9; density 0.2: 33728 x 1128 x 136 16.7 against 29.8.  On 64 sampled shapes it is taken for 30, 1.07 to 1.90 times as fast there.
 static int auto_gather_variant(const shflbw_weight* w, int N, bool allow_slab, int compute_units)
 {
     const int brow = w->brow, X = w->nrow / w->brow;

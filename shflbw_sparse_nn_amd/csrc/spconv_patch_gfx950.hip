@@ -9,8 +9,12 @@
 //      into registers (several batches in flight) and reads its B fragments from the rows the offsets name
 //      (transposing LDS reads; tap, stride and position are one added offset), MFMA, fp32 accumulators;
 //   3. the fp16 results go through LDS (pixel rows, filters in output order) to whole runs of the NHWC output.
-// What bounds it: the A stream (64 bytes per clock and compute unit from the L2) and the MFMAs are level for block
-// height 64, the LDS reads for 32 and 16; on small layers the chain of launch, patch, first fragments and stores.
+// What bounds it: the chain of these phases, with one workgroup per compute unit on layers of many channels.  16 x 14 x 14 x 512 ->
+// 2048, 3 x 3, block height 64, density 0.1 (19.3 us): patch 4.1, products 4.1 at the matrix cores' rate (88 % busy; the A
+// stream, 64 bytes per clock and compute unit from the L2, is level with them), results to LDS 2.3, 2-byte stores of
+// the permuted filters 3.2 (14.7 us per launch where the filters of a chunk are consecutive).  32 x 28 x 28 x 256 -> 512, stride 2,
+// block height 32, density 0.3 (15.7 us): 4.4, 5.2 (matrix cores 52 %, A stream 50 %, the rest LDS reads), 1.0, 1.8.  On small
+// layers launch, patch, first fragments and stores, a round trip each.
 #include "spconv_patch.h"
 
 #include <algorithm>
@@ -563,7 +567,8 @@ ConvPatchShape conv_patch_shape(int rows, const ConvPatchPlan& p)
 // a fit to 124 layers measured with 20 to 40 cuts each (10 % rms; the cut it picks is 4 % slower than the best one
 // measured on average).  Where the plane forms are estimated faster - many filters over few resident pixels (wide
 // filters over many channels), filters of several workgroups interleaved in the output - the cut is not `preferred`:
-// 7 x 54 x 54 x 584 -> 1024, 5 x 5, stride 2 takes 152 us here, 54 us there; 16 x 14 x 14 x 512 -> 2048 20 and 23 us.
+// 7 x 54 x 54 x 584 -> 1024, 5 x 5, stride 2 takes 152 us here, 54 us there; 16 x 14 x 14 x 512 -> 2048, which it takes, 20 and 23 us.
+// On 64 sampled layers it is preferred for 58, where the plane forms take 1.11 to 3.8 times as long.
 bool conv_patch_plan(const ConvPatchProblem& q, ConvPatchPlan* plan, const std::vector<ConvPatchShape>* held)
 {
     ConvPatchPlan best{};
