@@ -14,8 +14,7 @@ namespace shflbw {
 // position p of unit u.  The four units of a position lie side by side in LDS (8 bytes), which is what one lane of
 // the transposing LDS read supplies, so a tap is a plain offset whatever the stride, the batch and the alignment.
 struct ConvPatchPlan {
-    int valid;            // some patch fits the LDS
-    int preferred;        // ... and is estimated faster than the plane forms
+    int valid;            // some patch fits the LDS ...
     int col_blocks;       // 32-column blocks of a tile: 2 (16 positions x 4 units) or 1 (8 positions)
     int waves;            // waves of a workgroup
     int tile_h, tile_w;   // output positions of a unit
@@ -24,7 +23,6 @@ struct ConvPatchPlan {
     int step_h, step_w;   // patch positions between neighbouring output positions
     int patch_w, npos;    // columns and positions of the input patch of a unit
     int pitch;            // LDS bytes of one channel: 8 per position, an odd multiple of 8
-    int slack;            // LDS bytes behind the row of zeros that columns without a pixel may touch
     int groups, ksplit;   // waves = groups (rows) x ksplit (parts of the kept columns, a power of two: 1 << kshift)
     int kshift;
     int panels_per_wave;  // row units one wave computes one after the other
@@ -36,6 +34,8 @@ struct ConvPatchPlan {
     unsigned touch_bytes, touch_step; // last byte of the filter image a workgroup brings into the L2; bytes one round of an XCD's threads covers
     int lds_bytes;
     unsigned magic_bhw, magic_bw, magic_pw, magic_row, magic_chunks, magic_pg;
+    int preferred;        // ... and is estimated faster than the plane forms
+    int slack;            // LDS bytes behind the row of zeros that columns without a pixel may touch
 };
 
 // What the plan depends on.
