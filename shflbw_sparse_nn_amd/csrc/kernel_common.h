@@ -63,17 +63,23 @@ __device__ __forceinline__ void global_to_lds_16B(const void* gptr, uint32_t lds
                  : "m0");
 }
 
-// Same copy with the address split into a wave-uniform 64-bit base (scalar registers) and a
-// per-lane 32-bit byte offset: no vector-ALU address arithmetic is needed per copy, which
-// matters because vector-ALU work of one wave competes with the MFMAs of its SIMD neighbour.
+// The same copy through a buffer descriptor (scalar registers, so a copy takes no 64-bit address arithmetic of the lanes):
+// `lane_off` is a byte offset from the descriptor's base, and a lane whose offset is not below the descriptor's size brings 16
+// zeros into its piece of LDS instead of reading memory.
 template <int LDS_IMM>
-__device__ __forceinline__ void global_to_lds_16B_sbase(const void* sbase, uint32_t lane_off, uint32_t lds_base)
+__device__ __forceinline__ void buffer_to_lds_16B(int4_t desc, uint32_t lane_off, uint32_t lds_base)
 {
-    // LDS address = lds_base + LDS_IMM, formed directly in M0
-    asm volatile("s_add_i32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+    asm volatile("s_add_i32 m0, %2, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
                  :
-                 : "v"(lane_off), "s"(sbase), "s"(lds_base), "n"(LDS_IMM)
+                 : "v"(lane_off), "s"(desc), "s"(lds_base), "n"(LDS_IMM)
                  : "m0", "scc");
+}
+
+// descriptor of `bytes` bytes of plain memory from `base` on
+__device__ __forceinline__ int4_t buffer_descriptor(const void* base, uint32_t bytes)
+{
+    const uintptr_t p = (uintptr_t)base;
+    return int4_t{(int)(uint32_t)p, (int)(uint32_t)((p >> 32) & 0xffffu), (int)bytes, 0x00020000};
 }
 
 // the same copy with 4 bytes per lane: 256 bytes of consecutive LDS
