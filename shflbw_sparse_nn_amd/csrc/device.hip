@@ -810,9 +810,56 @@ void batch_planes_geometry(const shflbw_weight* f, int B, int stride, int Ho, in
 }
 
 //   form 4: the caller's tensors are C-H-W-B / F-H-W-B (the reference's), H and W bound input and output alike,
-//           the SpMM writes OFMap itself (its epilogue drops the padding columns, output_column());
+//           the SpMM writes OFMap itself (its epilogue drops the padding columns, output_column()); only for what
+//           chwb_gathers_input() leaves;
 //   form 2: the caller's tensors are NHWC with true stride and padding; the SpMM writes result_fm[f][(ho, wo, img)],
 //           a tile transpose writes OFMap.
+// Form 4 over the input itself (the state holds no planes): where the ids of its taps fit (chwb_tap_id) and the output does
+// not overwrite what is still to be gathered.
+bool chwb_gathers_input(const shflbw_weight* f, int B, int H, int W, const void* IFMap, const void* OFMap)
+{
+    const size_t pixels = (size_t)B * H * W * 2;
+    const char *in = (const char*)IFMap, *out = (const char*)OFMap;
+    const bool apart = in + pixels * f->C <= out || out + pixels * f->F <= in;
+    return apart && (long)f->R * f->S <= CHWB_MAX_TAPS &&
+           ((unsigned long long)f->C * H * W + (unsigned long long)f->R * W + f->S) * (unsigned long long)B * 2ull < 0x80000000ull;
+}
+
+int init_chwb_taps(shflbw_spconv_state* state, const shflbw_weight* f, int B, int H, int W, int stride, const void* IFMap, void* OFMap)
+{
+    const long ncols = (long)H * W * B; // columns of the GEMM: the output positions (ho, wo, b)
+    if (ncols > 0x7fffffffL) {
+        set_error("spconv_init: problem too large (%ld output positions)", ncols);
+        return SHFLBW_ERR_UNSUPPORTED;
+    }
+    const ConvChwbKernel* k = conv_chwb_kernel(f->brow, 0, f->nrow / f->brow, ncols, device_compute_units());
+    if (!k) {
+        set_error("spconv_init: no kernel for block size %d", f->brow);
+        return SHFLBW_ERR_UNSUPPORTED;
+    }
+    SHFLBW_HIP_TRY(k->prepare_taps());
+    state->middle_tile_cols = k->BN;
+    shflbw_weight* fw = const_cast<shflbw_weight*>(f); // the table of ids is bookkeeping of the handle (see init_planes)
+    std::lock_guard<std::mutex> scratch_guard(fw->scratch_lock);
+    const int key[5] = {FORM_CHWB, B, H, W, 0}; // the same for every stride
+    const int C = f->C, S = f->S;
+    const int *ids = nullptr, *ids_pm = nullptr;
+    int rc = conv_ids_for(fw, key, chwb_tap_id(0, CHWB_MAX_TAPS), [&](int kk) {
+        const int c = kk % C, tap = kk / C, r = tap / S, t = tap % S;
+        return chwb_tap_id((unsigned)((((long)c * H + r) * W + t) * (B / 8)), (unsigned)tap);
+    }, &ids, &ids_pm);
+    if (rc != SHFLBW_OK) return rc;
+    state->ncols = (int)ncols;
+    if ((rc = bind_middle(state, f, ncols, IFMap, OFMap, ids, ids_pm, (long)C * H * W * B)) != SHFLBW_OK) return rc;
+    state->shared_mem_size = (size_t)k->lds_bytes;
+    state->grid_dim[0] = (unsigned)((f->nrow / f->brow) * ((ncols + k->BN - 1) / k->BN));
+    state->block_dim[0] = (unsigned)k->threads;
+    state->grid_dim[1] = state->grid_dim[2] = 1;
+    state->block_dim[1] = state->block_dim[2] = 1;
+    state->init_success = 1;
+    return SHFLBW_OK;
+}
+
 int init_batch_planes(shflbw_spconv_state* state, const shflbw_weight* f, int B, int H, int W, int stride,
                       const void* IFMap, void* OFMap, int variant)
 {
@@ -825,6 +872,7 @@ int init_batch_planes(shflbw_spconv_state* state, const shflbw_weight* f, int B,
     if (variant == FORM_CHWB) { // H and W are the extents of the output grid and the bounds of the input (spconv/blockwise_format.h:111-115)
         state->Ho = H;
         state->Wo = W;
+        if (chwb_gathers_input(f, B, H, W, IFMap, OFMap)) return init_chwb_taps(state, f, B, H, W, stride, IFMap, OFMap);
     }
     BatchPlanes g;
     batch_planes_geometry(f, B, stride, state->Ho, state->Wo, &g);
@@ -1325,6 +1373,22 @@ int shflbw_spconv_exec(const shflbw_spconv_state* state, void* stream)
     if (state->variant == FORM_CHWB || state->variant == FORM_BPLANES) {
         const ConvChwbKernel* k = conv_chwb_kernel(state->brow, state->middle_tile_cols, 0, 0, 0);
         if (!k) return SHFLBW_ERR_UNSUPPORTED;
+        if (!state->planes) { // form 4 over the input itself
+            ChwbTapArgs t;
+            fill_spmm_launch_args(&state->spmm, k->BN, &t);
+            t.B = a.in;
+            t.alternate = 0;
+            t.batch = a.B, t.in_h = a.H, t.in_w = a.W;
+            t.taps_r = a.R, t.taps_s = a.S, t.stride = a.stride;
+            t.magic_batch = udiv_magic(a.B), t.magic_w = udiv_magic(a.W);
+            t.row_bits = 0;
+            for (int r = 0; r < a.R; r++) t.row_bits |= 1u << (r * a.S);
+            t.in_bytes = (unsigned)((size_t)a.C * a.H * a.W * a.B * 2);
+            if (t.X > 0) e = k->launch_taps(t, (hipStream_t)stream);
+            if (e == hipSuccess) return SHFLBW_OK;
+            set_error("spconv_exec: launch failed: %s", hipGetErrorString(e));
+            return SHFLBW_ERR_HIP;
+        }
         const bool nhwc = state->variant == FORM_BPLANES;
         e = nhwc ? launch_nhwc_to_planes(a, (half_t*)state->planes, state->plane_rows, state->plane_cols,
                                          state->plane_pitch, 1, (hipStream_t)stream, 1)

@@ -722,7 +722,12 @@ hipError_t launch_planes_to_nhwc(const half_t* dm, half_t* out, int F, int NP, i
 // F-H-W-B, batch innermost, H and W the extents of the OUTPUT grid and at the same time the bounds of the input
 // (out(ho, wo) reads in(ho*stride - R/2 + r, wo*stride - S/2 + t) where that lies inside H x W, zero elsewhere).
 // With the batch innermost both ends of the GEMM are contiguous: a kept vector k = (r, t, c) is a run of channel
-// c's plane at a constant offset, and a row of the result is a row of the output.  Two launches:
+// c's plane at a constant offset, and a row of the result is a row of the output.  One launch: the role-split SpMM over the
+// H * W * B output positions, whose producers gather the 16-byte pieces (8 images of one position) from the input itself and
+// fetch zeros where a tap lies outside the map (ws_producer, TAPS).  The padded copy it replaces was a launch, a write and a read of
+// the input, and a GEMM over the padded columns: 128 x 14 x 14 x 256 -> 256, 3 x 3, block height 64, density 0.1: 14.4-18.6 us with it,
+// 8.3-8.8 now; 32 x 55 x 27 x 360 -> 128, 1 x 7, stride 2: 68 and 20; 8 x 30 x 30 x 48 -> 32: 7.6 and 4.1.
+// Filters of more than CHWB_MAX_TAPS taps and inputs from 2^31 bytes on, which its ids cannot name, take two launches:
 //   1. chwb_to_planes_kernel: pure copy with zero fill into padded phase planes
 //        planes[phase (a, b)][c][(i * PW + j) * B + n] = in[c][i*stride + a - R/2][j*stride + b - S/2][n]
 //      with PHX = H + (R-1)/stride rows and PW = W + (S-1)/stride columns per plane: tap (r, t) of output (ho, wo)
@@ -767,9 +772,11 @@ hipError_t launch_chwb_to_planes(const half_t* in, half_t* planes, int B, int H,
     return hipGetLastError();
 }
 
-template <int V, int WN, int NCONS, int NPROD, int KT, int NSTAGE>
-__global__ void __launch_bounds__((NCONS + NPROD) * 64) spconv_chwb_kernel(SpmmLaunchArgs a)
+// Args: ChwbTapArgs gathers from the input itself, SpmmLaunchArgs from planes, with the columns of the padded grid.
+template <int V, int WN, int NCONS, int NPROD, int KT, int NSTAGE, typename Args>
+__global__ void __launch_bounds__((NCONS + NPROD) * 64) spconv_chwb_kernel(Args a)
 {
+    constexpr bool DMAP = !std::is_same<Args, ChwbTapArgs>::value;
     using Cfg = SpmmWsCfg<V, WN, NCONS, NPROD, KT, NSTAGE>;
     extern __shared__ __attribute__((aligned(1024))) char lds_raw[];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(SHFLBW_LDS char*)lds_raw;
@@ -785,39 +792,40 @@ __global__ void __launch_bounds__((NCONS + NPROD) * 64) spconv_chwb_kernel(SpmmL
     if (wave >= NCONS)
         ws_producer<Cfg, V, NCONS, NPROD, KT, NSTAGE>(a, lds0, lane, wave - NCONS, id_first, id_end, S);
     else if constexpr (V == 16)
-        ws_consumer16<Cfg, WN, NCONS, false, true>(a, lds0, lane, wave, id_first, id_end, S);
+        ws_consumer16<Cfg, WN, NCONS, false, DMAP>(a, lds0, lane, wave, id_first, id_end, S);
     else
-        ws_consumer<Cfg, V, WN, NCONS, false, true>(a, lds0, lane, wave, id_first, id_end, S);
+        ws_consumer<Cfg, V, WN, NCONS, false, DMAP>(a, lds0, lane, wave, id_first, id_end, S);
 }
 
-template <int V, int WN, int NCONS, int NPROD, int KT, int NSTAGE>
-static hipError_t launch_chwb(const SpmmLaunchArgs& a, hipStream_t stream)
+template <int V, int WN, int NCONS, int NPROD, int KT, int NSTAGE, typename Args>
+static hipError_t launch_chwb(const Args& a, hipStream_t stream)
 {
     using Cfg = SpmmWsCfg<V, WN, NCONS, NPROD, KT, NSTAGE>;
-    SpmmLaunchArgs b = a;
+    Args b = a;
     b.n_tiles = (a.N + Cfg::BN - 1) / Cfg::BN;
     const int T = a.X * b.n_tiles;
     int grid = a.num_cus > 0 ? a.num_cus : 256;
     grid = (grid / 8) * 8;
     const int need = ((T + 7) / 8) * 8;
     if (grid > need) grid = need;
-    hipLaunchKernelGGL((spconv_chwb_kernel<V, WN, NCONS, NPROD, KT, NSTAGE>), dim3(grid), dim3(Cfg::THREADS), Cfg::LDS_BYTES,
+    hipLaunchKernelGGL((spconv_chwb_kernel<V, WN, NCONS, NPROD, KT, NSTAGE, Args>), dim3(grid), dim3(Cfg::THREADS), Cfg::LDS_BYTES,
                        stream, b);
     return hipGetLastError();
 }
 
-template <int V, int WN, int NCONS, int NPROD, int KT, int NSTAGE>
+template <int V, int WN, int NCONS, int NPROD, int KT, int NSTAGE, typename Args>
 static hipError_t prepare_chwb()
 {
     using Cfg = SpmmWsCfg<V, WN, NCONS, NPROD, KT, NSTAGE>;
-    return hipFuncSetAttribute((const void*)spconv_chwb_kernel<V, WN, NCONS, NPROD, KT, NSTAGE>,
+    return hipFuncSetAttribute((const void*)spconv_chwb_kernel<V, WN, NCONS, NPROD, KT, NSTAGE, Args>,
                                hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS_BYTES);
 }
 
 #define SHFLBW_CHWB(V, WN, NC, NP, KT, NS)                                                                             \
     {                                                                                                                  \
-        V, WN* NC, (NC + NP) * 64, SpmmWsCfg<V, WN, NC, NP, KT, NS>::LDS_BYTES, &launch_chwb<V, WN, NC, NP, KT, NS>,  \
-            &prepare_chwb<V, WN, NC, NP, KT, NS>                                                                       \
+        V, WN* NC, (NC + NP) * 64, SpmmWsCfg<V, WN, NC, NP, KT, NS>::LDS_BYTES,                                       \
+            &launch_chwb<V, WN, NC, NP, KT, NS, SpmmLaunchArgs>, &prepare_chwb<V, WN, NC, NP, KT, NS, SpmmLaunchArgs>, \
+            &launch_chwb<V, WN, NC, NP, KT, NS, ChwbTapArgs>, &prepare_chwb<V, WN, NC, NP, KT, NS, ChwbTapArgs>        \
     }
 
 // (the widest tile of a block size first)

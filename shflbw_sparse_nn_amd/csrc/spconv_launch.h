@@ -82,8 +82,8 @@ inline int conv_xcd_sync_lines(int nx) { return 1 + nx * XCD_LINES; }
 // writes the XCD every workgroup of a launch of `blocks` workgroups runs on to out[blocks] (device memory)
 hipError_t launch_xcd_probe(int* out, int blocks, hipStream_t stream);
 
-// Batch-innermost (C-H-W-B in, F-H-W-B out) form of the convolution: the copy into padded phase planes and the
-// role-split kernel whose epilogue writes compact output rows.
+// Batch-innermost (C-H-W-B in, F-H-W-B out) form of the convolution: the role-split kernel that gathers from the input;
+// and the copy into padded phase planes with the kernel over those, whose epilogue writes compact output rows.
 hipError_t launch_chwb_to_planes(const half_t* in, half_t* planes, int B, int H, int W, int C, int R, int S, int stride,
                                  int PHX, int PW, int pitch, hipStream_t stream);
 struct ConvChwbKernel {
@@ -91,8 +91,10 @@ struct ConvChwbKernel {
     int BN;
     int threads;
     int lds_bytes;
-    hipError_t (*launch)(const SpmmLaunchArgs&, hipStream_t);
+    hipError_t (*launch)(const SpmmLaunchArgs&, hipStream_t); // over planes
     hipError_t (*prepare)();
+    hipError_t (*launch_taps)(const ChwbTapArgs&, hipStream_t); // over the input itself
+    hipError_t (*prepare_taps)();
 };
 const ConvChwbKernel* conv_chwb_kernel(int V, int tile_cols, long X, long ncols, int cus);
 

@@ -30,6 +30,19 @@ struct SpmmLaunchArgs {
                    // (pays when the rows of B under one column tile do not fit the XCD's L2)
 };
 
+// Convolution over batch-innermost tensors that gathers from the input itself (B points to it): the columns of the GEMM
+// are the output positions (ho, wo, b), a kept column is a channel plane and a tap, ids as chwb_tap_id() packs them.
+struct ChwbTapArgs : SpmmLaunchArgs {
+    int batch, in_h, in_w;      // batch, a multiple of 8; H and W bound input and output alike
+    int taps_r, taps_s, stride; // R * S <= CHWB_MAX_TAPS
+    unsigned magic_batch, magic_w; // udiv_magic of batch and in_w
+    unsigned row_bits;          // bits r * S for all r < R
+    unsigned in_bytes;          // of the whole input, below 2^31
+};
+constexpr int CHWB_MAX_TAPS = 31;  // a lane keeps one bit per tap; bit 31 is that of the padding slots, which no lane reads
+// units of 16 bytes from the lane's own position at tap (0, 0) of channel 0, and the tap
+constexpr int chwb_tap_id(unsigned units16, unsigned tap) { return (int)(units16 * 32u + tap); }
+
 struct SpmmVariant {
     int V;           // block size (rows per panel)
     int BN;          // output columns per workgroup

@@ -651,10 +651,15 @@ __device__ __forceinline__ void gather_rows4(int4_t k, uint32_t rowbytes, const 
 
 // Producer role: wave `pw` of NPROD issues its share of every stage of the workgroup's tile list (ids
 // id_first, id_first + S, ... < id_end; id = column tile * X + panel).
-template <typename Cfg, int V, int NCONS, int NPROD, int KT, int NSTAGE>
-__device__ __forceinline__ void ws_producer(const SpmmLaunchArgs& a, uint32_t lds0, int lane, int pw, int id_first,
+// TAPS (a ChwbTapArgs): rows are gathered from a batch-innermost feature map.  A lane's 16 bytes are 8 images of one output
+// position; its offset for a kept column is that of its position plus the id's, and where the id's tap lies outside the map at
+// this position - one bit per tap, worked out once per tile - the offset is moved past the end of the buffer, which fetches
+// zeros.  Three vector instructions a row in place of one; the copies, not the issue of instructions, set the pace.
+template <typename Cfg, int V, int NCONS, int NPROD, int KT, int NSTAGE, typename Args>
+__device__ __forceinline__ void ws_producer(const Args& a, uint32_t lds0, int lane, int pw, int id_first,
                                             int id_end, int S)
 {
+    constexpr bool TAPS = std::is_same<Args, ChwbTapArgs>::value;
     constexpr int BN = Cfg::BN, RPW = Cfg::RPW;
     constexpr int STAGE_BYTES = Cfg::STAGE_BYTES, B_BYTES = Cfg::B_BYTES;
     const int N = a.N, X = a.X;
@@ -716,7 +721,12 @@ __device__ __forceinline__ void ws_producer(const SpmmLaunchArgs& a, uint32_t ld
     // the offset -rowbytes + column = 2^32 - rowbytes + column, which lies past that end as long as K * rowbytes is at most
     // 2^32 - rowbytes (the launcher sees to it): it brings zeros like every other offset that is no part of B.  Ids that
     // were rewritten to something else than rows of B (planes) have no -1.
-    const int4_t map = buffer_descriptor(a.B, (uint32_t)a.K * rowbytes);
+    int4_t map;
+    if constexpr (TAPS)
+        map = buffer_descriptor(a.B, a.in_bytes);
+    else
+        map = buffer_descriptor(a.B, (uint32_t)a.K * rowbytes);
+    uint32_t outside[4] = {0, 0, 0, 0}; // TAPS: the taps that lie outside the map at the lane's position of copy j
     // Several rows per copy: all ones in the lanes of the q-th row.  Opaque, so that the ids are merged by bit operations: from
     // a chain of conditions the compiler makes branches over the lanes, fifty instructions per copy
     // (1024^3, density 0.25: 5.06 us with them, 4.40 without; 25 stages of 128 columns: 0.06 us less a stage).
@@ -742,8 +752,25 @@ __device__ __forceinline__ void ws_producer(const SpmmLaunchArgs& a, uint32_t ld
             const int lc = ((((pc >> 1) ^ row_xor32(key))) << 1) | (pc & 1);
             const int col = n0 + lc * 8;
             int c = col < N ? col : n0; // columns past N are never stored; any valid column of the tile will do
-            voff[j] = (uint32_t)c * 2;
+            if constexpr (TAPS) {
+                int pos, b, ho, wo;
+                fast_divmod(c, a.batch, a.magic_batch, pos, b);
+                fast_divmod(pos, a.in_w, a.magic_w, ho, wo);
+                const int h = ho * a.stride - (a.taps_r >> 1), w = wo * a.stride - (a.taps_s >> 1); // of tap (0, 0)
+                voff[j] = (uint32_t)((h * a.in_w + w) * a.batch + b) * 2u; // below zero for some: the sum with an inner tap's id is not
+                auto bits = [](int lo, int hi) { return ((1u << max(hi, 0)) - 1u) & ~((1u << max(lo, 0)) - 1u); };
+                const uint32_t cols = bits(-w, min(a.taps_s, a.in_w - w));
+                const uint32_t rows = a.row_bits & bits(-h * a.taps_s, min(a.taps_r, a.in_h - h) * a.taps_s);
+                outside[j] = ~(cols * rows); // the bits of cols at every row
+            } else {
+                voff[j] = (uint32_t)c * 2;
+            }
         }
+    };
+    // offset of the lane's piece of the row that id k names; past the end of the map where the tap lies outside
+    auto tap_off = [&](int k, int j) __attribute__((always_inline)) {
+        const uint32_t off = ((uint32_t)k >> 5) * 16u + voff[j];
+        return off | ((uint32_t)__builtin_amdgcn_sbfe((int)outside[j], (uint32_t)k & 31u, 1u) << 4);
     };
 
     // -- everything on the stage cadence, specialised on whether this producer also copies an A
@@ -763,15 +790,18 @@ __device__ __forceinline__ void ws_producer(const SpmmLaunchArgs& a, uint32_t ld
         auto stage = [&](int4_t ka, int4_t kb) __attribute__((always_inline)) {
             __builtin_amdgcn_s_waitcnt(vmcnt_imm((NSTAGE - 3) * MYOPS));
             wg_barrier();
-            if constexpr (Cfg::RPI > 1) {
+            if constexpr (TAPS || Cfg::RPI > 1) {
                 const int ks[8] = {ka.x, ka.y, ka.z, ka.w, kb.x, kb.y, kb.z, kb.w};
-                auto copy = [&](auto jj) __attribute__((always_inline)) { // fills the rows RPI * j and on, side by side in the lanes
+                auto copy = [&](auto jj) __attribute__((always_inline)) { // fills row j, or the rows RPI * j and on side by side in the lanes
                     constexpr int j = decltype(jj)::value;
                     if constexpr (j < Cfg::CPW) {
-                        int k = ks[Cfg::RPI * j] & part[0];
+                        int k = ks[j];
+                        if constexpr (Cfg::RPI > 1) {
+                            k = ks[Cfg::RPI * j] & part[0];
 #pragma unroll
-                        for (int q = 1; q < Cfg::RPI; q++) k |= ks[Cfg::RPI * j + q] & part[q];
-                        buffer_to_lds_16B<j * 0x400>(map, (uint32_t)k * rowbytes + voff[j & 3], sbp);
+                            for (int q = 1; q < Cfg::RPI; q++) k |= ks[Cfg::RPI * j + q] & part[q];
+                        }
+                        buffer_to_lds_16B<j * 0x400>(map, TAPS ? tap_off(k, j & 3) : (uint32_t)k * rowbytes + voff[j & 3], sbp);
                     }
                 };
                 copy(std::integral_constant<int, 0>{});
