@@ -294,6 +294,16 @@ static int plane_form_geometry(const shflbw_weight* f, int B, int H, int W, int 
     return SHFLBW_OK;
 }
 
+// Whether the results of a role-split launch are merged in the L2s (ordinary stores) instead of written through (device
+// scope): where rows of D start inside a line and D is at least three quarters of the eight L2s.  Block height 64,
+// K = 1640, density 0.1, written through / merged: 4096 x 1000 6.3 / 6.9 us, 4096 x 2008 10.4 / 10.9, 1024 x 8008 9.8 / 10.3 (16 MB);
+// 4096 x 4008 15.5 / 15.2, 16384 x 1000 16.0 / 15.1 (33 MB); 4096 x 8008 38.7 / 32.1.  On whole lines they are level for large D,
+// and 4096^3 takes 18.9 written through, 21.1 merged.
+static bool store_merges_lines(const void* D, int rows, int ldd)
+{
+    return (((uintptr_t)D | ((uintptr_t)ldd * 2)) & 127) != 0 && (size_t)rows * (size_t)ldd * 2 >= 24u << 20;
+}
+
 // launch arguments of the SpMM kernels from a state; BN is the tile width of the kernel that will run
 static void fill_spmm_launch_args(const shflbw_spmm_state* state, int BN, SpmmLaunchArgs* out)
 {
@@ -319,6 +329,7 @@ static void fill_spmm_launch_args(const shflbw_spmm_state* state, int BN, SpmmLa
     a.beta = state->args.beta;
     a.num_cus = device_compute_units();
     a.ldd = a.N;
+    a.merge_lines = store_merges_lines(a.D, a.M, a.ldd);
     a.dmap_row = a.dmap_valid = 0, a.dmap_magic = 0;
     // rows of B one column tile can touch: above about 2.5 MB they do not stay in the 4 MB L2 of an XCD
     // from one round of tiles to the next, and alternating the direction of the walk pays (measured:
@@ -1398,6 +1409,7 @@ int shflbw_spconv_exec(const shflbw_spconv_state* state, void* stream)
         fill_spmm_launch_args(&state->spmm, k->BN, &m);
         m.alternate = 0;
         m.ldd = a.Ho * a.Wo * a.B;                  // a row of the result: one filter, Ho x Wo x B values
+        m.merge_lines = store_merges_lines(m.D, m.M, m.ldd);
         m.dmap_row = state->plane_cols * a.B;       // columns of the GEMM per row of the padded output grid
         m.dmap_valid = a.Wo * a.B;                  // ... of which the first Wo x B are output values
         m.dmap_magic = udiv_magic(m.dmap_row);

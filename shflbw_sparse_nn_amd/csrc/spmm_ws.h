@@ -186,6 +186,15 @@ __device__ __forceinline__ void ws_consumer(const SpmmLaunchArgs& a, uint32_t ld
     constexpr int PRE = !RES || Cfg::WGS_PER_CU != 1 || Cfg::THREADS > 512 ? 0 : STEPS < 6 ? STEPS : 6;
     constexpr int PRE1 = PRE > 0 ? PRE : 1;
 
+    // Device scope, unless a.merge_lines: where the rows of D do not start at whole lines, a line is written in parts, by
+    // neighbouring store instructions, and each part written through is a write to memory of its own; ordinary stores merge in the
+    // L2 (4096 x 1640 x 16376, density 0.05, block height 128: 88.5 us written through, 63.5 merged; N = 16368: 73 and 57).
+    // What is dirty there when the launch ends is written back then, so this pays once D is larger than the L2s (see
+    // store_merges_lines).
+    auto store = [&](half_t* p, half8_t v, auto merge) __attribute__((always_inline)) {
+        store_result_16B<!XCD_LOCAL && !decltype(merge)::value>(p, v);
+    };
+
     struct Frags {
         half8_t a[MB], b[NB];
     };
@@ -332,7 +341,7 @@ __device__ __forceinline__ void ws_consumer(const SpmmLaunchArgs& a, uint32_t ld
         constexpr int LROWB = 128 + 16;
         const uint32_t wrl = epi + (lane & 15) * LROWB + (lane >> 5) * 8;
         const uint32_t rdl = epi + (lane >> 3) * LROWB + (lane & 7) * 16;
-        auto epi_lines = [&](int mb, auto scale, auto add_c) __attribute__((always_inline)) {
+        auto epi_lines = [&](int mb, auto scale, auto add_c, auto merge) __attribute__((always_inline)) {
             constexpr bool SCALE = decltype(scale)::value, ADDC = decltype(add_c)::value;
 #pragma unroll
             for (int np = 0; np < NB / 2; np++)
@@ -390,14 +399,14 @@ __device__ __forceinline__ void ws_consumer(const SpmmLaunchArgs& a, uint32_t ld
                     }
                     if (keep) {
 #pragma unroll
-                        for (int it = 0; it < 2; it++) store_result_16B<!XCD_LOCAL>(a.D + roff[it] + col, v[it]);
+                        for (int it = 0; it < 2; it++) store(a.D + roff[it] + col, v[it], merge);
                     }
                 }
         };
-        auto epi_block = [&](int mb, auto scale, auto add_c) __attribute__((always_inline)) {
+        auto epi_block = [&](int mb, auto scale, auto add_c, auto merge) __attribute__((always_inline)) {
             constexpr bool SCALE = decltype(scale)::value, ADDC = decltype(add_c)::value;
             if constexpr (LINES) {
-                epi_lines(mb, scale, add_c);
+                epi_lines(mb, scale, add_c, merge);
                 return;
             }
 #pragma unroll
@@ -454,7 +463,7 @@ __device__ __forceinline__ void ws_consumer(const SpmmLaunchArgs& a, uint32_t ld
                     }
                     if (keep) {
 #pragma unroll
-                        for (int it = 0; it < NIT; it++) store_result_16B<!XCD_LOCAL>(a.D + roff[it] + col, v[it]);
+                        for (int it = 0; it < NIT; it++) store(a.D + roff[it] + col, v[it], merge);
                     }
                 }
             }
@@ -467,16 +476,22 @@ __device__ __forceinline__ void ws_consumer(const SpmmLaunchArgs& a, uint32_t ld
         using T = std::true_type;
         using F = std::false_type;
         // one straight-line sequence over all 32-row blocks per specialisation
-        if constexpr (RES) {
+        auto epilogue = [&](auto merge) __attribute__((always_inline)) {
+            if constexpr (RES) {
 #pragma unroll
-            for (int mb = 0; mb < MB; mb++) epi_block(mb, T{}, T{});
-        } else if (alpha == 1.f) {
+                for (int mb = 0; mb < MB; mb++) epi_block(mb, T{}, T{}, merge);
+            } else if (alpha == 1.f) {
 #pragma unroll
-            for (int mb = 0; mb < MB; mb++) epi_block(mb, F{}, F{});
-        } else {
+                for (int mb = 0; mb < MB; mb++) epi_block(mb, F{}, F{}, merge);
+            } else {
 #pragma unroll
-            for (int mb = 0; mb < MB; mb++) epi_block(mb, T{}, F{});
-        }
+                for (int mb = 0; mb < MB; mb++) epi_block(mb, T{}, F{}, merge);
+            }
+        };
+        if (!XCD_LOCAL && a.merge_lines)
+            epilogue(T{});
+        else
+            epilogue(F{});
     }
 }
 
@@ -500,6 +515,11 @@ __device__ __forceinline__ void ws_consumer16(const SpmmLaunchArgs& a, uint32_t 
     }
     const uint32_t aoff = (uint32_t)(B_BYTES + lane * 16);
     const uint32_t epi = lds0 + Cfg::RING_BYTES + cw * Cfg::EPI_WAVE_BYTES;
+
+    // (see ws_consumer)
+    auto store = [&](half_t* p, half8_t v, auto merge) __attribute__((always_inline)) {
+        store_result_16B<!XCD_LOCAL && !decltype(merge)::value>(p, v);
+    };
 
     struct Frags {
         half8_t a, b[NB];
@@ -587,32 +607,38 @@ __device__ __forceinline__ void ws_consumer16(const SpmmLaunchArgs& a, uint32_t 
         size_t roff[2];
 #pragma unroll
         for (int it = 0; it < 2; it++) roff[it] = (size_t)__shfl(orow, it * 8 + (lane >> 3)) * a.ldd;
+        auto epilogue = [&](auto merge) __attribute__((always_inline)) {
 #pragma unroll
-        for (int h = 0; h < WN / 64; h++) {
+            for (int h = 0; h < WN / 64; h++) {
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                half4_t hv;
+                for (int q = 0; q < 4; q++) {
+                    half4_t hv;
 #pragma unroll
-                for (int e = 0; e < 4; e++) hv[e] = (half_t)scaled(acc[h * 4 + q][e], alpha, RES);
-                *(SHFLBW_LDS half4_t*)(uintptr_t)(wr + q * 32) = hv;
-            }
-            half8_t v[2];
-#pragma unroll
-            for (int it = 0; it < 2; it++) v[it] = *(SHFLBW_LDS half8_t*)(uintptr_t)(rd + it * 8 * EROWB);
-            int col = n0 + cw * WN + h * 64 + (lane & 7) * 8;
-            bool keep = col < N;
-            if (DMAP) keep = keep && output_column(a, col);
-            if (keep) {
-                if (RES) {
-#pragma unroll
-                    for (int it = 0; it < 2; it++)
-#pragma unroll
-                        for (int e = 0; e < 8; e++) v[it][e] = (half_t)((float)v[it][e] + beta * (float)c[h][it][e]);
+                    for (int e = 0; e < 4; e++) hv[e] = (half_t)scaled(acc[h * 4 + q][e], alpha, RES);
+                    *(SHFLBW_LDS half4_t*)(uintptr_t)(wr + q * 32) = hv;
                 }
+                half8_t v[2];
 #pragma unroll
-                for (int it = 0; it < 2; it++) store_result_16B<!XCD_LOCAL>(a.D + roff[it] + col, v[it]);
+                for (int it = 0; it < 2; it++) v[it] = *(SHFLBW_LDS half8_t*)(uintptr_t)(rd + it * 8 * EROWB);
+                int col = n0 + cw * WN + h * 64 + (lane & 7) * 8;
+                bool keep = col < N;
+                if (DMAP) keep = keep && output_column(a, col);
+                if (keep) {
+                    if (RES) {
+#pragma unroll
+                        for (int it = 0; it < 2; it++)
+#pragma unroll
+                            for (int e = 0; e < 8; e++) v[it][e] = (half_t)((float)v[it][e] + beta * (float)c[h][it][e]);
+                    }
+#pragma unroll
+                    for (int it = 0; it < 2; it++) store(a.D + roff[it] + col, v[it], merge);
+                }
             }
-        }
+        };
+        if (!XCD_LOCAL && a.merge_lines)
+            epilogue(std::true_type{});
+        else
+            epilogue(std::false_type{});
     }
 }
 
