@@ -294,14 +294,22 @@ static int plane_form_geometry(const shflbw_weight* f, int B, int H, int W, int 
     return SHFLBW_OK;
 }
 
-// Whether the results of a role-split launch are merged in the L2s (ordinary stores) instead of written through (device
-// scope): where rows of D start inside a line and D is at least three quarters of the eight L2s.  Block height 64,
-// K = 1640, density 0.1, written through / merged: 4096 x 1000 6.3 / 6.9 us, 4096 x 2008 10.4 / 10.9, 1024 x 8008 9.8 / 10.3 (16 MB);
-// 4096 x 4008 15.5 / 15.2, 16384 x 1000 16.0 / 15.1 (33 MB); 4096 x 8008 38.7 / 32.1.  On whole lines they are level for large D,
-// and 4096^3 takes 18.9 written through, 21.1 merged.
-static bool store_merges_lines(const void* D, int rows, int ldd)
+// How the role-split kernels store D.
+//  * Rows that do not start at whole lines: every line is written in parts, by neighbouring store instructions, and each part
+//    written through is a write to memory of its own.  Merged in the L2 once D is three quarters of the eight L2s, as what is
+//    dirty there when the launch ends is written back then.  us, through / merged, block height 64, K = 1640, density 0.1:
+//    4096 x 1000 6.3 / 6.9, 4096 x 2008 10.4 / 10.9, 1024 x 8008 9.8 / 10.3 (16 MB); 4096 x 4008 15.5 / 15.2, 16384 x 1000 16.0 / 15.1
+//    (33 MB); 4096 x 8008 38.7 / 32.1; block height 128, 4096 x 1640 x 16376, density 0.05: 88.5 / 63.5.
+//  * Whole lines: streamed from 96 MB on, if nothing reads D back at once; smaller results, also three of them in turn, stay in
+//    the Infinity Cache.  us, through / streamed, density 0.1, block height 64, K = 1640 or 2048: 16384 x 1024 12.5 / 12.9 (33 MB),
+//    6144 x 4096 30.8 / 30.3 (50 MB), 16384 x 2560 28.6 / 28.5, 16384 x 2816 34.3 / 33.0 (92 MB), 8192 x 6400 45 / 40, 8192 x 8192 58 / 50;
+//    block height 128: 16384 x 2048 23.5 / 26.0 (67 MB), 16384 x 2816 35.3 / 37.1, 8192 x 6400 74 / 69, 4096 x 16384 65 / 52; 16:
+//    16384 x 4096 110 / 89.  Merged: as written through for large D, 4096^3 21 / 25.
+static StoreMode result_store_mode(const void* D, int rows, int ldd, bool read_back)
 {
-    return (((uintptr_t)D | ((uintptr_t)ldd * 2)) & 127) != 0 && (size_t)rows * (size_t)ldd * 2 >= 24u << 20;
+    const size_t bytes = (size_t)rows * (size_t)ldd * 2;
+    if ((((uintptr_t)D | ((uintptr_t)ldd * 2)) & 127) != 0) return bytes >= 24u << 20 ? STORE_MERGE : STORE_THROUGH;
+    return bytes >= 96u << 20 && !read_back ? STORE_STREAM : STORE_THROUGH;
 }
 
 // launch arguments of the SpMM kernels from a state; BN is the tile width of the kernel that will run
@@ -329,7 +337,7 @@ static void fill_spmm_launch_args(const shflbw_spmm_state* state, int BN, SpmmLa
     a.beta = state->args.beta;
     a.num_cus = device_compute_units();
     a.ldd = a.N;
-    a.merge_lines = store_merges_lines(a.D, a.M, a.ldd);
+    a.store_mode = result_store_mode(a.D, a.M, a.ldd, a.ldb_bytes != a.N * 2); // (planes: the layout kernel behind it reads D)
     a.dmap_row = a.dmap_valid = 0, a.dmap_magic = 0;
     // rows of B one column tile can touch: above about 2.5 MB they do not stay in the 4 MB L2 of an XCD
     // from one round of tiles to the next, and alternating the direction of the walk pays (measured:
@@ -1388,6 +1396,7 @@ int shflbw_spconv_exec(const shflbw_spconv_state* state, void* stream)
             ChwbTapArgs t;
             fill_spmm_launch_args(&state->spmm, k->BN, &t);
             t.B = a.in;
+            t.store_mode = result_store_mode(t.D, t.M, t.ldd, false);
             t.alternate = 0;
             t.batch = a.B, t.in_h = a.H, t.in_w = a.W;
             t.taps_r = a.R, t.taps_s = a.S, t.stride = a.stride;
@@ -1409,7 +1418,7 @@ int shflbw_spconv_exec(const shflbw_spconv_state* state, void* stream)
         fill_spmm_launch_args(&state->spmm, k->BN, &m);
         m.alternate = 0;
         m.ldd = a.Ho * a.Wo * a.B;                  // a row of the result: one filter, Ho x Wo x B values
-        m.merge_lines = store_merges_lines(m.D, m.M, m.ldd);
+        m.store_mode = result_store_mode(m.D, m.M, m.ldd, nhwc);
         m.dmap_row = state->plane_cols * a.B;       // columns of the GEMM per row of the padded output grid
         m.dmap_valid = a.Wo * a.B;                  // ... of which the first Wo x B are output values
         m.dmap_magic = udiv_magic(m.dmap_row);

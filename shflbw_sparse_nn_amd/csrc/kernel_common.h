@@ -100,18 +100,23 @@ __device__ __forceinline__ void wait_vmcnt_fence()
 }
 
 // 16-byte store of result values.
-// DEVICE_SCOPE (the SpMM proper): the line is written through to memory instead of staying dirty in the XCD's L2,
-// where its later eviction would fall into the gathers of the next tile.  The compiler has no form of this store,
-// so it is inline assembly, and the compiler's hazard pass does not look inside: a vector-ALU write to the data
-// registers directly behind a store of more than 8 bytes needs wait states, which the s_nop supplies (the
-// registers are free for reuse after the statement).
-// Otherwise (results that workgroups of the same XCD read back in the same launch): an ordinary store, the line
-// stays in the XCD's L2.
-template <bool DEVICE_SCOPE = true>
+// THROUGH (device scope): the line is written through to memory instead of staying dirty in the XCD's L2, where its later
+// eviction would fall into the gathers of the next tile, and nothing is left to write back when the launch ends; this path
+// carries 2.7-2.9 TB/s, whatever the width of the tiles.  MERGE (an ordinary store): the line stays in the L2, where the parts of
+// a line that several instructions write meet, and where workgroups of the same XCD find it; 4.4-5 TB/s.  STREAM: the line
+// leaves the L2 first, so it does not push out what is still to be read, at 4.8-5.2 TB/s (64 columns wide: 3.4), but parts of a
+// line mostly leave one by one (rates: D alone, 8192 x 8192, tiles of 256 columns, more buffers than the Infinity Cache holds).
+// The compiler has no form of these stores, so they are inline assembly, and the compiler's hazard pass does not look
+// inside: a vector-ALU write to the data registers directly behind a store of more than 8 bytes needs wait states, which
+// the s_nop supplies (the registers are free for reuse after the statement).
+enum StoreMode { STORE_THROUGH = 0, STORE_MERGE = 1, STORE_STREAM = 2 };
+template <StoreMode MODE = STORE_THROUGH>
 __device__ __forceinline__ void store_result_16B(half_t* p, half8_t v)
 {
-    if constexpr (DEVICE_SCOPE)
+    if constexpr (MODE == STORE_THROUGH)
         asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" : : "v"(p), "v"(v) : "memory");
+    else if constexpr (MODE == STORE_STREAM)
+        asm volatile("global_store_dwordx4 %0, %1, off nt\n\ts_nop 1" : : "v"(p), "v"(v) : "memory");
     else
         asm volatile("global_store_dwordx4 %0, %1, off\n\ts_nop 1" : : "v"(p), "v"(v) : "memory");
 }

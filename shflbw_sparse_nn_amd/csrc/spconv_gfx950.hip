@@ -265,7 +265,7 @@ __global__ void __launch_bounds__(256) nhwc_to_planes_kernel(const half_t* __res
         },
         [&](int o, int q, half8_t v) { // destination row = channel c0 + o, positions p0 + 8q ..
             // written through (device scope): the planes do not wait dirty in the L2s for the end of the launch
-            if (c0 + o < g.C) store_result_16B<true>(dst + (size_t)(c0 + o) * g.pitch + p0 + q * 8, v);
+            if (c0 + o < g.C) store_result_16B<STORE_THROUGH>(dst + (size_t)(c0 + o) * g.pitch + p0 + q * 8, v);
         });
 }
 
@@ -289,7 +289,7 @@ __global__ void __launch_bounds__(256) planes_to_nhwc_kernel(const half_t* __res
             // written through: the output is not read again here, and nothing waits dirty for the end of the launch (a
             // streaming store was 1 % slower, an ordinary one 5 %)
             if (img < B && ho < Ho && wo < Wo && f < F)
-                store_result_16B<true>(out + ((size_t)(img * Ho + ho) * Wo + wo) * F + f, v);
+                store_result_16B<STORE_THROUGH>(out + ((size_t)(img * Ho + ho) * Wo + wo) * F + f, v);
         });
 }
 

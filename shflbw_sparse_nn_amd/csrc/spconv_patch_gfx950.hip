@@ -463,8 +463,8 @@ __global__ void __launch_bounds__(NW * 64, WPE) spconv_patch_kernel(ConvPatchArg
             }
             const int r = r0 + g8 + (li >> 3) * 32;
             const int pix0 = tout[cb * 16 + (li & 7)], pix1 = tout[cb * 16 + 8 + (li & 7)];
-            if (pix0 >= 0 && r < rows) store_result_16B<true>(a.out + (size_t)pix0 * a.F + row0 + r, __builtin_bit_cast(half8_t, first));
-            if (pix1 >= 0 && r < rows) store_result_16B<true>(a.out + (size_t)pix1 * a.F + row0 + r, __builtin_bit_cast(half8_t, second));
+            if (pix0 >= 0 && r < rows) store_result_16B<STORE_THROUGH>(a.out + (size_t)pix0 * a.F + row0 + r, __builtin_bit_cast(half8_t, first));
+            if (pix1 >= 0 && r < rows) store_result_16B<STORE_THROUGH>(a.out + (size_t)pix1 * a.F + row0 + r, __builtin_bit_cast(half8_t, second));
         }
     } else { // a chunk's filters are scattered over the pixel: 2-byte pieces in ascending order, merged in the L2
         constexpr int MAXQ = 8;

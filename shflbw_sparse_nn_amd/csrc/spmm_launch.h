@@ -22,7 +22,7 @@ struct SpmmLaunchArgs {
     const half_t* C;
     half_t* D;
     int ldd;                // values between two rows of C and D (N for the SpMM)
-    int merge_lines;        // D is stored without device scope: see store_merges_lines
+    int store_mode;         // a StoreMode: how the role-split kernels store D, see result_store_mode
     int dmap_row, dmap_valid; // batch-innermost convolution only: see output_column()
     unsigned dmap_magic;      // udiv magic of dmap_row
     float alpha, beta;

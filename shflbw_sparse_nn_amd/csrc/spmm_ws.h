@@ -186,13 +186,9 @@ __device__ __forceinline__ void ws_consumer(const SpmmLaunchArgs& a, uint32_t ld
     constexpr int PRE = !RES || Cfg::WGS_PER_CU != 1 || Cfg::THREADS > 512 ? 0 : STEPS < 6 ? STEPS : 6;
     constexpr int PRE1 = PRE > 0 ? PRE : 1;
 
-    // Device scope, unless a.merge_lines: where the rows of D do not start at whole lines, a line is written in parts, by
-    // neighbouring store instructions, and each part written through is a write to memory of its own; ordinary stores merge in the
-    // L2 (4096 x 1640 x 16376, density 0.05, block height 128: 88.5 us written through, 63.5 merged; N = 16368: 73 and 57).
-    // What is dirty there when the launch ends is written back then, so this pays once D is larger than the L2s (see
-    // store_merges_lines).
-    auto store = [&](half_t* p, half8_t v, auto merge) __attribute__((always_inline)) {
-        store_result_16B<!XCD_LOCAL && !decltype(merge)::value>(p, v);
+    // (XCD_LOCAL: other workgroups of the XCD read the result back from the L2)
+    auto store = [&](half_t* p, half8_t v, auto mode) __attribute__((always_inline)) {
+        store_result_16B<XCD_LOCAL ? STORE_MERGE : decltype(mode)::value>(p, v);
     };
 
     struct Frags {
@@ -341,7 +337,7 @@ __device__ __forceinline__ void ws_consumer(const SpmmLaunchArgs& a, uint32_t ld
         constexpr int LROWB = 128 + 16;
         const uint32_t wrl = epi + (lane & 15) * LROWB + (lane >> 5) * 8;
         const uint32_t rdl = epi + (lane >> 3) * LROWB + (lane & 7) * 16;
-        auto epi_lines = [&](int mb, auto scale, auto add_c, auto merge) __attribute__((always_inline)) {
+        auto epi_lines = [&](int mb, auto scale, auto add_c, auto mode) __attribute__((always_inline)) {
             constexpr bool SCALE = decltype(scale)::value, ADDC = decltype(add_c)::value;
 #pragma unroll
             for (int np = 0; np < NB / 2; np++)
@@ -399,14 +395,14 @@ __device__ __forceinline__ void ws_consumer(const SpmmLaunchArgs& a, uint32_t ld
                     }
                     if (keep) {
 #pragma unroll
-                        for (int it = 0; it < 2; it++) store(a.D + roff[it] + col, v[it], merge);
+                        for (int it = 0; it < 2; it++) store(a.D + roff[it] + col, v[it], mode);
                     }
                 }
         };
-        auto epi_block = [&](int mb, auto scale, auto add_c, auto merge) __attribute__((always_inline)) {
+        auto epi_block = [&](int mb, auto scale, auto add_c, auto mode) __attribute__((always_inline)) {
             constexpr bool SCALE = decltype(scale)::value, ADDC = decltype(add_c)::value;
             if constexpr (LINES) {
-                epi_lines(mb, scale, add_c, merge);
+                epi_lines(mb, scale, add_c, mode);
                 return;
             }
 #pragma unroll
@@ -463,7 +459,7 @@ __device__ __forceinline__ void ws_consumer(const SpmmLaunchArgs& a, uint32_t ld
                     }
                     if (keep) {
 #pragma unroll
-                        for (int it = 0; it < NIT; it++) store(a.D + roff[it] + col, v[it], merge);
+                        for (int it = 0; it < NIT; it++) store(a.D + roff[it] + col, v[it], mode);
                     }
                 }
             }
@@ -476,22 +472,24 @@ __device__ __forceinline__ void ws_consumer(const SpmmLaunchArgs& a, uint32_t ld
         using T = std::true_type;
         using F = std::false_type;
         // one straight-line sequence over all 32-row blocks per specialisation
-        auto epilogue = [&](auto merge) __attribute__((always_inline)) {
+        auto epilogue = [&](auto mode) __attribute__((always_inline)) {
             if constexpr (RES) {
 #pragma unroll
-                for (int mb = 0; mb < MB; mb++) epi_block(mb, T{}, T{}, merge);
+                for (int mb = 0; mb < MB; mb++) epi_block(mb, T{}, T{}, mode);
             } else if (alpha == 1.f) {
 #pragma unroll
-                for (int mb = 0; mb < MB; mb++) epi_block(mb, F{}, F{}, merge);
+                for (int mb = 0; mb < MB; mb++) epi_block(mb, F{}, F{}, mode);
             } else {
 #pragma unroll
-                for (int mb = 0; mb < MB; mb++) epi_block(mb, T{}, F{}, merge);
+                for (int mb = 0; mb < MB; mb++) epi_block(mb, T{}, F{}, mode);
             }
         };
-        if (!XCD_LOCAL && a.merge_lines)
-            epilogue(T{});
+        if (XCD_LOCAL || a.store_mode == STORE_THROUGH)
+            epilogue(std::integral_constant<StoreMode, STORE_THROUGH>{});
+        else if (a.store_mode == STORE_MERGE)
+            epilogue(std::integral_constant<StoreMode, STORE_MERGE>{});
         else
-            epilogue(F{});
+            epilogue(std::integral_constant<StoreMode, STORE_STREAM>{});
     }
 }
 
@@ -517,8 +515,8 @@ __device__ __forceinline__ void ws_consumer16(const SpmmLaunchArgs& a, uint32_t 
     const uint32_t epi = lds0 + Cfg::RING_BYTES + cw * Cfg::EPI_WAVE_BYTES;
 
     // (see ws_consumer)
-    auto store = [&](half_t* p, half8_t v, auto merge) __attribute__((always_inline)) {
-        store_result_16B<!XCD_LOCAL && !decltype(merge)::value>(p, v);
+    auto store = [&](half_t* p, half8_t v, auto mode) __attribute__((always_inline)) {
+        store_result_16B<XCD_LOCAL ? STORE_MERGE : decltype(mode)::value>(p, v);
     };
 
     struct Frags {
@@ -607,7 +605,7 @@ __device__ __forceinline__ void ws_consumer16(const SpmmLaunchArgs& a, uint32_t 
         size_t roff[2];
 #pragma unroll
         for (int it = 0; it < 2; it++) roff[it] = (size_t)__shfl(orow, it * 8 + (lane >> 3)) * a.ldd;
-        auto epilogue = [&](auto merge) __attribute__((always_inline)) {
+        auto epilogue = [&](auto mode) __attribute__((always_inline)) {
 #pragma unroll
             for (int h = 0; h < WN / 64; h++) {
 #pragma unroll
@@ -631,14 +629,16 @@ __device__ __forceinline__ void ws_consumer16(const SpmmLaunchArgs& a, uint32_t 
                             for (int e = 0; e < 8; e++) v[it][e] = (half_t)((float)v[it][e] + beta * (float)c[h][it][e]);
                     }
 #pragma unroll
-                    for (int it = 0; it < 2; it++) store(a.D + roff[it] + col, v[it], merge);
+                    for (int it = 0; it < 2; it++) store(a.D + roff[it] + col, v[it], mode);
                 }
             }
         };
-        if (!XCD_LOCAL && a.merge_lines)
-            epilogue(std::true_type{});
+        if (XCD_LOCAL || a.store_mode == STORE_THROUGH)
+            epilogue(std::integral_constant<StoreMode, STORE_THROUGH>{});
+        else if (a.store_mode == STORE_MERGE)
+            epilogue(std::integral_constant<StoreMode, STORE_MERGE>{});
         else
-            epilogue(std::false_type{});
+            epilogue(std::integral_constant<StoreMode, STORE_STREAM>{});
     }
 }
 
