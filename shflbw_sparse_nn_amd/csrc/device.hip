@@ -325,7 +325,8 @@ static void fill_spmm_launch_args(const shflbw_spmm_state* state, int BN, SpmmLa
     a.kidx = state->packed_indices;
     a.kidx_pm = state->packed_indices_pm;
     a.slab_ids = state->packed_slab;
-    a.slab_chunks = 1;
+    a.slab_chunks = 1, a.slab_by_chunk = 0;
+    a.groups = state->groups;
     a.panel_desc = state->panel_ptr;
     a.row_ids = state->args.A_row_indices;
     a.B = (const half_t*)state->args.B;
@@ -451,6 +452,7 @@ static int spmm_init_impl(shflbw_spmm_state* state, const shflbw_weight* w, int 
     state->packed_indices = (const int*)w->d_packed_indices;
     state->packed_indices_pm = (const int*)w->d_packed_indices_pm;
     state->packed_slab = w->packed_slab.empty() ? nullptr : (const int*)w->d_packed_slab;
+    state->groups = (int)(w->packed_indices.size() / 64);
     state->panel_ptr = (const int*)w->d_group_ptr;
     state->brow = w->brow;
     state->ldb_bytes = N * 2;

@@ -348,6 +348,47 @@ static hipError_t prepare_ws(const SpmmLaunchArgs&)
 // ---------------------------------------------------------------------------------------
 // slab form (all rows of a 64-column slab of B in LDS): launcher
 // ---------------------------------------------------------------------------------------
+// How the panels under a column tile are dealt to workgroups, which jobs an XCD shares, and how D is stored.
+template <int V>
+static void slab_plan(SpmmLaunchArgs& b, int cus)
+{
+    using Cfg = SpmmSlabCfg<V>;
+    const size_t d_bytes = (size_t)b.M * (size_t)b.ldd * 2;
+    const bool lines = (((uintptr_t)b.D | ((uintptr_t)b.ldd * 2)) & 127) == 0;
+    // As for the role-split kernels (result_store_mode).  us, through / merged / streamed, the better order of jobs each: whole lines,
+    // block height 32, density 0.2: 4096 x 1024 x 4096 17.0 / 18.1 / 17.2, 8192 x 768 x 8192 62 / 62 / 48; block height 16, 33728 x 777 x
+    // 1024 22.1 / 24.3 / 22.4, 20000 x 1000 x 6016 85 / 89 / 69.  Parts of lines: 8192 x 777 x 3000 (49 MB) 19.4 / 21.0 / 32, 33728 x 777 x
+    // 1000 (67 MB) 22.7 / 24.1 / 45, block height 32, 16384 x 800 x 2056 (67 MB) 42 / 35.5 / 49, 33728 x 1100 x 2104 136 / 123 / 121, 16:
+    // 20000 x 1000 x 6000 145 / 101 / 125.
+    b.store_mode = lines ? (d_bytes >= 96u << 20 ? STORE_STREAM : STORE_THROUGH) : d_bytes >= 64u << 20 ? STORE_MERGE : STORE_THROUGH;
+    // Chunks: at least as many as keep the panels of one wave within RID_REGS * 64 rows; then the number that takes the least
+    // rounds * (slab + panels of a wave), of the most that one, two and three rounds of the compute units have room for (us, from
+    // the phases of a wave).  33728 x 1100 x 2112, block height 32: 33 tiles x 9 chunks were two rounds, the second nearly empty, 91 us;
+    // 15 chunks 66.
+    const int rows_per_wg = Cfg::NW * Cfg::RID_REGS * 64, least = (b.M + rows_per_wg - 1) / rows_per_wg;
+    const double batches = 2.0 * b.groups / b.X; // of 32 slots, per panel
+    const double t_slab = 1.0 + 1.5e-3 * b.K, t_panel = V == 16 ? 0.30 + 0.12 * batches : 0.45 + 0.21 * batches;
+    double best = 0;
+    for (int r = 1; r <= 3; r++) {
+        const int c = std::max(1, std::min(b.X, std::max(least, cus * r / b.n_tiles)));
+        const int rounds = ((b.n_tiles * c + 7) / 8 * 8 + cus - 1) / cus;
+        const int wave_panels = ((b.X + c - 1) / c + Cfg::NW - 1) / Cfg::NW;
+        const double t = rounds * (t_slab + wave_panels * t_panel);
+        if (r == 1 || t < best * 0.95) best = t, b.slab_chunks = c;
+    }
+    // Order of the jobs.  An XCD owns T / 8 of them, side by side: by tile it reads few slabs and most of A, by chunk a part of A
+    // and most of B.  The order with fewer bytes into the L2s; by chunk where parts of lines are merged, as the tiles that
+    // share lines then lie on one XCD.  us, by tile / by chunk, block height 16: 33728 x 777 x 1024 (A 9 MB, B 1.6) 26.4 / 22.1, x 1000 29.6 /
+    // 22.7, 33728 x 1128 x 136 16.2 / 12.6; 8192 x 777 x 3000 (A 1.3, B 4.7) 19.4 / 20.8, 20000 x 1000 x 6000 merged 116 / 101; 32: 4096 x 1024 x
+    // 4096 (A 2.2, B 8.4) 17.0 / 19.3.
+    const int c = b.slab_chunks, per = std::max(1, (b.n_tiles * c + 7) / 8);
+    const double a_bytes = (double)b.groups * (64 * V * 2 + 256), slab_bytes = (double)Cfg::ROWB * b.K;
+    auto into_l2 = [&](double tiles, double chunks) { return tiles * slab_bytes + chunks / c * a_bytes; };
+    const double by_tile = into_l2(std::max(1.0, (double)per / c), std::min(c, per));
+    const double by_chunk = into_l2(std::min(b.n_tiles, per), std::max(1.0, (double)per / b.n_tiles));
+    b.slab_by_chunk = b.store_mode == STORE_MERGE || by_chunk < by_tile;
+}
+
 template <int V>
 static hipError_t launch_slab(const SpmmLaunchArgs& a, hipStream_t stream)
 {
@@ -355,22 +396,25 @@ static hipError_t launch_slab(const SpmmLaunchArgs& a, hipStream_t stream)
     if (a.K > Cfg::MAX_K || !a.slab_ids || a.K <= 0) return hipErrorInvalidValue;
     SpmmLaunchArgs b = a;
     b.n_tiles = (a.N + Cfg::BN - 1) / Cfg::BN;
-    // the panels under one column tile are dealt to as many workgroups as it takes to give every compute unit a job
-    // ... and so that the panels of one wave have at most RID_REGS * 64 rows
     const int cus = ((a.num_cus > 0 ? a.num_cus : 256) / 8) * 8;
-    const int rows_per_wg = Cfg::NW * Cfg::RID_REGS * 64;
-    b.slab_chunks = std::max(1, std::min(a.X, std::max(cus / b.n_tiles, (a.M + rows_per_wg - 1) / rows_per_wg)));
+    slab_plan<V>(b, cus);
     const int T = b.n_tiles * b.slab_chunks;
     const int grid = std::min(cus, ((T + 7) / 8) * 8);
-    hipLaunchKernelGGL((spmm_shflbw_slab_kernel<V>), dim3(grid), dim3(Cfg::THREADS), Cfg::lds_bytes(a.K), stream, b);
+    const auto kernel = b.store_mode == STORE_THROUGH ? &spmm_shflbw_slab_kernel<V, STORE_THROUGH>
+                        : b.store_mode == STORE_MERGE ? &spmm_shflbw_slab_kernel<V, STORE_MERGE>
+                                                      : &spmm_shflbw_slab_kernel<V, STORE_STREAM>;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(Cfg::THREADS), Cfg::lds_bytes(a.K), stream, b);
     return hipGetLastError();
 }
 
 template <int V>
 static hipError_t prepare_slab(const SpmmLaunchArgs&)
 {
-    return hipFuncSetAttribute((const void*)spmm_shflbw_slab_kernel<V>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               SpmmSlabCfg<V>::LDS_MAX);
+    for (const void* f : {(const void*)&spmm_shflbw_slab_kernel<V, STORE_THROUGH>, (const void*)&spmm_shflbw_slab_kernel<V, STORE_MERGE>,
+                          (const void*)&spmm_shflbw_slab_kernel<V, STORE_STREAM>})
+        if (hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, SpmmSlabCfg<V>::LDS_MAX); e != hipSuccess)
+            return e;
+    return hipSuccess;
 }
 
 #define SHFLBW_SLAB_VARIANT(V)                                                                                    \

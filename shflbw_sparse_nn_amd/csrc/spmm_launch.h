@@ -13,7 +13,9 @@ struct SpmmLaunchArgs {
     const int* kidx;        // private image: kept column ids, 64-slot padded per panel
     const int* kidx_pm;     // same ids, each 64-slot group reordered producer-major: [16p + 4j + r] = [16j + 4p + r]
     const int* slab_ids;    // slab kernel only: the ids as LDS offsets of slab rows, [group][pair of slots][step][2]
+    int groups;             // 64-slot groups of all panels
     int slab_chunks;        // slab kernel only: the panels are dealt to this many workgroups per column tile (launcher)
+    int slab_by_chunk;      // slab kernel only: jobs of one chunk of panels lie side by side instead of those of one column tile (launcher)
     const int* panel_desc;  // private image: per panel {MFMA k16 steps = ceil(nnz/16), first 64-slot group}
     const int* row_ids;     // M, or null when rows are not permuted
     const half_t* B;
@@ -22,7 +24,7 @@ struct SpmmLaunchArgs {
     const half_t* C;
     half_t* D;
     int ldd;                // values between two rows of C and D (N for the SpMM)
-    int store_mode;         // a StoreMode: how the role-split kernels store D, see result_store_mode
+    int store_mode;         // a StoreMode: how D is stored, see result_store_mode (slab kernel: slab_plan)
     int dmap_row, dmap_valid; // batch-innermost convolution only: see output_column()
     unsigned dmap_magic;      // udiv magic of dmap_row
     float alpha, beta;

@@ -14,7 +14,7 @@
 // A panel's 32 x 64 result goes through the wave's private staging area to D like in the role-split kernel.
 // Block height 16 (one 16x16x32 step of 32 slots per batch): a gathered value feeds only 16 MACs in the role-split kernel,
 // which is bound by the path from the L2 there (33728 x 777 x 1000, density 0.1: 329 MB of gathers for 67 MB of result,
-// 32.8 us; here 29.6, the time of the 138 MB that cross the fabric, every XCD reading all of A; 8192 x 384 x 4096: 28.7 and 17.3).
+// 32.8 us; here 24; 8192 x 384 x 4096: 28.7 and 17.3).
 #pragma once
 #include <type_traits>
 
@@ -48,7 +48,8 @@ struct SpmmSlabCfg {
     static constexpr int lds_bytes(int K) { return (((K + 7) & ~7) + 1) * ROWB + NW * EPI_WAVE_BYTES; }
 };
 
-template <int V_>
+// MODE: how D is stored.  An instance each: the end of a panel stands in the loop over the batches eight times.
+template <int V_, StoreMode MODE>
 __global__ void __launch_bounds__(SpmmSlabCfg<V_>::THREADS) spmm_shflbw_slab_kernel(SpmmLaunchArgs a)
 {
     using Cfg = SpmmSlabCfg<V_>;
@@ -64,8 +65,9 @@ __global__ void __launch_bounds__(SpmmSlabCfg<V_>::THREADS) spmm_shflbw_slab_ker
     const uint32_t epi = lds0 + (uint32_t)(Kp + 1) * ROWB + wave * Cfg::EPI_WAVE_BYTES;
     const SHFLBW_CONST int2_t* desc = (const SHFLBW_CONST int2_t*)(uintptr_t)a.panel_desc;
 
-    // jobs = (column tile, chunk of panels), chunk-minor; XCD x owns a contiguous range of them, so the
-    // workgroups of an XCD share a few slabs of B and, over all chunks, the whole of A in their L2
+    // jobs = (column tile, chunk of panels); XCD x owns a contiguous range of them.  Chunk-minor, the workgroups of an XCD
+    // share a few slabs of B and, over all chunks, the whole of A in their L2; tile-minor (slab_by_chunk), a few chunks of
+    // A and the whole of B (see slab_plan)
     const int chunks = a.slab_chunks, ppc = (X + chunks - 1) / chunks;
     const int T = a.n_tiles * chunks;
     const int per = (T + 7) >> 3, xcd = blockIdx.x & 7, S = gridDim.x >> 3;
@@ -98,7 +100,8 @@ __global__ void __launch_bounds__(SpmmSlabCfg<V_>::THREADS) spmm_shflbw_slab_ker
 
     bool first = true;
     for (int job = xcd * per + (blockIdx.x >> 3); job < job_end; job += S) {
-        const int nt = job / chunks, ch = job - nt * chunks;
+        const int major = job / (a.slab_by_chunk ? a.n_tiles : chunks), minor = job - major * (a.slab_by_chunk ? a.n_tiles : chunks);
+        const int nt = a.slab_by_chunk ? minor : major, ch = a.slab_by_chunk ? major : minor;
         const int n0 = nt * BN;
         // ---- the slab first, so that everything below runs while it is on its way: rows 8q .. 8q+7 per copy
         // instruction (lane l: row l / 8, 16-byte position l % 8)
@@ -142,9 +145,7 @@ __global__ void __launch_bounds__(SpmmSlabCfg<V_>::THREADS) spmm_shflbw_slab_ker
                 for (int i = 0; i < (V16 ? 4 : 16); i++) acc[nb][i] = 0.f;
         };
         // fp32 -> fp16 (one rounding) -> staging area, 16 rows of all 64 columns at a time -> rows of D, eight lanes
-        // to a row: every store instruction writes whole 128-byte lines where N is a multiple of 64.  Elsewhere the ends of
-        // a row segment are half lines, which streaming stores bring to memory twice (8192 x 777 x 3000, block height 16,
-        // density 0.1: 32.5 us with them, 23.2 with ordinary stores, 22.5 with device scope; N = 4096: 24, 21 and 20)
+        // to a row: every store instruction writes whole 128-byte lines where N is a multiple of 64 (how: see slab_plan)
         auto epilogue = [&]() __attribute__((always_inline)) {
             const int i0 = (p - pa) * V; // first row of the panel among the wave's rows
             int rid = ridreg[0];
@@ -189,8 +190,7 @@ __global__ void __launch_bounds__(SpmmSlabCfg<V_>::THREADS) spmm_shflbw_slab_ker
                         }
                     }
 #pragma unroll
-                    for (int it = 0; it < 2; it++) // D must not push A and the slabs out of the L2
-                        store_result_16B(a.D + roff[it] + col, v[it]);
+                    for (int it = 0; it < 2; it++) store_result_16B<MODE>(a.D + roff[it] + col, v[it]);
                 }
             }
         };
