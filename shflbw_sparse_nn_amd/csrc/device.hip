@@ -1238,7 +1238,7 @@ int conv_patch_for(shflbw_weight* fw, int B, int H, int W, int stride, int Ho, i
         ConvPatchArgs& a = g->args;
         a.p = plan;
         a.C = fw->C, a.F = fw->F, a.R = fw->R, a.S = fw->S;
-        a.in = nullptr, a.out = nullptr; // each launch's own
+        a.in = nullptr, a.out = nullptr, a.streams = 0; // each launch's own
         a.packedA = (const half8_t*)image->ptr;
         a.first_batch = image->first_batch;
         a.offs = image->offs;
@@ -1384,6 +1384,7 @@ int shflbw_spconv_exec(const shflbw_spconv_state* state, void* stream)
         if (!k) return SHFLBW_ERR_UNSUPPORTED;
         p.in = (const half_t*)state->args.IFMap;
         p.out = (half_t*)state->args.OFMap;
+        p.streams = conv_patch_streams((size_t)state->ncols * (size_t)p.F * 2);
         e = k->launch(p, (hipStream_t)stream);
         if (e == hipSuccess) return SHFLBW_OK;
         set_error("spconv_exec: launch failed: %s", hipGetErrorString(e));

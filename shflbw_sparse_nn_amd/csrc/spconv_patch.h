@@ -84,7 +84,14 @@ struct ConvPatchArgs {
     const unsigned short* dst;     // per stored row: its place among the staged rows of its workgroup
     const int* filt;               // per chunk and place: the filter (used when not dense)
     int dense;                     // the filters of a chunk are consecutive in the output
+    int streams;                   // ... and leave by streaming stores (conv_patch_streams)
 };
+
+// Outputs from 60 MB on are streamed where the filters of a workgroup are consecutive; smaller ones, also three of them in turn,
+// stay in the Infinity Cache and are written through.  1 x 1 on 64 channels, 56 x 56, us through / streamed: 16 -> 256 filters (26 MB)
+// 9.2 / 9.3, 32 images -> 240 (48 MB) 25.3 / 26.3, 32 -> 256 (51 MB) 15.0 / 15.0, 64 -> 160 (64 MB) 35.6 / 31.6, 44 -> 256 (71 MB) 21.6 / 17.2, 48 -> 240
+// (72 MB) 41.2 / 33.9, 64 -> 256 (103 MB) 36.0 / 25.0, 64 -> 304 (122 MB) 122 / 101.  (Ordinary stores: 25.1 for the 71 MB, 36.8 for the 103.)
+inline bool conv_patch_streams(size_t out_bytes) { return out_bytes >= 60u << 20; }
 
 // Packs the A fragments of `batches` batches from the weight's values (kept vectors one behind the other).  src: per batch and
 // slot the row unit's part of a kept vector, as a multiple of `rows` values; -1: zeros (a padding slot).

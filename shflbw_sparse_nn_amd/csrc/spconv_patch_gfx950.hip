@@ -446,26 +446,32 @@ __global__ void __launch_bounds__(NW * 64, WPE) spconv_patch_kernel(ConvPatchArg
     if (a.dense) { // transposing reads: a lane gets 8 consecutive filters of one of 16 pixels, twice, 32 filters apart; lanes
                    // 8..15 of each 16 then trade places so that a store writes whole 128-byte lines of 8 pixels
         const int nit = NB * 2 * ((rows + 63) >> 6);
-        for (int it = wave; it < nit; it += NW) {
-            const int cb = it & (NB * 2 - 1), r0 = (it / (NB * 2)) * 64, g8 = (lane >> 4) * 8;
-            int4_t v[2];
+        auto whole_lines = [&](auto mode) __attribute__((always_inline)) {
+            for (int it = wave; it < nit; it += NW) {
+                const int cb = it & (NB * 2 - 1), r0 = (it / (NB * 2)) * 64, g8 = (lane >> 4) * 8;
+                int4_t v[2];
 #pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const uint32_t at = stage + (uint32_t)(min(r0 + h * 32 + g8, rows - 8) + (li >> 2)) * SP + cb * 32 + (li & 3) * 8;
-                const half4_t lo = lds_read_tr16(at), hi = lds_read_tr16(at + 4 * SP);
-                v[h] = __builtin_bit_cast(int4_t, (half8_t)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-            }
-            int4_t first, second;
+                for (int h = 0; h < 2; h++) {
+                    const uint32_t at = stage + (uint32_t)(min(r0 + h * 32 + g8, rows - 8) + (li >> 2)) * SP + cb * 32 + (li & 3) * 8;
+                    const half4_t lo = lds_read_tr16(at), hi = lds_read_tr16(at + 4 * SP);
+                    v[h] = __builtin_bit_cast(int4_t, (half8_t)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+                }
+                int4_t first, second;
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                first[e] = __builtin_amdgcn_update_dpp(v[0][e], v[1][e], 0x128, 0xf, 0xc, false);  // row_ror:8 into lanes 8..15
-                second[e] = __builtin_amdgcn_update_dpp(v[1][e], v[0][e], 0x128, 0xf, 0x3, false); // ... into lanes 0..7
+                for (int e = 0; e < 4; e++) {
+                    first[e] = __builtin_amdgcn_update_dpp(v[0][e], v[1][e], 0x128, 0xf, 0xc, false);  // row_ror:8 into lanes 8..15
+                    second[e] = __builtin_amdgcn_update_dpp(v[1][e], v[0][e], 0x128, 0xf, 0x3, false); // ... into lanes 0..7
+                }
+                const int r = r0 + g8 + (li >> 3) * 32;
+                const int pix0 = tout[cb * 16 + (li & 7)], pix1 = tout[cb * 16 + 8 + (li & 7)];
+                if (pix0 >= 0 && r < rows) store_result_16B<decltype(mode)::value>(a.out + (size_t)pix0 * a.F + row0 + r, __builtin_bit_cast(half8_t, first));
+                if (pix1 >= 0 && r < rows) store_result_16B<decltype(mode)::value>(a.out + (size_t)pix1 * a.F + row0 + r, __builtin_bit_cast(half8_t, second));
             }
-            const int r = r0 + g8 + (li >> 3) * 32;
-            const int pix0 = tout[cb * 16 + (li & 7)], pix1 = tout[cb * 16 + 8 + (li & 7)];
-            if (pix0 >= 0 && r < rows) store_result_16B<STORE_THROUGH>(a.out + (size_t)pix0 * a.F + row0 + r, __builtin_bit_cast(half8_t, first));
-            if (pix1 >= 0 && r < rows) store_result_16B<STORE_THROUGH>(a.out + (size_t)pix1 * a.F + row0 + r, __builtin_bit_cast(half8_t, second));
-        }
+        };
+        if (a.streams)
+            whole_lines(std::integral_constant<StoreMode, STORE_STREAM>{});
+        else
+            whole_lines(std::integral_constant<StoreMode, STORE_THROUGH>{});
     } else { // a chunk's filters are scattered over the pixel: 2-byte pieces in ascending order, merged in the L2
         constexpr int MAXQ = 8;
         int f[MAXQ];
