@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -96,16 +97,15 @@ int upload(shflbw_weight* w)
 // compute units of the current device, looked up once per device
 static int device_compute_units()
 {
-    static std::mutex lock;
-    static int cached[64] = {};
+    static std::atomic<int> cached[64]; // two threads may look the same number up at once
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    std::lock_guard<std::mutex> guard(lock);
-    if (cached[dev] == 0) {
-        int n = 0;
-        cached[dev] = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0 ? n : 256;
+    int n = cached[dev].load(std::memory_order_relaxed);
+    if (n == 0) {
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+        cached[dev].store(n, std::memory_order_relaxed);
     }
-    return cached[dev];
+    return n;
 }
 
 // The variants of a block height lie side by side in the table.  Every initialisation and launch looks one up: the ranges

@@ -816,9 +816,8 @@ static hipError_t launch_chwb(const Args& a, hipStream_t stream)
 template <int V, int WN, int NCONS, int NPROD, int KT, int NSTAGE, typename Args>
 static hipError_t prepare_chwb()
 {
-    using Cfg = SpmmWsCfg<V, WN, NCONS, NPROD, KT, NSTAGE>;
-    return hipFuncSetAttribute((const void*)spconv_chwb_kernel<V, WN, NCONS, NPROD, KT, NSTAGE, Args>,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS_BYTES);
+    static std::atomic<unsigned long long> raised{0};
+    return raise_lds_limit(raised, {(const void*)spconv_chwb_kernel<V, WN, NCONS, NPROD, KT, NSTAGE, Args>}, SpmmWsCfg<V, WN, NCONS, NPROD, KT, NSTAGE>::LDS_BYTES);
 }
 
 #define SHFLBW_CHWB(V, WN, NC, NP, KT, NS)                                                                             \
@@ -877,9 +876,8 @@ static hipError_t launch_xcd(const SpmmLaunchArgs& a, const ConvXcdArgs& c, hipS
 template <int V, int WN, int NCONS, int NPROD, int KT, int NSTAGE>
 static hipError_t prepare_xcd()
 {
-    using Cfg = SpmmWsCfg<V, WN, NCONS, NPROD, KT, NSTAGE>;
-    return hipFuncSetAttribute((const void*)spconv_xcd_kernel<V, WN, NCONS, NPROD, KT, NSTAGE>,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS_BYTES);
+    static std::atomic<unsigned long long> raised{0};
+    return raise_lds_limit(raised, {(const void*)spconv_xcd_kernel<V, WN, NCONS, NPROD, KT, NSTAGE>}, SpmmWsCfg<V, WN, NCONS, NPROD, KT, NSTAGE>::LDS_BYTES);
 }
 
 #define SHFLBW_XCD(V, WN, NC, NP, KT, NS)                                                                            \
@@ -924,9 +922,8 @@ static hipError_t launch_conv(const SpconvLaunchArgs& a, hipStream_t stream)
 template <int V, int WN, int NWAVES, int KT>
 static hipError_t prepare_conv()
 {
-    using Cfg = SpconvCfg<V, WN, NWAVES, KT>;
-    return hipFuncSetAttribute((const void*)spconv_shflbw_kernel<V, WN, NWAVES, KT>,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS_BYTES);
+    static std::atomic<unsigned long long> raised{0};
+    return raise_lds_limit(raised, {(const void*)spconv_shflbw_kernel<V, WN, NWAVES, KT>}, SpconvCfg<V, WN, NWAVES, KT>::LDS_BYTES);
 }
 
 #define SHFLBW_CONV_VARIANT(V, WN, NW, KT)                                                          \

@@ -319,23 +319,14 @@ static hipError_t launch_ws(const SpmmLaunchArgs& a, hipStream_t stream)
     return hipGetLastError();
 }
 
-// Both instances: the beta of a state is a plain field, and the launch goes by what it holds then.  Once per device, so that
-// an initialisation makes no call into the driver for a limit that is already raised.
+// Both instances: the beta of a state is a plain field, and the launch goes by what it holds then.
 template <int V, int WN, int NCONS, int NPROD, int KT, int NSTAGE>
 static hipError_t prepare_ws(const SpmmLaunchArgs&)
 {
-    using Cfg = SpmmWsCfg<V, WN, NCONS, NPROD, KT, NSTAGE>;
-    static std::atomic<unsigned long long> raised{0}; // one bit per device
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
-    const unsigned long long bit = dev < 64 ? 1ull << dev : 0;
-    if (raised.load(std::memory_order_acquire) & bit) return hipSuccess;
-    for (const void* f : {(const void*)spmm_shflbw_ws_kernel<V, WN, NCONS, NPROD, KT, NSTAGE, false>,
-                          (const void*)spmm_shflbw_ws_kernel<V, WN, NCONS, NPROD, KT, NSTAGE, true>})
-        if ((e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS_BYTES)) != hipSuccess) return e;
-    raised.fetch_or(bit, std::memory_order_release);
-    return hipSuccess;
+    static std::atomic<unsigned long long> raised{0};
+    return raise_lds_limit(raised, {(const void*)spmm_shflbw_ws_kernel<V, WN, NCONS, NPROD, KT, NSTAGE, false>,
+                                    (const void*)spmm_shflbw_ws_kernel<V, WN, NCONS, NPROD, KT, NSTAGE, true>},
+                           SpmmWsCfg<V, WN, NCONS, NPROD, KT, NSTAGE>::LDS_BYTES);
 }
 
 #define SHFLBW_WS_VARIANT(V, WN, NC, NP, KT, NS)                                                             \
@@ -410,11 +401,10 @@ static hipError_t launch_slab(const SpmmLaunchArgs& a, hipStream_t stream)
 template <int V>
 static hipError_t prepare_slab(const SpmmLaunchArgs&)
 {
-    for (const void* f : {(const void*)&spmm_shflbw_slab_kernel<V, STORE_THROUGH>, (const void*)&spmm_shflbw_slab_kernel<V, STORE_MERGE>,
-                          (const void*)&spmm_shflbw_slab_kernel<V, STORE_STREAM>})
-        if (hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, SpmmSlabCfg<V>::LDS_MAX); e != hipSuccess)
-            return e;
-    return hipSuccess;
+    static std::atomic<unsigned long long> raised{0};
+    return raise_lds_limit(raised, {(const void*)&spmm_shflbw_slab_kernel<V, STORE_THROUGH>, (const void*)&spmm_shflbw_slab_kernel<V, STORE_MERGE>,
+                                    (const void*)&spmm_shflbw_slab_kernel<V, STORE_STREAM>},
+                           SpmmSlabCfg<V>::LDS_MAX);
 }
 
 #define SHFLBW_SLAB_VARIANT(V)                                                                                    \
@@ -449,9 +439,8 @@ static hipError_t launch_variant(const SpmmLaunchArgs& a, hipStream_t stream)
 template <int V, int WN, int NWAVES, int KT, int NSTAGE>
 static hipError_t prepare_variant(const SpmmLaunchArgs&)
 {
-    using Cfg = SpmmCfg<V, WN, NWAVES, KT, NSTAGE>;
-    return hipFuncSetAttribute((const void*)spmm_shflbw_kernel<V, WN, NWAVES, KT, NSTAGE>,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS_BYTES);
+    static std::atomic<unsigned long long> raised{0};
+    return raise_lds_limit(raised, {(const void*)spmm_shflbw_kernel<V, WN, NWAVES, KT, NSTAGE>}, SpmmCfg<V, WN, NWAVES, KT, NSTAGE>::LDS_BYTES);
 }
 
 #define SHFLBW_VARIANT(V, WN, NW, KT, NS)                                                                   \

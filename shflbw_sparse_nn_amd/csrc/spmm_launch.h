@@ -1,6 +1,10 @@
 // Launch-side description of the native SpMM tile variants (host + device shared).
 #pragma once
 #include <hip/hip_runtime.h>
+
+#include <atomic>
+#include <initializer_list>
+
 #include "kernel_common.h"
 
 namespace shflbw {
@@ -45,6 +49,21 @@ struct ChwbTapArgs : SpmmLaunchArgs {
 constexpr int CHWB_MAX_TAPS = 31;  // a lane keeps one bit per tap; bit 31 is that of the padding slots, which no lane reads
 // units of 16 bytes from the lane's own position at tap (0, 0) of channel 0, and the tap
 constexpr int chwb_tap_id(unsigned units16, unsigned tap) { return (int)(units16 * 32u + tap); }
+
+// Raises the dynamic-LDS limit of kernels, once per device (`raised`: one bit each): an initialisation makes no call into the
+// driver for a limit that is already raised.
+inline hipError_t raise_lds_limit(std::atomic<unsigned long long>& raised, std::initializer_list<const void*> kernels, int bytes)
+{
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    const unsigned long long bit = dev < 64 ? 1ull << dev : 0;
+    if (raised.load(std::memory_order_acquire) & bit) return hipSuccess;
+    for (const void* f : kernels)
+        if ((e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes)) != hipSuccess) return e;
+    raised.fetch_or(bit, std::memory_order_release);
+    return hipSuccess;
+}
 
 struct SpmmVariant {
     int V;           // block size (rows per panel)

@@ -236,15 +236,20 @@ static hipError_t launch_split(const SpmmLaunchArgs& a, hipStream_t stream)
     return launch_split_n<V16, 1>(a, stream);
 }
 
+template <bool V16, int NBK>
+static hipError_t prepare_split_n()
+{
+    using Cfg = SpmmSplitCfg<V16, NBK>;
+    static std::atomic<unsigned long long> raised{0};
+    return raise_lds_limit(raised, {(const void*)spmm_shflbw_split_kernel<V16, NBK>}, Cfg::lds_bytes(Cfg::MAX_WAVES));
+}
+
 template <bool V16>
 static hipError_t prepare_split(const SpmmLaunchArgs& a)
 {
     if constexpr (!V16)
-        if (split_wide_tiles(a))
-            return hipFuncSetAttribute((const void*)spmm_shflbw_split_kernel<false, 2>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       SpmmSplitCfg<false, 2>::lds_bytes(SpmmSplitCfg<false, 2>::MAX_WAVES));
-    return hipFuncSetAttribute((const void*)spmm_shflbw_split_kernel<V16, 1>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               SpmmSplitCfg<V16, 1>::lds_bytes(SpmmSplitCfg<V16, 1>::MAX_WAVES));
+        if (split_wide_tiles(a)) return prepare_split_n<V16, 2>();
+    return prepare_split_n<V16, 1>();
 }
 
 } // namespace shflbw

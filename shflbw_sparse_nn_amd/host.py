@@ -189,18 +189,20 @@ class SpmmBlockwiseOp:
         self._lib = capi.load()
         self.variant = variant
         self._state = capi.SpmmState()
+        self._ref, self._init, self._exec = C.byref(self._state), self._lib.shflbw_spmm_init_variant, self._lib.shflbw_spmm_exec
 
     def initialize(self, spmat, N, B, D, Cmat=None, alpha=1.0, beta=None):
         # the 4-argument form is alpha=1, beta=0; with C it is alpha=beta=1 (blockwise_op.h:143-159)
         if beta is None:
             beta = 0.0 if Cmat is None else 1.0
-        capi.check(self._lib.shflbw_spmm_init_variant(C.byref(self._state), spmat._h, N, B, Cmat, D, alpha, beta,
-                                                      self.variant))
+        if rc := self._init(self._ref, spmat._h, N, B, Cmat, D, alpha, beta, self.variant):
+            capi.check(rc)
         self._keep = spmat
         return self._state
 
     def __call__(self, stream=None):
-        capi.check(self._lib.shflbw_spmm_exec(C.byref(self._state), stream))
+        if rc := self._exec(self._ref, stream):
+            capi.check(rc)
 
 
 class SpconvBlockwiseOp:
@@ -211,14 +213,15 @@ class SpconvBlockwiseOp:
         self._lib = capi.load()
         self._state = capi.SpconvState()
         self._variant = variant
+        self._ref, self._exec = C.byref(self._state), self._lib.shflbw_spconv_exec
 
     def initialize(self, spfilter, B, H, W, stride, IFMap, OFMap, batch_innermost=False):
         """batch_innermost=True: the reference's C-H-W-B / F-H-W-B tensors and its bounds rule (H, W bound input and
         output alike); the form is then fixed."""
         if batch_innermost:
-            capi.check(self._lib.shflbw_spconv_init_chwb(C.byref(self._state), spfilter._h, B, H, W, stride, IFMap, OFMap))
+            capi.check(self._lib.shflbw_spconv_init_chwb(self._ref, spfilter._h, B, H, W, stride, IFMap, OFMap))
         else:
-            capi.check(self._lib.shflbw_spconv_init_variant(C.byref(self._state), spfilter._h, B, H, W, stride, IFMap,
+            capi.check(self._lib.shflbw_spconv_init_variant(self._ref, spfilter._h, B, H, W, stride, IFMap,
                                                             OFMap, self._variant))
         self._keep = spfilter
         return self._state
@@ -228,7 +231,8 @@ class SpconvBlockwiseOp:
         return self._state.Ho, self._state.Wo
 
     def __call__(self, stream=None):
-        capi.check(self._lib.shflbw_spconv_exec(C.byref(self._state), stream))
+        if rc := self._exec(self._ref, stream):
+            capi.check(rc)
 
     def check(self):
         """Waits for the device and raises if a launch of the fused form on this state did not run to completion."""
