@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -152,105 +153,111 @@ static bool spmm_variant_splits(const SpmmVariant* v) { return v && strncmp(v->n
 // few columns and holds to the same bound
 static bool spmm_variant_offsets32(const SpmmVariant* v) { return v && (v->name[0] == 'w' || spmm_variant_splits(v)); }
 
-// Tile choice when the caller does not force one: the table lists the preferred (persistent, 512 columns
-// wide) variant of every block size first.  When its tiles would occupy at most half of the compute units,
-// the role-split variant with 256-column tiles is taken instead (twice the tiles; measured 15-25 % faster
-// there, 5-20 % slower once the wide tiles fill the chip), and the one with 128-column tiles while even those
-// are no more than the compute units.
-// Block height 32 and at most SLAB_MAX_K columns: the slab variant moves less data between the L2 and the
-// compute units once a workgroup runs enough kept vectors over the 128 KiB slab it has to load first.  Taken
-// when (34 shapes measured with both kernels, each pair on one box)
-//  * a workgroup's panels keep at least 3 vectors per column of A on average (3.2: 5 % faster, 2.4: 5-20 %
-//    slower, 1.6: equal to 30 % slower: the slab load is not paid back),
-//  * A has at least 384 columns (at 256 B fits the L2, the gathers of the role-split kernel all hit, and the
-//    two kernels tie),
-//  * there are at least 32 column tiles, so that four or more workgroups of an XCD stream the same chunk of A
-//    at the same time and share it in their L2 (16 tiles: 15 % slower).
-// Inside these bounds: equal to 28 % faster (M = 4096, K = 1024, N = 4096, density 0.2: 15.1 against 16.5 us;
-// M = 8192, density 0.3: 31.3 against 38.7 us).
-// Block height 16 has no narrower tiles than 512 columns beside it and gathers twice as much per product: there the slab
-// variant is taken from 128 columns on (below, the split form) when (192 shapes)
-//  * a workgroup runs at least 24 panels (32 to 132: 1.0-1.9 times as fast) with at least one kept vector per column of A, or 16 panels
-//    with 2.5 (18 panels: 0.9 at 0.6 vectors, 1.2 at 5.5; 6 to 9 panels: 0.6-1.1), four where a fifth of the compute units would have
-//    no job (3.2: 8 % slower, 6.4: 5 % faster),
-//  * panels keep at least 32 vectors, or D is below 100 MB: with less to do per panel both wait for the stores of D, and the
-//    wider row segments of the role-split kernel are 5-15 % ahead (33728 x 96 x 2048: 38 against 46 us) where rows of D start at
-//    whole lines (15760 x 127 x 3864: 41 against 31 us).
-// On one box, density 0.1: 33728 x 777 x 1000 29.6 against 32.8 us; 8192 x 384 x 4096 17.3 against 28.7; 8192 x 777 x 3000 19.0 against
-// 24.9; density 0.2: 33728 x 1128 x 136 16.7 against 29.8.  On 64 sampled shapes it is taken for 30, 1.07 to 1.90 times as fast there.
-static int auto_gather_variant(const shflbw_weight* w, int N, bool allow_slab, int compute_units)
+// Tile choice when the caller does not force one: the variant with the least estimated time.  The weights are us, a fit per variant
+// (7-12 % rms) to 940 problems drawn over 512-33792 rows, 64-8192 columns of A, 8-16384 columns of B and densities of 0.02-0.5,
+// every variant of their block height timed over three sets of operands in turn.  Over those the estimate's choice takes 1.01
+// (block height 16), 1.02 (32, 64) and 1.01 times (128) the fastest variant's time on average.  The lines drawn by hand
+// before it - 128-column tiles while they do not outnumber the compute units, 256-column ones while the widest would fill at most
+// half of them, bounds for the slab and the split form - took 1.15, 1.10, 1.07 and 1.02 times, 3.3 at worst: above all many
+// panels over few columns ran on 512-column tiles (29632 x 761 x 64, density 0.47, block height 64: 16.1 us; 128-column tiles, two
+// workgroups per compute unit, 7.0), and block height 16 had no other width (6592 x 4295 x 544, density 0.03: 14.4; 256 columns 9.7).
+//
+//  role-split: base + tiles of a compute unit * (tile + stage * stages of 32 kept vectors) + d * (D at 5 TB/s); the tiles of a compute
+//    unit are `whole` parts the rounded-up number and the rest the mean, and where two workgroups share it a pair of tiles
+//    takes as long as one and (tile2 + stage2 * stages);
+//  slab: base + rounds * (slab + K / 1000 * row + panels of a wave * batches of 32 vectors * batch) + d * ...;
+//  split: base + rounds * (tile + (64 columns: wide) + steps of a wave * (step + (64 columns: wide_step))) + d * ...
+struct SpmmEstimate {
+    const char* name;
+    float base, tile, stage, whole, d, tile2, stage2;
+};
+static const SpmmEstimate g_estimates[] = {
+    {"ws16x128x4c4p_k32_s4", 2.97f, 0.708f, 0.271f, 1.f, 0.436f, 0.f, 0.f},
+    {"ws16x64x2c4p_k32_s6", 3.01f, 0.826f, 0.132f, 0.272f, 0.035f, 0.f, 0.082f},
+    {"ws16x64x4c4p_k32_s4", 3.03f, 0.735f, 0.152f, 0.153f, 0.249f, 0.f, 0.175f},
+    {"ws32x128x4c4p_k32_s4", 2.54f, 1.05f, 0.293f, 1.f, 0.605f, 0.f, 0.f},
+    {"ws32x32x4c4p_k32_s6", 3.0f, 0.787f, 0.123f, 0.109f, 0.406f, 0.f, 0.139f},
+    {"ws32x64x4c4p_k32_s3", 2.89f, 0.679f, 0.238f, 0.416f, 0.478f, 0.f, 0.264f},
+    {"ws32x64x4c4p_k32_s6", 2.81f, 0.763f, 0.185f, 0.809f, 0.565f, 0.f, 0.f},
+    {"ws64x128x4c4p_k32_s4", 2.28f, 1.8f, 0.349f, 1.f, 0.675f, 0.f, 0.f},
+    {"ws64x32x4c4p_k32_s4", 2.56f, 1.2f, 0.155f, 0.356f, 0.387f, 0.f, 0.246f},
+    {"ws64x32x4c4p_k32_s6", 3.24f, 0.348f, 0.171f, 1.f, 0.988f, 0.f, 0.f},
+    {"ws64x64x4c4p_k32_s3", 2.0f, 1.55f, 0.379f, 0.532f, 0.519f, 0.015f, 0.253f},
+    {"ws64x64x4c4p_k32_s6", 2.75f, 0.966f, 0.218f, 1.f, 0.652f, 0.f, 0.f},
+    {"ws128x32x4c4p_k32_s4", 2.62f, 1.05f, 0.206f, 0.658f, 0.703f, 0.33f, 0.382f},
+    {"ws128x32x4c4p_k32_s6", 2.51f, 1.19f, 0.2f, 1.f, 0.662f, 0.f, 0.f},
+    {"ws128x64x4c4p_k32_s6", 2.0f, 2.24f, 0.31f, 1.f, 0.512f, 0.f, 0.f},
+    // base, slab, row, -, batch, d
+    {"slab16x64", 2.63f, 0.991f, 0.667f, 0.f, 0.173f, 0.727f, 0.f},
+    {"slab32x64", 2.0f, 1.7f, 0.795f, 0.f, 0.175f, 0.944f, 0.f},
+    // base, tile, step, wide_step, wide, d
+    {"split16x32", 2.4f, 1.15f, 0.853f, 0.f, 0.f, 0.f, 0.f},
+    {"split32x32", 2.45f, 1.24f, 0.607f, 0.21f, 0.f, 1.19f, 0.f},
+    {"split64x32", 2.49f, 1.21f, 0.57f, 0.262f, 0.f, 1.27f, 0.f},
+    {"split128x32", 2.32f, 1.32f, 0.666f, 0.239f, 0.f, 0.944f, 0.f},
+};
+
+static double spmm_estimate(const SpmmVariant& v, const SpmmEstimate& e, bool splits, const shflbw_weight* w, int N, int compute_units)
 {
-    const int brow = w->brow, X = w->nrow / w->brow;
-    int count = 0;
-    const SpmmVariant* all = find_spmm_variant(brow, 0, &count);
-    if (allow_slab && !w->packed_slab.empty() && X > 0 && (brow == 16 ? N >= 128 : w->ncol >= 384)) {
-        for (int i = 0; i < count; i++) {
-            if (all[i].max_k >= w->ncol) {
-                const int cus = (compute_units / 8) * 8;
-                const int n_tiles = (N + all[i].BN - 1) / all[i].BN;
-                const int chunks = std::max(1, std::min(X, cus / n_tiles)); // as the launcher deals the panels
-                const double panels_per_wg = (double)X / chunks;
-                const double vectors_per_column = panels_per_wg * w->nnzb / ((double)X * w->ncol);
-                const double vectors = (double)w->nnzb / X;
-                if (brow == 16 ? panels_per_wg >= 16 && vectors_per_column >= (n_tiles * chunks < 0.8 * cus ? 4.0 : panels_per_wg < 24 ? 2.5 : 1.0) &&
-                                     (vectors >= 32 || 2.0 * w->nrow * N <= 100e6 || N % 64 != 0)
-                               : vectors_per_column >= 3.0 && n_tiles >= 32)
-                    return i;
-            }
-        }
+    const double X = w->nrow / w->brow, vectors = w->nnzb / X, t_d = 2.0 * w->nrow * N / 5e6;
+    const double cus = compute_units;
+    if (v.max_k > 0) {
+        const int groups = (int)(w->packed_indices.size() / 64);
+        const SlabDeal s = slab_deal(w->brow, (int)X, w->ncol, groups, (N + v.BN - 1) / v.BN, compute_units / 8 * 8);
+        return e.base + s.rounds * (e.tile + e.stage * w->ncol / 1000 + s.wave_panels * e.d * 2 * std::ceil(vectors / 64)) + e.tile2 * t_d;
     }
-    // the role-split variant of this block size with tiles of `bn` columns, -1 when there is none
-    auto role_split_with = [&](int bn) {
-        for (int i = 0; i < count; i++)
-            if (all[i].name[0] == 'w' && all[i].BN == bn) return i; // "ws..." names
-        return -1;
-    };
-    // small problems: 128-column tiles while they do not outnumber the compute units (39 shapes of block heights 32, 64
-    // and 128 measured against the wider tiles: 6-17 % faster up to one tile per compute unit, 10-25 % slower from two on)
-    if ((long)X * ((N + 127) / 128) <= compute_units) {
-        const int narrow = role_split_with(128);
-        if (narrow >= 0) return narrow;
+    if (splits) { // as launch_split cuts it
+        const bool v16 = w->brow == 16;
+        const double blocks = w->nrow / (v16 ? 16 : 32);
+        const bool wide = !v16 && N > 32 && blocks * ((N + 31) / 32) > cus;
+        const double grid = std::ceil(blocks / 8) * 8 * (wide ? (N + 63) / 64 : (N + 31) / 32), waves = grid <= cus ? 16 : 8;
+        const double steps = vectors / (v16 ? 32 : 16) / waves + 0.5;
+        return e.base + std::max(1.0, grid / (waves == 16 ? cus : 2 * cus)) * (e.tile + (e.stage + (wide ? e.whole : 0.f)) * steps) + e.tile2 * t_d;
     }
-    const SpmmVariant* first = find_spmm_variant(brow, 0, nullptr);
-    if (!first || first->BN != 512) return 0;
-    const long wide_tiles = (long)X * ((N + 511) / 512);
-    if (wide_tiles > compute_units / 2) return 0;
-    const int medium = role_split_with(256);
-    return medium >= 0 ? medium : 0;
+    const double per_cu = X * ((N + v.BN - 1) / v.BN) / cus, n = std::ceil(per_cu), mean = std::max(1.0, per_cu);
+    const double one = e.tile + e.stage * (vectors / 32 + 0.5);
+    double whole = n * one, rest = mean * one;
+    if (v.per_cu == 2) {
+        const double pair = one + e.tile2 + e.stage2 * (vectors / 32 + 0.5), pairs = std::floor(n / 2);
+        whole = pairs * pair + (n - 2 * pairs) * one;
+        rest = mean <= 2 ? one + (mean - 1) * (pair - one) : mean / 2 * pair;
+    }
+    return e.base + e.whole * whole + (1 - e.whole) * rest + e.d * t_d;
 }
 
-// Few columns: the split form (its waves split the kept vectors) where it is estimated to be at least a tenth faster than the
-// variant above.  Both estimates are us, fitted to 4 block heights x 7 weights x 6 widths from 8 to 512 columns:
-//  split: 4 + rounds * (0.6 + 0.03 * steps) with 32-column tiles (0.04 for block height 16), (0.9 + 0.052 * steps) with 64;
-//    rounds = workgroups per compute unit, steps of 16 kept vectors (32 for block height 16);
-//  above: 3.6 + rounds * (0.3 + 0.2 * stages) with 128-column tiles, (1.35 + 0.22 * stages) with wider ones for block height 32,
-//    1.7 from 64, (0.85 + 0.27 * stages) for 16; stages of 32 kept vectors.
-// 2048 x 8192, density 0.5, 8 columns: 8.1-10 us split, 30-37 us above; 8192 x 4096, density 0.3: 6.8 and 11.6-26; 4096 x 4096,
-// density 0.1: 5.1-5.4 and 6.2-7.4, with 256 columns 7.0 and 6.4; 16384 x 1024, density 0.1, block height 64, 64 columns: 5.7 and 4.7.
+// `spmm` false: what is multiplied are the planes of a convolution, which only the variants that gather rows by id can walk.
 static int auto_spmm_variant(const shflbw_weight* w, int N, bool spmm, int compute_units)
 {
-    const int general = auto_gather_variant(w, N, spmm, compute_units);
-    const int X = w->nrow / w->brow;
-    if (!spmm || N > 512 || X <= 0) return general;
-    int split = 0; // the split form is the last variant of its block height
-    find_spmm_variant(w->brow, 0, &split);
-    split--;
-    const SpmmVariant* g = find_spmm_variant(w->brow, general, nullptr);
-    if (!g || g->max_k > 0 || !spmm_variant_splits(find_spmm_variant(w->brow, split, nullptr))) return general;
-    const double cus = compute_units, vectors = (double)w->nnzb / X;
-    const bool v16 = w->brow == 16;
-    auto rounds = [cus](double workgroups) {
-        const double r = workgroups / cus;
-        return r <= 1 ? 1 : r <= 2 ? 2 : r;
+    struct Candidates { // of the four block heights, found once
+        struct One {
+            const SpmmVariant* v;
+            const SpmmEstimate* e;
+            int number;
+            bool splits;
+        };
+        std::vector<One> of[4];
+        Candidates()
+        {
+            for (int h = 0; h < 4; h++) {
+                int count = 0;
+                const SpmmVariant* all = find_spmm_variant(16 << h, 0, &count);
+                for (int i = 0; i < count; i++)
+                    for (const SpmmEstimate& e : g_estimates)
+                        if (strcmp(e.name, all[i].name) == 0) of[h].push_back({&all[i], &e, i, spmm_variant_splits(&all[i])});
+            }
+        }
     };
-    const double edge = g->BN <= 128 ? 0.3 : v16 ? 0.85 : w->brow == 32 ? 1.35 : 1.7;
-    const double stage = g->BN <= 128 ? 0.2 : v16 ? 0.27 : 0.22;
-    const double t_general = 3.6 + rounds(X * (double)((N + g->BN - 1) / g->BN)) * (edge + stage * vectors / 32);
-    const double blocks = w->nrow / (v16 ? 16.0 : 32.0), narrow = blocks * ((N + 31) / 32);
-    const double steps = vectors / (v16 ? 32 : 16);
-    const double t_split = v16 || N <= 32 || narrow <= cus ? 4 + rounds(narrow) * (0.6 + (v16 ? 0.04 : 0.03) * steps)
-                                                           : 4 + rounds(blocks * ((N + 63) / 64)) * (0.9 + 0.052 * steps);
-    return t_split < 0.9 * t_general ? split : general;
+    static const Candidates candidates;
+    const int h = w->brow == 16 ? 0 : w->brow == 32 ? 1 : w->brow == 64 ? 2 : w->brow == 128 ? 3 : -1;
+    if (h < 0 || w->nrow <= 0) return 0;
+    int best = 0;
+    double least = 0;
+    for (const auto& c : candidates.of[h]) {
+        if (c.v->max_k > 0 ? !spmm || w->packed_slab.empty() || w->ncol > c.v->max_k : c.splits && (!spmm || N > 1024)) continue;
+        const double t = spmm_estimate(*c.v, *c.e, c.splits, w, N, compute_units);
+        if (least == 0 || t < least) least = t, best = c.number;
+    }
+    return best;
 }
 
 // Geometry of the plane form of a convolution and the layout of its device scratch.

@@ -333,7 +333,7 @@ static hipError_t prepare_ws(const SpmmLaunchArgs&)
     {                                                                                                        \
         V, WN* NC, (NC + NP) * 64, SpmmWsCfg<V, WN, NC, NP, KT, NS>::LDS_BYTES,                               \
             "ws" #V "x" #WN "x" #NC "c" #NP "p_k" #KT "_s" #NS, &launch_ws<V, WN, NC, NP, KT, NS>,           \
-            &prepare_ws<V, WN, NC, NP, KT, NS>                                                                \
+            &prepare_ws<V, WN, NC, NP, KT, NS>, 0, SpmmWsCfg<V, WN, NC, NP, KT, NS>::WGS_PER_CU                 \
     }
 
 // ---------------------------------------------------------------------------------------
@@ -352,21 +352,7 @@ static void slab_plan(SpmmLaunchArgs& b, int cus)
     // 1000 (67 MB) 22.7 / 24.1 / 45, block height 32, 16384 x 800 x 2056 (67 MB) 42 / 35.5 / 49, 33728 x 1100 x 2104 136 / 123 / 121, 16:
     // 20000 x 1000 x 6000 145 / 101 / 125.
     b.store_mode = lines ? (d_bytes >= 96u << 20 ? STORE_STREAM : STORE_THROUGH) : d_bytes >= 64u << 20 ? STORE_MERGE : STORE_THROUGH;
-    // Chunks: at least as many as keep the panels of one wave within RID_REGS * 64 rows; then the number that takes the least
-    // rounds * (slab + panels of a wave), of the most that one, two and three rounds of the compute units have room for (us, from
-    // the phases of a wave).  33728 x 1100 x 2112, block height 32: 33 tiles x 9 chunks were two rounds, the second nearly empty, 91 us;
-    // 15 chunks 66.
-    const int rows_per_wg = Cfg::NW * Cfg::RID_REGS * 64, least = (b.M + rows_per_wg - 1) / rows_per_wg;
-    const double batches = 2.0 * b.groups / b.X; // of 32 slots, per panel
-    const double t_slab = 1.0 + 1.5e-3 * b.K, t_panel = V == 16 ? 0.30 + 0.12 * batches : 0.45 + 0.21 * batches;
-    double best = 0;
-    for (int r = 1; r <= 3; r++) {
-        const int c = std::max(1, std::min(b.X, std::max(least, cus * r / b.n_tiles)));
-        const int rounds = ((b.n_tiles * c + 7) / 8 * 8 + cus - 1) / cus;
-        const int wave_panels = ((b.X + c - 1) / c + Cfg::NW - 1) / Cfg::NW;
-        const double t = rounds * (t_slab + wave_panels * t_panel);
-        if (r == 1 || t < best * 0.95) best = t, b.slab_chunks = c;
-    }
+    b.slab_chunks = slab_deal(V, b.X, b.K, b.groups, b.n_tiles, cus).chunks;
     // Order of the jobs.  An XCD owns T / 8 of them, side by side: by tile it reads few slabs and most of A, by chunk a part of A
     // and most of B.  The order with fewer bytes into the L2s; by chunk where parts of lines are merged, as the tiles that
     // share lines then lie on one XCD.  us, by tile / by chunk, block height 16: 33728 x 777 x 1024 (A 9 MB, B 1.6) 26.4 / 22.1, x 1000 29.6 /
@@ -450,7 +436,7 @@ static hipError_t prepare_variant(const SpmmLaunchArgs&)
     }
 
 static const SpmmVariant g_variants[] = {
-    // block 64 (the first entry of a block size is the library's choice; measured order)
+    // block 64 (which one the library takes: auto_spmm_variant)
     SHFLBW_WS_VARIANT(64, 128, 4, 4, 32, 4),
     SHFLBW_WS_VARIANT(64, 128, 4, 4, 16, 5),
     SHFLBW_WS_VARIANT(64, 64, 4, 4, 32, 6),
@@ -468,6 +454,7 @@ static const SpmmVariant g_variants[] = {
     SHFLBW_VARIANT(64, 32, 4, 32, 3),
     SHFLBW_WS_VARIANT(64, 32, 4, 4, 32, 6), // 128-column tiles: problems too small for the wider ones
     SHFLBW_SPLIT_VARIANT(64), // few columns
+    SHFLBW_WS_VARIANT(64, 32, 4, 4, 32, 4), // 128-column tiles, two workgroups per compute unit
     // block 32
     SHFLBW_WS_VARIANT(32, 128, 4, 4, 32, 4),
     SHFLBW_WS_VARIANT(32, 128, 4, 4, 16, 6),
@@ -484,6 +471,8 @@ static const SpmmVariant g_variants[] = {
     SHFLBW_WS_VARIANT(16, 128, 4, 4, 32, 4),
     SHFLBW_SLAB_VARIANT(16), // weights of at most SLAB_MAX_K columns
     SHFLBW_SPLIT_VARIANT(16), // few columns
+    SHFLBW_WS_VARIANT(16, 64, 2, 4, 32, 6), // 128-column tiles, two workgroups per compute unit
+    SHFLBW_WS_VARIANT(16, 64, 4, 4, 32, 4), // two workgroups per compute unit
     // block 128
     SHFLBW_WS_VARIANT(128, 64, 4, 4, 32, 6),
     SHFLBW_WS_VARIANT(128, 64, 4, 4, 32, 5),
@@ -491,6 +480,7 @@ static const SpmmVariant g_variants[] = {
     SHFLBW_VARIANT(128, 32, 4, 32, 3),
     SHFLBW_WS_VARIANT(128, 32, 4, 4, 32, 6), // 128-column tiles: problems too small for the wider ones
     SHFLBW_SPLIT_VARIANT(128), // few columns
+    SHFLBW_WS_VARIANT(128, 32, 4, 4, 32, 4), // 128-column tiles, two workgroups per compute unit
 };
 
 // The row of zeros the padding slots gather.  `g_zero_row` is the host-side handle of the symbol; kernels get

@@ -74,9 +74,38 @@ struct SpmmVariant {
     hipError_t (*launch)(const SpmmLaunchArgs&, hipStream_t);
     hipError_t (*prepare)(const SpmmLaunchArgs&); // raises the dynamic-LDS limit of the kernels that `launch` may take (M, N, X are set)
     int max_k;               // 0, or the most columns of A the variant takes (it holds all rows of B in LDS)
+    int per_cu;              // role-split variants: workgroups a compute unit holds at once
 };
 
 const SpmmVariant* spmm_variants(int* count);
+
+// How the slab kernel deals X panels (groups of 64 slots in all) under n_tiles column tiles to workgroups: at least as many chunks
+// as keep the panels of one wave within the rows it has registers for; then the number that takes the least rounds * (slab + panels
+// of a wave), of the most that one, two and three rounds of the compute units have room for (us, from the phases of a wave).
+// 33728 x 1100 x 2112, block height 32: 33 tiles x 9 chunks were two rounds, the second nearly empty, 91 us; 15 chunks 66.
+constexpr int SLAB_WAVES = 8;          // of a workgroup
+constexpr int SLAB_WAVE_ROWS = 8 * 64; // rows of D a wave holds the places of
+struct SlabDeal {
+    int chunks, rounds, wave_panels;
+};
+inline SlabDeal slab_deal(int V, int X, int K, int groups, int n_tiles, int cus)
+{
+    const int least = (X * V + SLAB_WAVES * SLAB_WAVE_ROWS - 1) / (SLAB_WAVES * SLAB_WAVE_ROWS);
+    const double batches = 2.0 * groups / X; // of 32 slots, per panel
+    const double t_slab = 1.0 + 1.5e-3 * K, t_panel = V == 16 ? 0.30 + 0.12 * batches : 0.45 + 0.21 * batches;
+    SlabDeal best{};
+    double best_t = 0;
+    for (int r = 1; r <= 3; r++) {
+        const int most = cus * r / n_tiles, at_least = most > least ? most : least;
+        SlabDeal d;
+        d.chunks = at_least < 1 ? 1 : at_least > X ? X : at_least;
+        d.rounds = (int)(((long)n_tiles * d.chunks + 7) / 8 * 8 + cus - 1) / cus;
+        d.wave_panels = ((X + d.chunks - 1) / d.chunks + SLAB_WAVES - 1) / SLAB_WAVES;
+        const double t = d.rounds * (t_slab + d.wave_panels * t_panel);
+        if (r == 1 || t < best_t * 0.95) best_t = t, best = d;
+    }
+    return best;
+}
 
 // device address of the library's row of zeros on the current device (looked up once per device); null on failure
 const void* spmm_zero_row();

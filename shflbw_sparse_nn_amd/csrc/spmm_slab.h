@@ -31,13 +31,13 @@ struct SpmmSlabCfg {
     static constexpr int NA = V16 ? 1 : 2;   // A fragments, and MFMA steps, per batch of 32 slots
     static constexpr int BN = 64;            // columns of the slab
     static constexpr int ROWB = BN * 2;      // bytes of a slab row
-    static constexpr int NW = 8;             // waves of a workgroup
+    static constexpr int NW = SLAB_WAVES;    // waves of a workgroup
     static constexpr int THREADS = NW * 64;
     static constexpr int NB = V16 ? BN / 16 : BN / 32; // accumulator blocks
     static constexpr int NBUF = 8;           // batches a wave keeps in flight (even: the fragment sets alternate)
     static constexpr int FETCH_OPS = NA + 1; // loads per batch: A fragments and the offsets of a lane's slots
     static constexpr int PANEL_PASSES = V / 16;           // 16 rows of a panel's result are staged at a time
-    static constexpr int RID_REGS = 8;       // a wave's panels have at most RID_REGS * 64 rows
+    static constexpr int RID_REGS = SLAB_WAVE_ROWS / 64; // a wave's panels have at most RID_REGS * 64 rows
     static constexpr int EPI_ROWB = BN * 2 + 16;          // a staged row: all 64 columns and 16 bytes of padding
     static constexpr int EPI_WAVE_BYTES = 16 * EPI_ROWB;  // 16 rows at a time
     static constexpr int LDS_MAX = 160 * 1024;

@@ -179,7 +179,7 @@ __device__ __forceinline__ void ws_consumer(const SpmmLaunchArgs& a, uint32_t ld
     // L2s as with 64-byte row segments (4096 x 4096 x 4096, density 0.1: -2 %, -11 % at N = 16384, where every epilogue
     // runs beside other workgroups' gathers).  Not where two workgroups share a compute unit (128 registers per wave: it
     // spills).
-    constexpr bool LINES = SHFLBW_EPI_LINES && NB % 2 == 0 && 16 * (128 + 16) <= Cfg::EPI_WAVE_BYTES && Cfg::WGS_PER_CU == 1;
+    constexpr bool LINES = SHFLBW_EPI_LINES && NB % 2 == 0 && 16 * (128 + 16) <= Cfg::EPI_WAVE_BYTES;
     constexpr int CIT = LINES ? 2 : NIT;                            // pieces of C per epilogue step
     constexpr int STEPS = LINES ? MB * NB : MB * NB * (32 / ER);    // epilogue steps of a tile
     // ... whose pieces are in flight (beside 128 accumulators all eight would spill; waves with 128 registers have no room)
@@ -188,7 +188,8 @@ __device__ __forceinline__ void ws_consumer(const SpmmLaunchArgs& a, uint32_t ld
 
     // (XCD_LOCAL: other workgroups of the XCD read the result back from the L2)
     auto store = [&](half_t* p, half8_t v, auto mode) __attribute__((always_inline)) {
-        store_result_16B<XCD_LOCAL ? STORE_MERGE : decltype(mode)::value>(p, v);
+        constexpr StoreMode M = decltype(mode)::value;
+        store_result_16B<XCD_LOCAL || (M == STORE_STREAM && !LINES) ? STORE_MERGE : M>(p, v);
     };
 
     struct Frags {
