@@ -154,9 +154,9 @@ static bool spmm_variant_splits(const SpmmVariant* v) { return v && strncmp(v->n
 static bool spmm_variant_offsets32(const SpmmVariant* v) { return v && (v->name[0] == 'w' || spmm_variant_splits(v)); }
 
 // Tile choice when the caller does not force one: the variant with the least estimated time.  The weights are us, a fit per variant
-// (7-12 % rms) to 940 problems drawn over 512-33792 rows, 64-8192 columns of A, 8-16384 columns of B and densities of 0.02-0.5,
-// every variant of their block height timed over three sets of operands in turn.  Over those the estimate's choice takes 1.01
-// (block height 16), 1.02 (32, 64) and 1.01 times (128) the fastest variant's time on average.  The lines drawn by hand
+// (7-15 % rms) to 1390 problems drawn over 512-33792 rows, 64-8192 columns of A, 8-16384 columns of B and densities of 0.02-0.5,
+// every variant of their block height timed over three sets of operands in turn.  Over those the estimate's choice takes 1.01 (block
+// heights 16 and 128) and 1.02 times (32, 64) the fastest variant's time on average.  The lines drawn by hand
 // before it - 128-column tiles while they do not outnumber the compute units, 256-column ones while the widest would fill at most
 // half of them, bounds for the slab and the split form - took 1.15, 1.10, 1.07 and 1.02 times, 3.3 at worst: above all many
 // panels over few columns ran on 512-column tiles (29632 x 761 x 64, density 0.47, block height 64: 16.1 us; 128-column tiles, two
@@ -166,35 +166,39 @@ static bool spmm_variant_offsets32(const SpmmVariant* v) { return v && (v->name[
 //    unit are `whole` parts the rounded-up number and the rest the mean, and where two workgroups share it a pair of tiles
 //    takes as long as one and (tile2 + stage2 * stages);
 //  slab: base + rounds * (slab + K / 1000 * row + panels of a wave * batches of 32 vectors * batch) + d * ...;
-//  split: base + rounds * (tile + (64 columns: wide) + steps of a wave * (step + (64 columns: wide_step))) + d * ...
+//  split: base + rounds * (tile + steps of a wave * (step + (64 columns: wide_step))) + d * ...
 struct SpmmEstimate {
     const char* name;
+    int tiles; // 0; 1: only while its tiles do not outnumber the compute units; 2: only where they do
     float base, tile, stage, whole, d, tile2, stage2;
 };
 static const SpmmEstimate g_estimates[] = {
-    {"ws16x128x4c4p_k32_s4", 2.97f, 0.708f, 0.271f, 1.f, 0.436f, 0.f, 0.f},
-    {"ws16x64x2c4p_k32_s6", 3.01f, 0.826f, 0.132f, 0.272f, 0.035f, 0.f, 0.082f},
-    {"ws16x64x4c4p_k32_s4", 3.03f, 0.735f, 0.152f, 0.153f, 0.249f, 0.f, 0.175f},
-    {"ws32x128x4c4p_k32_s4", 2.54f, 1.05f, 0.293f, 1.f, 0.605f, 0.f, 0.f},
-    {"ws32x32x4c4p_k32_s6", 3.0f, 0.787f, 0.123f, 0.109f, 0.406f, 0.f, 0.139f},
-    {"ws32x64x4c4p_k32_s3", 2.89f, 0.679f, 0.238f, 0.416f, 0.478f, 0.f, 0.264f},
-    {"ws32x64x4c4p_k32_s6", 2.81f, 0.763f, 0.185f, 0.809f, 0.565f, 0.f, 0.f},
-    {"ws64x128x4c4p_k32_s4", 2.28f, 1.8f, 0.349f, 1.f, 0.675f, 0.f, 0.f},
-    {"ws64x32x4c4p_k32_s4", 2.56f, 1.2f, 0.155f, 0.356f, 0.387f, 0.f, 0.246f},
-    {"ws64x32x4c4p_k32_s6", 3.24f, 0.348f, 0.171f, 1.f, 0.988f, 0.f, 0.f},
-    {"ws64x64x4c4p_k32_s3", 2.0f, 1.55f, 0.379f, 0.532f, 0.519f, 0.015f, 0.253f},
-    {"ws64x64x4c4p_k32_s6", 2.75f, 0.966f, 0.218f, 1.f, 0.652f, 0.f, 0.f},
-    {"ws128x32x4c4p_k32_s4", 2.62f, 1.05f, 0.206f, 0.658f, 0.703f, 0.33f, 0.382f},
-    {"ws128x32x4c4p_k32_s6", 2.51f, 1.19f, 0.2f, 1.f, 0.662f, 0.f, 0.f},
-    {"ws128x64x4c4p_k32_s6", 2.0f, 2.24f, 0.31f, 1.f, 0.512f, 0.f, 0.f},
+    // The rings of three and four stages that let two workgroups share a compute unit are too short for one alone (128 columns
+    // 1.00-1.15 times, 256 columns up to 1.9 times the six stages' time, the more the longer the panels), and with more tiles than
+    // compute units the 128-column ones were ahead throughout (0.78-0.98 times).
+    {"ws16x128x4c4p_k32_s4", 0, 2.99f, 0.688f, 0.273f, 1.f, 0.442f, 0.f, 0.f},
+    {"ws16x64x2c4p_k32_s6", 0, 2.98f, 0.851f, 0.13f, 0.277f, 0.f, 0.f, 0.083f},
+    {"ws16x64x4c4p_k32_s4", 0, 3.06f, 0.7f, 0.158f, 0.149f, 0.329f, 0.f, 0.171f},
+    {"ws32x128x4c4p_k32_s4", 0, 2.56f, 1.05f, 0.295f, 1.f, 0.584f, 0.f, 0.f},
+    {"ws32x32x4c4p_k32_s6", 0, 2.94f, 0.873f, 0.124f, 0.137f, 0.318f, 0.f, 0.137f},
+    {"ws32x64x4c4p_k32_s3", 2, 2.49f, 0.f, 0.399f, 0.876f, 0.399f, 1.02f, 0.054f},
+    {"ws32x64x4c4p_k32_s6", 0, 2.86f, 0.756f, 0.188f, 0.773f, 0.531f, 0.f, 0.f},
+    {"ws64x128x4c4p_k32_s4", 0, 2.15f, 1.93f, 0.355f, 1.f, 0.653f, 0.f, 0.f},
+    {"ws64x32x4c4p_k32_s4", 2, 2.65f, 0.875f, 0.164f, 0.275f, 0.558f, 0.f, 0.257f},
+    {"ws64x32x4c4p_k32_s6", 1, 3.16f, 0.451f, 0.173f, 0.966f, 0.872f, 0.f, 0.f},
+    {"ws64x64x4c4p_k32_s3", 2, 2.0f, 1.67f, 0.288f, 0.353f, 0.457f, 0.f, 0.421f},
+    {"ws64x64x4c4p_k32_s6", 0, 2.65f, 1.06f, 0.224f, 1.f, 0.59f, 0.f, 0.f},
+    {"ws128x32x4c4p_k32_s4", 2, 3.17f, 0.967f, 0.366f, 0.334f, 0.156f, 1.61f, 0.302f},
+    {"ws128x32x4c4p_k32_s6", 1, 2.74f, 1.02f, 0.196f, 1.f, 0.712f, 0.f, 0.f},
+    {"ws128x64x4c4p_k32_s6", 0, 2.13f, 2.13f, 0.307f, 1.f, 0.521f, 0.f, 0.f},
     // base, slab, row, -, batch, d
-    {"slab16x64", 2.63f, 0.991f, 0.667f, 0.f, 0.173f, 0.727f, 0.f},
-    {"slab32x64", 2.0f, 1.7f, 0.795f, 0.f, 0.175f, 0.944f, 0.f},
-    // base, tile, step, wide_step, wide, d
-    {"split16x32", 2.4f, 1.15f, 0.853f, 0.f, 0.f, 0.f, 0.f},
-    {"split32x32", 2.45f, 1.24f, 0.607f, 0.21f, 0.f, 1.19f, 0.f},
-    {"split64x32", 2.49f, 1.21f, 0.57f, 0.262f, 0.f, 1.27f, 0.f},
-    {"split128x32", 2.32f, 1.32f, 0.666f, 0.239f, 0.f, 0.944f, 0.f},
+    {"slab16x64", 0, 2.41f, 1.33f, 0.561f, 0.f, 0.132f, 0.878f, 0.f},
+    {"slab32x64", 0, 2.0f, 1.71f, 0.765f, 0.f, 0.181f, 0.971f, 0.f},
+    // base, tile, step, wide_step, -, d
+    {"split16x32", 0, 2.45f, 1.1f, 0.901f, 0.f, 0.f, 0.007f, 0.f},
+    {"split32x32", 0, 2.46f, 1.21f, 0.641f, 0.194f, 0.f, 1.27f, 0.f},
+    {"split64x32", 0, 2.52f, 1.22f, 0.586f, 0.219f, 0.f, 1.25f, 0.f},
+    {"split128x32", 0, 2.43f, 1.28f, 0.618f, 0.254f, 0.f, 1.03f, 0.f},
 };
 
 static double spmm_estimate(const SpmmVariant& v, const SpmmEstimate& e, bool splits, const shflbw_weight* w, int N, int compute_units)
@@ -254,6 +258,8 @@ static int auto_spmm_variant(const shflbw_weight* w, int N, bool spmm, int compu
     double least = 0;
     for (const auto& c : candidates.of[h]) {
         if (c.v->max_k > 0 ? !spmm || w->packed_slab.empty() || w->ncol > c.v->max_k : c.splits && (!spmm || N > 1024)) continue;
+        const bool outnumber = (long)(w->nrow / w->brow) * ((N + c.v->BN - 1) / c.v->BN) > compute_units;
+        if (c.e->tiles != 0 && outnumber != (c.e->tiles == 2)) continue;
         const double t = spmm_estimate(*c.v, *c.e, c.splits, w, N, compute_units);
         if (least == 0 || t < least) least = t, best = c.number;
     }
@@ -860,13 +866,18 @@ int init_chwb_taps(shflbw_spconv_state* state, const shflbw_weight* f, int B, in
         set_error("spconv_init: problem too large (%ld output positions)", ncols);
         return SHFLBW_ERR_UNSUPPORTED;
     }
-    const ConvChwbKernel* k = conv_chwb_kernel(f->brow, 0, f->nrow / f->brow, ncols, device_compute_units());
+    // The cut of the SpMM of these sizes.  With three widths by the number of tiles, and one width for block height 16, us, before / now:
+    // 16 x 14 x 14 x 656 -> 32, 3 x 3, block height 16 20.4 / 11.9, 8 x 7 x 7 x 304 -> 1152, 5 x 5, 14.3 / 11.0; block height 32, 32 x 55 x 27 x
+    // 360 -> 128, 1 x 7, 20.1 / 18.5.
+    const int variant = auto_spmm_variant(f, (int)ncols, false, device_compute_units());
+    const SpmmVariant* v = find_spmm_variant(f->brow, variant, nullptr);
+    const ConvTapsKernel* k = v ? conv_taps_kernel(v->name) : nullptr;
     if (!k) {
         set_error("spconv_init: no kernel for block size %d", f->brow);
         return SHFLBW_ERR_UNSUPPORTED;
     }
-    SHFLBW_HIP_TRY(k->prepare_taps());
-    state->middle_tile_cols = k->BN;
+    SHFLBW_HIP_TRY(k->prepare());
+    state->middle_tile_cols = v->BN;
     shflbw_weight* fw = const_cast<shflbw_weight*>(f); // the table of ids is bookkeeping of the handle (see init_planes)
     std::lock_guard<std::mutex> scratch_guard(fw->scratch_lock);
     const int key[5] = {FORM_CHWB, B, H, W, 0}; // the same for every stride
@@ -879,9 +890,10 @@ int init_chwb_taps(shflbw_spconv_state* state, const shflbw_weight* f, int B, in
     if (rc != SHFLBW_OK) return rc;
     state->ncols = (int)ncols;
     if ((rc = bind_middle(state, f, ncols, IFMap, OFMap, ids, ids_pm, (long)C * H * W * B)) != SHFLBW_OK) return rc;
-    state->shared_mem_size = (size_t)k->lds_bytes;
-    state->grid_dim[0] = (unsigned)((f->nrow / f->brow) * ((ncols + k->BN - 1) / k->BN));
-    state->block_dim[0] = (unsigned)k->threads;
+    state->spmm.variant = variant;
+    state->shared_mem_size = (size_t)v->lds_bytes;
+    state->grid_dim[0] = (unsigned)((f->nrow / f->brow) * ((ncols + v->BN - 1) / v->BN));
+    state->block_dim[0] = (unsigned)v->threads;
     state->grid_dim[1] = state->grid_dim[2] = 1;
     state->block_dim[1] = state->block_dim[2] = 1;
     state->init_success = 1;
@@ -1400,11 +1412,12 @@ int shflbw_spconv_exec(const shflbw_spconv_state* state, void* stream)
     SpconvLaunchArgs a;
     fill_conv_launch_args(state, &a);
     if (state->variant == FORM_CHWB || state->variant == FORM_BPLANES) {
-        const ConvChwbKernel* k = conv_chwb_kernel(state->brow, state->middle_tile_cols, 0, 0, 0);
-        if (!k) return SHFLBW_ERR_UNSUPPORTED;
         if (!state->planes) { // form 4 over the input itself
+            const SpmmVariant* v = find_spmm_variant(state->brow, state->spmm.variant, nullptr);
+            const ConvTapsKernel* k = v ? conv_taps_kernel(v->name) : nullptr;
+            if (!k) return SHFLBW_ERR_UNSUPPORTED;
             ChwbTapArgs t;
-            fill_spmm_launch_args(&state->spmm, k->BN, &t);
+            fill_spmm_launch_args(&state->spmm, v->BN, &t);
             t.B = a.in;
             t.store_mode = result_store_mode(t.D, t.M, t.ldd, false);
             t.alternate = 0;
@@ -1414,11 +1427,13 @@ int shflbw_spconv_exec(const shflbw_spconv_state* state, void* stream)
             t.row_bits = 0;
             for (int r = 0; r < a.R; r++) t.row_bits |= 1u << (r * a.S);
             t.in_bytes = (unsigned)((size_t)a.C * a.H * a.W * a.B * 2);
-            if (t.X > 0) e = k->launch_taps(t, (hipStream_t)stream);
+            if (t.X > 0) e = k->launch(t, (hipStream_t)stream);
             if (e == hipSuccess) return SHFLBW_OK;
             set_error("spconv_exec: launch failed: %s", hipGetErrorString(e));
             return SHFLBW_ERR_HIP;
         }
+        const ConvChwbKernel* k = conv_chwb_kernel(state->brow, state->middle_tile_cols, 0, 0, 0);
+        if (!k) return SHFLBW_ERR_UNSUPPORTED;
         const bool nhwc = state->variant == FORM_BPLANES;
         e = nhwc ? launch_nhwc_to_planes(a, (half_t*)state->planes, state->plane_rows, state->plane_cols,
                                          state->plane_pitch, 1, (hipStream_t)stream, 1)

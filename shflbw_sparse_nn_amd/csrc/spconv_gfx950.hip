@@ -9,6 +9,8 @@
 // tap offset, fetches the 8 activations (zero outside the image) and stores them as one
 // 16-byte piece into the same swizzled [k][pixel] LDS layout the SpMM kernel uses, so the
 // matrix-core part (transposing LDS loads, 32x32x16 fp16 MFMA, fp32 accumulate) is shared.
+#include <cstring>
+
 #include "kernel_common.h"
 #include "spconv_launch.h"
 #include "spmm_ws.h"
@@ -774,7 +776,9 @@ hipError_t launch_chwb_to_planes(const half_t* in, half_t* planes, int B, int H,
 
 // Args: ChwbTapArgs gathers from the input itself, SpmmLaunchArgs from planes, with the columns of the padded grid.
 template <int V, int WN, int NCONS, int NPROD, int KT, int NSTAGE, typename Args>
-__global__ void __launch_bounds__((NCONS + NPROD) * 64) spconv_chwb_kernel(Args a)
+__global__ void
+__launch_bounds__((NCONS + NPROD) * 64, (SpmmWsCfg<V, WN, NCONS, NPROD, KT, NSTAGE>::WGS_PER_CU * (NCONS + NPROD) + 3) / 4)
+spconv_chwb_kernel(Args a)
 {
     constexpr bool DMAP = !std::is_same<Args, ChwbTapArgs>::value;
     using Cfg = SpmmWsCfg<V, WN, NCONS, NPROD, KT, NSTAGE>;
@@ -804,7 +808,7 @@ static hipError_t launch_chwb(const Args& a, hipStream_t stream)
     Args b = a;
     b.n_tiles = (a.N + Cfg::BN - 1) / Cfg::BN;
     const int T = a.X * b.n_tiles;
-    int grid = a.num_cus > 0 ? a.num_cus : 256;
+    int grid = (a.num_cus > 0 ? a.num_cus : 256) * Cfg::WGS_PER_CU;
     grid = (grid / 8) * 8;
     const int need = ((T + 7) / 8) * 8;
     if (grid > need) grid = need;
@@ -823,8 +827,7 @@ static hipError_t prepare_chwb()
 #define SHFLBW_CHWB(V, WN, NC, NP, KT, NS)                                                                             \
     {                                                                                                                  \
         V, WN* NC, (NC + NP) * 64, SpmmWsCfg<V, WN, NC, NP, KT, NS>::LDS_BYTES,                                       \
-            &launch_chwb<V, WN, NC, NP, KT, NS, SpmmLaunchArgs>, &prepare_chwb<V, WN, NC, NP, KT, NS, SpmmLaunchArgs>, \
-            &launch_chwb<V, WN, NC, NP, KT, NS, ChwbTapArgs>, &prepare_chwb<V, WN, NC, NP, KT, NS, ChwbTapArgs>        \
+            &launch_chwb<V, WN, NC, NP, KT, NS, SpmmLaunchArgs>, &prepare_chwb<V, WN, NC, NP, KT, NS, SpmmLaunchArgs>  \
     }
 
 // (the widest tile of a block size first)
@@ -857,6 +860,29 @@ const ConvChwbKernel* conv_chwb_kernel(int V, int tile_cols, long X, long ncols,
     if (X * ((ncols + 127) / 128) <= cus && (k = with(128))) return k;
     if (widest->BN == 512 && X * ((ncols + 511) / 512) <= cus / 2 && (k = with(256))) return k;
     return widest;
+}
+
+#define SHFLBW_CHWB_TAPS(V, WN, NC, NP, KT, NS)                                                                        \
+    {                                                                                                                  \
+        "ws" #V "x" #WN "x" #NC "c" #NP "p_k" #KT "_s" #NS, &launch_chwb<V, WN, NC, NP, KT, NS, ChwbTapArgs>,           \
+            &prepare_chwb<V, WN, NC, NP, KT, NS, ChwbTapArgs>                                                          \
+    }
+
+// one for every role-split variant the SpMM's choice knows
+static const ConvTapsKernel g_chwb_taps[] = {
+    SHFLBW_CHWB_TAPS(64, 128, 4, 4, 32, 4), SHFLBW_CHWB_TAPS(64, 64, 4, 4, 32, 6), SHFLBW_CHWB_TAPS(64, 64, 4, 4, 32, 3),
+    SHFLBW_CHWB_TAPS(64, 32, 4, 4, 32, 6),  SHFLBW_CHWB_TAPS(64, 32, 4, 4, 32, 4),
+    SHFLBW_CHWB_TAPS(32, 128, 4, 4, 32, 4), SHFLBW_CHWB_TAPS(32, 64, 4, 4, 32, 6), SHFLBW_CHWB_TAPS(32, 64, 4, 4, 32, 3),
+    SHFLBW_CHWB_TAPS(32, 32, 4, 4, 32, 6),
+    SHFLBW_CHWB_TAPS(16, 128, 4, 4, 32, 4), SHFLBW_CHWB_TAPS(16, 64, 4, 4, 32, 4), SHFLBW_CHWB_TAPS(16, 64, 2, 4, 32, 6),
+    SHFLBW_CHWB_TAPS(128, 64, 4, 4, 32, 6), SHFLBW_CHWB_TAPS(128, 32, 4, 4, 32, 6), SHFLBW_CHWB_TAPS(128, 32, 4, 4, 32, 4),
+};
+
+const ConvTapsKernel* conv_taps_kernel(const char* spmm_variant)
+{
+    for (const ConvTapsKernel& k : g_chwb_taps)
+        if (strcmp(k.spmm_variant, spmm_variant) == 0) return &k;
+    return nullptr;
 }
 
 template <int V, int WN, int NCONS, int NPROD, int KT, int NSTAGE>

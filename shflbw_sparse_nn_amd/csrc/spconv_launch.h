@@ -91,11 +91,15 @@ struct ConvChwbKernel {
     int BN;
     int threads;
     int lds_bytes;
-    hipError_t (*launch)(const SpmmLaunchArgs&, hipStream_t); // over planes
+    hipError_t (*launch)(const SpmmLaunchArgs&, hipStream_t);
     hipError_t (*prepare)();
-    hipError_t (*launch_taps)(const ChwbTapArgs&, hipStream_t); // over the input itself
-    hipError_t (*prepare_taps)();
 };
+struct ConvTapsKernel { // over the input itself, cut like a variant of the SpMM
+    const char* spmm_variant;
+    hipError_t (*launch)(const ChwbTapArgs&, hipStream_t);
+    hipError_t (*prepare)();
+};
+const ConvTapsKernel* conv_taps_kernel(const char* spmm_variant);
 const ConvChwbKernel* conv_chwb_kernel(int V, int tile_cols, long X, long ncols, int cus);
 
 // Stages 1 and 3 of the plane form of the convolution: NHWC input -> channel-major padded planes (one per
