@@ -1250,7 +1250,7 @@ int conv_patch_for(shflbw_weight* fw, int B, int H, int W, int stride, int Ho, i
         }
         const shflbw_weight::PatchPlaces* places = nullptr;
         if ((rc = patch_places_for(fw, plan.rows_wg, &places)) != SHFLBW_OK) return rc;
-        SHFLBW_HIP_TRY(conv_patch_kernel(RW, plan.col_blocks, plan.waves)->prepare());
+        SHFLBW_HIP_TRY(conv_patch_kernel(RW, plan.col_blocks, plan.waves, plan.deep)->prepare());
         // (an image beyond three quarters of an XCD's L2 is left to the ring past that)
         plan.touch_bytes = (unsigned)std::min<size_t>(image->touch, 3u << 20) - 4;
         plan.touch_step = (unsigned)(plan.jobs_per_xcd * plan.waves * 64) * 128u;
@@ -1399,7 +1399,7 @@ int shflbw_spconv_exec(const shflbw_spconv_state* state, void* stream)
     if (state->variant == FORM_PATCH) {
         ConvPatchArgs p;
         memcpy(&p, state->patch_launch, sizeof(p));
-        const ConvPatchKernel* k = conv_patch_kernel(conv_patch_unit_rows(state->brow), p.p.col_blocks, p.p.waves);
+        const ConvPatchKernel* k = conv_patch_kernel(conv_patch_unit_rows(state->brow), p.p.col_blocks, p.p.waves, p.p.deep);
         if (!k) return SHFLBW_ERR_UNSUPPORTED;
         p.in = (const half_t*)state->args.IFMap;
         p.out = (half_t*)state->args.OFMap;

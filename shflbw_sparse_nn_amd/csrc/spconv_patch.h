@@ -36,6 +36,7 @@ struct ConvPatchPlan {
     unsigned magic_bhw, magic_bw, magic_pw, magic_row, magic_chunks, magic_pg;
     int preferred;        // ... and is estimated faster than the plane forms
     int slack;            // LDS bytes behind the row of zeros that columns without a pixel may touch
+    int deep;             // the kernel with more batches in flight (see g_patch)
 };
 
 // What the plan depends on.
@@ -98,13 +99,13 @@ inline bool conv_patch_streams(size_t out_bytes) { return out_bytes >= 60u << 20
 hipError_t launch_patch_pack(const half_t* values, const int* src, half8_t* packedA, int rows, size_t batches, hipStream_t stream);
 
 struct ConvPatchKernel {
-    int RW, col_blocks, waves;
+    int RW, col_blocks, waves, deep;
     int per_cu; // workgroups of it the registers of a compute unit hold
     int ring, items; // batches a wave keeps in flight, patch items a thread keeps in flight
     hipError_t (*launch)(const ConvPatchArgs&, hipStream_t);
     hipError_t (*prepare)();
 };
-const ConvPatchKernel* conv_patch_kernel(int rows, int col_blocks, int waves);
+const ConvPatchKernel* conv_patch_kernel(int rows, int col_blocks, int waves, int deep);
 
 constexpr int CONV_PATCH_LDS_MAX = 160 * 1024;
 constexpr int CONV_PATCH_SLACK = 256;       // least LDS bytes behind the row of zeros

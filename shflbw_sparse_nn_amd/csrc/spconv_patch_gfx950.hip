@@ -539,14 +539,22 @@ static hipError_t prepare_patch()
                                CONV_PATCH_LDS_MAX);
 }
 
-#define SHFLBW_PATCH(RW, NB, NW, NBUF, U, WPE) {RW, NB, NW, WPE * 4 / NW, NBUF, U, &launch_patch<RW, NB, NW, NBUF, U, WPE>, &prepare_patch<RW, NB, NW, NBUF, U, WPE>}
+#define SHFLBW_PATCH(RW, NB, NW, NBUF, U, WPE, DEEP) {RW, NB, NW, DEEP, WPE * 4 / NW, NBUF, U, &launch_patch<RW, NB, NW, NBUF, U, WPE>, &prepare_patch<RW, NB, NW, NBUF, U, WPE>}
 
+// Workgroups of four waves keep two batches in flight: a deeper ring is more code to fetch at the start of every launch (24 x 24 x 24 x
+// 56 -> 32, 3 x 3, stride 2: 3.9 us, 4.4 with six batches), which only waves with many batches win back: for those the planner weighs
+// its cuts with the deep kernels.  us, before / now: 2 x 44 x 44 x 136 -> 96, 3 x 3, block height 32 6.5 / 5.1, 16 x 50 x 50 x 160 -> 256, 1 x 7,
+// 27.4 / 25.6, 3 x 14 x 30 x 224 -> 800, stride 2 6.8 / 6.1; block height 16: 8 x 26 x 52 x 48 -> 1216, stride 2 13.1 / 10.9, 8 x 45 x 41 x 24 -> 160
+// 9.0 / 7.5.  As many batches as the registers of the cut's workgroups hold without spilling; row units of 64, and of 16 over 64
+// columns, leave no room for them.
 static const ConvPatchKernel g_patch[] = {
-    SHFLBW_PATCH(16, 2, 8, 8, 5, 2), SHFLBW_PATCH(32, 2, 8, 8, 5, 2), SHFLBW_PATCH(64, 2, 8, 4, 5, 2),
-    SHFLBW_PATCH(16, 1, 8, 8, 5, 2), SHFLBW_PATCH(32, 1, 8, 8, 5, 2), SHFLBW_PATCH(64, 1, 8, 4, 5, 2),
-    SHFLBW_PATCH(16, 2, 4, 2, 2, 3), SHFLBW_PATCH(32, 2, 4, 2, 2, 2), SHFLBW_PATCH(64, 2, 4, 2, 2, 3),
-    SHFLBW_PATCH(16, 1, 4, 2, 2, 4), SHFLBW_PATCH(32, 1, 4, 2, 2, 4), SHFLBW_PATCH(64, 1, 4, 2, 2, 4),
+    SHFLBW_PATCH(16, 2, 8, 8, 5, 2, 0), SHFLBW_PATCH(32, 2, 8, 8, 5, 2, 0), SHFLBW_PATCH(64, 2, 8, 4, 5, 2, 0),
+    SHFLBW_PATCH(16, 1, 8, 8, 5, 2, 0), SHFLBW_PATCH(32, 1, 8, 8, 5, 2, 0), SHFLBW_PATCH(64, 1, 8, 4, 5, 2, 0),
+    SHFLBW_PATCH(16, 2, 4, 2, 2, 3, 0), SHFLBW_PATCH(32, 2, 4, 2, 2, 2, 0), SHFLBW_PATCH(64, 2, 4, 2, 2, 3, 0),
+    SHFLBW_PATCH(16, 1, 4, 2, 2, 4, 0), SHFLBW_PATCH(32, 1, 4, 2, 2, 4, 0), SHFLBW_PATCH(64, 1, 4, 2, 2, 4, 0),
+    SHFLBW_PATCH(32, 2, 4, 6, 2, 2, 1), SHFLBW_PATCH(16, 1, 4, 6, 2, 4, 1), SHFLBW_PATCH(32, 1, 4, 4, 2, 4, 1),
 };
+static int patch_deep_batches(int rows) { return rows == 16 ? 13 : 9; } // of a wave, from which on the deeper ring is taken
 
 // Estimated microseconds of the plane forms (three launches): the launches, the gathers of the SpMM, the two layout
 // passes.  The weights come from a fit to 124 measured layers (20 % rms).
@@ -596,7 +604,7 @@ bool conv_patch_plan(const ConvPatchProblem& q, ConvPatchPlan* plan, const std::
                 // on); else positions are packed
                 const int rl = tw <= 8 && th <= positions / 8 ? 8 : th == 1 ? 16 : tw;
                 ConvPatchPlan p{};
-                p.col_blocks = k.col_blocks, p.waves = k.waves;
+                p.col_blocks = k.col_blocks, p.waves = k.waves, p.deep = k.deep;
                 p.tile_h = th, p.tile_w = tw, p.row_len = rl;
                 p.blocks_w = (Wo + tw - 1) / tw;
                 const long blocks_hw = (long)((Ho + th - 1) / th) * p.blocks_w, units = B * blocks_hw;
@@ -643,6 +651,7 @@ bool conv_patch_plan(const ConvPatchProblem& q, ConvPatchPlan* plan, const std::
                         const double rounds = std::ceil((double)jobs / ((double)q.cus * wgs));
                         const double w = k.waves * act; // waves of a compute unit
                         const double nb = std::ceil(np * batches / p.ksplit);
+                        if (k.deep != (nb >= patch_deep_batches(rw) && conv_patch_kernel(rw, k.col_blocks, k.waves, 1) != nullptr)) continue;
                         const int steps = rw == 16 ? 1 : 2, mbw = rw == 64 ? 2 : 1, ncb = rw == 16 ? 2 * k.col_blocks : k.col_blocks;
                         const bool apart = rl == 8 || rl == 16; // rows of half a wave's positions lie in a line
                         const double t_mfma = steps * mbw * ncb * (rw == 16 ? 16 : 32) * w / 4 * 0.00045;
@@ -775,10 +784,10 @@ void ConvPatchOrder::of(const std::vector<int>& pair_of, std::vector<int>& order
     }
 }
 
-const ConvPatchKernel* conv_patch_kernel(int rows, int col_blocks, int waves)
+const ConvPatchKernel* conv_patch_kernel(int rows, int col_blocks, int waves, int deep)
 {
     for (const ConvPatchKernel& k : g_patch)
-        if (k.RW == rows && k.col_blocks == col_blocks && k.waves == waves) return &k;
+        if (k.RW == rows && k.col_blocks == col_blocks && k.waves == waves && k.deep == deep) return &k;
     return nullptr;
 }
 
