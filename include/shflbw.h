@@ -171,7 +171,7 @@ typedef struct shflbw_spmm_state {
     const int* panel_ptr;
     int brow;
     int ldb_bytes; /* distance in bytes between two rows of B that are one kept-column id apart: N * 2 */
-    const void* zero_row; /* 1 KiB of zeros inside the library (device memory): gathered for the padding slots */
+    const void* zero_row; /* 1 KiB of zeros inside the library (device memory): gathered for the padding slots by the variants without a buffer descriptor for B */
     const int* packed_slab; /* the ids as LDS offsets for the tile variants that hold B in LDS; NULL when the weight has too many columns */
     int groups; /* groups of 64 slots that the kept vectors of all panels fill */
 } shflbw_spmm_state;
@@ -286,8 +286,9 @@ int shflbw_spconv_exec(const shflbw_spconv_state* state, void* stream);
  * IFMap[c][hi][wi][b] and OFMap[f][ho][wo][b], batch innermost; H and W are the extents of the output grid and at
  * the same time the bounds of the input: out(ho, wo) reads in(ho*stride - R/2 + r, wo*stride - S/2 + s) where that lies
  * inside H x W and zero elsewhere (so IFMap holds C*H*W*B values and OFMap F*H*W*B, whatever the stride).
- * Precondition as in the reference's kernel (spconv/blockwise_kernel.h:200-207): B % 8 == 0.  exec launches a padded
- * copy of the input and one SpMM launch that writes OFMap directly (form 4 of shflbw_spconv_variant_name). */
+ * Precondition as in the reference's kernel (spconv/blockwise_kernel.h:200-207): B % 8 == 0.  exec launches one
+ * kernel that gathers from IFMap and writes OFMap (form 4 of shflbw_spconv_variant_name); for filters of more than 31 taps,
+ * inputs from 2 GiB on and an OFMap that overlaps IFMap a padded copy of the input and a kernel over that. */
 int shflbw_spconv_init_chwb(shflbw_spconv_state* state, const shflbw_weight* filter,
                             int B, int H, int W, int stride, const void* IFMap, void* OFMap);
 /* No counterpart in the reference.  For callers that cannot allocate device memory: code under HIP graph
