@@ -167,48 +167,54 @@ static bool spmm_variant_offsets32(const SpmmVariant* v) { return v && (v->name[
 //    takes as long as one and (tile2 + stage2 * stages);
 //  slab: base + rounds * (slab + K / 1000 * row + panels of a wave * batches of 32 vectors * batch) + d * ...;
 //  split: base + rounds * (tile + steps of a wave * (step + (64 columns: wide_step))) + d * ...
+//  With a C term c * (C at 5 TB/s) + c_tile * tiles (panels of a wave) more, fitted to 670 problems with one (9-16 % rms).  The variants differ in
+//  what C costs them: the slab form and the short rings read it in the epilogue.  Chosen as without it: 1.027 times the fastest variant on
+//  average, 1.36 at worst, with it 1.016 and 1.25 (24576 x 85 x 1848, block height 128, density 0.31: 64 us with 128 columns, 53 with 256;
+//  10464 x 89 x 2424, block height 16: slab 36, role-split 31); on 180 others 1.033 on average, now 1.020.
 struct SpmmEstimate {
     const char* name;
     int tiles; // 0; 1: only while its tiles do not outnumber the compute units; 2: only where they do
-    float base, tile, stage, whole, d, tile2, stage2;
+    float base, tile, stage, whole, d, tile2, stage2, c, c_tile;
 };
 static const SpmmEstimate g_estimates[] = {
     // The rings of three and four stages that let two workgroups share a compute unit are too short for one alone (128 columns
     // 1.00-1.15 times, 256 columns up to 1.9 times the six stages' time, the more the longer the panels), and with more tiles than
     // compute units the 128-column ones were ahead throughout (0.78-0.98 times).
-    {"ws16x128x4c4p_k32_s4", 0, 2.99f, 0.688f, 0.273f, 1.f, 0.442f, 0.f, 0.f},
-    {"ws16x64x2c4p_k32_s6", 0, 2.98f, 0.851f, 0.13f, 0.277f, 0.f, 0.f, 0.083f},
-    {"ws16x64x4c4p_k32_s4", 0, 3.06f, 0.7f, 0.158f, 0.149f, 0.329f, 0.f, 0.171f},
-    {"ws32x128x4c4p_k32_s4", 0, 2.56f, 1.05f, 0.295f, 1.f, 0.584f, 0.f, 0.f},
-    {"ws32x32x4c4p_k32_s6", 0, 2.94f, 0.873f, 0.124f, 0.137f, 0.318f, 0.f, 0.137f},
-    {"ws32x64x4c4p_k32_s3", 2, 2.49f, 0.f, 0.399f, 0.876f, 0.399f, 1.02f, 0.054f},
-    {"ws32x64x4c4p_k32_s6", 0, 2.86f, 0.756f, 0.188f, 0.773f, 0.531f, 0.f, 0.f},
-    {"ws64x128x4c4p_k32_s4", 0, 2.15f, 1.93f, 0.355f, 1.f, 0.653f, 0.f, 0.f},
-    {"ws64x32x4c4p_k32_s4", 2, 2.65f, 0.875f, 0.164f, 0.275f, 0.558f, 0.f, 0.257f},
-    {"ws64x32x4c4p_k32_s6", 1, 3.16f, 0.451f, 0.173f, 0.966f, 0.872f, 0.f, 0.f},
-    {"ws64x64x4c4p_k32_s3", 2, 2.0f, 1.67f, 0.288f, 0.353f, 0.457f, 0.f, 0.421f},
-    {"ws64x64x4c4p_k32_s6", 0, 2.65f, 1.06f, 0.224f, 1.f, 0.59f, 0.f, 0.f},
-    {"ws128x32x4c4p_k32_s4", 2, 3.17f, 0.967f, 0.366f, 0.334f, 0.156f, 1.61f, 0.302f},
-    {"ws128x32x4c4p_k32_s6", 1, 2.74f, 1.02f, 0.196f, 1.f, 0.712f, 0.f, 0.f},
-    {"ws128x64x4c4p_k32_s6", 0, 2.13f, 2.13f, 0.307f, 1.f, 0.521f, 0.f, 0.f},
-    // base, slab, row, -, batch, d
-    {"slab16x64", 0, 2.41f, 1.33f, 0.561f, 0.f, 0.132f, 0.878f, 0.f},
-    {"slab32x64", 0, 2.0f, 1.71f, 0.765f, 0.f, 0.181f, 0.971f, 0.f},
-    // base, tile, step, wide_step, -, d
-    {"split16x32", 0, 2.45f, 1.1f, 0.901f, 0.f, 0.f, 0.007f, 0.f},
-    {"split32x32", 0, 2.46f, 1.21f, 0.641f, 0.194f, 0.f, 1.27f, 0.f},
-    {"split64x32", 0, 2.52f, 1.22f, 0.586f, 0.219f, 0.f, 1.25f, 0.f},
-    {"split128x32", 0, 2.43f, 1.28f, 0.618f, 0.254f, 0.f, 1.03f, 0.f},
+    {"ws16x128x4c4p_k32_s4", 0, 2.99f, 0.688f, 0.273f, 1.f, 0.442f, 0.f, 0.f, 0.744f, 0.256f},
+    {"ws16x64x2c4p_k32_s6", 0, 2.98f, 0.851f, 0.13f, 0.277f, 0.f, 0.f, 0.083f, 0.977f, 0.f},
+    {"ws16x64x4c4p_k32_s4", 0, 3.06f, 0.7f, 0.158f, 0.149f, 0.329f, 0.f, 0.171f, 0.884f, 0.f},
+    {"ws32x128x4c4p_k32_s4", 0, 2.56f, 1.05f, 0.295f, 1.f, 0.584f, 0.f, 0.f, 0.874f, 0.612f},
+    {"ws32x32x4c4p_k32_s6", 0, 2.94f, 0.873f, 0.124f, 0.137f, 0.318f, 0.f, 0.137f, 1.09f, 0.f},
+    {"ws32x64x4c4p_k32_s3", 2, 2.49f, 0.f, 0.399f, 0.876f, 0.399f, 1.02f, 0.054f, 1.16f, 0.0154f},
+    {"ws32x64x4c4p_k32_s6", 0, 2.86f, 0.756f, 0.188f, 0.773f, 0.531f, 0.f, 0.f, 0.802f, 0.203f},
+    {"ws64x128x4c4p_k32_s4", 0, 2.15f, 1.93f, 0.355f, 1.f, 0.653f, 0.f, 0.f, 0.806f, 1.27f},
+    {"ws64x32x4c4p_k32_s4", 2, 2.65f, 0.875f, 0.164f, 0.275f, 0.558f, 0.f, 0.257f, 1.22f, 0.f},
+    {"ws64x32x4c4p_k32_s6", 1, 3.16f, 0.451f, 0.173f, 0.966f, 0.872f, 0.f, 0.f, 0.f, 0.00842f},
+    {"ws64x64x4c4p_k32_s3", 2, 2.0f, 1.67f, 0.288f, 0.353f, 0.457f, 0.f, 0.421f, 0.94f, 0.441f},
+    {"ws64x64x4c4p_k32_s6", 0, 2.65f, 1.06f, 0.224f, 1.f, 0.59f, 0.f, 0.f, 0.661f, 0.818f},
+    {"ws128x32x4c4p_k32_s4", 2, 3.17f, 0.967f, 0.366f, 0.334f, 0.156f, 1.61f, 0.302f, 1.33f, 0.f},
+    {"ws128x32x4c4p_k32_s6", 1, 2.74f, 1.02f, 0.196f, 1.f, 0.712f, 0.f, 0.f, 0.468f, 0.676f},
+    {"ws128x64x4c4p_k32_s6", 0, 2.13f, 2.13f, 0.307f, 1.f, 0.521f, 0.f, 0.f, 0.745f, 1.51f},
+    // base, slab, row, -, batch, d, -, c, c_panel
+    {"slab16x64", 0, 2.41f, 1.33f, 0.561f, 0.f, 0.132f, 0.878f, 0.f, 1.17f, 0.f},
+    {"slab32x64", 0, 2.0f, 1.71f, 0.765f, 0.f, 0.181f, 0.971f, 0.f, 1.12f, 0.0686f},
+    // base, tile, step, wide_step, -, d, -, c, -
+    {"split16x32", 0, 2.45f, 1.1f, 0.901f, 0.f, 0.f, 0.007f, 0.f, 2.94f, 0.f},
+    {"split32x32", 0, 2.46f, 1.21f, 0.641f, 0.194f, 0.f, 1.27f, 0.f, 0.911f, 0.f},
+    {"split64x32", 0, 2.52f, 1.22f, 0.586f, 0.219f, 0.f, 1.25f, 0.f, 0.999f, 0.f},
+    {"split128x32", 0, 2.43f, 1.28f, 0.618f, 0.254f, 0.f, 1.03f, 0.f, 0.994f, 0.f},
 };
 
-static double spmm_estimate(const SpmmVariant& v, const SpmmEstimate& e, bool splits, const shflbw_weight* w, int N, int compute_units)
+static double spmm_estimate(const SpmmVariant& v, const SpmmEstimate& e, bool splits, const shflbw_weight* w, int N, bool residual, int compute_units)
 {
     const double X = w->nrow / w->brow, vectors = w->nnzb / X, t_d = 2.0 * w->nrow * N / 5e6;
     const double cus = compute_units;
+    auto with_c = [&](double t, double tiles) { return residual ? t + e.c * t_d + e.c_tile * tiles : t; };
     if (v.max_k > 0) {
         const int groups = (int)(w->packed_indices.size() / 64);
         const SlabDeal s = slab_deal(w->brow, (int)X, w->ncol, groups, (N + v.BN - 1) / v.BN, compute_units / 8 * 8);
-        return e.base + s.rounds * (e.tile + e.stage * w->ncol / 1000 + s.wave_panels * e.d * 2 * std::ceil(vectors / 64)) + e.tile2 * t_d;
+        return with_c(e.base + s.rounds * (e.tile + e.stage * w->ncol / 1000 + s.wave_panels * e.d * 2 * std::ceil(vectors / 64)) + e.tile2 * t_d,
+                      (double)s.rounds * s.wave_panels);
     }
     if (splits) { // as launch_split cuts it
         const bool v16 = w->brow == 16;
@@ -216,7 +222,8 @@ static double spmm_estimate(const SpmmVariant& v, const SpmmEstimate& e, bool sp
         const bool wide = !v16 && N > 32 && blocks * ((N + 31) / 32) > cus;
         const double grid = std::ceil(blocks / 8) * 8 * (wide ? (N + 63) / 64 : (N + 31) / 32), waves = grid <= cus ? 16 : 8;
         const double steps = vectors / (v16 ? 32 : 16) / waves + 0.5;
-        return e.base + std::max(1.0, grid / (waves == 16 ? cus : 2 * cus)) * (e.tile + (e.stage + (wide ? e.whole : 0.f)) * steps) + e.tile2 * t_d;
+        const double rounds = std::max(1.0, grid / (waves == 16 ? cus : 2 * cus));
+        return with_c(e.base + rounds * (e.tile + (e.stage + (wide ? e.whole : 0.f)) * steps) + e.tile2 * t_d, rounds);
     }
     const double per_cu = X * ((N + v.BN - 1) / v.BN) / cus, n = std::ceil(per_cu), mean = std::max(1.0, per_cu);
     const double one = e.tile + e.stage * (vectors / 32 + 0.5);
@@ -226,11 +233,11 @@ static double spmm_estimate(const SpmmVariant& v, const SpmmEstimate& e, bool sp
         whole = pairs * pair + (n - 2 * pairs) * one;
         rest = mean <= 2 ? one + (mean - 1) * (pair - one) : mean / 2 * pair;
     }
-    return e.base + e.whole * whole + (1 - e.whole) * rest + e.d * t_d;
+    return with_c(e.base + e.whole * whole + (1 - e.whole) * rest + e.d * t_d, e.whole * n + (1 - e.whole) * mean);
 }
 
 // `spmm` false: what is multiplied are the planes of a convolution, which only the variants that gather rows by id can walk.
-static int auto_spmm_variant(const shflbw_weight* w, int N, bool spmm, int compute_units)
+static int auto_spmm_variant(const shflbw_weight* w, int N, bool spmm, bool residual, int compute_units)
 {
     struct Candidates { // of the four block heights, found once
         struct One {
@@ -260,7 +267,7 @@ static int auto_spmm_variant(const shflbw_weight* w, int N, bool spmm, int compu
         if (c.v->max_k > 0 ? !spmm || w->packed_slab.empty() || w->ncol > c.v->max_k : c.splits && (!spmm || N > 1024)) continue;
         const bool outnumber = (long)(w->nrow / w->brow) * ((N + c.v->BN - 1) / c.v->BN) > compute_units;
         if (c.e->tiles != 0 && outnumber != (c.e->tiles == 2)) continue;
-        const double t = spmm_estimate(*c.v, *c.e, c.splits, w, N, compute_units);
+        const double t = spmm_estimate(*c.v, *c.e, c.splits, w, N, residual, compute_units);
         if (least == 0 || t < least) least = t, best = c.number;
     }
     return best;
@@ -414,7 +421,7 @@ static int spmm_init_impl(shflbw_spmm_state* state, const shflbw_weight* w, int 
     // the role-split kernels address the rows of B with 32-bit byte offsets
     const bool wide_b = (unsigned long long)w->ncol * (unsigned long long)N * 2ull + (unsigned long long)N * 2ull > 0xffffffffull;
     if (variant < 0) {
-        variant = auto_spmm_variant(w, N, !gather_only, compute_units);
+        variant = auto_spmm_variant(w, N, !gather_only, beta != 0.f, compute_units);
         if (wide_b) { // first variant of this block size with 64-bit addressing (block height 16 has none: refused below)
             int n = 0;
             find_spmm_variant(w->brow, variant = 0, &n);
@@ -869,7 +876,7 @@ int init_chwb_taps(shflbw_spconv_state* state, const shflbw_weight* f, int B, in
     // The cut of the SpMM of these sizes.  With three widths by the number of tiles, and one width for block height 16, us, before / now:
     // 16 x 14 x 14 x 656 -> 32, 3 x 3, block height 16 20.4 / 11.9, 8 x 7 x 7 x 304 -> 1152, 5 x 5, 14.3 / 11.0; block height 32, 32 x 55 x 27 x
     // 360 -> 128, 1 x 7, 20.1 / 18.5.
-    const int variant = auto_spmm_variant(f, (int)ncols, false, device_compute_units());
+    const int variant = auto_spmm_variant(f, (int)ncols, false, false, device_compute_units());
     const SpmmVariant* v = find_spmm_variant(f->brow, variant, nullptr);
     const ConvTapsKernel* k = v ? conv_taps_kernel(v->name) : nullptr;
     if (!k) {
