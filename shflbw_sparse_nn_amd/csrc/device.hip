@@ -387,7 +387,8 @@ const char* shflbw_spmm_variant_name(int brow, int variant)
 
 // `gather_only`: the caller will point the gather at something other than a K x N matrix (the planes of a
 // convolution, ids rewritten as element offsets), which only the variants that gather rows by id can walk: the
-// variants that hold all K rows of B in LDS are left out of the automatic choice and refused when forced.
+// variants that hold all K rows of B in LDS are left out of the automatic choice and refused when forced.  There is no
+// K x N matrix then, and its size bounds nothing: the caller keeps what its ids address below 4 GiB.
 static int spmm_init_impl(shflbw_spmm_state* state, const shflbw_weight* w, int N, const void* B, const void* C, void* D,
                           float alpha, float beta, int variant, bool gather_only)
 {
@@ -419,7 +420,8 @@ static int spmm_init_impl(shflbw_spmm_state* state, const shflbw_weight* w, int 
     }
     const int X = w->nrow / w->brow, compute_units = device_compute_units();
     // the role-split kernels address the rows of B with 32-bit byte offsets
-    const bool wide_b = (unsigned long long)w->ncol * (unsigned long long)N * 2ull + (unsigned long long)N * 2ull > 0xffffffffull;
+    const bool wide_b =
+        !gather_only && (unsigned long long)w->ncol * (unsigned long long)N * 2ull + (unsigned long long)N * 2ull > 0xffffffffull;
     if (variant < 0) {
         variant = auto_spmm_variant(w, N, !gather_only, beta != 0.f, compute_units);
         if (wide_b) { // first variant of this block size with 64-bit addressing (block height 16 has none: refused below)
@@ -706,12 +708,12 @@ int conv_bulk_for(shflbw_weight* fw, const int (&key)[5], const void* in, const 
 }
 
 // Sets up the SpMM launch in the middle of a plane form: N columns, the planes as B, `result` as D, the rewritten ids
-// (element offsets: one id apart is one value apart) and `id_space` as the extent the ids address.
+// (element offsets: one id apart is one value apart) and `id_space` as the extent the ids address, below 2^31 values
+// (every caller's size check).  `variant`: of the SpMM's variants, -1 for the library's choice among those that gather rows by id.
 int bind_middle(shflbw_spconv_state* state, const shflbw_weight* f, long N, const void* planes, void* result,
-                const int* ids, const int* ids_pm, long id_space)
+                const int* ids, const int* ids_pm, long id_space, int variant = -1)
 {
-    // only the variants that gather rows by id can walk the planes; the first one of the block size (role-split)
-    int rc = spmm_init_impl(&state->spmm, f, (int)N, planes, nullptr, result, 1.f, 0.f, -1, true);
+    int rc = spmm_init_impl(&state->spmm, f, (int)N, planes, nullptr, result, 1.f, 0.f, variant, true);
     if (rc != SHFLBW_OK) return rc;
     state->spmm.packed_indices = ids;
     state->spmm.packed_indices_pm = ids_pm;
@@ -896,8 +898,7 @@ int init_chwb_taps(shflbw_spconv_state* state, const shflbw_weight* f, int B, in
     }, &ids, &ids_pm);
     if (rc != SHFLBW_OK) return rc;
     state->ncols = (int)ncols;
-    if ((rc = bind_middle(state, f, ncols, IFMap, OFMap, ids, ids_pm, (long)C * H * W * B)) != SHFLBW_OK) return rc;
-    state->spmm.variant = variant;
+    if ((rc = bind_middle(state, f, ncols, IFMap, OFMap, ids, ids_pm, (long)C * H * W * B, variant)) != SHFLBW_OK) return rc;
     state->shared_mem_size = (size_t)v->lds_bytes;
     state->grid_dim[0] = (unsigned)((f->nrow / f->brow) * ((ncols + v->BN - 1) / v->BN));
     state->block_dim[0] = (unsigned)v->threads;
