@@ -286,21 +286,24 @@ struct PlaneForm {
     size_t total_bytes() const { return planes_bytes + dm_bytes + 2 * ids_bytes; }
 };
 
+// `rows` channel rows of `pitch` values and a row of zeros behind them: within the 4 GiB of 32-bit byte offsets?
+static bool planes_fit(long rows, long pitch) { return rows < 0x7fffffffL / pitch; }
+
 static int plane_form_geometry(const shflbw_weight* f, int B, int H, int W, int stride, PlaneForm* g)
 {
     const int s = stride, ph = f->R / 2, pw = f->S / 2;
+    g->copies = (f->S - 1) / s >= 1 ? 2 : 1;
+    if (s > 5 || g->copies * s * s > 32) {
+        set_error("spconv: stride %d has too many phase planes for the plane form", s);
+        return SHFLBW_ERR_UNSUPPORTED;
+    }
     g->PH = (H + 2 * ph + s - 1) / s;
     g->PW = ((W + 2 * pw + s - 1) / s + 7) / 8 * 8;
     g->np = (long)B * g->PH * g->PW;
     const long max_shift = (long)((f->R - 1) / s) * g->PW + (f->S - 1) / s; // largest tap offset
     g->pitch = (g->np + max_shift + 8 + 63) / 64 * 64;
-    g->copies = (f->S - 1) / s >= 1 ? 2 : 1;
-    if (g->copies * s * s > 32) {
-        set_error("spconv: stride %d has too many phase planes for the plane form", s);
-        return SHFLBW_ERR_UNSUPPORTED;
-    }
     g->rows = (long)g->copies * s * s * f->C;
-    if (g->np > 0x7fffffffL || (unsigned long long)(g->rows + 1) * (unsigned long long)g->pitch * 2ull > 0xffffffffull) {
+    if (g->np > 0x7fffffffL || !planes_fit(g->rows, g->pitch)) {
         set_error("spconv: problem too large for the plane form (%ld rows of %ld positions)", g->rows, g->pitch);
         return SHFLBW_ERR_UNSUPPORTED;
     }
@@ -922,6 +925,10 @@ int init_batch_planes(shflbw_spconv_state* state, const shflbw_weight* f, int B,
         state->Wo = W;
         if (chwb_gathers_input(f, B, H, W, IFMap, OFMap)) return init_chwb_taps(state, f, B, H, W, stride, IFMap, OFMap);
     }
+    if (stride > 5792) { // stride^2 planes of 64 values or more: beyond 4 GiB
+        set_error("spconv_init: stride %d has too many phase planes", stride);
+        return SHFLBW_ERR_UNSUPPORTED;
+    }
     BatchPlanes g;
     batch_planes_geometry(f, B, stride, state->Ho, state->Wo, &g);
     // the SpMM in the middle: tile width by the size of the GEMM, as for the SpMM proper
@@ -934,7 +941,7 @@ int init_batch_planes(shflbw_spconv_state* state, const shflbw_weight* f, int B,
     state->middle_tile_cols = k->BN;
     const int s = stride, C = f->C, S = f->S;
     const long pitch = (g.np + g.max_shift + 8 + 63) / 64 * 64;
-    if (g.ncols > 0x7fffffffL || (unsigned long long)(g.rows + 1) * (unsigned long long)pitch * 2ull > 0xffffffffull) {
+    if (g.ncols > 0x7fffffffL || !planes_fit(g.rows, pitch)) {
         set_error("spconv_init: problem too large (%ld channel rows of %ld values)", g.rows, pitch);
         return SHFLBW_ERR_UNSUPPORTED;
     }
@@ -986,11 +993,15 @@ struct FusedForm {
 
 int fused_form_geometry(const shflbw_weight* f, int B, int stride, int Ho, int Wo, int nx, FusedForm* g)
 {
+    if (stride > 5) {
+        set_error("spconv_init: stride %d has too many phase planes for the fused form", stride);
+        return SHFLBW_ERR_UNSUPPORTED;
+    }
     batch_planes_geometry(f, B, stride, Ho, Wo, &g->g);
     g->nx = nx;
     g->cx = ((g->g.ncols + nx - 1) / nx + 63) / 64 * 64;
     g->pitch = (g->cx + g->g.max_shift + 63) / 64 * 64;
-    if (stride * stride > 32 || g->g.ncols > 0x7fffffffL ||
+    if (g->g.ncols > 0x7fffffffL ||
         (unsigned long long)(g->g.rows + 1) * (unsigned long long)g->pitch * 2ull > 0x7fffffffull ||
         (unsigned long long)f->F * (unsigned long long)g->cx > 0x7fffffffull) {
         set_error("spconv_init: problem too large for the fused form (%ld channel rows of %ld values per XCD)", g->g.rows, g->pitch);
