@@ -288,7 +288,8 @@ int shflbw_spconv_exec(const shflbw_spconv_state* state, void* stream);
  * inside H x W and zero elsewhere (so IFMap holds C*H*W*B values and OFMap F*H*W*B, whatever the stride).
  * Precondition as in the reference's kernel (spconv/blockwise_kernel.h:200-207): B % 8 == 0.  exec launches one
  * kernel that gathers from IFMap and writes OFMap (form 4 of shflbw_spconv_variant_name); for filters of more than 31 taps,
- * inputs from 2 GiB on and an OFMap that overlaps IFMap a padded copy of the input and a kernel over that. */
+ * inputs from 2 GiB on, maps on which max(H, W) * stride * S leaves an int (strides past the map aside) and an OFMap that overlaps
+ * IFMap a padded copy of the input and a kernel over that. */
 int shflbw_spconv_init_chwb(shflbw_spconv_state* state, const shflbw_weight* filter,
                             int B, int H, int W, int stride, const void* IFMap, void* OFMap);
 /* No counterpart in the reference.  For callers that cannot allocate device memory: code under HIP graph

@@ -855,20 +855,20 @@ void batch_planes_geometry(const shflbw_weight* f, int B, int stride, int Ho, in
     g->max_shift = ((long)((f->R - 1) / s) * g->PW + (f->S - 1) / s) * B;
 }
 
-//   form 4: the caller's tensors are C-H-W-B / F-H-W-B (the reference's), H and W bound input and output alike,
-//           the SpMM writes OFMap itself (its epilogue drops the padding columns, output_column()); only for what
-//           chwb_gathers_input() leaves;
-//   form 2: the caller's tensors are NHWC with true stride and padding; the SpMM writes result_fm[f][(ho, wo, img)],
-//           a tile transpose writes OFMap.
-// Form 4 over the input itself (the state holds no planes): where the ids of its taps fit (chwb_tap_id) and the output does
-// not overwrite what is still to be gathered.
-bool chwb_gathers_input(const shflbw_weight* f, int B, int H, int W, const void* IFMap, const void* OFMap)
+// Strides past the map read it at the first row and column only, whatever they are: one such stride stands for all.
+long chwb_stride(int H, int W, int R, int S, int stride) { return std::min((long)stride, (long)H + W + R + S); }
+
+// Form 4 over the input itself (the state holds no planes): where the ids of its taps fit (chwb_tap_id), the output does
+// not overwrite what is still to be gathered, and the input row of every position times the width of the filter stays
+// within an int (by which the kernel tells the taps outside the map).
+bool chwb_gathers_input(const shflbw_weight* f, int B, int H, int W, int stride, const void* IFMap, const void* OFMap)
 {
     const size_t pixels = (size_t)B * H * W * 2;
     const char *in = (const char*)IFMap, *out = (const char*)OFMap;
     const bool apart = in + pixels * f->C <= out || out + pixels * f->F <= in;
     return apart && (long)f->R * f->S <= CHWB_MAX_TAPS &&
-           ((unsigned long long)f->C * H * W + (unsigned long long)f->R * W + f->S) * (unsigned long long)B * 2ull < 0x80000000ull;
+           ((unsigned long long)f->C * H * W + (unsigned long long)f->R * W + f->S) * (unsigned long long)B * 2ull < 0x80000000ull &&
+           std::max(H, W) * chwb_stride(H, W, f->R, f->S, stride) * f->S < 0x7fffffffL;
 }
 
 int init_chwb_taps(shflbw_spconv_state* state, const shflbw_weight* f, int B, int H, int W, int stride, const void* IFMap, void* OFMap)
@@ -911,6 +911,11 @@ int init_chwb_taps(shflbw_spconv_state* state, const shflbw_weight* f, int B, in
     return SHFLBW_OK;
 }
 
+//   form 4: the caller's tensors are C-H-W-B / F-H-W-B (the reference's), H and W bound input and output alike,
+//           the SpMM writes OFMap itself (its epilogue drops the padding columns, output_column()); only for what
+//           chwb_gathers_input() leaves;
+//   form 2: the caller's tensors are NHWC with true stride and padding; the SpMM writes result_fm[f][(ho, wo, img)],
+//           a tile transpose writes OFMap.
 int init_batch_planes(shflbw_spconv_state* state, const shflbw_weight* f, int B, int H, int W, int stride,
                       const void* IFMap, void* OFMap, int variant)
 {
@@ -923,7 +928,7 @@ int init_batch_planes(shflbw_spconv_state* state, const shflbw_weight* f, int B,
     if (variant == FORM_CHWB) { // H and W are the extents of the output grid and the bounds of the input (spconv/blockwise_format.h:111-115)
         state->Ho = H;
         state->Wo = W;
-        if (chwb_gathers_input(f, B, H, W, IFMap, OFMap)) return init_chwb_taps(state, f, B, H, W, stride, IFMap, OFMap);
+        if (chwb_gathers_input(f, B, H, W, stride, IFMap, OFMap)) return init_chwb_taps(state, f, B, H, W, stride, IFMap, OFMap);
     }
     if (stride > 5792) { // stride^2 planes of 64 values or more: beyond 4 GiB
         set_error("spconv_init: stride %d has too many phase planes", stride);
@@ -1441,7 +1446,7 @@ int shflbw_spconv_exec(const shflbw_spconv_state* state, void* stream)
             t.store_mode = result_store_mode(t.D, t.M, t.ldd, false);
             t.alternate = 0;
             t.batch = a.B, t.in_h = a.H, t.in_w = a.W;
-            t.taps_r = a.R, t.taps_s = a.S, t.stride = a.stride;
+            t.taps_r = a.R, t.taps_s = a.S, t.stride = (int)chwb_stride(a.H, a.W, a.R, a.S, a.stride);
             t.magic_batch = udiv_magic(a.B), t.magic_w = udiv_magic(a.W);
             t.row_bits = 0;
             for (int r = 0; r < a.R; r++) t.row_bits |= 1u << (r * a.S);

@@ -784,7 +784,7 @@ __device__ __forceinline__ void ws_producer(const Args& a, uint32_t lds0, int la
                 fast_divmod(c, a.batch, a.magic_batch, pos, b);
                 fast_divmod(pos, a.in_w, a.magic_w, ho, wo);
                 const int h = ho * a.stride - (a.taps_r >> 1), w = wo * a.stride - (a.taps_s >> 1); // of tap (0, 0)
-                voff[j] = (uint32_t)((h * a.in_w + w) * a.batch + b) * 2u; // below zero for some: the sum with an inner tap's id is not
+                voff[j] = (((uint32_t)h * a.in_w + w) * a.batch + b) * 2u; // below zero for some: the sum with an inner tap's id is not
                 auto bits = [](int lo, int hi) { return ((1u << max(hi, 0)) - 1u) & ~((1u << max(lo, 0)) - 1u); };
                 const uint32_t cols = bits(-w, min(a.taps_s, a.in_w - w));
                 const uint32_t rows = a.row_bits & bits(-h * a.taps_s, min(a.taps_r, a.in_h - h) * a.taps_s);
