@@ -207,7 +207,7 @@ int main(int argc, char** argv)
         q.kept_per_panel = (double)v[5] / (l.F / l.V);
         ConvPatchPlan p{};
         if (!conv_patch_plan(q, &p)) return 1;
-        printf("%d %d %d %d %d %d\n", conv_patch_unit_rows(l.V), p.col_blocks, p.waves, p.panels_per_wave, p.ksplit, p.chunks);
+        printf("%d %d %d %d %d %d %d\n", conv_patch_unit_rows(l.V), p.col_blocks, p.waves, p.panels_per_wave, p.ksplit, p.chunks, p.deep);
         return 0;
     }
     const int bad = reads_stay_inside() + orders_follow_the_rule() + plans_keep_to_held_shapes();
