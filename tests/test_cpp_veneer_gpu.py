@@ -41,6 +41,17 @@ def test_reference_example_flows(torch_gpu):
     assert out.count("Passed") == 7 and "Failed" not in out
 
 
+@pytest.mark.gpu
+def test_batch_innermost_every_cut(torch_gpu):
+    # every kernel that gathers from a batch-innermost input, also those the library's choice takes at other sizes only
+    out = _run("test_chwb_cuts", 110)
+    passed = [l.split(":")[0] for l in out.splitlines() if l.endswith(" Passed")]
+    names = set(passed)
+    per_height = {v: sum(n.startswith("ws%dx" % v) for n in names) for v in (16, 32, 64, 128)}
+    assert per_height == {16: 3, 32: 4, 64: 5, 128: 3}
+    assert all(passed.count(n) >= 8 for n in names) and "Failed" not in out
+
+
 BENCH = os.path.join(ROOT, "shflbw_sparse_nn_amd", "block_sparse", "benchmark")
 
 

@@ -1,5 +1,6 @@
-"""The batch-innermost convolution (C-H-W-B in, F-H-W-B out): the launch that gathers from the input itself, at the edges of
-its rule (31 taps, overlapping tensors) and of its tiles, bit for bit on integer data against the oracle."""
+"""The batch-innermost convolution (C-H-W-B in, F-H-W-B out): the launch that gathers from the input itself, in the cuts that the
+library takes, at the edges of its rule (31 taps, overlapping tensors), bit for bit on integer data against the oracle.  Its
+kernels, each by name: tests/cpp/test_chwb_cuts.cc."""
 import numpy as np
 import pytest
 
@@ -14,10 +15,10 @@ pytestmark = pytest.mark.gpu
     (8, 9, 40, 3, 32, 1, 31, 1, 32, 0.5, False),     # as many taps as a lane keeps bits for
     (8, 9, 17, 3, 32, 4, 8, 1, 32, 0.5, True),       # one more: planes
     (16, 11, 6, 5, 64, 7, 7, 2, 64, 0.3, True),
-    (40, 13, 7, 12, 128, 5, 5, 2, 128, 0.2, False),  # tiles of 128 columns whose pieces belong to several positions
-    (128, 14, 14, 16, 256, 3, 3, 1, 64, 0.1, False), # tiles of 512 columns
+    (40, 13, 7, 12, 128, 5, 5, 2, 128, 0.2, False),  # tiles whose pieces belong to several positions
+    (128, 14, 14, 16, 256, 3, 3, 1, 64, 0.1, False),
     (64, 14, 14, 9, 256, 3, 3, 3, 32, 0.3, False),   # tiles of 256 columns
-    (24, 30, 30, 7, 640, 2, 4, 1, 64, 0.2, False),   # even extents, a last tile of 96 columns
+    (24, 30, 30, 7, 640, 2, 4, 1, 64, 0.2, False),   # even extents, a ragged last tile
     (104, 15, 15, 4, 48, 1, 1, 2, 16, 0.9, False),
     (8, 5, 6, 70, 64, 3, 1, 2, 32, 0.0, False),      # panels that keep next to nothing
 ])
