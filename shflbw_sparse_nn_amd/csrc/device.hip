@@ -1624,7 +1624,7 @@ static const char* const g_spconv_forms[FORM_COUNT] = {
     "direct",                 // 1: one kernel, im2col gather from NHWC in the tile loads
     "bplanes+spmm+transpose", // 2: NHWC tensors, planes and result with the batch innermost (batch a multiple of 8): three launches
     "bplanes-fused",          // 3: the steps of form 2 in one persistent launch, every XCD on its own columns
-    "chwb-planes+spmm",       // 4: the reference's batch-innermost tensors (shflbw_spconv_init_chwb only): one launch over the input; padded copy and SpMM where its ids do not fit
+    "chwb",                   // 4: the reference's batch-innermost tensors (shflbw_spconv_init_chwb only): one launch over the input; padded copy and SpMM where its ids do not fit
     "patch",                  // 5: one launch, the input patch of a workgroup's pixels in LDS, channel-major
 };
 

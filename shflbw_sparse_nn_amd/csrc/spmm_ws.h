@@ -177,8 +177,8 @@ __device__ __forceinline__ void ws_consumer(const SpmmLaunchArgs& a, uint32_t ld
     // Whole lines: with an even number of 32-column blocks, 16 rows of two neighbouring blocks are staged at a time
     // (rows of 128 bytes + 16) and eight lanes store one 128-byte line of a row: half as many write requests to the
     // L2s as with 64-byte row segments (4096 x 4096 x 4096, density 0.1: -2 %, -11 % at N = 16384, where every epilogue
-    // runs beside other workgroups' gathers).  Not where two workgroups share a compute unit (128 registers per wave: it
-    // spills).
+    // runs beside other workgroups' gathers).  The variants whose workgroups share a compute unit have room for it too: none
+    // spills with its 128 registers per wave.
     constexpr bool LINES = SHFLBW_EPI_LINES && NB % 2 == 0 && 16 * (128 + 16) <= Cfg::EPI_WAVE_BYTES;
     constexpr int CIT = LINES ? 2 : NIT;                            // pieces of C per epilogue step
     constexpr int STEPS = LINES ? MB * NB : MB * NB * (32 / ER);    // epilogue steps of a tile
@@ -694,8 +694,8 @@ __device__ __forceinline__ void ws_producer(const Args& a, uint32_t lds0, int la
     // A wave issues roughly one instruction every five to six cycles, whatever the kind, and
     // the workgroup advances one stage per producer round: the round is kept to the copies,
     // one multiply and one add per gathered row, and a handful of scalar bookkeeping.
-    //  * addresses are a 64-bit base in scalar registers plus a 32-bit per-lane offset; the
-    //    row offset id * row bytes goes into the lane offset (B must be smaller than 4 GiB);
+    //  * rows are addressed by 32-bit lane offsets into a buffer descriptor in scalar registers; the
+    //    row offset id * row bytes goes into the lane offset (B and one row more: less than 4 GiB);
     //  * the stream is walked group by group (64 slots = up to four stages of one tile); the
     //    16 ids a producer needs for the next group are fetched by one scalar load at the
     //    start of the current group and first touched when that group is finished, several

@@ -1,4 +1,4 @@
-"""D from 24 MB on whose rows do not start at whole lines is stored without device scope (store_merges_lines): both sides of the
+"""D from 24 MB on whose rows do not start at whole lines is merged in the L2 (result_store_mode): both sides of the
 rule, every block height, with and without C, rows and a base that start inside a line, against exact integer products."""
 import numpy as np
 import pytest
