@@ -153,87 +153,121 @@ static bool spmm_variant_splits(const SpmmVariant* v) { return v && strncmp(v->n
 // few columns and holds to the same bound
 static bool spmm_variant_offsets32(const SpmmVariant* v) { return v && (v->name[0] == 'w' || spmm_variant_splits(v)); }
 
-// Tile choice when the caller does not force one: the variant with the least estimated time.  The weights are us, a fit per variant
-// (7-15 % rms) to 1390 problems drawn over 512-33792 rows, 64-8192 columns of A, 8-16384 columns of B and densities of 0.02-0.5,
-// every variant of their block height timed over three sets of operands in turn.  Over those the estimate's choice takes 1.01 (block
-// heights 16 and 128) and 1.02 times (32, 64) the fastest variant's time on average.  The lines drawn by hand
-// before it - 128-column tiles while they do not outnumber the compute units, 256-column ones while the widest would fill at most
-// half of them, bounds for the slab and the split form - took 1.15, 1.10, 1.07 and 1.02 times, 3.3 at worst: above all many
-// panels over few columns ran on 512-column tiles (29632 x 761 x 64, density 0.47, block height 64: 16.1 us; 128-column tiles, two
-// workgroups per compute unit, 7.0), and block height 16 had no other width (6592 x 4295 x 544, density 0.03: 14.4; 256 columns 9.7).
+// Tile choice when the caller does not force one: the variant with the least estimated time.  The weights are us, fitted to 13 620 problems
+// (profiles/spmm_estimate_fit.py draws, times and fits them: 64-65536 rows, 64-16384 columns of A, 8-131072 of B, densities of 0.02-0.5,
+// up to four times the work of 8192 x 4096 x 16384 at block height 128, a fifth of them with a C term; every variant of their block
+// height timed over three sets of operands in turn), so that the variant with the least estimate takes little longer than the
+// fastest one; no weight says what its part costs by itself.  Over 4620 problems drawn and timed after the fit the choice takes
+// 1.009 times the fastest variant's time (geometric mean), more than 1.1 times on 86.
+// Before: a least-squares fit to 1390 problems up to the work of the largest case, with one D term however D is stored and the
+// mean number of tiles for long panels that two workgroups of a compute unit share: 1.023 times, more than 1.1 times on 384.  It took
+// narrow tiles where D is large (12416 x 69 x 63096, block height 128, density 0.05: 794 us, now 553; 5952 x 744 x 64552, 64: 340 and 299) and where
+// long panels fill a few compute units twice (5472 x 3207 x 368, 32, 0.37: 19.2 and 15.7).  The lines drawn by hand before that
+// (bounds on tiles, columns and kept vectors) take 1.09 times on average and 2.9 at worst, above all for many panels over few
+// columns on 512-column tiles (29632 x 761 x 64, density 0.47, block height 64: 16.1 us; 128-column tiles 7.0).
 //
-//  role-split: base + tiles of a compute unit * (tile + stage * stages of 32 kept vectors) + d * (D at 5 TB/s); the tiles of a compute
-//    unit are `whole` parts the rounded-up number and the rest the mean, and where two workgroups share it a pair of tiles
-//    takes as long as one and (tile2 + stage2 * stages);
-//  slab: base + rounds * (slab + K / 1000 * row + panels of a wave * batches of 32 vectors * batch) + d * ...;
-//  split: base + rounds * (tile + steps of a wave * (step + (64 columns: wide_step))) + d * ...
-//  With a C term c * (C at 5 TB/s) + c_tile * tiles (panels of a wave) more, fitted to 670 problems with one (9-16 % rms).  The variants differ in
-//  what C costs them: the slab form and the short rings read it in the epilogue.  Chosen as without it: 1.027 times the fastest variant on
-//  average, 1.36 at worst, with it 1.016 and 1.25 (24576 x 85 x 1848, block height 128, density 0.31: 64 us with 128 columns, 53 with 256;
-//  10464 x 89 x 2424, block height 16: slab 36, role-split 31); on 180 others 1.033 on average, now 1.020.
-struct SpmmEstimate {
-    const char* name;
-    int tiles; // 0; 1: only while its tiles do not outnumber the compute units; 2: only where they do
-    float base, tile, stage, whole, d, tile2, stage2, c, c_tile;
+//  role-split: base + tiles of a compute unit * (tile + stage * stages of 32 kept vectors) + D.  The tiles of a compute unit are
+//    their number rounded up.  Where two workgroups share one, a second tile beside the first counts as second.tile and second.stage,
+//    its presence costs second.start, and per tile, other than per stage, the mean number counts;
+//  slab: base + rounds * (slab + K / 1000 * row + panels of a wave * (panel + batches of 32 vectors * batch)) + D;
+//  split: base + rounds * (tile + steps of a wave * (step + (64 columns: wide_step))) + D;
+//  D: its bytes at 5 TB/s times the weight of the way it is stored (by StoreMode), and what exceeds the Infinity Cache times `beyond`.
+//  With a C term c * (C at 5 TB/s) and c_tile for every tile (round of the split form, panel of a wave) more.
+struct StoreWeights {
+    float by_mode[3], beyond;
+    double of(StoreMode mode, double t_d) const { return by_mode[mode] * t_d + beyond * std::max(0.0, t_d - 53.7); }
 };
-static const SpmmEstimate g_estimates[] = {
-    // The rings of three and four stages that let two workgroups share a compute unit are too short for one alone (128 columns
-    // 1.00-1.15 times, 256 columns up to 1.9 times the six stages' time, the more the longer the panels), and with more tiles than
-    // compute units the 128-column ones were ahead throughout (0.78-0.98 times).
-    {"ws16x128x4c4p_k32_s4", 0, 2.99f, 0.688f, 0.273f, 1.f, 0.442f, 0.f, 0.f, 0.744f, 0.256f},
-    {"ws16x64x2c4p_k32_s6", 0, 2.98f, 0.851f, 0.13f, 0.277f, 0.f, 0.f, 0.083f, 0.977f, 0.f},
-    {"ws16x64x4c4p_k32_s4", 0, 3.06f, 0.7f, 0.158f, 0.149f, 0.329f, 0.f, 0.171f, 0.884f, 0.f},
-    {"ws32x128x4c4p_k32_s4", 0, 2.56f, 1.05f, 0.295f, 1.f, 0.584f, 0.f, 0.f, 0.874f, 0.612f},
-    {"ws32x32x4c4p_k32_s6", 0, 2.94f, 0.873f, 0.124f, 0.137f, 0.318f, 0.f, 0.137f, 1.09f, 0.f},
-    {"ws32x64x4c4p_k32_s3", 2, 2.49f, 0.f, 0.399f, 0.876f, 0.399f, 1.02f, 0.054f, 1.16f, 0.0154f},
-    {"ws32x64x4c4p_k32_s6", 0, 2.86f, 0.756f, 0.188f, 0.773f, 0.531f, 0.f, 0.f, 0.802f, 0.203f},
-    {"ws64x128x4c4p_k32_s4", 0, 2.15f, 1.93f, 0.355f, 1.f, 0.653f, 0.f, 0.f, 0.806f, 1.27f},
-    {"ws64x32x4c4p_k32_s4", 2, 2.65f, 0.875f, 0.164f, 0.275f, 0.558f, 0.f, 0.257f, 1.22f, 0.f},
-    {"ws64x32x4c4p_k32_s6", 1, 3.16f, 0.451f, 0.173f, 0.966f, 0.872f, 0.f, 0.f, 0.f, 0.00842f},
-    {"ws64x64x4c4p_k32_s3", 2, 2.0f, 1.67f, 0.288f, 0.353f, 0.457f, 0.f, 0.421f, 0.94f, 0.441f},
-    {"ws64x64x4c4p_k32_s6", 0, 2.65f, 1.06f, 0.224f, 1.f, 0.59f, 0.f, 0.f, 0.661f, 0.818f},
-    {"ws128x32x4c4p_k32_s4", 2, 3.17f, 0.967f, 0.366f, 0.334f, 0.156f, 1.61f, 0.302f, 1.33f, 0.f},
-    {"ws128x32x4c4p_k32_s6", 1, 2.74f, 1.02f, 0.196f, 1.f, 0.712f, 0.f, 0.f, 0.468f, 0.676f},
-    {"ws128x64x4c4p_k32_s6", 0, 2.13f, 2.13f, 0.307f, 1.f, 0.521f, 0.f, 0.f, 0.745f, 1.51f},
-    // base, slab, row, -, batch, d, -, c, c_panel
-    {"slab16x64", 0, 2.41f, 1.33f, 0.561f, 0.f, 0.132f, 0.878f, 0.f, 1.17f, 0.f},
-    {"slab32x64", 0, 2.0f, 1.71f, 0.765f, 0.f, 0.181f, 0.971f, 0.f, 1.12f, 0.0686f},
-    // base, tile, step, wide_step, -, d, -, c, -
-    {"split16x32", 0, 2.45f, 1.1f, 0.901f, 0.f, 0.f, 0.007f, 0.f, 2.94f, 0.f},
-    {"split32x32", 0, 2.46f, 1.21f, 0.641f, 0.194f, 0.f, 1.27f, 0.f, 0.911f, 0.f},
-    {"split64x32", 0, 2.52f, 1.22f, 0.586f, 0.219f, 0.f, 1.25f, 0.f, 0.999f, 0.f},
-    {"split128x32", 0, 2.43f, 1.28f, 0.618f, 0.254f, 0.f, 1.03f, 0.f, 0.994f, 0.f},
+struct SecondTile {
+    float start, tile, stage;
+    double tiles(double mean) const { return mean <= 2 ? 1 + (mean - 1) * tile : mean / 2 * (1 + tile); }
+    double stages(double n) const { return std::floor(n / 2) * (1 + stage) + n - 2 * std::floor(n / 2); }
+};
+struct RoleSplitEstimate {
+    const char* name;
+    float base, tile, stage;
+    StoreWeights d;
+    float c, c_tile;
+    SecondTile second; // variants with two workgroups per compute unit only
+};
+struct SlabEstimate {
+    const char* name;
+    float base, slab, row, panel, batch;
+    StoreWeights d;
+    float c, c_panel;
+};
+struct SplitEstimate {
+    const char* name;
+    float base, tile, step, wide_step, d, c, c_round;
+};
+static const RoleSplitEstimate g_role_split_estimates[] = {
+    {"ws16x128x4c4p_k32_s4", 2.21f, 0.746f, 0.323f, {0.967f, 0.677f, 0.f, 0.f}, 0.607f, 0.277f},
+    {"ws16x64x4c4p_k32_s4", 1.44f, 1.02f, 0.204f, {0.0306f, 0.f, 0.f, 0.591f}, 0.f, 0.373f, {0.297f, 0.28f, 0.79f}},
+    {"ws16x64x2c4p_k32_s6", 1.6f, 0.701f, 0.167f, {0.f, 0.f, 0.f, 0.f}, 0.f, 0.279f, {0.413f, 0.425f, 0.395f}},
+    {"ws32x128x4c4p_k32_s4", 1.74f, 1.22f, 0.355f, {0.962f, 0.727f, 0.0583f, 0.18f}, 0.627f, 1.02f},
+    {"ws32x64x4c4p_k32_s3", 1.21f, 1.19f, 0.409f, {0.13f, 0.203f, 0.f, 2.84f}, 0.434f, 0.573f, {0.114f, 0.316f, 0.436f}},
+    {"ws32x64x4c4p_k32_s6", 1.11f, 1.43f, 0.223f, {0.00974f, 0.f, 0.f, 0.f}, 0.255f, 0.602f},
+    {"ws32x32x4c4p_k32_s6", 1.29f, 1.06f, 0.171f, {0.0221f, 0.f, 0.f, 0.704f}, 0.609f, 0.287f, {0.32f, 0.203f, 0.502f}},
+    {"ws64x128x4c4p_k32_s4", 1.82f, 2.09f, 0.433f, {0.503f, 0.566f, 0.286f, 0.342f}, 0.939f, 0.813f},
+    {"ws64x64x4c4p_k32_s3", 0.f, 2.09f, 0.557f, {0.56f, 0.578f, 0.0858f, 1.18f}, 0.692f, 1.55f, {0.857f, 0.f, 0.f}},
+    {"ws64x64x4c4p_k32_s6", 1.58f, 1.33f, 0.263f, {0.454f, 0.758f, 0.222f, 0.307f}, 0.144f, 1.72f},
+    {"ws64x32x4c4p_k32_s4", 1.22f, 0.464f, 0.25f, {0.802f, 0.959f, 0.603f, 0.922f}, 0.603f, 0.678f, {0.853f, 0.418f, 0.334f}},
+    {"ws64x32x4c4p_k32_s6", 1.12f, 1.48f, 0.195f, {0.0511f, 0.f, 0.f, 0.09f}, 0.307f, 0.546f},
+    {"ws128x64x4c4p_k32_s6", 1.52f, 2.51f, 0.342f, {0.355f, 0.469f, 0.395f, 0.286f}, 0.711f, 1.26f},
+    {"ws128x32x4c4p_k32_s4", 0.f, 2.96f, 0.276f, {0.418f, 0.397f, 0.383f, 1.28f}, 1.14f, 0.82f, {1.1f, 0.f, 0.66f}},
+    {"ws128x32x4c4p_k32_s6", 1.42f, 2.07f, 0.24f, {0.322f, 0.323f, 0.f, 0.537f}, 0.37f, 0.99f},
+};
+static const SlabEstimate g_slab_estimates[] = {
+    {"slab16x64", 0.0239f, 2.81f, 1.54f, 0.f, 0.186f, {0.824f, 0.761f, 0.584f, 0.104f}, 0.835f, 0.235f},
+    {"slab32x64", 2.03f, 0.681f, 1.84f, 0.604f, 0.216f, {0.633f, 0.527f, 0.357f, 0.166f}, 1.12f, 0.231f},
+};
+static const SplitEstimate g_split_estimates[] = {
+    {"split16x32", 0.494f, 1.68f, 0.846f, 0.2f, 3.68f, 1.28f, 0.189f},
+    {"split32x32", 0.693f, 2.39f, 0.574f, 0.297f, 0.66f, 0.06f, 0.191f},
+    {"split64x32", 1.47f, 1.6f, 0.651f, 0.47f, 0.518f, 0.f, 0.451f},
+    {"split128x32", 0.558f, 1.32f, 0.929f, 0.832f, 1.37f, 0.968f, 0.492f},
 };
 
-static double spmm_estimate(const SpmmVariant& v, const SpmmEstimate& e, bool splits, const shflbw_weight* w, int N, bool residual, int compute_units)
+static StoreMode result_store_mode(const void* D, int rows, int ldd, bool read_back);
+
+// What an estimate depends on.
+struct SpmmProblem {
+    const shflbw_weight* w;
+    int N, X, cus;
+    double vectors; // kept per panel
+    double t_d;     // D (and C) at 5 TB/s
+    bool residual;
+};
+
+static double estimate(const SpmmVariant& v, const RoleSplitEstimate& e, const SpmmProblem& q)
 {
-    const double X = w->nrow / w->brow, vectors = w->nnzb / X, t_d = 2.0 * w->nrow * N / 5e6;
-    const double cus = compute_units;
-    auto with_c = [&](double t, double tiles) { return residual ? t + e.c * t_d + e.c_tile * tiles : t; };
-    if (v.max_k > 0) {
-        const int groups = (int)(w->packed_indices.size() / 64);
-        const SlabDeal s = slab_deal(w->brow, (int)X, w->ncol, groups, (N + v.BN - 1) / v.BN, compute_units / 8 * 8);
-        return with_c(e.base + s.rounds * (e.tile + e.stage * w->ncol / 1000 + s.wave_panels * e.d * 2 * std::ceil(vectors / 64)) + e.tile2 * t_d,
-                      (double)s.rounds * s.wave_panels);
-    }
-    if (splits) { // as launch_split cuts it
-        const bool v16 = w->brow == 16;
-        const double blocks = w->nrow / (v16 ? 16 : 32);
-        const bool wide = !v16 && N > 32 && blocks * ((N + 31) / 32) > cus;
-        const double grid = std::ceil(blocks / 8) * 8 * (wide ? (N + 63) / 64 : (N + 31) / 32), waves = grid <= cus ? 16 : 8;
-        const double steps = vectors / (v16 ? 32 : 16) / waves + 0.5;
-        const double rounds = std::max(1.0, grid / (waves == 16 ? cus : 2 * cus));
-        return with_c(e.base + rounds * (e.tile + (e.stage + (wide ? e.whole : 0.f)) * steps) + e.tile2 * t_d, rounds);
-    }
-    const double per_cu = X * ((N + v.BN - 1) / v.BN) / cus, n = std::ceil(per_cu), mean = std::max(1.0, per_cu);
-    const double one = e.tile + e.stage * (vectors / 32 + 0.5);
-    double whole = n * one, rest = mean * one;
-    if (v.per_cu == 2) {
-        const double pair = one + e.tile2 + e.stage2 * (vectors / 32 + 0.5), pairs = std::floor(n / 2);
-        whole = pairs * pair + (n - 2 * pairs) * one;
-        rest = mean <= 2 ? one + (mean - 1) * (pair - one) : mean / 2 * pair;
-    }
-    return with_c(e.base + e.whole * whole + (1 - e.whole) * rest + e.d * t_d, e.whole * n + (1 - e.whole) * mean);
+    const double mean = (double)q.X * ((q.N + v.BN - 1) / v.BN) / q.cus, n = std::ceil(mean);
+    const bool two = v.per_cu == 2;
+    const double tiles = two ? e.second.tiles(std::max(1.0, mean)) : n, stages = two ? e.second.stages(n) : n;
+    const double t = e.base + e.tile * tiles + e.stage * (q.vectors / 32 + 0.5) * stages + (two && n >= 2 ? e.second.start : 0.f) +
+                     e.d.of(result_store_mode(nullptr, q.w->nrow, q.N, false), q.t_d);
+    return q.residual ? t + e.c * q.t_d + e.c_tile * tiles : t;
+}
+
+static double estimate(const SpmmVariant& v, const SlabEstimate& e, const SpmmProblem& q)
+{
+    const SlabDeal s = slab_deal(q.w->brow, q.X, q.w->ncol, (int)(q.w->packed_indices.size() / 64), (q.N + v.BN - 1) / v.BN, q.cus / 8 * 8);
+    const double panels = (double)s.rounds * s.wave_panels;
+    const double t = e.base + s.rounds * (e.slab + e.row * q.w->ncol / 1000) + panels * (e.panel + e.batch * 2 * std::ceil(q.vectors / 64)) +
+                     e.d.of(slab_store_mode(nullptr, q.w->nrow, q.N), q.t_d);
+    return q.residual ? t + e.c * q.t_d + e.c_panel * panels : t;
+}
+
+static double estimate(const SpmmVariant&, const SplitEstimate& e, const SpmmProblem& q) // as launch_split cuts it
+{
+    const bool v16 = q.w->brow == 16;
+    const double blocks = q.w->nrow / (v16 ? 16 : 32);
+    const bool wide = !v16 && q.N > 32 && blocks * ((q.N + 31) / 32) > q.cus;
+    const double grid = std::ceil(blocks / 8) * 8 * (wide ? (q.N + 63) / 64 : (q.N + 31) / 32);
+    const int waves = grid <= q.cus ? 16 : 8;
+    const double steps = q.vectors / (v16 ? 32 : 16) / waves + 0.5;
+    const double mean = std::max(1.0, grid / (waves == 16 ? q.cus : 2 * q.cus)), rounds = 0.5 * (mean + std::ceil(mean));
+    const double t = e.base + rounds * (e.tile + (e.step + (wide ? e.wide_step : 0.f)) * steps) + e.d * q.t_d;
+    return q.residual ? t + e.c * q.t_d + e.c_round * rounds : t;
 }
 
 // `spmm` false: what is multiplied are the planes of a convolution, which only the variants that gather rows by id can walk.
@@ -242,9 +276,10 @@ static int auto_spmm_variant(const shflbw_weight* w, int N, bool spmm, bool resi
     struct Candidates { // of the four block heights, found once
         struct One {
             const SpmmVariant* v;
-            const SpmmEstimate* e;
             int number;
-            bool splits;
+            const RoleSplitEstimate* role_split; // one of the three
+            const SlabEstimate* slab;
+            const SplitEstimate* split;
         };
         std::vector<One> of[4];
         Candidates()
@@ -252,22 +287,29 @@ static int auto_spmm_variant(const shflbw_weight* w, int N, bool spmm, bool resi
             for (int h = 0; h < 4; h++) {
                 int count = 0;
                 const SpmmVariant* all = find_spmm_variant(16 << h, 0, &count);
-                for (int i = 0; i < count; i++)
-                    for (const SpmmEstimate& e : g_estimates)
-                        if (strcmp(e.name, all[i].name) == 0) of[h].push_back({&all[i], &e, i, spmm_variant_splits(&all[i])});
+                for (int i = 0; i < count; i++) {
+                    for (const RoleSplitEstimate& e : g_role_split_estimates)
+                        if (strcmp(e.name, all[i].name) == 0) of[h].push_back({&all[i], i, &e, nullptr, nullptr});
+                    for (const SlabEstimate& e : g_slab_estimates)
+                        if (strcmp(e.name, all[i].name) == 0) of[h].push_back({&all[i], i, nullptr, &e, nullptr});
+                    for (const SplitEstimate& e : g_split_estimates)
+                        if (strcmp(e.name, all[i].name) == 0) of[h].push_back({&all[i], i, nullptr, nullptr, &e});
+                }
             }
         }
     };
     static const Candidates candidates;
     const int h = w->brow == 16 ? 0 : w->brow == 32 ? 1 : w->brow == 64 ? 2 : w->brow == 128 ? 3 : -1;
     if (h < 0 || w->nrow <= 0) return 0;
+    SpmmProblem q{w, N, w->nrow / w->brow, compute_units, 0, 2.0 * w->nrow * N / 5e6, residual};
+    q.vectors = (double)w->nnzb / q.X;
     int best = 0;
     double least = 0;
     for (const auto& c : candidates.of[h]) {
-        if (c.v->max_k > 0 ? !spmm || w->packed_slab.empty() || w->ncol > c.v->max_k : c.splits && (!spmm || N > 1024)) continue;
-        const bool outnumber = (long)(w->nrow / w->brow) * ((N + c.v->BN - 1) / c.v->BN) > compute_units;
-        if (c.e->tiles != 0 && outnumber != (c.e->tiles == 2)) continue;
-        const double t = spmm_estimate(*c.v, *c.e, c.splits, w, N, residual, compute_units);
+        if (!c.role_split && !spmm) continue;
+        if (c.slab && (w->packed_slab.empty() || w->ncol > c.v->max_k)) continue;
+        if (c.split && N > 1024) continue;
+        const double t = c.role_split ? estimate(*c.v, *c.role_split, q) : c.slab ? estimate(*c.v, *c.slab, q) : estimate(*c.v, *c.split, q);
         if (least == 0 || t < least) least = t, best = c.number;
     }
     return best;
@@ -880,7 +922,8 @@ int init_chwb_taps(shflbw_spconv_state* state, const shflbw_weight* f, int B, in
     }
     // The cut of the SpMM of these sizes.  With three widths by the number of tiles, and one width for block height 16, us, before / now:
     // 16 x 14 x 14 x 656 -> 32, 3 x 3, block height 16 20.4 / 11.9, 8 x 7 x 7 x 304 -> 1152, 5 x 5, 14.3 / 11.0; block height 32, 32 x 55 x 27 x
-    // 360 -> 128, 1 x 7, 20.1 / 18.5.
+    // 360 -> 128, 1 x 7, 20.1 / 18.5.  The estimate was fitted to no convolution; over 500 drawn layers, every cut timed, its choice takes
+    // 1.010 times the fastest cut's time, 1.25 at worst.
     const int variant = auto_spmm_variant(f, (int)ncols, false, false, device_compute_units());
     const SpmmVariant* v = find_spmm_variant(f->brow, variant, nullptr);
     const ConvTapsKernel* k = v ? conv_taps_kernel(v->name) : nullptr;

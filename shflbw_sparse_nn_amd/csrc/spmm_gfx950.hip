@@ -344,14 +344,7 @@ template <int V>
 static void slab_plan(SpmmLaunchArgs& b, int cus)
 {
     using Cfg = SpmmSlabCfg<V>;
-    const size_t d_bytes = (size_t)b.M * (size_t)b.ldd * 2;
-    const bool lines = (((uintptr_t)b.D | ((uintptr_t)b.ldd * 2)) & 127) == 0;
-    // As for the role-split kernels (result_store_mode).  us, through / merged / streamed, the better order of jobs each: whole lines,
-    // block height 32, density 0.2: 4096 x 1024 x 4096 17.0 / 18.1 / 17.2, 8192 x 768 x 8192 62 / 62 / 48; block height 16, 33728 x 777 x
-    // 1024 22.1 / 24.3 / 22.4, 20000 x 1000 x 6016 85 / 89 / 69.  Parts of lines: 8192 x 777 x 3000 (49 MB) 19.4 / 21.0 / 32, 33728 x 777 x
-    // 1000 (67 MB) 22.7 / 24.1 / 45, block height 32, 16384 x 800 x 2056 (67 MB) 42 / 35.5 / 49, 33728 x 1100 x 2104 136 / 123 / 121, 16:
-    // 20000 x 1000 x 6000 145 / 101 / 125.
-    b.store_mode = lines ? (d_bytes >= 96u << 20 ? STORE_STREAM : STORE_THROUGH) : d_bytes >= 64u << 20 ? STORE_MERGE : STORE_THROUGH;
+    b.store_mode = slab_store_mode(b.D, b.M, b.ldd);
     b.slab_chunks = slab_deal(V, b.X, b.K, b.groups, b.n_tiles, cus).chunks;
     // Order of the jobs.  An XCD owns T / 8 of them, side by side: by tile it reads few slabs and most of A, by chunk a part of A
     // and most of B.  The order with fewer bytes into the L2s; by chunk where parts of lines are merged, as the tiles that

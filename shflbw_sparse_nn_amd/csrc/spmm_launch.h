@@ -107,6 +107,18 @@ inline SlabDeal slab_deal(int V, int X, int K, int groups, int n_tiles, int cus)
     return best;
 }
 
+// How the slab kernel stores D, as result_store_mode for the role-split kernels.  us, through / merged / streamed, the better order of
+// jobs each: whole lines, block height 32, density 0.2: 4096 x 1024 x 4096 17.0 / 18.1 / 17.2, 8192 x 768 x 8192 62 / 62 / 48; block height 16,
+// 33728 x 777 x 1024 22.1 / 24.3 / 22.4, 20000 x 1000 x 6016 85 / 89 / 69.  Parts of lines: 8192 x 777 x 3000 (49 MB) 19.4 / 21.0 / 32, 33728 x
+// 777 x 1000 (67 MB) 22.7 / 24.1 / 45, block height 32, 16384 x 800 x 2056 (67 MB) 42 / 35.5 / 49, 33728 x 1100 x 2104 136 / 123 / 121, 16:
+// 20000 x 1000 x 6000 145 / 101 / 125.
+inline StoreMode slab_store_mode(const void* D, int rows, int ldd)
+{
+    const size_t bytes = (size_t)rows * (size_t)ldd * 2;
+    if ((((uintptr_t)D | ((uintptr_t)ldd * 2)) & 127) != 0) return bytes >= 64u << 20 ? STORE_MERGE : STORE_THROUGH;
+    return bytes >= 96u << 20 ? STORE_STREAM : STORE_THROUGH;
+}
+
 // device address of the library's row of zeros on the current device (looked up once per device); null on failure
 const void* spmm_zero_row();
 
