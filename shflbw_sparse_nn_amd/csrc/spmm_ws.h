@@ -485,6 +485,8 @@ __device__ __forceinline__ void ws_consumer(const SpmmLaunchArgs& a, uint32_t ld
                 for (int mb = 0; mb < MB; mb++) epi_block(mb, T{}, F{}, mode);
             }
         };
+        // (Three sequences in one kernel, not an instance each as for the slab form: 0.92 to 1.03 times the time of a kernel with the
+        // first alone, 1.002 on average over 33 pairs of variant and problem; 1024^3, density 0.25: 4.33 against 4.25 us.)
         if (XCD_LOCAL || a.store_mode == STORE_THROUGH)
             epilogue(std::integral_constant<StoreMode, STORE_THROUGH>{});
         else if (a.store_mode == STORE_MERGE)
