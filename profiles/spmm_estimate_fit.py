@@ -5,8 +5,7 @@ g_role_split_estimates, g_slab_estimates and g_split_estimates in csrc/device.hi
     python profiles/spmm_estimate_fit.py check OUT...         the library's choice as it was when OUT was timed, against the fastest
     python profiles/spmm_estimate_fit.py fit V OUT...         weights for block height V, as rows of the tables
 
-The tables hold what `fit` gave for seeds 1000, 2000 and 3000 (without the `large` problems of the first two); the form of the estimate
-was chosen on seed 4000, and seeds 5000 and 6000 were timed with the library that holds the tables.
+The tables hold what `fit` gave for seeds 1000, 2000 and 3000; seeds from 6000 on were timed with the library that holds the tables.
 """
 import json
 import math
@@ -137,7 +136,9 @@ def features(p, name):
     V, N, X = p["V"], p["N"], p["M"] // p["V"]
     vectors, t_d, c, kind = p["nnzb"] / X, 2.0 * p["M"] * N / 5e6, float(p["residual"]), kind_of(name)
     d_bytes, lines = 2 * p["M"] * N, N * 2 % 128 == 0
-    mode = (2 if d_bytes >= 96 << 20 else 0) if lines else (1 if d_bytes >= (64 if kind == "slab" else 24) << 20 else 0)
+    all_bytes = d_bytes * (2 if p["residual"] else 1) + 2 * p["K"] * N
+    half_lines = re.match(r"ws(32|64|128)x32x4c", name) and d_bytes >= 24 << 20
+    mode = (2 if d_bytes >= 96 << 20 else 0) if lines else (1 if all_bytes >= 80 << 20 or half_lines else 0)
     D = [t_d * (mode == m) for m in range(3)] + [max(0.0, t_d - 53.7)]
     if kind == "slab":
         batches = 2 * math.ceil(vectors / 64)

@@ -227,7 +227,9 @@ static const SplitEstimate g_split_estimates[] = {
     {"split128x32", 0.558f, 1.32f, 0.929f, 0.832f, 1.37f, 0.968f, 0.492f},
 };
 
-static StoreMode result_store_mode(const void* D, int rows, int ldd, bool read_back);
+static StoreMode result_store_mode(const void* D, int rows, int ldd, size_t others, bool narrow, bool read_back);
+// role-split tiles of 128 columns, but for block height 16, are stored by half lines (ws_consumer)
+static bool stores_half_lines(int brow, int tile_cols) { return brow != 16 && tile_cols == 128; }
 
 // What an estimate depends on.
 struct SpmmProblem {
@@ -236,6 +238,7 @@ struct SpmmProblem {
     double vectors; // kept per panel
     double t_d;     // D (and C) at 5 TB/s
     bool residual;
+    size_t others;  // bytes of B and C
 };
 
 static double estimate(const SpmmVariant& v, const RoleSplitEstimate& e, const SpmmProblem& q)
@@ -244,7 +247,7 @@ static double estimate(const SpmmVariant& v, const RoleSplitEstimate& e, const S
     const bool two = v.per_cu == 2;
     const double tiles = two ? e.second.tiles(std::max(1.0, mean)) : n, stages = two ? e.second.stages(n) : n;
     const double t = e.base + e.tile * tiles + e.stage * (q.vectors / 32 + 0.5) * stages + (two && n >= 2 ? e.second.start : 0.f) +
-                     e.d.of(result_store_mode(nullptr, q.w->nrow, q.N, false), q.t_d);
+                     e.d.of(result_store_mode(nullptr, q.w->nrow, q.N, q.others, stores_half_lines(q.w->brow, v.BN), false), q.t_d);
     return q.residual ? t + e.c * q.t_d + e.c_tile * tiles : t;
 }
 
@@ -253,7 +256,7 @@ static double estimate(const SpmmVariant& v, const SlabEstimate& e, const SpmmPr
     const SlabDeal s = slab_deal(q.w->brow, q.X, q.w->ncol, (int)(q.w->packed_indices.size() / 64), (q.N + v.BN - 1) / v.BN, q.cus / 8 * 8);
     const double panels = (double)s.rounds * s.wave_panels;
     const double t = e.base + s.rounds * (e.slab + e.row * q.w->ncol / 1000) + panels * (e.panel + e.batch * 2 * std::ceil(q.vectors / 64)) +
-                     e.d.of(slab_store_mode(nullptr, q.w->nrow, q.N), q.t_d);
+                     e.d.of(slab_store_mode(nullptr, q.w->nrow, q.N, q.others), q.t_d);
     return q.residual ? t + e.c * q.t_d + e.c_panel * panels : t;
 }
 
@@ -301,7 +304,7 @@ static int auto_spmm_variant(const shflbw_weight* w, int N, bool spmm, bool resi
     static const Candidates candidates;
     const int h = w->brow == 16 ? 0 : w->brow == 32 ? 1 : w->brow == 64 ? 2 : w->brow == 128 ? 3 : -1;
     if (h < 0 || w->nrow <= 0) return 0;
-    SpmmProblem q{w, N, w->nrow / w->brow, compute_units, 0, 2.0 * w->nrow * N / 5e6, residual};
+    SpmmProblem q{w, N, w->nrow / w->brow, compute_units, 0, 2.0 * w->nrow * N / 5e6, residual, ((size_t)w->ncol + (residual ? w->nrow : 0)) * N * 2};
     q.vectors = (double)w->nnzb / q.X;
     int best = 0;
     double least = 0;
@@ -359,21 +362,23 @@ static int plane_form_geometry(const shflbw_weight* f, int B, int H, int W, int 
     return SHFLBW_OK;
 }
 
-// How the role-split kernels store D.
+// How the role-split kernels store D.  `others`: bytes of B and C.
 //  * Rows that do not start at whole lines: every line is written in parts, by neighbouring store instructions, and each part
-//    written through is a write to memory of its own.  Merged in the L2 once D is three quarters of the eight L2s, as what is
-//    dirty there when the launch ends is written back then.  us, through / merged, block height 64, K = 1640, density 0.1:
-//    4096 x 1000 6.3 / 6.9, 4096 x 2008 10.4 / 10.9, 1024 x 8008 9.8 / 10.3 (16 MB); 4096 x 4008 15.5 / 15.2, 16384 x 1000 16.0 / 15.1
-//    (33 MB); 4096 x 8008 38.7 / 32.1; block height 128, 4096 x 1640 x 16376, density 0.05: 88.5 / 63.5.
+//    written through is a write of its own to the Infinity Cache, or to memory where that does not hold the line.  Merged in the L2
+//    where it will not: where three such problems in turn, 3 * (B + C + D), do not fit its 256 MB.  Merged / through, 600 drawn
+//    problems with D of 8 to 300 MB (955 pairs with a variant without C, 397 with): 0.92 by this rule, 6 pairs above 1.05; with
+//    the line at D >= 24 MB, as before, 0.92 and 85, up to 1.22 (32 x 1184 x 279 x 13792, 33 MB, short panels: 9.8 us through, 12.0).
+//    Narrow tiles, whose stores are half lines, from 24 MB on (0.92 below the other line).
 //  * Whole lines: streamed from 96 MB on, if nothing reads D back at once; smaller results, also three of them in turn, stay in
 //    the Infinity Cache.  us, through / streamed, density 0.1, block height 64, K = 1640 or 2048: 16384 x 1024 12.5 / 12.9 (33 MB),
 //    6144 x 4096 30.8 / 30.3 (50 MB), 16384 x 2560 28.6 / 28.5, 16384 x 2816 34.3 / 33.0 (92 MB), 8192 x 6400 45 / 40, 8192 x 8192 58 / 50;
 //    block height 128: 16384 x 2048 23.5 / 26.0 (67 MB), 16384 x 2816 35.3 / 37.1, 8192 x 6400 74 / 69, 4096 x 16384 65 / 52; 16:
 //    16384 x 4096 110 / 89.  Merged: as written through for large D, 4096^3 21 / 25.
-static StoreMode result_store_mode(const void* D, int rows, int ldd, bool read_back)
+static StoreMode result_store_mode(const void* D, int rows, int ldd, size_t others, bool narrow, bool read_back)
 {
     const size_t bytes = (size_t)rows * (size_t)ldd * 2;
-    if ((((uintptr_t)D | ((uintptr_t)ldd * 2)) & 127) != 0) return bytes >= 24u << 20 ? STORE_MERGE : STORE_THROUGH;
+    if ((((uintptr_t)D | ((uintptr_t)ldd * 2)) & 127) != 0)
+        return bytes + others >= STORE_MERGE_BYTES || (narrow && bytes >= 24u << 20) ? STORE_MERGE : STORE_THROUGH;
     return bytes >= 96u << 20 && !read_back ? STORE_STREAM : STORE_THROUGH;
 }
 
@@ -403,7 +408,8 @@ static void fill_spmm_launch_args(const shflbw_spmm_state* state, int BN, SpmmLa
     a.beta = state->args.beta;
     a.num_cus = device_compute_units();
     a.ldd = a.N;
-    a.store_mode = result_store_mode(a.D, a.M, a.ldd, a.ldb_bytes != a.N * 2); // (planes: the layout kernel behind it reads D)
+    a.store_mode = result_store_mode(a.D, a.M, a.ldd, bytes_of_b_and_c(a), stores_half_lines(state->brow, BN),
+                                     a.ldb_bytes != a.N * 2); // (planes: the layout kernel behind it reads D)
     a.dmap_row = a.dmap_valid = 0, a.dmap_magic = 0;
     // rows of B one column tile can touch: above about 2.5 MB they do not stay in the 4 MB L2 of an XCD
     // from one round of tiles to the next, and alternating the direction of the walk pays (measured:
@@ -1486,7 +1492,7 @@ int shflbw_spconv_exec(const shflbw_spconv_state* state, void* stream)
             ChwbTapArgs t;
             fill_spmm_launch_args(&state->spmm, v->BN, &t);
             t.B = a.in;
-            t.store_mode = result_store_mode(t.D, t.M, t.ldd, false);
+            t.store_mode = result_store_mode(t.D, t.M, t.ldd, bytes_of_b_and_c(t), stores_half_lines(state->brow, v->BN), false);
             t.alternate = 0;
             t.batch = a.B, t.in_h = a.H, t.in_w = a.W;
             t.taps_r = a.R, t.taps_s = a.S, t.stride = (int)chwb_stride(a.H, a.W, a.R, a.S, a.stride);
@@ -1510,7 +1516,7 @@ int shflbw_spconv_exec(const shflbw_spconv_state* state, void* stream)
         fill_spmm_launch_args(&state->spmm, k->BN, &m);
         m.alternate = 0;
         m.ldd = a.Ho * a.Wo * a.B;                  // a row of the result: one filter, Ho x Wo x B values
-        m.store_mode = result_store_mode(m.D, m.M, m.ldd, nhwc);
+        m.store_mode = result_store_mode(m.D, m.M, m.ldd, bytes_of_b_and_c(m), stores_half_lines(state->brow, k->BN), nhwc);
         m.dmap_row = state->plane_cols * a.B;       // columns of the GEMM per row of the padded output grid
         m.dmap_valid = a.Wo * a.B;                  // ... of which the first Wo x B are output values
         m.dmap_magic = udiv_magic(m.dmap_row);

@@ -344,7 +344,7 @@ template <int V>
 static void slab_plan(SpmmLaunchArgs& b, int cus)
 {
     using Cfg = SpmmSlabCfg<V>;
-    b.store_mode = slab_store_mode(b.D, b.M, b.ldd);
+    b.store_mode = slab_store_mode(b.D, b.M, b.ldd, bytes_of_b_and_c(b));
     b.slab_chunks = slab_deal(V, b.X, b.K, b.groups, b.n_tiles, cus).chunks;
     // Order of the jobs.  An XCD owns T / 8 of them, side by side: by tile it reads few slabs and most of A, by chunk a part of A
     // and most of B.  The order with fewer bytes into the L2s; by chunk where parts of lines are merged, as the tiles that

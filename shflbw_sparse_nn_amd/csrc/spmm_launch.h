@@ -107,15 +107,19 @@ inline SlabDeal slab_deal(int V, int X, int K, int groups, int n_tiles, int cus)
     return best;
 }
 
+// Bytes of B, C and D from which on three problems in turn leave the Infinity Cache (256 MB).
+constexpr size_t STORE_MERGE_BYTES = 80u << 20;
+inline size_t bytes_of_b_and_c(const SpmmLaunchArgs& a) { return (size_t)a.K * a.ldb_bytes + (a.beta != 0.f ? (size_t)a.M * a.ldd * 2 : 0); }
+
 // How the slab kernel stores D, as result_store_mode for the role-split kernels.  us, through / merged / streamed, the better order of
 // jobs each: whole lines, block height 32, density 0.2: 4096 x 1024 x 4096 17.0 / 18.1 / 17.2, 8192 x 768 x 8192 62 / 62 / 48; block height 16,
-// 33728 x 777 x 1024 22.1 / 24.3 / 22.4, 20000 x 1000 x 6016 85 / 89 / 69.  Parts of lines: 8192 x 777 x 3000 (49 MB) 19.4 / 21.0 / 32, 33728 x
-// 777 x 1000 (67 MB) 22.7 / 24.1 / 45, block height 32, 16384 x 800 x 2056 (67 MB) 42 / 35.5 / 49, 33728 x 1100 x 2104 136 / 123 / 121, 16:
-// 20000 x 1000 x 6000 145 / 101 / 125.
-inline StoreMode slab_store_mode(const void* D, int rows, int ldd)
+// 33728 x 777 x 1024 22.1 / 24.3 / 22.4, 20000 x 1000 x 6016 85 / 89 / 69.  Parts of lines: 8192 x 777 x 3000 (49 MB) 19.4 / 21.0 / 32, block
+// height 32, 33728 x 1100 x 2104 136 / 123 / 121, 16: 20000 x 1000 x 6000 145 / 101 / 125; merged / through over 191 drawn problems: 0.88 by
+// this rule, 1.02 at worst, with the line at D >= 64 MB, as before, 0.89 and 1.15 (16592 x 76 x 2848, block height 16, 95 MB: 21.7 and 24.1 us).
+inline StoreMode slab_store_mode(const void* D, int rows, int ldd, size_t others)
 {
     const size_t bytes = (size_t)rows * (size_t)ldd * 2;
-    if ((((uintptr_t)D | ((uintptr_t)ldd * 2)) & 127) != 0) return bytes >= 64u << 20 ? STORE_MERGE : STORE_THROUGH;
+    if ((((uintptr_t)D | ((uintptr_t)ldd * 2)) & 127) != 0) return bytes + others >= STORE_MERGE_BYTES ? STORE_MERGE : STORE_THROUGH;
     return bytes >= 96u << 20 ? STORE_STREAM : STORE_THROUGH;
 }
 

@@ -1,5 +1,6 @@
-"""D from 24 MB on whose rows do not start at whole lines is merged in the L2 (result_store_mode): both sides of the
-rule, every block height, with and without C, rows and a base that start inside a line, against exact integer products."""
+"""D whose rows do not start at whole lines is merged in the L2 where B, C and D are 80 MiB or more, under narrow tiles where D is 24 MiB
+(result_store_mode): both sides of the rule, every block height, with and without C, rows and a base that start inside a line,
+against exact integer products."""
 import numpy as np
 import pytest
 
@@ -10,10 +11,14 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("V", [16, 32, 64, 128])
 @pytest.mark.parametrize("M,N,offset,residual", [
-    (4096, 3080, 0, False),   # 25.2 MB, rows start inside a line
+    (4096, 3080, 0, False),   # D of 25.2 MB, rows start inside a line: merged under narrow tiles
     (4096, 3080, 0, True),
     (4096, 2920, 0, False),   # 23.9 MB: written through
     (4096, 3136, 8, False),   # rows of whole lines from a base that is not at one
+    (4096, 8008, 0, False),   # B and D 80.9 MiB: merged under all tiles
+    (4096, 7912, 0, False),   # 79.9 MiB
+    (4096, 8064, 8, False),
+    (4096, 4616, 0, True),    # with C 82.7 MiB
     (256, 49160, 0, True),
 ])
 def test_ragged_rows(torch_gpu, V, M, N, offset, residual):

@@ -9,7 +9,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("V,M,K,N,per,residual", [
-    (16, 33728, 777, 1000, 12, False),   # A larger than B: by chunk, parts of lines merged (67 MB)
+    (16, 33728, 777, 1000, 12, False),   # A larger than B: by chunk, parts of lines, written through (67 MB)
+    (16, 33728, 777, 1304, 12, False),   # ... merged (88 MB, with B 86 MiB)
     (16, 20000, 1128, 136, 9, True),     # by chunk, written through; three column tiles, the last one of 8 columns
     (16, 8192, 384, 4096, 12, False),    # by tile, written through
     (16, 4096, 400, 12352, 5, False),    # by tile, streamed (101 MB)
