@@ -191,7 +191,8 @@ def fit(V, data):
         us[rows[name][0], j] = rows[name][2]
     best = us.min(1).values
     loss_of = torch.where(torch.isinf(us), torch.zeros_like(us), us / best[:, None] - 1).clamp(max=1.5)
-    for steps, weight, tau, lr in ((2500, 0, 1, .03), (2500, 10, .04, .03), (1200, 30, .03, .01), (1200, 60, .02, .01), (2400, 100, .015, .01)):
+    for steps, weight, tau, lr in ((2500, 0, 1, .03), (2500, 10, .04, .03), (1200, 30, .03, .01), (1200, 60, .02, .01), (2400, 100, .015, .01),
+                                   (2400, 200, .01, .01)):
         opt = torch.optim.Adam(theta.values(), lr=lr)
         for step in range(steps):
             if step == steps * 6 // 10:

@@ -153,17 +153,17 @@ static bool spmm_variant_splits(const SpmmVariant* v) { return v && strncmp(v->n
 // few columns and holds to the same bound
 static bool spmm_variant_offsets32(const SpmmVariant* v) { return v && (v->name[0] == 'w' || spmm_variant_splits(v)); }
 
-// Tile choice when the caller does not force one: the variant with the least estimated time.  The weights are us, fitted to 13 620 problems
+// Tile choice when the caller does not force one: the variant with the least estimated time.  The weights are us, fitted to 13 860 problems
 // (profiles/spmm_estimate_fit.py draws, times and fits them: 64-65536 rows, 64-16384 columns of A, 8-131072 of B, densities of 0.02-0.5,
 // up to four times the work of 8192 x 4096 x 16384 at block height 128, a fifth of them with a C term; every variant of their block
 // height timed over three sets of operands in turn), so that the variant with the least estimate takes little longer than the
 // fastest one; no weight says what its part costs by itself.  Over 4620 problems drawn and timed after the fit the choice takes
-// 1.009 times the fastest variant's time (geometric mean), more than 1.1 times on 86.
+// 1.009 times the fastest variant's time (geometric mean), more than 1.1 times on 61.
 // Before: a least-squares fit to 1390 problems up to the work of the largest case, with one D term however D is stored and the
-// mean number of tiles for long panels that two workgroups of a compute unit share: 1.023 times, more than 1.1 times on 384.  It took
+// mean number of tiles for long panels that two workgroups of a compute unit share: 1.021 times, more than 1.1 times on 323.  It took
 // narrow tiles where D is large (12416 x 69 x 63096, block height 128, density 0.05: 794 us, now 553; 5952 x 744 x 64552, 64: 340 and 299) and where
 // long panels fill a few compute units twice (5472 x 3207 x 368, 32, 0.37: 19.2 and 15.7).  The lines drawn by hand before that
-// (bounds on tiles, columns and kept vectors) take 1.09 times on average and 2.9 at worst, above all for many panels over few
+// (bounds on tiles, columns and kept vectors) take 1.09 times on average and 2.8 at worst, above all for many panels over few
 // columns on 512-column tiles (29632 x 761 x 64, density 0.47, block height 64: 16.1 us; 128-column tiles 7.0).
 //
 //  role-split: base + tiles of a compute unit * (tile + stage * stages of 32 kept vectors) + D.  The tiles of a compute unit are
@@ -200,31 +200,31 @@ struct SplitEstimate {
     float base, tile, step, wide_step, d, c, c_round;
 };
 static const RoleSplitEstimate g_role_split_estimates[] = {
-    {"ws16x128x4c4p_k32_s4", 2.21f, 0.746f, 0.323f, {0.967f, 0.677f, 0.f, 0.f}, 0.607f, 0.277f},
-    {"ws16x64x4c4p_k32_s4", 1.44f, 1.02f, 0.204f, {0.0306f, 0.f, 0.f, 0.591f}, 0.f, 0.373f, {0.297f, 0.28f, 0.79f}},
-    {"ws16x64x2c4p_k32_s6", 1.6f, 0.701f, 0.167f, {0.f, 0.f, 0.f, 0.f}, 0.f, 0.279f, {0.413f, 0.425f, 0.395f}},
-    {"ws32x128x4c4p_k32_s4", 1.74f, 1.22f, 0.355f, {0.962f, 0.727f, 0.0583f, 0.18f}, 0.627f, 1.02f},
-    {"ws32x64x4c4p_k32_s3", 1.21f, 1.19f, 0.409f, {0.13f, 0.203f, 0.f, 2.84f}, 0.434f, 0.573f, {0.114f, 0.316f, 0.436f}},
-    {"ws32x64x4c4p_k32_s6", 1.11f, 1.43f, 0.223f, {0.00974f, 0.f, 0.f, 0.f}, 0.255f, 0.602f},
-    {"ws32x32x4c4p_k32_s6", 1.29f, 1.06f, 0.171f, {0.0221f, 0.f, 0.f, 0.704f}, 0.609f, 0.287f, {0.32f, 0.203f, 0.502f}},
-    {"ws64x128x4c4p_k32_s4", 1.82f, 2.09f, 0.433f, {0.503f, 0.566f, 0.286f, 0.342f}, 0.939f, 0.813f},
-    {"ws64x64x4c4p_k32_s3", 0.f, 2.09f, 0.557f, {0.56f, 0.578f, 0.0858f, 1.18f}, 0.692f, 1.55f, {0.857f, 0.f, 0.f}},
-    {"ws64x64x4c4p_k32_s6", 1.58f, 1.33f, 0.263f, {0.454f, 0.758f, 0.222f, 0.307f}, 0.144f, 1.72f},
-    {"ws64x32x4c4p_k32_s4", 1.22f, 0.464f, 0.25f, {0.802f, 0.959f, 0.603f, 0.922f}, 0.603f, 0.678f, {0.853f, 0.418f, 0.334f}},
-    {"ws64x32x4c4p_k32_s6", 1.12f, 1.48f, 0.195f, {0.0511f, 0.f, 0.f, 0.09f}, 0.307f, 0.546f},
-    {"ws128x64x4c4p_k32_s6", 1.52f, 2.51f, 0.342f, {0.355f, 0.469f, 0.395f, 0.286f}, 0.711f, 1.26f},
-    {"ws128x32x4c4p_k32_s4", 0.f, 2.96f, 0.276f, {0.418f, 0.397f, 0.383f, 1.28f}, 1.14f, 0.82f, {1.1f, 0.f, 0.66f}},
-    {"ws128x32x4c4p_k32_s6", 1.42f, 2.07f, 0.24f, {0.322f, 0.323f, 0.f, 0.537f}, 0.37f, 0.99f},
+    {"ws16x128x4c4p_k32_s4", 2.04f, 0.747f, 0.317f, {1.05f, 0.578f, 0.f, 0.f}, 0.661f, 0.298f},
+    {"ws16x64x4c4p_k32_s4", 1.74f, 0.637f, 0.215f, {0.f, 0.0566f, 0.f, 0.0226f}, 0.f, 0.286f, {0.286f, 0.922f, 0.619f}},
+    {"ws16x64x2c4p_k32_s6", 2.12f, 0.396f, 0.161f, {0.f, 0.113f, 0.f, 0.f}, 0.421f, 0.176f, {0.0802f, 1.49f, 0.402f}},
+    {"ws32x128x4c4p_k32_s4", 2.06f, 0.893f, 0.364f, {0.941f, 1.11f, 0.729f, 0.f}, 0.726f, 0.722f},
+    {"ws32x64x4c4p_k32_s3", 1.35f, 0.871f, 0.429f, {0.202f, 0.638f, 0.f, 0.227f}, 0.409f, 0.617f, {0.296f, 0.429f, 0.343f}},
+    {"ws32x64x4c4p_k32_s6", 1.32f, 1.38f, 0.22f, {0.0374f, 0.0822f, 0.f, 0.f}, 0.235f, 0.524f},
+    {"ws32x32x4c4p_k32_s6", 1.56f, 0.948f, 0.165f, {0.f, 0.23f, 0.f, 0.28f}, 0.487f, 0.311f, {0.193f, 0.28f, 0.569f}},
+    {"ws64x128x4c4p_k32_s4", 1.67f, 1.99f, 0.478f, {0.659f, 0.718f, 0.461f, 0.228f}, 0.599f, 1.49f},
+    {"ws64x64x4c4p_k32_s3", 0.444f, 1.38f, 0.586f, {0.635f, 0.899f, 0.169f, 0.586f}, 0.657f, 1.49f, {0.838f, 0.0779f, 0.f}},
+    {"ws64x64x4c4p_k32_s6", 1.49f, 1.4f, 0.295f, {0.379f, 0.636f, 0.129f, 0.281f}, 0.271f, 1.36f},
+    {"ws64x32x4c4p_k32_s4", 1.32f, 0.44f, 0.247f, {0.677f, 1.03f, 0.591f, 0.594f}, 0.211f, 0.928f, {0.758f, 0.624f, 0.419f}},
+    {"ws64x32x4c4p_k32_s6", 1.02f, 1.48f, 0.207f, {0.f, 0.f, 0.f, 0.0376f}, 0.00714f, 0.764f},
+    {"ws128x64x4c4p_k32_s6", 0.27f, 3.63f, 0.415f, {0.251f, 0.00972f, 0.f, 0.55f}, 0.543f, 1.14f},
+    {"ws128x32x4c4p_k32_s4", 0.f, 2.74f, 0.297f, {0.515f, 0.339f, 0.339f, 0.896f}, 1.03f, 0.923f, {0.967f, 0.0828f, 0.816f}},
+    {"ws128x32x4c4p_k32_s6", 0.694f, 2.52f, 0.268f, {0.372f, 0.471f, 0.0712f, 0.f}, 0.296f, 1.13f},
 };
 static const SlabEstimate g_slab_estimates[] = {
-    {"slab16x64", 0.0239f, 2.81f, 1.54f, 0.f, 0.186f, {0.824f, 0.761f, 0.584f, 0.104f}, 0.835f, 0.235f},
-    {"slab32x64", 2.03f, 0.681f, 1.84f, 0.604f, 0.216f, {0.633f, 0.527f, 0.357f, 0.166f}, 1.12f, 0.231f},
+    {"slab16x64", 1.52f, 1.19f, 2.22f, 0.f, 0.168f, {0.894f, 1.05f, 0.604f, 0.0739f}, 0.0722f, 0.624f},
+    {"slab32x64", 0.f, 2.91f, 1.98f, 0.211f, 0.235f, {0.89f, 0.794f, 0.83f, 0.376f}, 0.374f, 0.848f},
 };
 static const SplitEstimate g_split_estimates[] = {
-    {"split16x32", 0.494f, 1.68f, 0.846f, 0.2f, 3.68f, 1.28f, 0.189f},
-    {"split32x32", 0.693f, 2.39f, 0.574f, 0.297f, 0.66f, 0.06f, 0.191f},
-    {"split64x32", 1.47f, 1.6f, 0.651f, 0.47f, 0.518f, 0.f, 0.451f},
-    {"split128x32", 0.558f, 1.32f, 0.929f, 0.832f, 1.37f, 0.968f, 0.492f},
+    {"split16x32", 0.78f, 1.57f, 0.843f, 0.2f, 3.67f, 0.f, 0.205f},
+    {"split32x32", 1.03f, 2.2f, 0.541f, 0.306f, 0.579f, 0.8f, 0.263f},
+    {"split64x32", 1.02f, 2.07f, 0.634f, 0.502f, 0.642f, 0.f, 0.608f},
+    {"split128x32", 0.333f, 1.5f, 0.775f, 0.798f, 1.68f, 1.12f, 0.501f},
 };
 
 static StoreMode result_store_mode(const void* D, int rows, int ldd, size_t others, bool narrow, bool read_back);
@@ -929,7 +929,7 @@ int init_chwb_taps(shflbw_spconv_state* state, const shflbw_weight* f, int B, in
     // The cut of the SpMM of these sizes.  With three widths by the number of tiles, and one width for block height 16, us, before / now:
     // 16 x 14 x 14 x 656 -> 32, 3 x 3, block height 16 20.4 / 11.9, 8 x 7 x 7 x 304 -> 1152, 5 x 5, 14.3 / 11.0; block height 32, 32 x 55 x 27 x
     // 360 -> 128, 1 x 7, 20.1 / 18.5.  The estimate was fitted to no convolution; over 500 drawn layers, every cut timed, its choice takes
-    // 1.010 times the fastest cut's time, 1.25 at worst.
+    // 1.013 times the fastest cut's time, 1.24 at worst.
     const int variant = auto_spmm_variant(f, (int)ncols, false, false, device_compute_units());
     const SpmmVariant* v = find_spmm_variant(f->brow, variant, nullptr);
     const ConvTapsKernel* k = v ? conv_taps_kernel(v->name) : nullptr;
