@@ -368,7 +368,7 @@ static int plane_form_geometry(const shflbw_weight* f, int B, int H, int W, int 
 //    where it will not: where three such problems in turn, 3 * (B + C + D), do not fit its 256 MB.  Merged / through, 600 drawn
 //    problems with D of 8 to 300 MB (955 pairs with a variant without C, 397 with): 0.92 by this rule, 6 pairs above 1.05; with
 //    the line at D >= 24 MB, as before, 0.92 and 85, up to 1.22 (32 x 1184 x 279 x 13792, 33 MB, short panels: 9.8 us through, 12.0).
-//    Narrow tiles, whose stores are half lines, from 24 MB on (0.92 below the other line).
+//    Narrow tiles, whose stores are half lines, from 24 MB on (0.88 below the other line).
 //  * Whole lines: streamed from 96 MB on, if nothing reads D back at once; smaller results, also three of them in turn, stay in
 //    the Infinity Cache.  us, through / streamed, density 0.1, block height 64, K = 1640 or 2048: 16384 x 1024 12.5 / 12.9 (33 MB),
 //    6144 x 4096 30.8 / 30.3 (50 MB), 16384 x 2560 28.6 / 28.5, 16384 x 2816 34.3 / 33.0 (92 MB), 8192 x 6400 45 / 40, 8192 x 8192 58 / 50;
