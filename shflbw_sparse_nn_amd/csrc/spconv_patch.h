@@ -57,7 +57,8 @@ ConvPatchShape conv_patch_shape(int rows, const ConvPatchPlan& p);
 inline int conv_patch_group(int rows) { return rows == 16 ? 8 : 4; }
 
 // Fills `plan`; false when no patch fits the LDS (with `held`: none of these shapes) or the sizes leave 32-bit indexes.
-bool conv_patch_plan(const ConvPatchProblem& q, ConvPatchPlan* plan, const std::vector<ConvPatchShape>* held = nullptr);
+// `wide_cuts` false: the plan without the wide kernels, which a check holds the other one against.
+bool conv_patch_plan(const ConvPatchProblem& q, ConvPatchPlan* plan, const std::vector<ConvPatchShape>* held = nullptr, bool wide_cuts = true);
 
 // Order of the kept columns of a row panel that keeps the LDS reads of a group of rows apart (see the definition).
 struct ConvPatchOrder {

@@ -715,10 +715,10 @@ ConvPatchShape conv_patch_shape(int rows, const ConvPatchPlan& p)
 // filters over many channels), filters of several workgroups interleaved in the output - the cut is not `preferred`:
 // 7 x 54 x 54 x 584 -> 1024, 5 x 5, stride 2 takes 152 us here, 54 us there; 16 x 14 x 14 x 512 -> 2048, which it takes, 20 and 23 us.
 // On 64 sampled layers it is preferred for 58, where the plane forms take 1.11 to 3.8 times as long.
-bool conv_patch_plan(const ConvPatchProblem& q, ConvPatchPlan* plan, const std::vector<ConvPatchShape>* held)
+bool conv_patch_plan(const ConvPatchProblem& q, ConvPatchPlan* plan, const std::vector<ConvPatchShape>* held, bool wide_cuts)
 {
     ConvPatchPlan best{};
-    double best_cost = 0, best_plain = 0;
+    double best_cost = 0, best_plain = 0, best_other = HUGE_VAL; // best_other: of the cuts that are not wide
     const bool flat = q.R == 1 && q.S == 1 && q.stride == 1; // every pixel for itself: one long row
     const unsigned long long in_bytes = (unsigned long long)q.B * q.H * q.W * q.C * 2;
     if (in_bytes > 0xffffff00ull || (unsigned long long)q.B * q.Ho * q.Wo > 0x7fffffffull) return false;
@@ -731,7 +731,7 @@ bool conv_patch_plan(const ConvPatchProblem& q, ConvPatchPlan* plan, const std::
         if (k.RW != rw) continue;
         const bool wide = k.deep == CONV_PATCH_WIDE;
         const int np_wide = (nunits + k.waves - 1) / k.waves; // row units of a wave with all filters in one workgroup
-        if (wide && (!q.permuted || np_wide <= conv_patch_units(rw) || np_wide > k.units)) continue;
+        if (wide && (!wide_cuts || !q.permuted || np_wide <= conv_patch_units(rw) || np_wide > k.units)) continue;
         const int positions = 8 * k.col_blocks;
         for (int th = 1; th <= std::min(positions, Ho); th++)
             for (int tw = 1; tw <= std::min(positions / th, Wo); tw++) {
@@ -807,14 +807,18 @@ bool conv_patch_plan(const ConvPatchProblem& q, ConvPatchPlan* plan, const std::
                         if (!best.valid || cost < best_cost) {
                             best = p, best_cost = cost;
                             best_plain = 2.9 + plain * (1 + (rounds - 1) * 1.16) + jobs * 1.0e-5;
+                            if (!wide) best_other = cost; // (the wide kernels come last: they do not stand in the way of another cut)
                             best.valid = 1;
                         }
                     }
             }
     }
     if (!best.valid) return false;
-    // (without the wide kernels' weights, which were fitted against chunks: 52 x 16 x 16 x 792 -> 1792, 1 x 1: 40.9 us here, 36.0 there)
-    best.preferred = best_plain <= conv_planes_estimate(q);
+    // Without the wide kernels' weights, which were fitted against chunks (52 x 16 x 16 x 792 -> 1792, 1 x 1: 40.9 us here, 36.0 there); but a
+    // layer that the form would take in chunks is not lost to the plane forms because a wide cut is estimated faster still.  Of 39450
+    // sampled layers 9 are such; on these and five more the wide cut takes 0.47 to 0.99 times the plane forms' time and 0.77 to
+    // 1.07 times that of the chunks: 23 x 38 x 38 x 168 -> 1984, 1 x 1, block height 64 77.9 us, planes 101.7, chunks 90.1.
+    best.preferred = std::min(best_plain, best_other) <= conv_planes_estimate(q);
     best.H = H, best.W = W, best.Ho = Ho, best.Wo = Wo, best.stride = q.stride;
     best.pad_h = q.R / 2, best.pad_w = q.S / 2;
     best.skip = q.stride > q.R || q.stride > q.S;

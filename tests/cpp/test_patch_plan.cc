@@ -1,6 +1,7 @@
 // The planner of the convolution's patch form on the CPU: what a workgroup of the cut it picks would read from LDS, for
 // seeded random layers.  The walk below restates the kernel's addressing (position -> column offset, kept column -> row).
 #include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -193,6 +194,42 @@ int plans_keep_to_held_shapes()
     return bad + (other < 500);
 }
 
+// Wide cuts are a further choice of the patch form: a layer that takes the form without them takes it with them.
+int wide_cuts_keep_the_form()
+{
+    // permuted layers whose wide cut is estimated ahead of the best other one by its own weights, and behind the plane forms without them
+    std::vector<Layer> layers{{64, 1984, 184, 1, 1, 1, 32, 38, 26, 1, 22.6 / 184}, {64, 1984, 168, 1, 1, 1, 23, 38, 38, 1, 0.06},
+                              {32, 1920, 304, 1, 1, 1, 57, 19, 19, 1, 0.19},       {128, 1920, 328, 1, 1, 1, 31, 31, 31, 1, 0.09},
+                              {32, 1984, 120, 1, 1, 1, 46, 29, 29, 1, 0.22}};
+    std::mt19937 rng(11);
+    auto spread = [&](int lo, int hi) { return std::exp(std::log((double)lo) + rng() % 10000 / 10000.0 * std::log((double)hi / lo)); };
+    for (int t = 0; t < 2500; t++) {
+        Layer l{};
+        l.V = 16 << rng() % 4;
+        l.F = std::max(512 / l.V + 1, (int)(spread(512, 2048) / l.V)) * l.V;
+        l.C = 8 * (int)spread(2, 128);
+        l.R = l.S = 1 + 2 * (int)(rng() % 3);
+        if (rng() % 6 == 0) l.R = 1, l.S = 7;
+        l.permuted = 1, l.B = (int)spread(1, 128), l.H = (int)spread(5, 56), l.W = rng() % 2 ? l.H : (int)spread(5, 56);
+        l.stride = rng() % 10 < 7 ? 1 : 2, l.density = spread(5, 50) / 100;
+        layers.push_back(l);
+    }
+    int bad = 0, wide = 0;
+    for (const Layer& l : layers) {
+        ConvPatchPlan with{}, without{};
+        if (!conv_patch_plan(problem(l), &without, nullptr, false)) continue;
+        bad += without.deep == CONV_PATCH_WIDE;
+        if (!conv_patch_plan(problem(l), &with) || (without.preferred && !with.preferred)) {
+            if (bad++ < 8)
+                printf("Failed: V %d F %d C %d %dx%d map %d x %dx%d stride %d density %g: the plane forms take it from a wide cut\n", l.V, l.F, l.C,
+                       l.R, l.S, l.B, l.H, l.W, l.stride, l.density);
+        }
+        wide += with.deep == CONV_PATCH_WIDE;
+    }
+    printf("wide cuts: %d layers, %d left to the plane forms for one\n", wide, bad);
+    return bad + (wide < 500);
+}
+
 } // namespace
 
 // test_patch_plan: the checks above.  test_patch_plan cut V F C R S nnzb permuted B H W stride: the cut of one layer, as
@@ -210,7 +247,7 @@ int main(int argc, char** argv)
         printf("%d %d %d %d %d %d %d\n", conv_patch_unit_rows(l.V), p.col_blocks, p.waves, p.panels_per_wave, p.ksplit, p.chunks, p.deep);
         return 0;
     }
-    const int bad = reads_stay_inside() + orders_follow_the_rule() + plans_keep_to_held_shapes();
+    const int bad = reads_stay_inside() + orders_follow_the_rule() + plans_keep_to_held_shapes() + wide_cuts_keep_the_form();
     printf(bad ? "FAILED\n" : "ALL PASSED\n");
     return bad != 0;
 }
