@@ -759,10 +759,10 @@ bool conv_patch_plan(const ConvPatchProblem& q, ConvPatchPlan* plan, const std::
                 p.slack = (int)std::max<long>(CONV_PATCH_SLACK, last - (q.C + 1L) * p.pitch);
                 const long slab = (long)(q.C + 1) * p.pitch + p.slack;
                 if (slab > CONV_PATCH_LDS_MAX) continue;
-                // what the patch of a single workgroup takes: a cut cannot be better than that
+                // what the patch of a single workgroup takes, for a wide cut by its weight: a cut cannot be better than that
                 const double rounds_patch = std::ceil((double)((p.npos + 7) / 8 * ((q.C + 63) / 64)) / (k.waves * k.items));
                 const double start = 1.0 + (k.waves == 8 ? 1.15 : 0), patch_bytes = q.C * p.npos * 8 * 5.3e-6;
-                if (best.valid && 2.9 + start + patch_bytes + rounds_patch * 0.7 >= best_cost) continue;
+                if (best.valid && 2.9 + (start + patch_bytes + rounds_patch * 0.7) * (wide ? 0.65 : 1) >= best_cost) continue;
                 for (int groups = k.waves; groups >= (wide ? k.waves : 1); groups >>= 1)
                     for (int np = wide ? np_wide : 1; np <= k.units; np = wide ? k.units + 1 : np << 1) {
                         p.groups = groups, p.ksplit = k.waves / groups, p.panels_per_wave = np;
