@@ -174,6 +174,7 @@ typedef struct shflbw_spmm_state {
     const void* zero_row; /* 1 KiB of zeros inside the library (device memory): gathered for the padding slots by the variants without a buffer descriptor for B */
     const int* packed_slab; /* the ids as LDS offsets for the tile variants that hold B in LDS; NULL when the weight has too many columns */
     int groups; /* groups of 64 slots that the kept vectors of all panels fill */
+    int half_panels; /* panels of the first of two parts of about the same work, or 0 */
 } shflbw_spmm_state;
 
 /* C may be NULL when beta == 0.  variant < 0 selects automatically. */

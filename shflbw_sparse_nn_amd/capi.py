@@ -58,7 +58,8 @@ class SpmmState(C.Structure):
                 ("init_success", C.c_int), ("variant", C.c_int), ("args", _SpmmArgs),
                 ("packed_values", C.c_void_p), ("packed_indices", C.c_void_p), ("packed_indices_pm", C.c_void_p),
                 ("panel_ptr", C.c_void_p), ("brow", C.c_int), ("ldb_bytes", C.c_int), ("zero_row", C.c_void_p),
-                ("packed_slab", C.c_void_p), ("groups", C.c_int)]
+                ("packed_slab", C.c_void_p), ("groups", C.c_int),
+                ("half_panels", C.c_int)]
 
 
 class _SpconvArgs(C.Structure):

@@ -398,6 +398,7 @@ static void fill_spmm_launch_args(const shflbw_spmm_state* state, int BN, SpmmLa
     a.slab_ids = state->packed_slab;
     a.slab_chunks = 1, a.slab_panels = a.X, a.slab_by_chunk = 0;
     a.groups = state->groups;
+    a.half_panels = state->half_panels;
     a.panel_desc = state->panel_ptr;
     a.row_ids = state->args.A_row_indices;
     a.B = (const half_t*)state->args.B;
@@ -527,6 +528,7 @@ static int spmm_init_impl(shflbw_spmm_state* state, const shflbw_weight* w, int 
     state->packed_indices_pm = (const int*)w->d_packed_indices_pm;
     state->packed_slab = w->packed_slab.empty() ? nullptr : (const int*)w->d_packed_slab;
     state->groups = (int)(w->packed_indices.size() / 64);
+    state->half_panels = w->half_panels;
     state->panel_ptr = (const int*)w->d_group_ptr;
     state->brow = w->brow;
     state->ldb_bytes = N * 2;

@@ -286,8 +286,8 @@ spmm_shflbw_ws_kernel(SpmmLaunchArgs a)
     const int S = gridDim.x >> 3;
     int id_first, id_end, t_step = 1, t_first = 0;
     if constexpr (HALVES) {
-        const int p0 = (xcd & 1) * (a.X >> 1), part = xcd >> 1;
-        a.X = (xcd & 1) ? a.X - p0 : a.X >> 1;
+        const int p0 = (xcd & 1) * a.half_panels, part = xcd >> 1;
+        a.X = (xcd & 1) ? a.X - p0 : a.half_panels;
         a.magic_x = (xcd & 1) ? a.magic_halves[1] : a.magic_halves[0];
         a.panel_desc += 2 * p0;
         if (a.row_ids) {
@@ -336,7 +336,7 @@ spmm_shflbw_ws_kernel(SpmmLaunchArgs a)
 static bool panel_halves(const SpmmLaunchArgs& a, int S)
 {
     const size_t a_bytes = (size_t)a.groups * 64 * (a.M / a.X) * 2;
-    if (a.store_mode != STORE_STREAM || a.X < 2 || a_bytes <= 6u << 20 || a_bytes > 10u << 20) return false;
+    if (a.store_mode != STORE_STREAM || a.half_panels <= 0 || a.half_panels >= a.X || a_bytes <= 6u << 20 || a_bytes > 10u << 20) return false;
     return a.X <= 40 || ((size_t)a.ldd * 2 % (32u << 10) == 0 && 2 * S % a.X == 0);
 }
 
@@ -372,7 +372,7 @@ static hipError_t launch_ws(const SpmmLaunchArgs& a, hipStream_t stream)
             kernel = b.beta == 0.f  ? &spmm_shflbw_ws_kernel<V, WN, NCONS, NPROD, KT, NSTAGE, C_NONE, true>
                      : streams_c(b) ? &spmm_shflbw_ws_kernel<V, WN, NCONS, NPROD, KT, NSTAGE, C_STREAMED, true>
                                     : &spmm_shflbw_ws_kernel<V, WN, NCONS, NPROD, KT, NSTAGE, C_CACHED, true>;
-            b.magic_halves[0] = udiv_magic(b.X >> 1), b.magic_halves[1] = udiv_magic(b.X - (b.X >> 1));
+            b.magic_halves[0] = udiv_magic(b.half_panels), b.magic_halves[1] = udiv_magic(b.X - b.half_panels);
             b.alternate = 0; // no second round under a column tile
         }
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream, b);

@@ -16,7 +16,8 @@ struct SpmmLaunchArgs {
     int M, N, K;
     int X;       // row panels = M / V
     unsigned magic_x; // udiv_magic of X
-    unsigned magic_halves[2]; // ... of the panels of the two halves, where they are cut in two (launcher)
+    int half_panels;          // panels of the first of two parts of about the same work, 0: no such cut (spmm_half_panels)
+    unsigned magic_halves[2]; // udiv_magic of the panels of either part (launcher, where they are taken apart)
     int n_tiles; // column tiles, filled by the launcher
     unsigned magic_tiles; // split kernel: udiv_magic of n_tiles; slab kernel: of the number that job numbers are cut by, n_tiles or slab_chunks (launcher)
     int split_shift;      // split kernel only: log2 of the 32-row blocks of a panel (launcher)

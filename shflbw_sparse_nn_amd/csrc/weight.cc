@@ -224,6 +224,20 @@ static void order_for_slab16(const int* ids, int nnz, int* ord)
 //   V == 16 (16x16x32 tiles): step s covers slots 32s..32s+31; lane l holds row l%16,
 //     slots 32s + 8*(l/16) + 0..7.
 // ---------------------------------------------------------------------------------
+int spmm_half_panels(const int* indptr, int X)
+{
+    auto larger_part = [&](int first) { // over half of the work
+        auto work = [&](int panels) { return (double)(indptr[panels] - indptr[0]) + 280.0 * panels; };
+        return 2 * std::max(work(first), work(X) - work(first)) / work(X);
+    };
+    if (X < 2) return 0;
+    int first = X / 2;
+    if (larger_part(first) > 1.03)
+        for (int p = 1; p < X; p++)
+            if (larger_part(p) < larger_part(first)) first = p;
+    return larger_part(first) <= 1.05 ? first : 0;
+}
+
 int build_packed_image(shflbw_weight* w)
 {
     if (w->bcol != 1) {
@@ -246,6 +260,7 @@ int build_packed_image(shflbw_weight* w)
         w->panel_desc[2 * i] = (w->indptr[i + 1] - w->indptr[i] + 15) / 16;
         w->panel_desc[2 * i + 1] = w->group_ptr[i];
     }
+    w->half_panels = spmm_half_panels(w->indptr.data(), X);
     const size_t slots = (size_t)w->group_ptr[X] * 64;
     w->packed_indices.assign(slots, 0);
     w->packed_indices_pm.assign(slots, 0);
