@@ -382,8 +382,7 @@ static StoreMode result_store_mode(const void* D, int rows, int ldd, size_t othe
     return bytes >= 96u << 20 && !read_back ? STORE_STREAM : STORE_THROUGH;
 }
 
-// launch arguments of the SpMM kernels from a state; BN is the tile width of the kernel that will run
-static void fill_spmm_launch_args(const shflbw_spmm_state* state, int BN, SpmmLaunchArgs* out)
+void fill_spmm_launch_args(const shflbw_spmm_state* state, int BN, SpmmLaunchArgs* out)
 {
     SpmmLaunchArgs& a = *out;
     a.M = state->args.M;

@@ -6,6 +6,7 @@
 #include <initializer_list>
 
 #include "kernel_common.h"
+#include "shflbw.h"
 
 namespace shflbw {
 
@@ -131,6 +132,36 @@ inline StoreMode slab_store_mode(const void* D, int rows, int ldd, size_t others
     if ((((uintptr_t)D | ((uintptr_t)ldd * 2)) & 127) != 0) return bytes + others >= STORE_MERGE_BYTES ? STORE_MERGE : STORE_THROUGH;
     return bytes >= 96u << 20 ? STORE_STREAM : STORE_THROUGH;
 }
+
+// Whether the panels are cut in two halves that the XCDs work on apart.  With all panels under one column tile after the other every
+// XCD reads the whole of A once per column tile, from the Infinity Cache where A exceeds the L2, and the 32 workgroups of an XCD store
+// pieces of one column tile at a time.  Halves help large results of block height 128
+//  * with at most 40 panels, where half of A stays in the L2 from tile to tile and the workgroups of an XCD are on two column tiles
+//    at a time, for a second trip of B.  us, whole / halves: 4096 x 2775 x 14592, density 0.32 130 / 118, 4096 x 4245 x 19456, 0.28 203 / 188,
+//    3584 x 6898 x 15808, 0.13 115 / 108, with C 5120 x 3195 x 12032, 0.19 106 / 102; but with the whole of A nearly there, 3712 x 4465 x 28672, 0.14
+//    (4.7 MB) 170 / 183, with more panels, 6656 x 4389 x 31744, 0.13 298 / 316, 7552 x 5327 x 9728, 0.07 83 / 88;
+//  * where the pitch of D is a multiple of 32 KiB, which puts a column tile's pieces of all rows into the same few channels of the
+//    memory (with C, 8192 x 4096 x N, 0.1: N = 14336 176, 16384 221, 20480 252), if the half goes evenly into the workgroups of an XCD, so that no
+//    round is on two column tiles by a part: the XCDs of a half then are on neighbouring column tiles.  8192 x 4096 x 16384 with C 221 / 202,
+//    without 168 / 151, 8192 x 1536 x 16384, 0.25 with C 218 / 192, 8192 x 4096 x 32768 with C 418 / 398; 8192 x 4096 x 20480 with C 252 / 264.
+inline bool panel_halves(const SpmmLaunchArgs& a, int S)
+{
+    const size_t a_bytes = (size_t)a.groups * 64 * (a.M / a.X) * 2;
+    if (a.store_mode != STORE_STREAM || a.half_panels <= 0 || a.half_panels >= a.X || a_bytes <= 6u << 20 || a_bytes > 10u << 20) return false;
+    return a.X <= 40 || ((size_t)a.ldd * 2 % (32u << 10) == 0 && 2 * S % a.X == 0);
+}
+
+// Whether C is streamed past the caches: where D is, and B, C and D are twice the Infinity Cache, nothing of C lasts until a next
+// pass.  us, cached / streamed: block height 64, 8192 x 4096 x 16384, density 0.1 (670 MB) 256 / 233, 16384 x 4096 x 8192, 0.05 (604 MB) 177 / 170, 14144 x 1186 x
+// 13824, 0.16 (815 MB) 239 / 230; 128: 32768 x 2048 x 4096, 0.1 (553 MB) 146 / 143; but 64, 9152 x 1339 x 12288, 0.17 (482 MB) 142 / 146, 11584 x 1908 x 9216,
+// 0.13 (462 MB) 134 / 146, and D in parts of lines, 128, 17280 x 6409 x 13928, 0.025 342 / 369.
+inline bool streams_c(const SpmmLaunchArgs& a)
+{
+    return a.store_mode == STORE_STREAM && bytes_of_b_and_c(a) + (size_t)a.M * a.ldd * 2 >= 512u << 20;
+}
+
+// Launch arguments of the SpMM kernels from a state; BN is the tile width of the kernel that will run.
+void fill_spmm_launch_args(const shflbw_spmm_state* state, int BN, SpmmLaunchArgs* out);
 
 // device address of the library's row of zeros on the current device (looked up once per device); null on failure
 const void* spmm_zero_row();

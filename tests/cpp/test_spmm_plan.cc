@@ -1,10 +1,13 @@
 // How the SpMM goes about the panels of a weight, on the CPU.
 #include <algorithm>
 #include <cstdio>
+#include <cstdlib>
+#include <cstring>
 #include <functional>
 #include <random>
 #include <vector>
 
+#include "csrc/spmm_launch.h"
 #include "csrc/weight_internal.h"
 
 using namespace shflbw;
@@ -52,10 +55,38 @@ int parts_are_even()
     return bad + (uneven < 50) + (none < 20);
 }
 
+// The launch of a product with the 256-column variant of block height 128 (of another one: its wide variant) on 256 compute units.
+SpmmLaunchArgs launch_of(int V, int K, int N, const std::vector<int>& indptr, bool permuted, bool residual)
+{
+    const int X = (int)indptr.size() - 1;
+    shflbw_spmm_state s;
+    memset(&s, 0, sizeof(s));
+    s.args.M = X * V, s.args.N = N, s.args.K = K;
+    s.args.D = (void*)(uintptr_t)0x10000; // whole lines; never dereferenced
+    s.args.A_row_indices = permuted ? indptr.data() : nullptr;
+    s.args.alpha = 1.f, s.args.beta = residual ? 1.f : 0.f;
+    s.brow = V, s.ldb_bytes = N * 2;
+    for (int i = 0; i < X; i++) s.groups += (indptr[i + 1] - indptr[i] + 63) / 64;
+    s.half_panels = spmm_half_panels(indptr.data(), X);
+    SpmmLaunchArgs a;
+    fill_spmm_launch_args(&s, 256, &a);
+    return a;
+}
+
 } // namespace
 
-int main()
+// test_spmm_plan: the checks above.  test_spmm_plan launch V K N permuted residual < kept vectors of every panel: whether C is streamed, panels
+// of the first half (0: not in halves).
+int main(int argc, char** argv)
 {
+    if (argc == 7 && !strcmp(argv[1], "launch")) {
+        std::vector<int> p(1, 0);
+        for (int n; scanf("%d", &n) == 1;) p.push_back(p.back() + n);
+        const bool residual = atoi(argv[6]);
+        const SpmmLaunchArgs a = launch_of(atoi(argv[2]), atoi(argv[3]), atoi(argv[4]), p, atoi(argv[5]), residual);
+        printf("%d %d\n", residual && streams_c(a), panel_halves(a, 32) ? a.half_panels : 0);
+        return 0;
+    }
     const int bad = parts_are_even();
     printf(bad ? "FAILED\n" : "ALL PASSED\n");
     return bad != 0;

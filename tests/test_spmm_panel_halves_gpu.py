@@ -1,51 +1,24 @@
 """Large D over few long panels: the XCDs take the panels in halves (panel_halves): both sides of the rule, odd numbers of
 panels, column tiles that do and do not divide by four, panels that keep nothing, rows permuted and not, against exact
 integer products."""
-import numpy as np
 import pytest
 
-import shflbw_sparse_nn_amd as S
+from tests import spmm_large
 
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("V,X,N,per,permuted,residual", [
-    (128, 33, 12288, 800, True, False),   # halves of 16 and 17 panels, 48 column tiles
-    (128, 33, 12352, 800, False, True),   # a last tile of 64 columns; 49 column tiles: ranges that split a column tile
-    (128, 33, 32768, 800, True, True),    # C streamed
-    (128, 64, 16384, 420, True, False),   # a pitch of 32 KiB, as many panels to a half as an XCD has workgroups
-    (128, 64, 16448, 420, False, False),  # another pitch: not halved
-    (128, 9, 46080, 3300, True, True),    # fewer panels than workgroups of an XCD
-    (64, 33, 24576, 1400, False, False),  # a block height that is not halved
+@pytest.mark.parametrize("V,X,N,per,permuted,residual,first", [
+    (128, 33, 12288, 800, True, False, 16),   # halves of 16 and 17 panels, 48 column tiles
+    (128, 33, 12352, 800, False, True, 16),   # a last tile of 64 columns; 49 column tiles: ranges that split a column tile
+    (128, 33, 32768, 800, True, True, 16),    # C streamed
+    (128, 64, 16384, 420, True, False, 32),   # a pitch of 32 KiB, as many panels to a half as an XCD has workgroups
+    (128, 64, 16448, 420, False, False, 0),   # another pitch: not halved
+    (128, 9, 46080, 3300, True, True, 4),     # fewer panels than workgroups of an XCD
+    (64, 33, 24576, 1400, False, False, 0),   # a block height that is not halved
 ])
-def test_panel_halves(torch_gpu, V, X, N, per, permuted, residual):
-    torch = torch_gpu
-    M, K = V * X, 2 * per
-    rng = np.random.default_rng(V + X + N)
-    kept = [0 if p == X - 2 else per - (p % 3) * 40 if p % 2 else per + 30 for p in range(X)]
-    cols = [np.sort(rng.choice(K, n, replace=False)) for n in kept]
-    values = [rng.integers(-1, 2, size=(n, V)).astype(np.float16) for n in kept]
-    perm = rng.permutation(M).astype(np.int32) if permuted else None
-    w = S.BlockwiseSpMatrix()
-    w.set(M, K, V, 1, np.concatenate([[0], np.cumsum(kept)]).astype(np.int32), np.concatenate(cols).astype(np.int32),
-          np.concatenate(values).reshape(-1), perm)
-    w.transform_and_sync_device()
-    B = torch.from_numpy(rng.integers(-1, 2, size=(K, N)).astype(np.float16)).cuda()
-    C = torch.from_numpy(rng.integers(-4, 5, size=(M, N)).astype(np.float16)).cuda() if residual else None
-    dense = torch.zeros((M, K), dtype=torch.float32)
-    rows = torch.from_numpy((perm if permuted else np.arange(M)).astype(np.int64)).reshape(X, V)
-    for p in range(X):
-        dense[rows[p][:, None], torch.from_numpy(cols[p])[None, :]] = torch.from_numpy(values[p].T.astype(np.float32))
-    ref = (dense.cuda() @ B.float()).half()  # sums of at most 3330 products of -1, 0 and 1, in practice below 2^11: exact
-    assert float(ref.abs().max()) < 2000
-    if residual:
-        ref += C
-    D = torch.empty((M, N), dtype=torch.float16, device="cuda")
-    names = S.spmm_variants(V)
-    for variant in [-1] + [i for i, n in enumerate(names) if n in ("ws128x64x4c4p_k32_s6", "ws64x128x4c4p_k32_s4")]:
-        op = S.SpmmBlockwiseOp(variant)
-        op.initialize(w, N, B.data_ptr(), D.data_ptr(), C.data_ptr() if residual else None)
-        for _ in range(2):
-            D.fill_(float("nan"))
-            op(torch.cuda.current_stream().cuda_stream)
-            assert torch.equal(D, ref), names[variant] if variant >= 0 else "the library's choice"
+def test_panel_halves(torch_gpu, V, X, N, per, permuted, residual, first):
+    kept, K = spmm_large.lengths(X, per), 2 * per
+    if V == 128:
+        assert spmm_large.launch(V, kept, K, N, permuted, residual)[1] == first
+    spmm_large.check(torch_gpu, V, kept, K, N, permuted, residual)

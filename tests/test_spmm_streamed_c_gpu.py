@@ -1,47 +1,19 @@
 """C is streamed where B, C and D are twice the Infinity Cache (streams_c), against exact integer products."""
-import numpy as np
 import pytest
 
-import shflbw_sparse_nn_amd as S
+from tests import spmm_large
 
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("V,X,N,per,permuted,residual", [
-    (128, 33, 32768, 700, True, True),
-    (128, 33, 14336, 700, False, True),  # cached
-    (64, 33, 61440, 1400, False, True),
-    (32, 64, 61440, 150, True, True),
-    (16, 64, 122880, 150, True, True),
+@pytest.mark.parametrize("V,X,N,per,permuted,residual,streamed", [
+    (128, 33, 32768, 700, True, True, 1),
+    (128, 33, 14336, 700, False, True, 0),  # cached
+    (64, 33, 61440, 1400, False, True, 1),
+    (32, 64, 61440, 150, True, True, 1),
+    (16, 64, 122880, 150, True, True, 1),
 ])
-def test_streamed_c(torch_gpu, V, X, N, per, permuted, residual):
-    torch = torch_gpu
-    M, K = V * X, 2 * per
-    rng = np.random.default_rng(V + X + N)
-    kept = [0 if p == X - 2 else per - (p % 3) * 40 if p % 2 else per + 30 for p in range(X)]
-    cols = [np.sort(rng.choice(K, n, replace=False)) for n in kept]
-    values = [rng.integers(-1, 2, size=(n, V)).astype(np.float16) for n in kept]
-    perm = rng.permutation(M).astype(np.int32) if permuted else None
-    w = S.BlockwiseSpMatrix()
-    w.set(M, K, V, 1, np.concatenate([[0], np.cumsum(kept)]).astype(np.int32), np.concatenate(cols).astype(np.int32),
-          np.concatenate(values).reshape(-1), perm)
-    w.transform_and_sync_device()
-    B = torch.from_numpy(rng.integers(-1, 2, size=(K, N)).astype(np.float16)).cuda()
-    C = torch.from_numpy(rng.integers(-4, 5, size=(M, N)).astype(np.float16)).cuda() if residual else None
-    dense = torch.zeros((M, K), dtype=torch.float32)
-    rows = torch.from_numpy((perm if permuted else np.arange(M)).astype(np.int64)).reshape(X, V)
-    for p in range(X):
-        dense[rows[p][:, None], torch.from_numpy(cols[p])[None, :]] = torch.from_numpy(values[p].T.astype(np.float32))
-    ref = (dense.cuda() @ B.float()).half()  # sums of at most 2730 products of -1, 0 and 1, in practice below 2^11: exact
-    assert float(ref.abs().max()) < 2000
-    if residual:
-        ref += C
-    D = torch.empty((M, N), dtype=torch.float16, device="cuda")
-    names = S.spmm_variants(V)
-    for variant in [-1] + [i for i, n in enumerate(names) if n in ("ws128x64x4c4p_k32_s6", "ws64x128x4c4p_k32_s4")]:
-        op = S.SpmmBlockwiseOp(variant)
-        op.initialize(w, N, B.data_ptr(), D.data_ptr(), C.data_ptr() if residual else None)
-        for _ in range(2):
-            D.fill_(float("nan"))
-            op(torch.cuda.current_stream().cuda_stream)
-            assert torch.equal(D, ref), names[variant] if variant >= 0 else "the library's choice"
+def test_streamed_c(torch_gpu, V, X, N, per, permuted, residual, streamed):
+    kept, K = spmm_large.lengths(X, per), 2 * per
+    assert spmm_large.launch(V, kept, K, N, permuted, residual)[0] == streamed
+    spmm_large.check(torch_gpu, V, kept, K, N, permuted, residual)
