@@ -346,7 +346,6 @@ static hipError_t launch_ws(const SpmmLaunchArgs& a, hipStream_t stream)
                      : streams_c(b) ? &spmm_shflbw_ws_kernel<V, WN, NCONS, NPROD, KT, NSTAGE, C_STREAMED, true>
                                     : &spmm_shflbw_ws_kernel<V, WN, NCONS, NPROD, KT, NSTAGE, C_CACHED, true>;
             b.magic_halves[0] = udiv_magic(b.half_panels), b.magic_halves[1] = udiv_magic(b.X - b.half_panels);
-            b.alternate = 0; // no second round under a column tile
         }
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream, b);
     return hipGetLastError();

@@ -44,7 +44,9 @@ struct SpmmLaunchArgs {
     float alpha, beta;
     int num_cus; // compute units of the device (persistent kernels size their grid with it)
     int alternate; // role-split kernels: walk every second tile of a workgroup from its last stage to its first
-                   // (pays when the rows of B under one column tile do not fit the XCD's L2)
+                   // (pays when the rows of B under one column tile do not fit the XCD's L2; in halves too, where a workgroup's next
+                   // tile is another column tile of the same panels, whose A it then finds: us, one way / alternating: 8192 x
+                   // 8192 x 16384, 0.07 226 / 222, with C 271 / 259, 5120 x 8192 x 16384, 0.11 198 / 189, with C 217 / 208)
 };
 
 // Convolution over batch-innermost tensors that gathers from the input itself (B points to it): the columns of the GEMM

@@ -22,3 +22,13 @@ def test_panel_halves(torch_gpu, V, X, N, per, permuted, residual, first):
     if V == 128:
         assert spmm_large.launch(V, kept, K, N, permuted, residual)[1] == first
     spmm_large.check(torch_gpu, V, kept, K, N, permuted, residual)
+
+
+@pytest.mark.parametrize("X,N,per,residual,first", [
+    (33, 12288, 800, False, 16),
+    (64, 16384, 420, True, 32),
+])
+def test_stages_in_alternating_order(torch_gpu, X, N, per, residual, first):
+    kept, K = spmm_large.lengths(X, per), 5400  # rows of B under a column tile: 2.8 MB
+    assert spmm_large.launch(128, kept, K, N, True, residual)[1] == first
+    spmm_large.check(torch_gpu, 128, kept, K, N, True, residual)
