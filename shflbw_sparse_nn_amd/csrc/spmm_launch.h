@@ -135,22 +135,27 @@ inline StoreMode slab_store_mode(const void* D, int rows, int ldd, size_t others
     return bytes >= 96u << 20 ? STORE_STREAM : STORE_THROUGH;
 }
 
-// Whether the panels are cut in two halves that the XCDs work on apart.  With all panels under one column tile after the other every
-// XCD reads the whole of A once per column tile, from the Infinity Cache where A exceeds the L2, and the 32 workgroups of an XCD store
-// pieces of one column tile at a time.  Halves help large results of block height 128
-//  * with at most 40 panels, where half of A stays in the L2 from tile to tile and the workgroups of an XCD are on two column tiles
-//    at a time, for a second trip of B.  us, whole / halves: 4096 x 2775 x 14592, density 0.32 130 / 118, 4096 x 4245 x 19456, 0.28 203 / 188,
-//    3584 x 6898 x 15808, 0.13 115 / 108, with C 5120 x 3195 x 12032, 0.19 106 / 102; but with the whole of A nearly there, 3712 x 4465 x 28672, 0.14
-//    (4.7 MB) 170 / 183, with more panels, 6656 x 4389 x 31744, 0.13 298 / 316, 7552 x 5327 x 9728, 0.07 83 / 88;
+// Whether the panels are cut in two halves that the XCDs work on apart; S: workgroups of an XCD.  With all panels under one column tile
+// after the other every XCD reads the whole of A once per column tile, from the Infinity Cache where A exceeds the L2, and its
+// workgroups store pieces of one column tile at a time.  In halves it reads half of A and is on two column tiles at a time, or its
+// neighbours are on other ones, for a second trip of B.  That helps large results of block height 128 with an A of at most 10 MB, half of
+// which stays in an L2 for the most part.  Times of halves over whole panels, 436 problems, from 24 panels on where nothing else is said:
+//  * where A is longer than 6 MB and there are at most 40 panels, two column tiles to a round: 0.95 to 1.04, 0.988 on average (4096 x
+//    2775 x 14592, density 0.32 120 us / 113, 3456 x 2890 x 20544, 0.26 184 / 175, 4608 x 4960 x 27840, 0.15, with C 272 / 283).  41 to 47
+//    panels 0.94 to 1.04, 1.00; from 48 on 0.95 to 1.13, 1.03; an A of 4.5 to 6 MB 0.89 to 1.04, 0.99, above 10 MB 0.97 to 1.03, 0.99; 14
+//    to 23 panels, three column tiles and more, 0.96 to 1.05, 0.995; below that the larger part decides;
 //  * where the pitch of D is a multiple of 32 KiB, which puts a column tile's pieces of all rows into the same few channels of the
-//    memory (with C, 8192 x 4096 x N, 0.1: N = 14336 176, 16384 221, 20480 252), if the half goes evenly into the workgroups of an XCD, so that no
-//    round is on two column tiles by a part: the XCDs of a half then are on neighbouring column tiles.  8192 x 4096 x 16384 with C 221 / 202,
-//    without 168 / 151, 8192 x 1536 x 16384, 0.25 with C 218 / 192, 8192 x 4096 x 32768 with C 418 / 398; 8192 x 4096 x 20480 with C 252 / 264.
+//    memory; in halves the workgroups of an XCD, or those of its neighbours, are on other column tiles.  An A longer than 6 MB without C
+//    0.91 to 1.02, 0.97, with C 0.88 to 1.01, 0.955 (8192 x 4500 x 16384, 0.085, with C 234 us / 214, without 178 / 173; 16384 x 4096 x 16384,
+//    0.059 367 / 339 and 268 / 252; above 10 MB 0.93 to 1.06, 0.98); a shorter one with C and permuted rows 0.76 to 1.06, 0.89 (14336 x
+//    2048 x 16384, 0.027 274 / 218), rows not permuted 0.91 to 1.13, 0.985, without C 0.71 to 1.11, 0.94; below 24 panels 0.85 to 1.11, 0.98.
 inline bool panel_halves(const SpmmLaunchArgs& a, int S)
 {
     const size_t a_bytes = (size_t)a.groups * 64 * (a.M / a.X) * 2;
-    if (a.store_mode != STORE_STREAM || a.half_panels <= 0 || a.half_panels >= a.X || a_bytes <= 6u << 20 || a_bytes > 10u << 20) return false;
-    return a.X <= 40 || ((size_t)a.ldd * 2 % (32u << 10) == 0 && 2 * S % a.X == 0);
+    if (a.store_mode != STORE_STREAM || a.half_panels <= 0 || a.half_panels >= a.X || 4 * a.X < 3 * S || a_bytes > 10u << 20) return false;
+    const bool long_a = a_bytes > 6u << 20;
+    if ((size_t)a.ldd * 2 % (32u << 10) == 0) return long_a || (a.beta != 0.f && a.row_ids != nullptr);
+    return long_a && 4 * a.X <= 5 * S;
 }
 
 // Whether C is streamed past the caches: where D is, and B, C and D are twice the Infinity Cache, nothing of C lasts until a next
