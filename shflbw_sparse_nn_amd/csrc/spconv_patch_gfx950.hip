@@ -799,11 +799,13 @@ bool conv_patch_plan(const ConvPatchProblem& q, ConvPatchPlan* plan, const std::
                         const double t_out = values * (!q.permuted || p.chunks == 1 ? 5.0e-5 : 1.5e-4) +
                                              (p.ksplit > 1 ? k.waves * rw * cols * 4.0 * act * 1.0e-5 : 0);
                         const double plain = start + t_patch + t_main + t_out;
-                        // What surrounds the products costs the wide kernels less than this sum says, with the weights below by sampled layers
-                        // near the line: 122 that switch from chunks by it take 0.47 to 1.08 times the time, 0.82 on average, three of them more than 1.02.  (0.65 alone: 42 of 71 switch, two of
-                        // many products 1.05 and 1.14 times as long; 0.55 and 1.2: 41, three 1.07 to 1.14.)
+                        // What surrounds the products costs the wide kernels less than this sum says, with the weights below by sampled
+                        // layers near the line (0.65 alone: two of 42 that switch, of many products, 1.05 and 1.14 times as long; 0.55
+                        // and 1.2: three 1.07 to 1.14); and a tie of the estimates goes to the chunks: 263 of 550 layers switch, 0.33 to 1.03
+                        // times the time, 0.77 on average, two of them more than 1.02 (without the hundredth 280, ten of them up to 1.23:
+                        // small layers of 576 filters, 9 x 46 x 5 x 144, 1 x 1 5.2 us, 6.4 on a wide cut).
                         const double one = wide ? std::min(plain, (start + t_patch + t_out) * 0.65 + t_main * 1.25) : plain;
-                        const double cost = 2.9 + one * (1 + (rounds - 1) * 1.16) + jobs * 1.0e-5;
+                        const double cost = (2.9 + one * (1 + (rounds - 1) * 1.16) + jobs * 1.0e-5) * (wide ? 1.01 : 1);
                         if (!best.valid || cost < best_cost) {
                             best = p, best_cost = cost;
                             best_plain = 2.9 + plain * (1 + (rounds - 1) * 1.16) + jobs * 1.0e-5;
