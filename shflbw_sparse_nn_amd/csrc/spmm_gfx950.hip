@@ -317,7 +317,7 @@ spmm_shflbw_ws_kernel(SpmmLaunchArgs a)
     }
 
     if constexpr (V == 16)
-        ws_consumer16<Cfg, WN, NCONS, false, false, RES>(a, lds0, lane, wave, id_first, id_end, S);
+        ws_consumer16<Cfg, WN, NCONS, false, false, RES>(a, lds0, lane, wave, id_first, id_end, S, t_step, t_first);
     else
         ws_consumer<Cfg, V, WN, NCONS, false, false, RES>(a, lds0, lane, wave, id_first, id_end, S, t_step, t_first);
 }
