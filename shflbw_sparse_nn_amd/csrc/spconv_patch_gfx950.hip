@@ -494,8 +494,6 @@ __global__ void __launch_bounds__(NW * 64, WPE) spconv_patch_kernel(ConvPatchArg
         for (int j = 0; j < NBUF; j++) pass_through(buf[j]);
     }
 
-    // the filters a lane stores below, asked for here: in front of the stores the trip to memory stood in the chain
-    constexpr int MAXQ = 8;
     const int row0 = ch * P.rows_wg, rows = min(P.rows_wg, a.F - row0);
 
     // ---- results: one LDS row per filter, in output order (a lane holds four columns, the four units of a position, of
@@ -591,6 +589,7 @@ __global__ void __launch_bounds__(NW * 64, WPE) spconv_patch_kernel(ConvPatchArg
         else
             whole_lines(std::integral_constant<StoreMode, STORE_THROUGH>{});
     } else { // a chunk's filters are scattered over the pixel: 2-byte pieces in ascending order, merged in the L2
+        constexpr int MAXQ = 8;
         int f[MAXQ];
 #pragma unroll
         for (int q = 0; q < MAXQ; q++) f[q] = q * 64 + lane < rows ? a.filt[row0 + q * 64 + lane] : -1;
@@ -668,13 +667,15 @@ static hipError_t prepare_patch()
 // columns, leave no room for them.
 //
 // Wide kernels (the last ones): a permuted filter of more rows than the waves of a workgroup otherwise compute leaves in 2-byte stores from
-// every workgroup of a column tile, and what bounds those is the L2s' writes: 64 lanes of one of six workgroups reach thirteen
-// pieces of 64 bytes (17 x 18 x 14 x 208 -> 1472, 1 x 1: 4.9 of a workgroup's 8.4 us).  With up to four times the row units a wave, over
-// 32 columns, or twice over 64, one workgroup has all filters of its pixels and stores whole lines.  A unit's results go to LDS behind the patch as
-// the unit is finished: held in registers as in the other kernels they would not fit beside the ring.  us, in chunks / wide: that
-// layer 12.6 / 9.3, 88 x 8 x 23 x 216 -> 1344, 3 x 3, block height 64 43.1 / 25.2, 43 x 13 x 27 x 824 -> 1184, 1 x 1, 32 38.4 / 24.5, 120 x 14 x 25 x 80 ->
-// 608, 1 x 1, 16 32.3 / 24.3, 16 x 33 x 33 x 192 -> 1536, 1 x 7, 128 55.0 / 45.8; 64 columns: 24 x 13 x 25 x 176 -> 832, 1 x 7, 32 21.5 / 12.6 (19.5 over 32
-// columns), 8 x 54 x 54 x 240 -> 640, 3 x 3, 64 31.6 (41.2); all of 40 sampled layers that the estimate takes them for 1.03 to 1.7 times as fast.  Layers of few pixels, which would leave compute units idle, stay in chunks.
+// every workgroup of a column tile, and what bounds those is the L2s' writes: 64 lanes of one of six workgroups reach thirteen pieces of 64
+// bytes (17 x 18 x 14 x 208 -> 1472, 1 x 1: 4.9 of a workgroup's 8.4 us).  With up to four times the row units a wave, over 32 columns, or
+// twice over 64, one workgroup has all filters of its pixels and stores whole lines.  A unit's results go to LDS behind the patch as the
+// unit is finished: held in registers as in the other kernels they would not fit beside the ring.  us, in chunks / wide: that layer 12.6 /
+// 9.3, 88 x 8 x 23 x 216 -> 1344, 3 x 3, block height 64 43.1 / 25.2, 43 x 13 x 27 x 824 -> 1184, 1 x 1, 32 38.4 / 24.5, 120 x 14 x 25 x 80
+// -> 608, 1 x 1, 16 32.3 / 24.3, 16 x 33 x 33 x 192 -> 1536, 1 x 7, 128 55.0 / 45.8; 64 columns: 24 x 13 x 25 x 176 -> 832, 1 x 7, 32 21.5
+// / 12.6 (19.5 over 32 columns), 8 x 54 x 54 x 240 -> 640, 3 x 3, 64 31.6 (41.2); sampled layers: see the estimate.  Layers of few pixels,
+// which would leave compute units idle, stay in chunks, and so do filters of 2048 rows: a row of a result takes 80 bytes of LDS, which
+// leaves no room for a patch.
 static const ConvPatchKernel g_patch[] = {
     SHFLBW_PATCH(16, 2, 8, 8, 5, 2, 0), SHFLBW_PATCH(32, 2, 8, 8, 5, 2, 0), SHFLBW_PATCH(64, 2, 8, 4, 5, 2, 0),
     SHFLBW_PATCH(16, 1, 8, 8, 5, 2, 0), SHFLBW_PATCH(32, 1, 8, 8, 5, 2, 0), SHFLBW_PATCH(64, 1, 8, 4, 5, 2, 0),

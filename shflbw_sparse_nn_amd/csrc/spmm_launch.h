@@ -20,7 +20,7 @@ struct SpmmLaunchArgs {
     int half_panels;          // panels of the first of two parts of about the same work, 0: no such cut (spmm_half_panels)
     unsigned magic_halves[2]; // udiv_magic of the panels of either part (launcher, where they are taken apart)
     int n_tiles; // column tiles, filled by the launcher
-    unsigned magic_tiles; // split kernel: udiv_magic of n_tiles; slab kernel: of the number that job numbers are cut by, n_tiles or slab_chunks (launcher)
+    unsigned magic_tiles; // split kernel: udiv_magic of n_tiles; slab kernel: of what job numbers are cut by, n_tiles or slab_chunks (launcher)
     int split_shift;      // split kernel only: log2 of the 32-row blocks of a panel (launcher)
     const half8_t* packedA; // private image: A fragments in register order
     const int* kidx;        // private image: kept column ids, 64-slot padded per panel
@@ -158,10 +158,12 @@ inline bool panel_halves(const SpmmLaunchArgs& a, int S)
     return long_a && 4 * a.X <= 5 * S;
 }
 
-// Whether C is streamed past the caches: where D is, and B, C and D are twice the Infinity Cache, nothing of C lasts until a next
-// pass.  us, cached / streamed: block height 64, 8192 x 4096 x 16384, density 0.1 (670 MB) 256 / 233, 16384 x 4096 x 8192, 0.05 (604 MB) 177 / 170, 14144 x 1186 x
-// 13824, 0.16 (815 MB) 239 / 230; 128: 32768 x 2048 x 4096, 0.1 (553 MB) 146 / 143; but 64, 9152 x 1339 x 12288, 0.17 (482 MB) 142 / 146, 11584 x 1908 x 9216,
-// 0.13 (462 MB) 134 / 146, and D in parts of lines, 128, 17280 x 6409 x 13928, 0.025 342 / 369.
+// Whether C is streamed past the caches: where D is, and B, C and D are twice the Infinity Cache, nothing of C lasts until a next pass. us,
+// cached / streamed: block height 64, 8192 x 4096 x 16384, density 0.1 (670 MB) 256 / 233, 16384 x 4096 x 8192, 0.05 (604 MB) 177 / 170,
+// 14144 x 1186 x 13824, 0.16 (815 MB) 239 / 230; 128: 32768 x 2048 x 4096, 0.1 (553 MB) 146 / 143; but 64, 9152 x 1339 x 12288, 0.17 (482
+// MB) 142 / 146, 11584 x 1908 x 9216, 0.13 (462 MB) 134 / 146, and D in parts of lines, 128, 17280 x 6409 x 13928, 0.025 342 / 369.  45
+// drawn problems above the line, over three sets of operands in turn 0.90 to 1.00 times as long streamed, over one set 0.90 to 1.03 (9920 x
+// 120 x 14272 119 / 123); below it, from 400 MB, 0.95 to 1.01 and 0.94 to 1.34.
 inline bool streams_c(const SpmmLaunchArgs& a)
 {
     return a.store_mode == STORE_STREAM && bytes_of_b_and_c(a) + (size_t)a.M * a.ldd * 2 >= 512u << 20;

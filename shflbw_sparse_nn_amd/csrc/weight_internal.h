@@ -162,12 +162,13 @@ inline void interleave8(const uint16_t* const (&v)[8], int rows, uint16_t* out)
 
 // Panels of the first of two parts of about the same work that the panels are cut into, in order: equal numbers of panels where that puts
 // at most 1.03 times half of the work into the larger part, else the cut that comes closest to half; 0 where that has more than 1.05 times
-// half.  The SpMM of block height 128 may give each part to one half of the GPU (panel_halves), and then takes as long as the larger
-// one.  A panel's work is its kept vectors and, for storing its rows, 280 more (the tile and stage
-// weights of that kernel's estimate: 3.63 us a tile, 0.415 us 32 vectors).  us, no parts / equal numbers of panels / cut by work:
-// 4096 x 2775 x 14592, density 0.32, the first half of the panels keeping twice as many 136 / 127 / 116, a density falling from 1.5 to 0.5 of the
-// mean 139 / 131 / 111, 8192 x 4096 x 16384, 0.1, with C, these two 226 / 221 / 203 and 225 / 224 / 202, the last panel keeping six times
-// as many 338 / 438 / 218, the first half 1.05 times the mean (larger part 1.03) 219 / 204 / 208.  With larger parts of 1.2, 1.11 and 1.08 times half of the work 5, 9 and 13 panels lost 1.29, 1.06 and 1.09.
+// half.  The SpMM of block height 128 may give each part to one half of the GPU (panel_halves), and then takes as long as the larger one.
+// A panel's work is its kept vectors and, for storing its rows, 280 more (the tile and stage weights of that kernel's estimate: 3.63 us a
+// tile, 0.415 us 32 vectors).  us, no parts / equal numbers of panels / cut by work: 4096 x 2775 x 14592, density 0.32, the first half of
+// the panels keeping twice as many 136 / 127 / 116, a density falling from 1.5 to 0.5 of the mean 139 / 131 / 111, 8192 x 4096 x 16384,
+// 0.1, with C, these two 226 / 221 / 203 and 225 / 224 / 202, the last panel keeping six times as many 338 / 438 / 218, the first half 1.05
+// times the mean (larger part 1.03) 219 / 204 / 208.  With larger parts of 1.2, 1.11 and 1.08 times half of the work 5, 9 and 13 panels
+// lost 1.29, 1.06 and 1.09.
 int spmm_half_panels(const int* indptr, int X);
 
 // builds group_ptr / packed_indices / packed_values from the host arrays
