@@ -161,7 +161,7 @@ inline bool panel_halves(const SpmmLaunchArgs& a, int S)
 // Whether C is streamed past the caches: where D is, and B, C and D are twice the Infinity Cache, nothing of C lasts until a next pass. us,
 // cached / streamed: block height 64, 8192 x 4096 x 16384, density 0.1 (670 MB) 256 / 233, 16384 x 4096 x 8192, 0.05 (604 MB) 177 / 170,
 // 14144 x 1186 x 13824, 0.16 (815 MB) 239 / 230; 128: 32768 x 2048 x 4096, 0.1 (553 MB) 146 / 143; but 64, 9152 x 1339 x 12288, 0.17 (482
-// MB) 142 / 146, 11584 x 1908 x 9216, 0.13 (462 MB) 134 / 146, and D in parts of lines, 128, 17280 x 6409 x 13928, 0.025 342 / 369.  45
+// MB) 142 / 146, 11584 x 1908 x 9216, 0.13 (462 MB) 134 / 146, and D in parts of lines, 128, 17280 x 6409 x 13928, 0.025 342 / 369.  50
 // drawn problems above the line, over three sets of operands in turn 0.90 to 1.00 times as long streamed, over one set 0.90 to 1.03 (9920 x
 // 120 x 14272 119 / 123); below it, from 400 MB, 0.95 to 1.01 and 0.94 to 1.34.
 inline bool streams_c(const SpmmLaunchArgs& a)
