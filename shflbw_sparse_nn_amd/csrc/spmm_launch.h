@@ -17,7 +17,6 @@ struct SpmmLaunchArgs {
     int M, N, K;
     int X;       // row panels = M / V
     unsigned magic_x; // udiv_magic of X
-    int half_panels;          // panels of the first of two parts of about the same work, 0: no such cut (spmm_half_panels)
     unsigned magic_halves[2]; // udiv_magic of the panels of either part (launcher, where they are taken apart)
     int n_tiles; // column tiles, filled by the launcher
     unsigned magic_tiles; // split kernel: udiv_magic of n_tiles; slab kernel: of what job numbers are cut by, n_tiles or slab_chunks (launcher)
@@ -47,6 +46,9 @@ struct SpmmLaunchArgs {
                    // (pays when the rows of B under one column tile do not fit the XCD's L2; in halves too, where a workgroup's next
                    // tile is another column tile of the same panels, whose A it then finds: us, one way / alternating: 8192 x
                    // 8192 x 16384, 0.07 226 / 222, with C 271 / 259, 5120 x 8192 x 16384, 0.11 198 / 189, with C 217 / 208)
+    int half_panels; // panels of the first of two parts of about the same work, 0: no such cut (spmm_half_panels).  Stands last: eight
+                     // bytes more in front of the pointers cost the smallest products 0.18 us (1024^3, density 0.25: 4.24 / 4.42),
+                     // the loads of the arguments fall into other lines
 };
 
 // Convolution over batch-innermost tensors that gathers from the input itself (B points to it): the columns of the GEMM
