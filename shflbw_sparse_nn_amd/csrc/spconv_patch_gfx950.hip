@@ -10,11 +10,11 @@
 //      (transposing LDS reads; tap, stride and position are one added offset), MFMA, fp32 accumulators;
 //   3. the fp16 results go through LDS (pixel rows, filters in output order) to whole runs of the NHWC output.
 // What bounds it: the chain of these phases, with one workgroup per compute unit on layers of many channels.  16 x 14 x 14 x 512 ->
-// 2048, 3 x 3, block height 64, density 0.1 (18.2 us; us after a wave's start): arguments 0.65, patch asked for until 1.9 (160 KB at the
-// 64 bytes a clock of a compute unit) and in LDS at 3.7, products 4.1 at the matrix cores' rate (the A stream is level with them), the
+// 2048, 3 x 3, block height 64, density 0.1 (17.6 us; us after a wave's start): arguments 0.7, patch asked for until 1.9 (160 KB at the
+// 64 bytes a clock of a compute unit) and in LDS at 3.5, products 4.4 near the matrix cores' rate (the A stream is level with them), the
 // slowest wave 0.8 later, results to LDS 0.8, 2-byte stores of the permuted filters 3.5, bound by the pieces of 64 bytes that the L2s
-// write (consecutive 2-byte stores: 2.0).  32 x 28 x 28 x 256 -> 512, stride 2, block height 32, density 0.3 (14.3 us): 0.7, 3.9, 4.4 (matrix
-// cores 52 %, A stream 50 %, the rest LDS reads), 0.4, 0.4, 1.9.  On small layers launch, patch, first fragments and stores, a round trip
+// write (consecutive 2-byte stores: 2.0).  32 x 28 x 28 x 256 -> 512, stride 2, block height 32, density 0.3 (14.0 us): 0.7, 3.7, 4.8 (matrix
+// cores 56 %, A stream 54 %, the rest LDS reads), 0.5, 0.4, 1.9.  On small layers launch, patch, first fragments and stores, a round trip
 // each.
 #include "spconv_patch.h"
 
@@ -715,7 +715,7 @@ ConvPatchShape conv_patch_shape(int rows, const ConvPatchPlan& p)
 // measured on average).  Where the plane forms are estimated faster - many filters over few resident pixels (wide
 // filters over many channels), filters of several workgroups interleaved in the output - the cut is not `preferred`:
 // 7 x 54 x 54 x 584 -> 1024, 5 x 5, stride 2 takes 152 us here, 54 us there; 16 x 14 x 14 x 512 -> 2048, which it takes, 20 and 23 us.
-// On 64 sampled layers it is preferred for 58, where the plane forms take 1.11 to 3.8 times as long.
+// On 64 sampled layers it is preferred for 60, where the plane forms take 1.2 to 4.0 times as long.
 bool conv_patch_plan(const ConvPatchProblem& q, ConvPatchPlan* plan, const std::vector<ConvPatchShape>* held, bool wide_cuts)
 {
     ConvPatchPlan best{};
