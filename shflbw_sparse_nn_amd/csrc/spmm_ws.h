@@ -109,7 +109,8 @@ __device__ __forceinline__ bool output_column(const SpmmLaunchArgs& a, int& col)
 // Walks the tile ids id, id+S, ... < end of one workgroup and keeps the descriptor of the
 // current and of the following tile in scalar registers, so a tile switch never waits for memory.  The division by X is a
 // multiplication: as integer divisions, some thirty instructions each at five clocks, three of them stood in front of a workgroup's first
-// copies and at every tile switch (128 x 14 x 14 x 256 -> 256, form 4: 9.00 us, 8.87 without; 1024^3, density 0.25: 4.33, 4.29).
+// copies and at every tile switch (128 x 14 x 14 x 256 -> 256, form 4: 9.00 us, 8.87 without; 1024^3, density 0.25: no difference beyond
+// the noise of 1 %).
 struct TileWalker {
     int id, end, S, X;
     unsigned magic_x;
